@@ -144,6 +144,7 @@ struct anuga_domain {
     bool mixed = false;
     // quantities
     double *eta = nullptr;
+    double *field = nullptr;   // [N] behind eta: staging of one quantity in the caller's order
     DeQ *A = nullptr;   // step state / rk2 backup: {w, uh, vh, z}
     DeQ *B = nullptr;   // rk2 substep state
     DeQ *C = nullptr;   // rk3 middle-substep state of the fused kernels (allocated on demand)
@@ -957,7 +958,8 @@ static int domain_alloc(const anuga_params *params, int64_t S64, const int64_t *
     DCHK(dalloc(&d->nb, N));
     DCHK(dalloc(&d->cen, N));
     DCHK(dalloc(&d->area, N));
-    DCHK(dalloc(&d->eta, N));
+    DCHK(dalloc(&d->eta, 2 * (size_t)N));
+    d->field = d->eta + N;
     DCHK(dalloc(&d->A, N));
     DCHK(dalloc(&d->B, N));
     for (int q = 0; q < 3; q++) DCHK(dalloc(&d->ex[q], N));
@@ -1494,38 +1496,50 @@ static int scenario_ok(anuga_domain *d, int64_t s)
     return ANUGA_OK;
 }
 
+// One quantity of scenario s crosses as 8 B per triangle through the device
+// staging buffer `field` in the caller's order; a kernel reorders it.
 static int set_centroids(anuga_domain *d, int s, int quantity, const double *values)
 {
     if (!values) return fail(d, ANUGA_E_ARG, "values is NULL");
     const int N = d->ntri[s], kb = d->kbeg[s];
-    const int *perm = d->perm.data() + kb;
-    if (quantity == ANUGA_FRICTION) {
-        std::vector<double> t(N);
-        for (int p = 0; p < N; p++) t[p] = values[perm[p]];
-        HIPCHK(d, hipStreamSynchronize(d->stream));
-        HIPCHK(d, hipMemcpy(d->eta + kb, t.data(), N * sizeof(double), hipMemcpyHostToDevice));
-        return ANUGA_OK;
-    }
     const int slot = record_slot(quantity);
-    if (slot < 0) return fail(d, ANUGA_E_ARG, "quantity cannot be set");
-    // the bed is part of both state buffers; the others of the current one
-    DeQ *bufs[2] = {d->substate ? d->B : d->A, slot == 3 ? (d->substate ? d->A : d->B) : nullptr};
-    for (DeQ *buf : bufs) {
-        if (!buf) continue;
-        std::vector<DeQ> h;
-        int rc = download_records(d, buf, kb, N, h);
-        if (rc) return rc;
-        for (int p = 0; p < N; p++) (&h[p].w)[slot] = values[perm[p]];
-        HIPCHK(d, hipMemcpy(buf + kb, h.data(), N * sizeof(DeQ), hipMemcpyHostToDevice));
+    if (slot < 0 && quantity != ANUGA_FRICTION)
+        return fail(d, ANUGA_E_ARG, "quantity cannot be set");
+    double *v = d->eta + kb, *v2 = nullptr;
+    int stride = 1;
+    if (slot >= 0) {
+        // the bed is part of both state buffers; the others of the current one
+        stride = sizeof(DeQ) / sizeof(double);
+        v = reinterpret_cast<double *>((d->substate ? d->B : d->A) + kb) + slot;
+        if (slot == 3) v2 = reinterpret_cast<double *>((d->substate ? d->A : d->B) + kb) + slot;
     }
-    if (slot == 3 && d->mixed) {
+    HIPCHK(d, hipMemcpyAsync(d->field, values, N * sizeof(double), hipMemcpyHostToDevice,
+                             d->stream));
+    hipLaunchKernelGGL(de_set_field, dim3((N + DE_BLOCK - 1) / DE_BLOCK), dim3(DE_BLOCK), 0,
+                       d->stream, N, d->caller + kb, d->field, stride, v, v2);
+    if (slot == 3 && d->mixed)
         // bed offsets of the mixed flux's local datum
         hipLaunchKernelGGL(de_bed_offsets, dim3((N + DE_BLOCK - 1) / DE_BLOCK), dim3(DE_BLOCK), 0,
                            d->stream, kb, kb + N, d->nb, d->A, (DeGeoF32 *)d->gf);
-        int rc = launch_check(d);
-        if (rc) return rc;
-        HIPCHK(d, hipStreamSynchronize(d->stream));
-    }
+    int rc = launch_check(d);
+    if (rc) return rc;
+    HIPCHK(d, hipStreamSynchronize(d->stream));
+    return ANUGA_OK;
+}
+
+// v[k * stride] of the n triangles from kb (v at triangle kb; height: the depth
+// of the records at v) to the host in the caller's order
+static int download_field(anuga_domain *d, int kb, int n, const double *v, int stride,
+                          double *values, bool height = false)
+{
+    auto kern = height ? de_get_field<true> : de_get_field<false>;
+    hipLaunchKernelGGL(kern, dim3((n + DE_BLOCK - 1) / DE_BLOCK), dim3(DE_BLOCK), 0, d->stream, n,
+                       d->caller + kb, v, stride, d->field);
+    int rc = launch_check(d);
+    if (rc) return rc;
+    HIPCHK(d, hipMemcpyAsync(values, d->field, n * sizeof(double), hipMemcpyDeviceToHost,
+                             d->stream));
+    HIPCHK(d, hipStreamSynchronize(d->stream));
     return ANUGA_OK;
 }
 
@@ -1533,22 +1547,15 @@ static int get_centroids(anuga_domain *d, int s, int quantity, double *values)
 {
     if (!values) return fail(d, ANUGA_E_ARG, "values is NULL");
     const int N = d->ntri[s], kb = d->kbeg[s];
-    const int *perm = d->perm.data() + kb;
-    if (quantity == ANUGA_FRICTION) {
-        std::vector<double> t(N);
-        HIPCHK(d, hipStreamSynchronize(d->stream));
-        HIPCHK(d, hipMemcpy(t.data(), d->eta + kb, N * sizeof(double), hipMemcpyDeviceToHost));
-        for (int p = 0; p < N; p++) values[perm[p]] = t[p];
-        return ANUGA_OK;
-    }
     const int slot = record_slot(quantity);
-    if (slot < 0 && quantity != ANUGA_HEIGHT) return fail(d, ANUGA_E_ARG, "unknown quantity");
-    std::vector<DeQ> h;
-    int rc = download_records(d, d->substate ? d->B : d->A, kb, N, h);
-    if (rc) return rc;
-    for (int p = 0; p < N; p++)
-        values[perm[p]] = slot >= 0 ? (&h[p].w)[slot] : std::fmax(h[p].w - h[p].z, 0.0);
-    return ANUGA_OK;
+    if (slot < 0 && quantity != ANUGA_HEIGHT && quantity != ANUGA_FRICTION)
+        return fail(d, ANUGA_E_ARG, "unknown quantity");
+    const double *v = quantity == ANUGA_FRICTION
+                          ? d->eta + kb
+                          : reinterpret_cast<const double *>((d->substate ? d->B : d->A) + kb) +
+                                std::max(slot, 0);
+    const int stride = quantity == ANUGA_FRICTION ? 1 : sizeof(DeQ) / sizeof(double);
+    return download_field(d, kb, N, v, stride, values, quantity == ANUGA_HEIGHT);
 }
 
 static int set_boundary(anuga_domain *d, int s, const int32_t *kind, const double *dirichlet_values)
@@ -3346,23 +3353,15 @@ int anuga_adjoint_gradient(anuga_domain *d, const double *dloss_dstage, double *
             if (rc) return rc;
         }
     }
+    int rc = ANUGA_OK;
+    if (grad_friction && (rc = download_field(d, 0, N, a->nbar, 1, grad_friction))) return rc;
+    if (grad_elevation && (rc = download_field(d, 0, N, a->zbar, 1, grad_elevation))) return rc;
+    if (grad_state0)
+        for (int q = 0; q < 3; q++)
+            if ((rc = download_field(d, 0, N, a->lam + (size_t)q * N, 1,
+                                     grad_state0 + (size_t)q * N)))
+                return rc;
     HIPCHK(d, hipStreamSynchronize(d->stream));
-    std::vector<double> h(n3);
-    auto unpermute = [&](const double *src, double *dst) {
-        for (int p = 0; p < N; p++) dst[d->perm[p]] = src[p];
-    };
-    if (grad_friction) {
-        HIPCHK(d, hipMemcpy(h.data(), a->nbar, N * sizeof(double), hipMemcpyDeviceToHost));
-        unpermute(h.data(), grad_friction);
-    }
-    if (grad_elevation) {
-        HIPCHK(d, hipMemcpy(h.data(), a->zbar, N * sizeof(double), hipMemcpyDeviceToHost));
-        unpermute(h.data(), grad_elevation);
-    }
-    if (grad_state0) {
-        HIPCHK(d, hipMemcpy(h.data(), a->lam, n3 * sizeof(double), hipMemcpyDeviceToHost));
-        for (int q = 0; q < 3; q++) unpermute(h.data() + (size_t)q * N, grad_state0 + (size_t)q * N);
-    }
     return ANUGA_OK;
 }
 

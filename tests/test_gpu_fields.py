@@ -1,0 +1,54 @@
+"""Centroid quantities between the caller's and the library's order on the
+device (de_set_field, de_get_field), against the values as they were given:
+copies, so bit for bit, at sizes around one workgroup and for every quantity,
+in a single scenario and in an ensemble whose scenarios start on workgroup
+boundaries."""
+
+import numpy as np
+import pytest
+
+from anuga_core_amd.domain import Domain
+from anuga_core_amd.ensemble import Ensemble
+from anuga_core_amd.mesh import Mesh, rectangular
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ("stage", "xmomentum", "ymomentum", "elevation", "friction")
+
+
+def _values(N, seed):
+    rng = np.random.default_rng(seed)
+    q = {n: rng.standard_normal(N) for n in NAMES}
+    q["stage"][::7] = -np.inf
+    q["xmomentum"][::5] = np.nan
+    q["ymomentum"][::3] = -0.0
+    return q
+
+
+def _same(a, b):
+    return np.array_equal(a.view(np.int64), b.view(np.int64))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("cells", [1, 127, 128, 129, 300])
+def test_domain_fields_round_trip(cells, precision):
+    mesh = Mesh(*rectangular(cells, 1, float(cells), 1.0))
+    d = Domain(mesh=mesh, precision=precision)
+    q = _values(mesh.number_of_triangles, cells)
+    for n in NAMES:
+        d.set_quantity(n, q[n], location="centroids")
+    for n in NAMES:
+        assert _same(d.get_quantity(n).centroid_values, q[n]), n
+    depth = np.fmax(q["stage"] - q["elevation"], 0.0)
+    assert np.array_equal(d.get_quantity("height").centroid_values, depth)
+
+
+def test_ensemble_fields_round_trip():
+    meshes = [Mesh(*rectangular(c, 1, float(c), 1.0)) for c in (128, 1, 200, 127)]
+    e = Ensemble(meshes)
+    qs = [_values(m.number_of_triangles, 10 + s) for s, m in enumerate(meshes)]
+    for s, m in enumerate(meshes):
+        e.set_scenario(s, m, qs[s], {t: "reflective" for t in m.get_boundary_tags()})
+    for s in range(len(meshes)):
+        for n in NAMES:
+            assert _same(e.get_quantity(s, n), qs[s][n]), (s, n)
