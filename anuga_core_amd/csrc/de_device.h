@@ -200,6 +200,12 @@ struct DeControl {
     int grows, gcap;
 };
 
+// rows of the per-block partials, part[row][blocks]: CFL timestep, boundary
+// inflow of the first, second and third substep, protect's mass or the volume
+enum { DE_P_DT = 0, DE_P_BF0, DE_P_MASS, DE_P_BF1, DE_P_BF2, DE_P_ROWS };
+// contiguous chunks of a scenario's blocks in the reductions
+#define DE_RCHUNKS 32
+
 // control block of the scenario that owns logical block lb
 __device__ __forceinline__ DeControl *de_ctl(DeControl *ctl, const int *scen, int lb)
 {

@@ -42,7 +42,7 @@ thread_local std::string g_create_error;
 // ---------------------------------------------------------------------------
 static const int64_t kNoAllocMaxN = int64_t(1) << 27;
 static const int kNoAllocCtl = 32;                        // doubles for the DeControl
-static const int kNoAllocChunks = 3 * DE_RCHUNKS;         // the first stage's results
+static const int kNoAllocChunks = 3 * DE_RCHUNKS;         // the first stage's results (one row)
 static const int64_t kNoAllocDoubles =
     kNoAllocCtl + kNoAllocChunks + (kNoAllocMaxN + DE_BLOCK - 1) / DE_BLOCK;
 static_assert(sizeof(DeControl) <= kNoAllocCtl * sizeof(double), "control block size");
@@ -81,6 +81,7 @@ struct RateOp {
 
 struct anuga_domain {
     int N = 0, M = 0, nblocks = 0;   // N: internal triangles incl. padding; M: boundary edges
+    int max_blocks = 0;              // the largest scenario's blocks
     int S = 1;                       // scenarios
     anuga_params P{};
     hipStream_t stream = nullptr;
@@ -155,8 +156,8 @@ struct anuga_domain {
     double *bval = nullptr;             // [3 slots][3][M]
     long long bsstride = 0;             // 0, or 3M once per-substep boundary values are set
     std::vector<signed char> hbkind;    // host copy of bkind
-    double *part = nullptr;   // [3][nblocks]: dt, bflux, mass
-    double *chunks = nullptr; // [3][S][DE_RCHUNKS]: the reduction's first stage
+    double *part = nullptr;   // [DE_P_ROWS][nblocks]
+    double *chunks = nullptr; // [DE_P_ROWS][S][DE_RCHUNKS]: the reduction's first stage
     DeControl *ctl = nullptr; // [S] device step control
     unsigned long long *dneg = nullptr;
     DeControl *hctl = nullptr;          // [S] pinned host mirror of ctl
@@ -578,6 +579,18 @@ static DeMesh dev_mesh(const anuga_domain *d)
     return m;
 }
 
+// a row of the per-block partials (DE_P_*)
+static double *part_row(const anuga_domain *d, int row)
+{
+    return d->part + (size_t)row * d->nblocks;
+}
+
+template <int SUB>
+static double *bflux_row(const anuga_domain *d)
+{
+    return part_row(d, SUB == 0 ? DE_P_BF0 : (SUB == 3 ? DE_P_BF2 : DE_P_BF1));
+}
+
 static dim3 scenario_grid(const anuga_domain *d)
 {
     return dim3((d->S + 63) / 64);
@@ -590,11 +603,11 @@ static void launch_extrapolate(anuga_domain *d, DeQ *S)
     if (d->mixed)
         hipLaunchKernelGGL(de_extrapolate<float>, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->E, d->flags,
-                           d->part + 2 * (size_t)d->nblocks, d->ctl);
+                           part_row(d, DE_P_MASS), d->ctl);
     else
         hipLaunchKernelGGL(de_extrapolate<double>, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->E, d->flags,
-                           d->part + 2 * (size_t)d->nblocks, d->ctl);
+                           part_row(d, DE_P_MASS), d->ctl);
     timer_end(d, T_EXTRAP);
 }
 
@@ -613,19 +626,18 @@ static void launch_flux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
             hipLaunchKernelGGL((de_flux<double, SUB, true>), dim3(d->nblocks), dim3(DE_BLOCK), 0,
                                d->stream, dev_mesh(d), dev_params(d->P), S, d->eta,
                                (const double *)d->E, bc, d->flags, d->ex[0], d->ex[1],
-                               d->ex[2], bk, out, d->ctl, d->part, d->part + d->nblocks,
+                               d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
                                d->dneg);
         else
             hipLaunchKernelGGL((de_flux<double, SUB>), dim3(d->nblocks), dim3(DE_BLOCK), 0,
                                d->stream, dev_mesh(d), dev_params(d->P), S, d->eta,
                                (const double *)d->E, bc, d->flags, d->ex[0], d->ex[1],
-                               d->ex[2], bk, out, d->ctl, d->part, d->part + d->nblocks,
+                               d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
                                d->dneg);
     } else
         hipLaunchKernelGGL((de_flux_mixed<SUB>), dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->eta, (const DeEdgeRec32 *)d->E,
-                           bc, d->flags, d->ex[0], d->ex[1], d->ex[2], bk, out, d->ctl, d->part,
-                           d->part + d->nblocks, d->dneg);
+                           bc, d->flags, d->ex[0], d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d), d->dneg);
 }
 
 template <class T>
@@ -656,16 +668,15 @@ static void launch_xflux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
         const size_t lds = ((size_t)DE_BLOCK + (size_t)d->hcap) * (sizeof(double) + 12 * sizeof(float));
         hipLaunchKernelGGL(de_xflux_mixed<SUB>, dim3(d->nblocks), dim3(DE_BLOCK), lds, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->eta, tl, bc, d->flags, d->ex[0],
-                           d->ex[1], d->ex[2], bk, out, d->ctl, d->part, d->part + d->nblocks,
-                           d->part + 2 * (size_t)d->nblocks, d->dneg);
+                           d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
+                           part_row(d, DE_P_MASS), d->dneg);
     } else if (d->rw || d->P.low_froude || d->P.use_sloped_mannings) {
         // the general instantiation: walls, low_froude, sloped friction
         const size_t lds = (12 * (size_t)DE_BLOCK + 12 * (size_t)d->hcap) * sizeof(double) +
                            (((size_t)DE_BLOCK + d->hcap + 7) & ~(size_t)7);
         hipLaunchKernelGGL((de_xflux<SUB, true>), dim3(d->nblocks), dim3(DE_BLOCK), lds,
                            d->stream, dev_mesh(d), dev_params(d->P), S, d->eta, tl, bc, d->flags,
-                           d->ex[0], d->ex[1], d->ex[2], bk, out, d->ctl, d->part,
-                           d->part + d->nblocks, d->part + 2 * (size_t)d->nblocks, d->dneg,
+                           d->ex[0], d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d), part_row(d, DE_P_MASS), d->dneg,
                            (double *)d->E);
     } else if (d->mirror && d->tedge && d->edge_once) {
         // each edge's flux once: tile and halo edge values, then the tile's
@@ -674,14 +685,14 @@ static void launch_xflux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
         auto kern = (d->vgeom && d->vx) ? de_xflux_e<SUB, true> : de_xflux_e<SUB, false>;
         hipLaunchKernelGGL(kern, dim3(d->nblocks), dim3(DE_BLOCK), lds, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->eta, tl, bc, d->flags, d->ex[0],
-                           d->ex[1], d->ex[2], bk, out, d->ctl, d->part, d->part + d->nblocks,
-                           d->part + 2 * (size_t)d->nblocks, d->dneg);
+                           d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
+                           part_row(d, DE_P_MASS), d->dneg);
     } else {
         const size_t lds = (12 * (size_t)DE_BLOCK + 12 * (size_t)d->hcap) * sizeof(double);
         hipLaunchKernelGGL(de_xflux<SUB>, dim3(d->nblocks), dim3(DE_BLOCK), lds, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->eta, tl, bc, d->flags, d->ex[0],
-                           d->ex[1], d->ex[2], bk, out, d->ctl, d->part, d->part + d->nblocks,
-                           d->part + 2 * (size_t)d->nblocks, d->dneg, (double *)d->E);
+                           d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
+                           part_row(d, DE_P_MASS), d->dneg, (double *)d->E);
     }
 }
 
@@ -714,36 +725,80 @@ static void launch_flux(anuga_domain *d, int substep, DeQ *S, DeQ *bk = nullptr,
     timer_end(d, substep ? T_FLUX1 : T_FLUX0);
 }
 
-static void launch_update(anuga_domain *d, DeQ *S, DeQ *out)
+// Whether a scenario's partials are few enough for one workgroup to reduce
+// (de_reduce, de_finish_step, de_update without the chunk stage).
+static bool reduce_direct(const anuga_domain *d)
+{
+    return d->max_blocks <= DE_DIRECT_BLOCKS;
+}
+
+template <bool SLOPED>
+static void launch_update_t(anuga_domain *d, DeQ *S, DeQ *out, int dt)
+{
+    const double *pdt = dt == DE_DT_CHUNKS ? d->chunks : part_row(d, DE_P_DT);
+    auto kern = dt == DE_DT_GIVEN    ? de_update<SLOPED, DE_DT_GIVEN>
+                : dt == DE_DT_DIRECT ? de_update<SLOPED, DE_DT_DIRECT>
+                                     : de_update<SLOPED, DE_DT_CHUNKS>;
+    hipLaunchKernelGGL(kern, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream, d->scen,
+                       dev_params(d->P), S, d->eta, d->flags, d->ex[0], d->ex[1], d->ex[2],
+                       d->ctl, out, d->dneg, pdt, (const double *)d->E, d->N, d->vx);
+}
+
+// dt: DE_DT_*, where the timestep comes from
+static void launch_update(anuga_domain *d, DeQ *S, DeQ *out, int dt = DE_DT_GIVEN)
 {
     if (out == d->B) d->backup_valid = false;
     timer_begin(d, T_UPDATE);
-    if (d->P.use_sloped_mannings && !d->mixed)
-        hipLaunchKernelGGL((de_update<true>), dim3(d->nblocks), dim3(DE_BLOCK), 0,
-                           d->stream, d->scen, dev_params(d->P), S, d->eta, d->flags, d->ex[0],
-                           d->ex[1], d->ex[2], d->ctl, out, d->dneg, (const double *)d->E, d->N,
-                           d->vx);
-    else
-        hipLaunchKernelGGL(de_update<false>, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream,
-                           d->scen, dev_params(d->P), S, d->eta, d->flags, d->ex[0], d->ex[1],
-                           d->ex[2], d->ctl, out, d->dneg);
+    if (d->P.use_sloped_mannings && !d->mixed) launch_update_t<true>(d, S, out, dt);
+    else launch_update_t<false>(d, S, out, dt);
     timer_end(d, T_UPDATE);
 }
 
-static void launch_reduce(anuga_domain *d, int mode)
+// Reduce a row of the partials to the control blocks: MODE DE_R_* (DE_R_FLUX0:
+// the CFL timestep and protect's mass too).
+template <int MODE>
+static void launch_reduce(anuga_domain *d, int row)
 {
-    const double *pdt = d->part, *pbf = d->part + d->nblocks;
-    const double *pm = d->part + 2 * (size_t)d->nblocks;
-    typedef void (*Chunks)(const double *, const double *, const double *, const DeControl *,
-                           double *);
-    typedef void (*Final)(const double *, DeControl *);
-    const Chunks kc[5] = {de_reduce_chunks<0>, de_reduce_chunks<1>, de_reduce_chunks<2>,
-                          de_reduce_chunks<3>, de_reduce_chunks<4>};
-    const Final kf[5] = {de_reduce_final<0>, de_reduce_final<1>, de_reduce_final<2>,
-                         de_reduce_final<3>, de_reduce_final<4>};
-    hipLaunchKernelGGL(kc[mode], dim3(DE_RCHUNKS, d->S), dim3(256), 0, d->stream, pdt, pbf, pm,
-                       d->ctl, d->chunks);
-    hipLaunchKernelGGL(kf[mode], dim3(d->S), dim3(64), 0, d->stream, d->chunks, d->ctl);
+    constexpr bool FIRST = MODE == DE_R_FLUX0;
+    const dim3 g(d->S), b(DE_RED_THREADS);
+    if (reduce_direct(d)) {
+        hipLaunchKernelGGL((de_reduce<MODE, false>), g, b, 0, d->stream, d->part, d->nblocks, row,
+                           d->ctl);
+        return;
+    }
+    const int live = MODE != DE_R_MASS && MODE != DE_R_VOLUME;
+    hipLaunchKernelGGL((de_reduce_chunks<FIRST, FIRST ? 2 : 1>), dim3(DE_RCHUNKS, d->S), dim3(256),
+                       0, d->stream, d->part, d->nblocks, row, (int)DE_P_MASS, 0, live, d->ctl,
+                       d->chunks);
+    hipLaunchKernelGGL((de_reduce<MODE, true>), g, b, 0, d->stream, d->chunks, d->nblocks, row,
+                       d->ctl);
+}
+
+template <int METHOD>
+static void launch_finish_t(anuga_domain *d)
+{
+    const dim3 g(d->S), b(DE_RED_THREADS);
+    double *hist = d->S == 1 ? d->hist : nullptr;
+    if (reduce_direct(d)) {
+        hipLaunchKernelGGL((de_finish_step<METHOD, false>), g, b, 0, d->stream, d->part,
+                           d->nblocks, d->ctl, hist);
+        return;
+    }
+    hipLaunchKernelGGL((de_reduce_chunks<false, METHOD>), dim3(DE_RCHUNKS, d->S), dim3(256), 0,
+                       d->stream, d->part, d->nblocks, (int)DE_P_BF0, (int)DE_P_BF1,
+                       (int)DE_P_BF2, 1, d->ctl, d->chunks);
+    hipLaunchKernelGGL((de_finish_step<METHOD, true>), g, b, 0, d->stream, d->chunks, d->nblocks,
+                       d->ctl, hist);
+}
+
+// the end of a device-controlled step
+static void launch_finish(anuga_domain *d)
+{
+    switch (d->P.timestep_fluxcalls) {
+    case 1: launch_finish_t<1>(d); break;
+    case 2: launch_finish_t<2>(d); break;
+    default: launch_finish_t<3>(d); break;
+    }
 }
 
 static void launch_control(anuga_domain *d, void (*k)(DeControl *, int))
@@ -754,7 +809,7 @@ static void launch_control(anuga_domain *d, void (*k)(DeControl *, int))
 static void launch_volume(anuga_domain *d, DeQ *S)
 {
     hipLaunchKernelGGL(de_volume, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream, d->scen, d->ctl,
-                       S, d->area, d->part + 2 * (size_t)d->nblocks);
+                       S, d->area, part_row(d, DE_P_MASS));
 }
 
 // leave device-controlled mode before host-controlled launches
@@ -766,10 +821,10 @@ static void ensure_live(anuga_domain *d)
     }
 }
 
-// One device-controlled step of every scenario: both substeps, the timestep
-// on the device and the end-of-step bookkeeping. Every kernel returns at once
-// for a scenario whose done flag is set.
-static void enqueue_later_substeps(anuga_domain *d)
+// The substeps after the first, with the timestep in the control blocks;
+// `reduce`: their boundary fluxes are reduced here (host-sequenced steps), not
+// at the end of the step.
+static void enqueue_later_substeps(anuga_domain *d, bool reduce)
 {
     if (d->P.timestep_fluxcalls == 2) {
         if (fused(d)) {
@@ -778,23 +833,23 @@ static void enqueue_later_substeps(anuga_domain *d)
             launch_extrapolate(d, d->B);
             launch_flux(d, 1, d->B, d->A, d->A);
         }
-        launch_reduce(d, 1);
+        if (reduce) launch_reduce<DE_R_FLUX1>(d, DE_P_BF1);
     } else if (d->P.timestep_fluxcalls == 3) {
         if (fused(d) && d->C) {
             // the middle substep writes C, not B in place: other tiles are
             // still extrapolating B
             launch_xflux(d, 2, d->B, d->A, d->C);
-            launch_reduce(d, 1);
             launch_xflux(d, 3, d->C, d->A, d->A);
-            launch_reduce(d, 4);
-            return;
+        } else {
+            launch_extrapolate(d, d->B);
+            launch_flux(d, 2, d->B, d->A, d->B);
+            launch_extrapolate(d, d->B);
+            launch_flux(d, 3, d->B, d->A, d->A);
         }
-        launch_extrapolate(d, d->B);
-        launch_flux(d, 2, d->B, d->A, d->B);
-        launch_reduce(d, 1);
-        launch_extrapolate(d, d->B);
-        launch_flux(d, 3, d->B, d->A, d->A);
-        launch_reduce(d, 4);
+        if (reduce) {
+            launch_reduce<DE_R_FLUX1>(d, DE_P_BF1);
+            launch_reduce<DE_R_FLUX2>(d, DE_P_BF2);
+        }
     }
 }
 
@@ -821,6 +876,9 @@ static void launch_operators(anuga_domain *d)
     for (const RateOp &o : d->ops) launch_operator(d, o);
 }
 
+// One device-controlled step of every scenario: the substeps, the timestep on
+// the device and the end-of-step bookkeeping. Every kernel returns at once for
+// a scenario whose done flag is set.
 static void enqueue_device_step(anuga_domain *d)
 {
     const bool rk = d->P.timestep_fluxcalls > 1;
@@ -830,13 +888,13 @@ static void enqueue_device_step(anuga_domain *d)
         launch_extrapolate(d, d->A);
         launch_flux(d, 0, d->A);
     }
-    launch_reduce(d, 0);
-    launch_control(d, de_timestep);
-    launch_update(d, d->A, rk ? d->B : d->A);
-    enqueue_later_substeps(d);
+    if (!reduce_direct(d))
+        hipLaunchKernelGGL((de_reduce_chunks<true, 0>), dim3(DE_RCHUNKS, d->S), dim3(256), 0,
+                           d->stream, d->part, d->nblocks, 0, 0, 0, 1, d->ctl, d->chunks);
+    launch_update(d, d->A, rk ? d->B : d->A, reduce_direct(d) ? DE_DT_DIRECT : DE_DT_CHUNKS);
+    enqueue_later_substeps(d, false);
     launch_operators(d);
-    hipLaunchKernelGGL(de_finish_step, scenario_grid(d), dim3(64), 0, d->stream, d->ctl, d->S,
-                       d->S == 1 ? d->hist : nullptr);
+    launch_finish(d);
     if (d->G)
         hipLaunchKernelGGL(de_sample_gauges<false>, dim3(1), dim3(256), 0, d->stream, d->ctl,
                            d->G, d->gtri, d->A, 0.0, d->gtimes, d->gvals);
@@ -928,6 +986,7 @@ static int domain_alloc(const anuga_params *params, int64_t S64, const int64_t *
     d->nbnd.resize(S);
     for (int s = 0; s < S; s++) {
         d->ntri[s] = (int)ntri[s];
+        d->max_blocks = std::max(d->max_blocks, (d->ntri[s] + DE_BLOCK - 1) / DE_BLOCK);
         d->nbnd[s] = (int)nbnd[s];
     }
     d->mesh_set.assign(S, 0);
@@ -978,8 +1037,8 @@ static int domain_alloc(const anuga_params *params, int64_t S64, const int64_t *
     DCHK(dalloc(&d->flags, N));
     DCHK(dalloc(&d->bkind, M));
     DCHK(dalloc(&d->bval, 9 * (size_t)M));   // three substep slots
-    DCHK(dalloc(&d->part, 3 * (size_t)d->nblocks));
-    DCHK(dalloc(&d->chunks, 3 * (size_t)S * DE_RCHUNKS));
+    DCHK(dalloc(&d->part, DE_P_ROWS * (size_t)d->nblocks));
+    DCHK(dalloc(&d->chunks, DE_P_ROWS * (size_t)S * DE_RCHUNKS));
     DCHK(dalloc(&d->ctl, S));
     DCHK(dalloc(&d->dsetup, S));
     DCHK(dalloc(&d->dneg, 1));
@@ -1018,7 +1077,7 @@ static int domain_alloc(const anuga_params *params, int64_t S64, const int64_t *
     DCHK(hipMemset(d->flags, DE_F_KEEP, N));
     DCHK(hipMemset(d->bkind, 0, std::max(M, 1)));
     DCHK(hipMemset(d->bval, 0, 9 * (size_t)std::max(M, 1) * sizeof(double)));
-    DCHK(hipMemset(d->part, 0, 3 * (size_t)d->nblocks * sizeof(double)));
+    DCHK(hipMemset(d->part, 0, DE_P_ROWS * (size_t)d->nblocks * sizeof(double)));
     DCHK(hipMemset(d->dneg, 0, sizeof(unsigned long long)));
     std::memset(d->hctl, 0, S * sizeof(DeControl));
     std::memset(d->hsetup, 0, S * sizeof(DeBatchSetup));
@@ -1713,7 +1772,7 @@ static int distribute(anuga_domain *d)
     DeQ *S = d->substate ? d->B : d->A;
     launch_extrapolate(d, S);
     launch_materialize(d, S);
-    launch_reduce(d, 2);
+    launch_reduce<DE_R_MASS>(d, DE_P_MASS);
     int rc = launch_check(d);
     if (rc) return rc;
     return sync_scalars(d);
@@ -1723,7 +1782,7 @@ static int volumes(anuga_domain *d)
 {
     DeQ *S = d->substate ? d->B : d->A;
     launch_volume(d, S);
-    launch_reduce(d, 3);
+    launch_reduce<DE_R_VOLUME>(d, DE_P_MASS);
     int rc = launch_check(d);
     if (rc) return rc;
     return sync_scalars(d);
@@ -1783,21 +1842,22 @@ static void adj_stages(anuga_domain *d, AdjRun *a, const DeQ *X)
     const size_t N = d->N;
     DeBoundary bc{d->bkind, d->bval, d->M, 0};
     const DeParams p = dev_params(d->P);
-    double *pm = d->part + 2 * (size_t)d->nblocks;
+    double *pm = part_row(d, DE_P_MASS);
     hipLaunchKernelGGL(de_extrapolate<double>, g, b, 0, d->stream, dev_mesh(d), p, X, a->E0, a->f0,
                        pm, d->ctl);
     hipLaunchKernelGGL((de_flux<double, 0>), g, b, 0, d->stream, dev_mesh(d), p, X, d->eta,
                        a->E0, bc, a->f0, a->ex0, a->ex0 + N, a->ex0 + 2 * N, nullptr, nullptr,
                        d->ctl,
-                       d->part, d->part + d->nblocks, a->neg);
-    hipLaunchKernelGGL(de_update<false>, g, b, 0, d->stream, d->scen, p, X, d->eta, a->f0, a->ex0,
-                       a->ex0 + N, a->ex0 + 2 * N, d->ctl, a->S1, a->neg);
+                       part_row(d, DE_P_DT), part_row(d, DE_P_BF0), a->neg);
+    hipLaunchKernelGGL((de_update<false, DE_DT_GIVEN>), g, b, 0, d->stream, d->scen, p, X, d->eta,
+                       a->f0, a->ex0, a->ex0 + N, a->ex0 + 2 * N, d->ctl, a->S1, a->neg, nullptr,
+                       nullptr, 0, nullptr);
     hipLaunchKernelGGL(de_extrapolate<double>, g, b, 0, d->stream, dev_mesh(d), p, a->S1, a->E1,
                        a->f1, pm, d->ctl);
     hipLaunchKernelGGL((de_flux<double, 0>), g, b, 0, d->stream, dev_mesh(d), p, a->S1, d->eta,
                        a->E1, bc, a->f1, a->ex1, a->ex1 + N, a->ex1 + 2 * N, nullptr, nullptr,
                        d->ctl,
-                       d->part, d->part + d->nblocks, a->neg);
+                       part_row(d, DE_P_DT), part_row(d, DE_P_BF0), a->neg);
 }
 
 // lam (adjoint of the step's result, [3][N]) -> adjoint of its start X
@@ -2600,7 +2660,7 @@ int anuga_compute_fluxes(anuga_domain *d, double *flux_timestep)
         launch_extrapolate(d, d->A);
         launch_flux(d, 0, d->A);
     }
-    launch_reduce(d, 0);
+    launch_reduce<DE_R_FLUX0>(d, DE_P_BF0);
     rc = launch_check(d);
     if (rc) return rc;
     rc = sync_scalars(d);
@@ -2646,7 +2706,7 @@ static int later_substeps(anuga_domain *d, double dt, int64_t *num_negative, int
         return fail(d, ANUGA_E_STATE, "substeps of another timestepping method");
     if (d->substate != 1) return fail(d, ANUGA_E_STATE, "second substep without a first");
     hipLaunchKernelGGL(de_set_dt, dim3(1), dim3(64), 0, d->stream, d->ctl, dt);
-    enqueue_later_substeps(d);
+    enqueue_later_substeps(d, true);
     hipLaunchKernelGGL(de_integrate, dim3(1), dim3(64), 0, d->stream, d->ctl, method);
     rc = launch_check(d);
     if (rc) return rc;
@@ -2681,9 +2741,8 @@ static int lts_fluxes(anuga_domain *d, double *flux_timestep)
     DeBoundary bc{d->bkind, d->bval, d->M, d->bsstride};
     hipLaunchKernelGGL(de_flux_lts, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream, dev_mesh(d),
                        dev_params(d->P), d->A, (const double *)d->E, bc, d->flags, d->ex[0],
-                       d->ex[1], d->ex[2], d->lts, d->lts_call, d->ctl, d->part,
-                       d->part + d->nblocks);
-    launch_reduce(d, 0);
+                       d->ex[1], d->ex[2], d->lts, d->lts_call, d->ctl, part_row(d, DE_P_DT), part_row(d, DE_P_BF0));
+    launch_reduce<DE_R_FLUX0>(d, DE_P_BF0);
     int rc = launch_check(d);
     if (rc) return rc;
     rc = sync_scalars(d);
@@ -2837,7 +2896,10 @@ int anuga_compute_fluxes_ext_central(anuga_domain *d, double timestep, double *f
     }
     const int sub = (int)(d->op_flux_calls % d->P.timestep_fluxcalls);
     launch_flux(d, 0, d->A);
-    launch_reduce(d, sub == 0 ? 0 : (sub == 1 ? 1 : 4));
+    // every call evaluates substep 0's kernel, so its row of the partials
+    if (sub == 0) launch_reduce<DE_R_FLUX0>(d, DE_P_BF0);
+    else if (sub == 1) launch_reduce<DE_R_FLUX1>(d, DE_P_BF0);
+    else launch_reduce<DE_R_FLUX2>(d, DE_P_BF0);
     rc = launch_check(d);
     if (rc) return rc;
     rc = sync_scalars(d);
@@ -3007,14 +3069,20 @@ int anuga_water_volume_noalloc(int64_t N, const double *stage, const double *ele
     DeControl *ctl = reinterpret_cast<DeControl *>(sc);
     double *chunks = sc + kNoAllocCtl, *part = chunks + kNoAllocChunks;
     const int n = (int)N, nb = (int)((N + DE_BLOCK - 1) / DE_BLOCK);
-    // the reduction of anuga_get_water_volume (de_volume, MODE 3), over the
+    // the reduction of anuga_get_water_volume (de_volume, DE_R_VOLUME), over the
     // caller's arrays
     hipLaunchKernelGGL(de_control_init, dim3(1), dim3(64), 0, st, ctl, n, nb);
     hipLaunchKernelGGL(de_volume_arrays, dim3(nb), dim3(DE_BLOCK), 0, st, n, stage, elevation,
                        area, part);
-    hipLaunchKernelGGL(de_reduce_chunks<3>, dim3(DE_RCHUNKS, 1), dim3(256), 0, st, part, part,
-                       part, ctl, chunks);
-    hipLaunchKernelGGL(de_reduce_final<3>, dim3(1), dim3(64), 0, st, chunks, ctl);
+    if (nb <= DE_DIRECT_BLOCKS) {
+        hipLaunchKernelGGL((de_reduce<DE_R_VOLUME, false>), dim3(1), dim3(DE_RED_THREADS), 0, st,
+                           part, nb, 0, ctl);
+    } else {
+        hipLaunchKernelGGL((de_reduce_chunks<false, 1>), dim3(DE_RCHUNKS, 1), dim3(256), 0, st,
+                           part, nb, 0, 0, 0, 0, ctl, chunks);
+        hipLaunchKernelGGL((de_reduce<DE_R_VOLUME, true>), dim3(1), dim3(DE_RED_THREADS), 0, st,
+                           chunks, nb, 0, ctl);
+    }
     hipLaunchKernelGGL(de_copy_volume, dim3(1), dim3(64), 0, st, ctl, volume);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)

@@ -18,7 +18,9 @@
 //   de_update       friction + update + fix_negative_cells
 //                   (sw_domain_orig.c:2805-2838, quantity.c:772-822,
 //                   sw_domain_orig.c:2890-2910).
-//   de_reduce       fixed-order reduction of the per-block partials.
+//                   In device-controlled steps it forms the timestep too.
+//   de_reduce_chunks, de_reduce, de_finish_step  fixed-order reduction of the
+//                   per-block partials; the last also ends the step.
 //   de_xflux,       extrapolation and flux fused over compact tiles (the
 //   de_xflux_mixed  bisection order): a workgroup extrapolates its
 //                   triangles and their halo into LDS and gathers the fluxes
@@ -1833,27 +1835,116 @@ de_xflux_mixed(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__
                                part_mass, lb);
 }
 
+// Generic_Domain.update_timestep (generic_domain.py:2349-2415): the timestep
+// before the clamps, min(CFL * flux_dt, max_dt), and the step's timestep,
+// clamped to the final time and the next yield time. Reads nothing that
+// de_commit_timestep writes.
+__device__ __forceinline__ double de_cfl_timestep(const DeControl *c, double flux_dt)
+{
+    const double a = c->cfl * (c->fixed_flux_dt > 0.0 ? c->fixed_flux_dt : flux_dt);
+    return (c->max_dt < a) ? c->max_dt : a;
+}
+
+__device__ __forceinline__ double de_clamped_timestep(const DeControl *c, double ts)
+{
+    if (c->t + ts > c->finaltime) ts = c->finaltime - c->t;
+    if (c->t + ts > c->yieldtime) ts = c->yieldtime - c->t;
+    return ts;
+}
+
+// the rest of update_timestep, by one thread of a scenario: the recorded
+// extremes, the small-step counter with its first-order switch and its
+// exception (reported as DE_ERR_SMALL_TIMESTEP), and the results
+__device__ __forceinline__ void de_commit_timestep(DeControl *c, double flux_dt, double ts,
+                                                   double dt)
+{
+    c->rec_max = (c->rec_max > ts) ? c->rec_max : ts;      // max(timestep, recorded_max)
+    c->rec_min = (c->rec_min < ts) ? c->rec_min : ts;      // min(timestep, recorded_min)
+    if (ts < c->min_dt) {
+        c->smallsteps += 1;
+        if (c->smallsteps > c->max_smallsteps) {
+            c->smallsteps = 0;
+            if (c->order == 1) atomicOr(&c->status, DE_ERR_SMALL_TIMESTEP);
+            else c->order = 1;
+        }
+    } else {
+        c->smallsteps = 0;
+        if (c->order == 1 && c->default_order == 2) c->order = 2;
+    }
+    c->flux_dt = flux_dt;
+    c->dt = dt;
+}
+
+// where de_update takes the timestep from: the control block (host-sequenced
+// steps), or update_timestep over the minimum of the scenario's per-block CFL
+// partials, read directly (at most DE_DIRECT_BLOCKS of them) or as the chunk
+// results of de_reduce_chunks<0>
+enum { DE_DT_GIVEN = 0, DE_DT_DIRECT, DE_DT_CHUNKS };
+
 // friction + update + fix_negative_cells from the explicit updates of substep 0;
-// `out` may alias `q` (Euler, in place: each thread reads then writes its own record)
-template <bool SLOPED = false>
+// `out` may alias `q` (Euler, in place: each thread reads then writes its own record).
+// With DT, every workgroup forms the step's timestep for itself from pdt, the
+// CFL partials or chunk results, and the scenario's first one records it: the
+// reduction and update_timestep cost no launches of their own. The control
+// fields that the others read are not the ones it writes. Each launch in the
+// graph of a step takes about 4.6 us however small: with the end of the step
+// reduced in de_finish_step, a DE0 step has 3 launches instead of 6 and a DE1
+// step 4 instead of 9 (6 above DE_DIRECT_BLOCKS); 120 DE1 steps of 90k
+// triangles with two reads went from 16.5 to 10.5 ms, a 40k DE0 run of 205
+// steps from 13.7 to 10.3 ms. The minimum's loads and barrier hide behind the
+// triangle's own records, requested first: 66.5 us at 4M triangles, 67.0
+// without it.
+template <bool SLOPED, int DT>
 __global__ void __launch_bounds__(DE_BLOCK)
 de_update(const int *__restrict__ scen, DeParams p, const DeQ *q, const double *__restrict__ eta,
           const unsigned char *__restrict__ flags, const double *__restrict__ exw,
           const double *__restrict__ exuh, const double *__restrict__ exvh, DeControl *ctl,
-          DeQ *out, unsigned long long *__restrict__ nneg, const double *__restrict__ E = nullptr,
-          int N = 0, const double *__restrict__ vx = nullptr)
+          DeQ *out, unsigned long long *__restrict__ nneg, const double *__restrict__ pdt,
+          const double *__restrict__ E = nullptr, int N = 0,
+          const double *__restrict__ vx = nullptr)
 {
     const int lb = xcd_block();
-    DeControl *cb = de_ctl(ctl, scen, lb);
+    const int sc = scen ? scen[lb] : 0;
+    DeControl *cb = ctl + sc;
     if (cb->done) return;
     const int k = lb * DE_BLOCK + threadIdx.x;
-    if (k >= cb->kend) return;
-    const double dt = cb->dt;
-    int *err = &cb->status;
-    const DeCentroid c = de_centroid(q[k], flags[k]);
+    const bool on = k < cb->kend;
+    DeQ qk{0.0, 0.0, 0.0, 0.0};
+    unsigned f = 0;
+    double n = 0.0, e0 = 0.0, e1 = 0.0, e2 = 0.0;
+    if (on) {
+        qk = q[k];
+        f = flags[k];
+        n = eta[k];
+        e0 = exw[k];
+        e1 = exuh[k];
+        e2 = exvh[k];
+    }
+    double dt;
+    if constexpr (DT == DE_DT_GIVEN) {
+        dt = cb->dt;
+    } else {
+        __shared__ double red[DE_BLOCK / 64];
+        double m = 1.0e100;
+        if constexpr (DT == DE_DT_DIRECT) {
+            for (int i = cb->bbeg + (int)threadIdx.x; i < cb->bend; i += DE_BLOCK)
+                m = fmin(m, pdt[i]);
+        } else if (threadIdx.x < DE_RCHUNKS) {
+            m = pdt[(size_t)sc * DE_RCHUNKS + threadIdx.x];
+        }
+        m = de_wave_min(m);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+        __syncthreads();
+        m = red[0];
+        for (int i = 1; i < DE_BLOCK / 64; i++) m = fmin(m, red[i]);
+        const double ts = de_cfl_timestep(cb, m);
+        dt = de_clamped_timestep(cb, ts);
+        if (lb == cb->bbeg && threadIdx.x == 0) de_commit_timestep(cb, m, ts, dt);
+    }
+    if (!on) return;
     DeSlope sl{false, 0.0, 0.0};
     if constexpr (SLOPED) sl = de_sloped_bed(E, N, k, vx);
-    out[k] = de_advance(c, eta[k], exw[k], exuh[k], exvh[k], dt, p, err, nneg, sl);
+    out[k] = de_advance(de_centroid(qk, f), n, e0, e1, e2, dt, p, &cb->status, nneg, sl);
 }
 
 // ---------------------------------------------------------------------------
@@ -1958,90 +2049,148 @@ de_fix_negative(int kend, DeQ *__restrict__ q, unsigned long long *__restrict__ 
     }
 }
 
-// Fixed-order reduction of the per-block partials into the control blocks,
-// in two stages so that many CUs read the partials: de_reduce_chunks splits
-// each scenario's blocks into DE_RCHUNKS contiguous chunks, one 256-thread
-// workgroup each; de_reduce_final adds a scenario's chunk results. MODE 0:
-// flux_dt, bflux0, mass (first substep); 1: bflux1 (second substep);
-// 2: mass (distribute); 3: volume; 4: bflux2 (third substep). The order of
-// the additions depends only on the scenario's block count.
-#define DE_RCHUNKS 32
-template <int MODE>
+// Fixed-order reduction of the per-block partials part[row][nblocks], row
+// DE_P_*, into the control blocks. Each scenario's blocks split into
+// DE_RCHUNKS contiguous chunks; a chunk's partials are added in a fixed order,
+// then the chunk results. The order depends only on the scenario's block
+// count. Up to DE_DIRECT_BLOCKS blocks (a chunk of at most 64, one per lane)
+// one workgroup per scenario reduces them in a single launch (4.6 us, at any
+// such size); above, de_reduce_chunks gives each chunk its own workgroup so
+// that many CUs read the partials, and a second stage adds the chunk results.
+// Both give the same bits.
+#define DE_DIRECT_BLOCKS (64 * DE_RCHUNKS)
+
+// what a reduction leaves in the control block
+enum { DE_R_FLUX0 = 0, DE_R_FLUX1, DE_R_MASS, DE_R_VOLUME, DE_R_FLUX2 };
+
+// One workgroup per chunk (blockIdx.x) and scenario (blockIdx.y): the CFL
+// minimum if DT, and the sums of NR rows, each to chunks[row][scenario][chunk].
+// live: nothing for scenarios that are done.
+template <bool DT, int NR>
 __global__ void __launch_bounds__(256)
-de_reduce_chunks(const double *__restrict__ part_dt, const double *__restrict__ part_bf,
-                 const double *__restrict__ part_mass, const DeControl *__restrict__ ctl,
-                 double *__restrict__ chunks)
+de_reduce_chunks(const double *__restrict__ part, int nblocks, int r0, int r1, int r2, int live,
+                 const DeControl *__restrict__ ctl, double *__restrict__ chunks)
 {
-    constexpr bool DT = MODE == 0, BF = MODE <= 1 || MODE == 4;
-    constexpr bool MS = MODE == 0 || MODE == 2 || MODE == 3;
-    __shared__ double s0[4], s1[4], s2[4];
+    __shared__ double red[4][4];
     const int sc = blockIdx.y, c = blockIdx.x, S = gridDim.y;
     const DeControl *cb = ctl + sc;
-    double a = 1.0e100, b = 0.0, m = 0.0;
-    if (!((MODE < 2 || MODE == 4) && cb->done)) {
-        const int b0 = cb->bbeg, b1 = cb->bend;
-        const int len = (b1 - b0 + DE_RCHUNKS - 1) / DE_RCHUNKS;
-        const int c0 = b0 + c * len, c1 = min(b1, c0 + len);
-        for (int i = c0 + (int)threadIdx.x; i < c1; i += 256) {
-            if (DT) a = fmin(a, part_dt[i]);
-            if (BF) b += part_bf[i];
-            if (MS) m += part_mass[i];
-        }
+    if (live && cb->done) return;
+    const int rows[3] = {r0, r1, r2};
+    double a = 1.0e100, b[3] = {0.0, 0.0, 0.0};
+    const int b0 = cb->bbeg, b1 = cb->bend;
+    const int len = (b1 - b0 + DE_RCHUNKS - 1) / DE_RCHUNKS;
+    const int c0 = b0 + c * len, c1 = min(b1, c0 + len);
+    for (int i = c0 + (int)threadIdx.x; i < c1; i += 256) {
+        if (DT) a = fmin(a, part[(size_t)DE_P_DT * nblocks + i]);
+#pragma unroll
+        for (int r = 0; r < NR; r++) b[r] += part[(size_t)rows[r] * nblocks + i];
     }
-    a = de_wave_min(a);
-    b = de_wave_sum(b);
-    m = de_wave_sum(m);
+    if (DT) a = de_wave_min(a);
+#pragma unroll
+    for (int r = 0; r < NR; r++) b[r] = de_wave_sum(b[r]);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (lane == 0) {
-        s0[wv] = a;
-        s1[wv] = b;
-        s2[wv] = m;
+        red[3][wv] = a;
+#pragma unroll
+        for (int r = 0; r < NR; r++) red[r][wv] = b[r];
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int k = 1; k < 4; k++) {
-            s0[0] = fmin(s0[0], s0[k]);
-            s1[0] += s1[k];
-            s2[0] += s2[k];
-        }
         const size_t o = (size_t)sc * DE_RCHUNKS + c, n = (size_t)S * DE_RCHUNKS;
-        chunks[o] = s0[0];
-        chunks[n + o] = s1[0];
-        chunks[2 * n + o] = s2[0];
+        if (DT) {
+            for (int k = 1; k < 4; k++) red[3][0] = fmin(red[3][0], red[3][k]);
+            chunks[DE_P_DT * n + o] = red[3][0];
+        }
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            for (int k = 1; k < 4; k++) red[r][0] += red[r][k];
+            chunks[rows[r] * n + o] = red[r][0];
+        }
     }
 }
 
-template <int MODE>
-__global__ void __launch_bounds__(64)
-de_reduce_final(const double *__restrict__ chunks, DeControl *ctl)
+#define DE_RED_THREADS 512
+// The sums of NR rows of one scenario's partials, by one workgroup of
+// DE_RED_THREADS threads (every thread gets them): the chunk results are read
+// (CHUNKS) or formed here, a wave per chunk and a lane per block.
+template <bool CHUNKS, int NR>
+__device__ __forceinline__ void de_reduce_rows(const double *__restrict__ src, int nblocks,
+                                               const DeControl *cb, int sc, int S,
+                                               const int rows[3], double (*res)[DE_RCHUNKS],
+                                               double sum[3])
 {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (!CHUNKS) {
+        const int b0 = cb->bbeg, b1 = cb->bend;
+        const int len = (b1 - b0 + DE_RCHUNKS - 1) / DE_RCHUNKS;
+        constexpr int PER = DE_RCHUNKS / (DE_RED_THREADS / 64);
+        double x[PER][3];
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            const int c = wv + j * (DE_RED_THREADS / 64);
+            const int i = b0 + c * len + lane;
+            const bool in = lane < len && i < b1;
+#pragma unroll
+            for (int r = 0; r < NR; r++)
+                x[j][r] = in ? src[(size_t)rows[r] * nblocks + i] : 0.0;
+        }
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+#pragma unroll
+            for (int r = 0; r < NR; r++) {
+                const double v = de_wave_sum_nz(x[j][r]);
+                if (lane == 0) res[r][wv + j * (DE_RED_THREADS / 64)] = v;
+            }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        double v = 0.0;
+        if (lane < DE_RCHUNKS)
+            v = CHUNKS ? src[((size_t)rows[r] * S + sc) * DE_RCHUNKS + lane] : res[r][lane];
+        sum[r] = __shfl(de_wave_sum_nz(v), 0, 64);
+    }
+}
+
+// A reduction to the control block outside device-controlled steps: MODE
+// DE_R_*, of the row (and for DE_R_FLUX0 the CFL timesteps and protect's
+// mass). src: the partials, or the chunk results (CHUNKS).
+template <int MODE, bool CHUNKS>
+__global__ void __launch_bounds__(DE_RED_THREADS)
+de_reduce(const double *__restrict__ src, int nblocks, int row, DeControl *ctl)
+{
+    __shared__ double res[3][DE_RCHUNKS], red[DE_RED_THREADS / 64];
     const int sc = blockIdx.x, S = gridDim.x, t = threadIdx.x;
     DeControl *cb = ctl + sc;
-    if ((MODE < 2 || MODE == 4) && cb->done) return;
-    const size_t o = (size_t)sc * DE_RCHUNKS + t, n = (size_t)S * DE_RCHUNKS;
-    double a = 1.0e100, b = 0.0, m = 0.0;
-    if (t < DE_RCHUNKS) {
-        a = chunks[o];
-        b = chunks[n + o];
-        m = chunks[2 * n + o];
-    }
-    a = de_wave_min(a);
-    b = de_wave_sum(b);
-    m = de_wave_sum(m);
-    if (t == 0) {
-        if (MODE == 0) {
-            cb->flux_dt = a;
-            cb->bflux0 = b;
-            cb->mass = m;
-        } else if (MODE == 1) {
-            cb->bflux1 = b;
-        } else if (MODE == 2) {
-            cb->mass = m;
-        } else if (MODE == 3) {
-            cb->volume = m;
+    const bool live = MODE == DE_R_FLUX0 || MODE == DE_R_FLUX1 || MODE == DE_R_FLUX2;
+    if (live && cb->done) return;
+    double sum[3];
+    const int rows[3] = {row, DE_P_MASS, 0};
+    de_reduce_rows<CHUNKS, MODE == DE_R_FLUX0 ? 2 : 1>(src, nblocks, cb, sc, S, rows, res, sum);
+    if (MODE == DE_R_FLUX0) {
+        double a = 1.0e100;
+        if (CHUNKS) {
+            if (t < DE_RCHUNKS) a = src[((size_t)DE_P_DT * S + sc) * DE_RCHUNKS + t];
         } else {
-            cb->bflux2 = b;
+            for (int i = cb->bbeg + t; i < cb->bend; i += DE_RED_THREADS)
+                a = fmin(a, src[(size_t)DE_P_DT * nblocks + i]);
         }
+        a = de_wave_min(a);
+        if ((t & 63) == 0) red[t >> 6] = a;
+        __syncthreads();
+        if (t == 0) {
+            for (int i = 1; i < DE_RED_THREADS / 64; i++) red[0] = fmin(red[0], red[i]);
+            cb->flux_dt = red[0];
+            cb->bflux0 = sum[0];
+            cb->mass = sum[1];
+        }
+        return;
+    }
+    if (t == 0) {
+        if (MODE == DE_R_FLUX1) cb->bflux1 = sum[0];
+        else if (MODE == DE_R_MASS) cb->mass = sum[0];
+        else if (MODE == DE_R_VOLUME) cb->volume = sum[0];
+        else cb->bflux2 = sum[0];
     }
 }
 
@@ -2061,50 +2210,33 @@ __device__ __forceinline__ double de_flux_integral(double integral, double dt, i
     return integral + 1.0 / 6.0 * dt * (s0 + s1 + 4.0 * s2);
 }
 
-// Generic_Domain.update_timestep (generic_domain.py:2349-2415) on the device:
-// CFL and max-timestep limit, recorded extremes, the small-step counter with
-// its first-order switch and its exception (reported as DE_ERR_SMALL_TIMESTEP),
-// and the clamps to the final time and the next yield time.
-__global__ void de_timestep(DeControl *ctl, int S)
+// End of a step, one workgroup per scenario: the boundary flux sums of the
+// METHOD's substeps and their integral (boundary_flux_integral_operator.py:
+// 39-49), relative_time += dt, timestep history (one scenario only), and the
+// yield / final-time test of _evolve_base (generic_domain.py:1855-1895) that
+// turns the scenario's next steps into no-ops.
+template <int METHOD, bool CHUNKS>
+__global__ void __launch_bounds__(DE_RED_THREADS)
+de_finish_step(const double *__restrict__ src, int nblocks, DeControl *ctl, double *hist)
 {
-    DeControl *c = de_scenario(ctl, S);
-    if (!c || c->done) return;
-    const double flux_dt = c->fixed_flux_dt > 0.0 ? c->fixed_flux_dt : c->flux_dt;
-    const double a = c->cfl * flux_dt;
-    double ts = (c->max_dt < a) ? c->max_dt : a;           // min(CFL * flux_dt, max_dt)
-    c->rec_max = (c->rec_max > ts) ? c->rec_max : ts;      // max(timestep, recorded_max)
-    c->rec_min = (c->rec_min < ts) ? c->rec_min : ts;      // min(timestep, recorded_min)
-    if (ts < c->min_dt) {
-        c->smallsteps += 1;
-        if (c->smallsteps > c->max_smallsteps) {
-            c->smallsteps = 0;
-            if (c->order == 1) c->status |= DE_ERR_SMALL_TIMESTEP;
-            else c->order = 1;
-        }
-    } else {
-        c->smallsteps = 0;
-        if (c->order == 1 && c->default_order == 2) c->order = 2;
-    }
-    if (c->t + ts > c->finaltime) ts = c->finaltime - c->t;
-    if (c->t + ts > c->yieldtime) ts = c->yieldtime - c->t;
-    c->dt = ts;
-}
-
-// End of a step: boundary flux integral (boundary_flux_integral_operator.py:39-49),
-// relative_time += dt, timestep history (one scenario only), and the yield /
-// final-time test of _evolve_base (generic_domain.py:1855-1895) that turns the
-// scenario's next steps into no-ops.
-__global__ void de_finish_step(DeControl *ctl, int S, double *hist)
-{
-    DeControl *c = de_scenario(ctl, S);
-    if (!c || c->done) return;
+    __shared__ double res[3][DE_RCHUNKS];
+    const int sc = blockIdx.x, S = gridDim.x;
+    DeControl *c = ctl + sc;
+    if (c->done) return;
+    double sum[3] = {0.0, 0.0, 0.0};
+    const int rows[3] = {DE_P_BF0, DE_P_BF1, DE_P_BF2};
+    de_reduce_rows<CHUNKS, METHOD>(src, nblocks, c, sc, S, rows, res, sum);
+    if (threadIdx.x) return;
+    c->bflux0 = sum[0];
+    if (METHOD > 1) c->bflux1 = sum[1];
+    if (METHOD > 2) c->bflux2 = sum[2];
     const double dt = c->dt;
-    c->integral = de_flux_integral(c->integral, dt, c->method, c->bflux0, c->bflux1, c->bflux2);
+    c->integral = de_flux_integral(c->integral, dt, METHOD, sum[0], sum[1], sum[2]);
     c->t = c->t + dt;
     if (hist && c->nsteps < c->hist_cap) hist[c->nsteps] = dt;
     c->nsteps += 1;
     if (c->t >= c->finaltime - c->eps) {
-        if (c->t > c->finaltime) c->status |= DE_ERR_OVERSHOOT;
+        if (c->t > c->finaltime) atomicOr(&c->status, DE_ERR_OVERSHOOT);
         c->done = 1;
     } else if (c->t >= c->yieldtime) {
         c->done = 2;
