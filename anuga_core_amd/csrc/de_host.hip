@@ -61,6 +61,16 @@ const char *kTimerNames[] = {"extrapolate", "flux0", "update", "flux1", "xflux0"
 enum { T_EXTRAP = 0, T_FLUX0, T_UPDATE, T_FLUX1, T_XFLUX0, T_XFLUX1, T_COUNT };
 const int kTimerRing = 64;
 
+// Steps of a run that come back with their timesteps in the one copy that ends
+// the run (longer histories take a copy of their own).
+const int kHostHist = 512;
+// Steps per captured graph. A run of fewer than kGraphMin steps is launched
+// kernel by kernel: at 400 and at 40k triangles (DE0, 3 launches a step) 18.0
+// and 19.0 us a step, with a graph of one step 21.5 and 22.9, of 8 steps 17.4
+// and 18.7, of 32 steps 17.1 and 18.5; 90k triangles, DE1: 41.3, 45.2, 40.4,
+// 40.3. Capturing 8 steps takes 45 to 100 us once.
+const int kGraphSteps = 8, kGraphMin = 64;
+
 }  // namespace
 
 // a Rate_operator's device data
@@ -159,18 +169,24 @@ struct anuga_domain {
     double *part = nullptr;   // [DE_P_ROWS][nblocks]
     double *chunks = nullptr; // [DE_P_ROWS][S][DE_RCHUNKS]: the reduction's first stage
     DeControl *ctl = nullptr; // [S] device step control
-    unsigned long long *dneg = nullptr;
-    DeControl *hctl = nullptr;          // [S] pinned host mirror of ctl
-    unsigned long long *hneg = nullptr; // pinned host mirror of *dneg
+    unsigned long long *dneg = nullptr; // fix_negative count, behind ctl
+    // one pinned allocation: the mirror of ctl and of the counter behind it,
+    // then hsetup, hhist and the staging of the boundary values' three slots
+    DeControl *hctl = nullptr;          // [S] host mirror of ctl
+    unsigned long long *hneg = nullptr; // host mirror of *dneg
     DeBatchSetup *dsetup = nullptr;     // [S] time control of a step run
-    DeBatchSetup *hsetup = nullptr;     // [S] pinned staging of dsetup
+    DeBatchSetup *hsetup = nullptr;     // [S] staging of dsetup
+    double *hhist = nullptr;            // [kHostHist] the history of a run of steps
+    double *hbval = nullptr;            // [3][3][M] boundary values on their way to bval
+    bool bval_sent[3] = {false, false, false};   // slot not known to have arrived
     double *hist = nullptr;             // device timestep history of a step run (S == 1)
     int64_t hist_cap = 0;
     bool done_on_device = false;        // a step run may have left done flags set
-    hipGraph_t graph = nullptr;         // one captured device-controlled step
+    hipGraph_t graph = nullptr;         // kGraphSteps captured device-controlled steps
     hipGraphExec_t graph_exec = nullptr;
     bool use_graph = true;
 
+    double host_dt = 0.0;     // the timestep of the last first substep (substate 1)
     int substate = 0;         // 0: at a step boundary (state in A); 1: rk2 substep state in B
     // per-operation calls (the reference's call order): the semi-implicit
     // momentum updates (allocated on first use), whether B holds a backup of
@@ -733,37 +749,42 @@ static bool reduce_direct(const anuga_domain *d)
 }
 
 template <bool SLOPED>
-static void launch_update_t(anuga_domain *d, DeQ *S, DeQ *out, int dt)
+static void launch_update_t(anuga_domain *d, DeQ *S, DeQ *out, int dt, double host_dt)
 {
     const double *pdt = dt == DE_DT_CHUNKS ? d->chunks : part_row(d, DE_P_DT);
     auto kern = dt == DE_DT_GIVEN    ? de_update<SLOPED, DE_DT_GIVEN>
+                : dt == DE_DT_HOST   ? de_update<SLOPED, DE_DT_HOST>
                 : dt == DE_DT_DIRECT ? de_update<SLOPED, DE_DT_DIRECT>
                                      : de_update<SLOPED, DE_DT_CHUNKS>;
     hipLaunchKernelGGL(kern, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream, d->scen,
                        dev_params(d->P), S, d->eta, d->flags, d->ex[0], d->ex[1], d->ex[2],
-                       d->ctl, out, d->dneg, pdt, (const double *)d->E, d->N, d->vx);
+                       d->ctl, out, d->dneg, pdt, host_dt,
+                       (int)(d->P.timestep_fluxcalls == 1), (const double *)d->E, d->N, d->vx);
 }
 
-// dt: DE_DT_*, where the timestep comes from
-static void launch_update(anuga_domain *d, DeQ *S, DeQ *out, int dt = DE_DT_GIVEN)
+// dt: DE_DT_*, where the timestep comes from; host_dt: the timestep of
+// DE_DT_HOST
+static void launch_update(anuga_domain *d, DeQ *S, DeQ *out, int dt = DE_DT_GIVEN,
+                          double host_dt = 0.0)
 {
     if (out == d->B) d->backup_valid = false;
     timer_begin(d, T_UPDATE);
-    if (d->P.use_sloped_mannings && !d->mixed) launch_update_t<true>(d, S, out, dt);
-    else launch_update_t<false>(d, S, out, dt);
+    if (d->P.use_sloped_mannings && !d->mixed) launch_update_t<true>(d, S, out, dt, host_dt);
+    else launch_update_t<false>(d, S, out, dt, host_dt);
     timer_end(d, T_UPDATE);
 }
 
 // Reduce a row of the partials to the control blocks: MODE DE_R_* (DE_R_FLUX0:
-// the CFL timestep and protect's mass too).
+// the CFL timestep and protect's mass too); integrate: the timestepping method
+// whose step this reduction completes (its boundary flux integral), or 0.
 template <int MODE>
-static void launch_reduce(anuga_domain *d, int row)
+static void launch_reduce(anuga_domain *d, int row, int integrate = 0)
 {
     constexpr bool FIRST = MODE == DE_R_FLUX0;
     const dim3 g(d->S), b(DE_RED_THREADS);
     if (reduce_direct(d)) {
         hipLaunchKernelGGL((de_reduce<MODE, false>), g, b, 0, d->stream, d->part, d->nblocks, row,
-                           d->ctl);
+                           integrate, d->ctl);
         return;
     }
     const int live = MODE != DE_R_MASS && MODE != DE_R_VOLUME;
@@ -771,7 +792,7 @@ static void launch_reduce(anuga_domain *d, int row)
                        0, d->stream, d->part, d->nblocks, row, (int)DE_P_MASS, 0, live, d->ctl,
                        d->chunks);
     hipLaunchKernelGGL((de_reduce<MODE, true>), g, b, 0, d->stream, d->chunks, d->nblocks, row,
-                       d->ctl);
+                       integrate, d->ctl);
 }
 
 template <int METHOD>
@@ -822,8 +843,8 @@ static void ensure_live(anuga_domain *d)
 }
 
 // The substeps after the first, with the timestep in the control blocks;
-// `reduce`: their boundary fluxes are reduced here (host-sequenced steps), not
-// at the end of the step.
+// `reduce`: their boundary fluxes are reduced here and the step's integral is
+// advanced (host-sequenced steps), not at the end of the step.
 static void enqueue_later_substeps(anuga_domain *d, bool reduce)
 {
     if (d->P.timestep_fluxcalls == 2) {
@@ -833,7 +854,7 @@ static void enqueue_later_substeps(anuga_domain *d, bool reduce)
             launch_extrapolate(d, d->B);
             launch_flux(d, 1, d->B, d->A, d->A);
         }
-        if (reduce) launch_reduce<DE_R_FLUX1>(d, DE_P_BF1);
+        if (reduce) launch_reduce<DE_R_FLUX1>(d, DE_P_BF1, 2);
     } else if (d->P.timestep_fluxcalls == 3) {
         if (fused(d) && d->C) {
             // the middle substep writes C, not B in place: other tiles are
@@ -848,7 +869,7 @@ static void enqueue_later_substeps(anuga_domain *d, bool reduce)
         }
         if (reduce) {
             launch_reduce<DE_R_FLUX1>(d, DE_P_BF1);
-            launch_reduce<DE_R_FLUX2>(d, DE_P_BF2);
+            launch_reduce<DE_R_FLUX2>(d, DE_P_BF2, 3);
         }
     }
 }
@@ -908,14 +929,35 @@ static void drop_graph(anuga_domain *d)
     d->graph = nullptr;
 }
 
-// read the control blocks and counters; raise a pending device error
+// nsteps device-controlled steps into the stream
+static int enqueue_device_steps(anuga_domain *d, int64_t nsteps)
+{
+    const bool graph = d->use_graph && !d->timing && (d->graph_exec || nsteps >= kGraphMin);
+    if (graph && !d->graph_exec) {
+        HIPCHK(d, hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
+        for (int i = 0; i < kGraphSteps; i++) enqueue_device_step(d);
+        hipGraph_t g = nullptr;
+        HIPCHK(d, hipStreamEndCapture(d->stream, &g));
+        d->graph = g;
+        HIPCHK(d, hipGraphInstantiate(&d->graph_exec, d->graph, nullptr, nullptr, 0));
+    }
+    int64_t i = 0;
+    if (graph)
+        for (; i + kGraphSteps <= nsteps; i += kGraphSteps)
+            HIPCHK(d, hipGraphLaunch(d->graph_exec, d->stream));
+    for (; i < nsteps; i++) enqueue_device_step(d);
+    return ANUGA_OK;
+}
+
+// read the control blocks and the counter behind them; raise a pending device
+// error
 static int sync_scalars(anuga_domain *d)
 {
-    HIPCHK(d, hipMemcpyAsync(d->hctl, d->ctl, d->S * sizeof(DeControl), hipMemcpyDeviceToHost,
-                             d->stream));
-    HIPCHK(d, hipMemcpyAsync(d->hneg, d->dneg, sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                             d->stream));
+    HIPCHK(d, hipMemcpyAsync(d->hctl, d->ctl,
+                             d->S * sizeof(DeControl) + sizeof(unsigned long long),
+                             hipMemcpyDeviceToHost, d->stream));
     HIPCHK(d, hipStreamSynchronize(d->stream));
+    for (bool &sent : d->bval_sent) sent = false;
     int e = 0;
     for (int s = 0; s < d->S; s++) e |= d->hctl[s].status;
     if (e) {
@@ -1039,12 +1081,20 @@ static int domain_alloc(const anuga_params *params, int64_t S64, const int64_t *
     DCHK(dalloc(&d->bval, 9 * (size_t)M));   // three substep slots
     DCHK(dalloc(&d->part, DE_P_ROWS * (size_t)d->nblocks));
     DCHK(dalloc(&d->chunks, DE_P_ROWS * (size_t)S * DE_RCHUNKS));
-    DCHK(dalloc(&d->ctl, S));
+    // the control blocks with the fix_negative counter behind them
+    DCHK(hipMalloc((void **)&d->ctl, S * sizeof(DeControl) + sizeof(unsigned long long)));
+    d->dneg = reinterpret_cast<unsigned long long *>(d->ctl + S);
     DCHK(dalloc(&d->dsetup, S));
-    DCHK(dalloc(&d->dneg, 1));
-    DCHK(hipHostMalloc((void **)&d->hctl, S * sizeof(DeControl), hipHostMallocDefault));
-    DCHK(hipHostMalloc((void **)&d->hsetup, S * sizeof(DeBatchSetup), hipHostMallocDefault));
-    DCHK(hipHostMalloc((void **)&d->hneg, sizeof(unsigned long long), hipHostMallocDefault));
+    static_assert(sizeof(DeControl) % 8 == 0 && sizeof(DeBatchSetup) % 8 == 0, "pinned layout");
+    const size_t hctl_bytes = S * sizeof(DeControl) + sizeof(unsigned long long);
+    const size_t hsetup_bytes = S * sizeof(DeBatchSetup);
+    DCHK(hipHostMalloc((void **)&d->hctl,
+                       hctl_bytes + hsetup_bytes + (kHostHist + 9 * (size_t)M) * sizeof(double),
+                       hipHostMallocDefault));
+    d->hneg = reinterpret_cast<unsigned long long *>(d->hctl + S);
+    d->hsetup = reinterpret_cast<DeBatchSetup *>(d->hneg + 1);
+    d->hhist = reinterpret_cast<double *>(d->hsetup + S);
+    d->hbval = d->hhist + kHostHist;
     if (S > 1) {
         DCHK(dalloc(&d->scen, d->nblocks));
         std::vector<int> bs(d->nblocks, 0);
@@ -1078,9 +1128,7 @@ static int domain_alloc(const anuga_params *params, int64_t S64, const int64_t *
     DCHK(hipMemset(d->bkind, 0, std::max(M, 1)));
     DCHK(hipMemset(d->bval, 0, 9 * (size_t)std::max(M, 1) * sizeof(double)));
     DCHK(hipMemset(d->part, 0, DE_P_ROWS * (size_t)d->nblocks * sizeof(double)));
-    DCHK(hipMemset(d->dneg, 0, sizeof(unsigned long long)));
-    std::memset(d->hctl, 0, S * sizeof(DeControl));
-    std::memset(d->hsetup, 0, S * sizeof(DeBatchSetup));
+    std::memset(d->hctl, 0, hctl_bytes + hsetup_bytes);
     for (int s = 0; s < S; s++) {
         DeControl &c = d->hctl[s];
         c.kbeg = d->kbeg[s];
@@ -1088,8 +1136,7 @@ static int domain_alloc(const anuga_params *params, int64_t S64, const int64_t *
         c.bbeg = d->kbeg[s] / DE_BLOCK;
         c.bend = (c.kend + DE_BLOCK - 1) / DE_BLOCK;
     }
-    DCHK(hipMemcpy(d->ctl, d->hctl, S * sizeof(DeControl), hipMemcpyHostToDevice));
-    *d->hneg = 0;
+    DCHK(hipMemcpy(d->ctl, d->hctl, hctl_bytes, hipMemcpyHostToDevice));
     {
         const char *g = std::getenv("ANUGA_HIP_GRAPH");
         d->use_graph = !(g && g[0] == '0');
@@ -1697,10 +1744,11 @@ static int evolve_steps(anuga_domain *d, int64_t max_steps, const anuga_time_con
         d->hist = nullptr;
         d->hist_cap = 0;
         drop_graph(d);
-        HIPCHK(d, dalloc(&d->hist, (size_t)max_steps));
-        d->hist_cap = max_steps;
+        const int64_t cap = std::max<int64_t>(max_steps, kHostHist);
+        HIPCHK(d, dalloc(&d->hist, (size_t)cap));
+        d->hist_cap = cap;
     }
-    HIPCHK(d, hipStreamSynchronize(d->stream));   // the staging buffer is free again
+    if (d->S > 1) HIPCHK(d, hipStreamSynchronize(d->stream));   // the staging is free again
     for (int s = 0; s < d->S; s++) {
         DeBatchSetup &b = d->hsetup[s];
         b.t = st[s].relative_time;
@@ -1721,27 +1769,24 @@ static int evolve_steps(anuga_domain *d, int64_t max_steps, const anuga_time_con
         b.method = (int)d->P.timestep_fluxcalls;
         b.stop_reached = stop_reached ? 1 : 0;
     }
-    HIPCHK(d, hipMemcpyAsync(d->dsetup, d->hsetup, d->S * sizeof(DeBatchSetup),
-                             hipMemcpyHostToDevice, d->stream));
-    hipLaunchKernelGGL(de_setup_batch, scenario_grid(d), dim3(64), 0, d->stream, d->ctl, d->S,
-                       d->dsetup);
+    if (d->S > 1) {
+        HIPCHK(d, hipMemcpyAsync(d->dsetup, d->hsetup, d->S * sizeof(DeBatchSetup),
+                                 hipMemcpyHostToDevice, d->stream));
+        hipLaunchKernelGGL(de_setup_batch, scenario_grid(d), dim3(64), 0, d->stream, d->ctl, d->S,
+                           d->dsetup);
+    } else {
+        hipLaunchKernelGGL(de_setup_one, dim3(1), dim3(64), 0, d->stream, d->ctl, d->hsetup[0]);
+    }
     d->done_on_device = true;
-
-    const bool graph = d->use_graph && !d->timing;
-    if (graph && !d->graph_exec && max_steps > 0) {
-        HIPCHK(d, hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
-        enqueue_device_step(d);
-        hipGraph_t g = nullptr;
-        HIPCHK(d, hipStreamEndCapture(d->stream, &g));
-        d->graph = g;
-        HIPCHK(d, hipGraphInstantiate(&d->graph_exec, d->graph, nullptr, nullptr, 0));
-    }
-    for (int64_t i = 0; i < max_steps; i++) {
-        if (graph) HIPCHK(d, hipGraphLaunch(d->graph_exec, d->stream));
-        else enqueue_device_step(d);
-    }
+    rc = enqueue_device_steps(d, max_steps);
+    if (rc) return rc;
     rc = launch_check(d);
     if (rc) return rc;
+    // the history crosses before the one synchronisation of the run
+    const bool short_hist = dt_history && max_steps <= kHostHist;
+    if (short_hist && max_steps > 0)
+        HIPCHK(d, hipMemcpyAsync(d->hhist, d->hist, max_steps * sizeof(double),
+                                 hipMemcpyDeviceToHost, d->stream));
     rc = sync_scalars(d);
     for (int s = 0; s < d->S; s++) {
         const DeControl &c = d->hctl[s];
@@ -1757,9 +1802,9 @@ static int evolve_steps(anuga_domain *d, int64_t max_steps, const anuga_time_con
     }
     if (d->G) d->grows_host += d->hctl[0].nsteps;
     if (dt_history && d->hctl[0].nsteps > 0) {
-        HIPCHK(d, hipMemcpy(dt_history, d->hist,
-                            (size_t)std::min<int64_t>(d->hctl[0].nsteps, max_steps) * sizeof(double),
-                            hipMemcpyDeviceToHost));
+        const size_t n = (size_t)std::min<int64_t>(d->hctl[0].nsteps, max_steps);
+        if (short_hist) std::memcpy(dt_history, d->hhist, n * sizeof(double));
+        else HIPCHK(d, hipMemcpy(dt_history, d->hist, n * sizeof(double), hipMemcpyDeviceToHost));
     }
     return rc;
 }
@@ -1851,7 +1896,7 @@ static void adj_stages(anuga_domain *d, AdjRun *a, const DeQ *X)
                        part_row(d, DE_P_DT), part_row(d, DE_P_BF0), a->neg);
     hipLaunchKernelGGL((de_update<false, DE_DT_GIVEN>), g, b, 0, d->stream, d->scen, p, X, d->eta,
                        a->f0, a->ex0, a->ex0 + N, a->ex0 + 2 * N, d->ctl, a->S1, a->neg, nullptr,
-                       nullptr, 0, nullptr);
+                       0.0, 0, nullptr, 0, nullptr);
     hipLaunchKernelGGL(de_extrapolate<double>, g, b, 0, d->stream, dev_mesh(d), p, a->S1, a->E1,
                        a->f1, pm, d->ctl);
     hipLaunchKernelGGL((de_flux<double, 0>), g, b, 0, d->stream, dev_mesh(d), p, a->S1, d->eta,
@@ -1938,14 +1983,12 @@ void anuga_destroy(anuga_domain *d)
                     d->scen, d->tstart, d->thalo, d->tslot, d->rw, d->rwd, d->caller, d->vx, d->node_start, d->node_tri, d->iperm_dev,
                     d->out_f32, d->gtri, d->gtimes, d->gvals, d->sub_idx, d->sub_val, d->eta, d->A, d->B, d->C, d->E, d->flags,
                     d->ex[0], d->ex[1], d->ex[2], d->bkind, d->bval, d->part, d->chunks, d->ctl, d->dsetup,
-                    d->dneg, d->hist, d->si[0], d->si[1], d->testart, d->tesplit, d->tedge,
+                    d->hist, d->si[0], d->si[1], d->testart, d->tesplit, d->tedge,
                     d->lts.e0, d->lts.e1, d->lts.e2, d->lts.pg, d->lts.et, d->lts.fuf,
                     d->lts.acf, d->lts.tmin, d->lts.unf};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (d->hctl) hipHostFree(d->hctl);
-    if (d->hsetup) hipHostFree(d->hsetup);
-    if (d->hneg) hipHostFree(d->hneg);
     for (int t = 0; t < T_COUNT; t++) {
         for (auto e : d->timers[t].start) hipEventDestroy(e);
         for (auto e : d->timers[t].stop) hipEventDestroy(e);
@@ -2080,12 +2123,18 @@ int anuga_set_boundary_values(anuga_domain *d, int64_t slot, const double *value
     if (slot < 0 || slot > 2) return fail(d, ANUGA_E_ARG, "slot must be 0, 1 or 2");
     if (M > 0 && !values) return fail(d, ANUGA_E_ARG, "values is NULL");
     if (M == 0) return ANUGA_OK;
-    std::vector<double> v(3 * (size_t)M);
+    // through pinned staging, in stream order: nothing waits unless the slot's
+    // last upload may still be on its way
+    if (d->bval_sent[slot]) {
+        HIPCHK(d, hipStreamSynchronize(d->stream));
+        for (bool &sent : d->bval_sent) sent = false;
+    }
+    double *v = d->hbval + (size_t)slot * 3 * M;
     for (int j = 0; j < M; j++)
         for (int q = 0; q < 3; q++) v[(size_t)q * M + j] = values[3 * (size_t)j + q];
-    HIPCHK(d, hipStreamSynchronize(d->stream));
-    HIPCHK(d, hipMemcpy(d->bval + (size_t)slot * 3 * M, v.data(), 3 * (size_t)M * sizeof(double),
-                        hipMemcpyHostToDevice));
+    HIPCHK(d, hipMemcpyAsync(d->bval + (size_t)slot * 3 * M, v, 3 * (size_t)M * sizeof(double),
+                             hipMemcpyHostToDevice, d->stream));
+    d->bval_sent[slot] = true;
     if (slot > 0 && d->bsstride == 0) {
         d->bsstride = 3 * (long long)M;
         drop_graph(d);
@@ -2688,9 +2737,9 @@ int anuga_update_conserved_quantities(anuga_domain *d, double dt, int64_t *num_n
     if (d->substate != 0) return fail(d, ANUGA_E_STATE, "update called twice in a step");
     ensure_live(d);
     const bool rk = d->P.timestep_fluxcalls > 1;
-    hipLaunchKernelGGL(de_set_dt, dim3(1), dim3(64), 0, d->stream, d->ctl, dt);
-    launch_update(d, d->A, rk ? d->B : d->A);
-    if (!rk) hipLaunchKernelGGL(de_integrate, dim3(1), dim3(64), 0, d->stream, d->ctl, 1);
+    // records dt and, for euler, advances the boundary flux integral
+    launch_update(d, d->A, rk ? d->B : d->A, DE_DT_HOST, dt);
+    d->host_dt = dt;
     rc = launch_check(d);
     if (rc) return rc;
     if (rk) d->substate = 1;
@@ -2705,9 +2754,10 @@ static int later_substeps(anuga_domain *d, double dt, int64_t *num_negative, int
     if (d->P.timestep_fluxcalls != method)
         return fail(d, ANUGA_E_STATE, "substeps of another timestepping method");
     if (d->substate != 1) return fail(d, ANUGA_E_STATE, "second substep without a first");
-    hipLaunchKernelGGL(de_set_dt, dim3(1), dim3(64), 0, d->stream, d->ctl, dt);
+    // the first substep's update left its dt in the control block
+    if (!(dt == d->host_dt))
+        hipLaunchKernelGGL(de_set_dt, dim3(1), dim3(64), 0, d->stream, d->ctl, dt);
     enqueue_later_substeps(d, true);
-    hipLaunchKernelGGL(de_integrate, dim3(1), dim3(64), 0, d->stream, d->ctl, method);
     rc = launch_check(d);
     if (rc) return rc;
     d->substate = 0;
@@ -3076,12 +3126,12 @@ int anuga_water_volume_noalloc(int64_t N, const double *stage, const double *ele
                        area, part);
     if (nb <= DE_DIRECT_BLOCKS) {
         hipLaunchKernelGGL((de_reduce<DE_R_VOLUME, false>), dim3(1), dim3(DE_RED_THREADS), 0, st,
-                           part, nb, 0, ctl);
+                           part, nb, 0, 0, ctl);
     } else {
         hipLaunchKernelGGL((de_reduce_chunks<false, 1>), dim3(DE_RCHUNKS, 1), dim3(256), 0, st,
                            part, nb, 0, 0, 0, 0, ctl, chunks);
         hipLaunchKernelGGL((de_reduce<DE_R_VOLUME, true>), dim3(1), dim3(DE_RED_THREADS), 0, st,
-                           chunks, nb, 0, ctl);
+                           chunks, nb, 0, 0, ctl);
     }
     hipLaunchKernelGGL(de_copy_volume, dim3(1), dim3(64), 0, st, ctl, volume);
     hipError_t e = hipGetLastError();

@@ -1835,6 +1835,15 @@ de_xflux_mixed(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__
                                part_mass, lb);
 }
 
+// boundary_flux_integral_operator.__call__ (boundary_flux_integral_operator.py:46-62)
+__device__ __forceinline__ double de_flux_integral(double integral, double dt, int method,
+                                                   double s0, double s1, double s2)
+{
+    if (method == 1) return integral + dt * s0;
+    if (method == 2) return integral + 0.5 * dt * (s0 + s1);
+    return integral + 1.0 / 6.0 * dt * (s0 + s1 + 4.0 * s2);
+}
+
 // Generic_Domain.update_timestep (generic_domain.py:2349-2415): the timestep
 // before the clamps, min(CFL * flux_dt, max_dt), and the step's timestep,
 // clamped to the final time and the next yield time. Reads nothing that
@@ -1875,11 +1884,11 @@ __device__ __forceinline__ void de_commit_timestep(DeControl *c, double flux_dt,
     c->dt = dt;
 }
 
-// where de_update takes the timestep from: the control block (host-sequenced
-// steps), or update_timestep over the minimum of the scenario's per-block CFL
+// where de_update takes the timestep from: the control block, the host (which
+// it then records, and for euler advances the boundary flux integral), or update_timestep over the minimum of the scenario's per-block CFL
 // partials, read directly (at most DE_DIRECT_BLOCKS of them) or as the chunk
 // results of de_reduce_chunks<0>
-enum { DE_DT_GIVEN = 0, DE_DT_DIRECT, DE_DT_CHUNKS };
+enum { DE_DT_GIVEN = 0, DE_DT_HOST, DE_DT_DIRECT, DE_DT_CHUNKS };
 
 // friction + update + fix_negative_cells from the explicit updates of substep 0;
 // `out` may alias `q` (Euler, in place: each thread reads then writes its own record).
@@ -1900,7 +1909,7 @@ de_update(const int *__restrict__ scen, DeParams p, const DeQ *q, const double *
           const unsigned char *__restrict__ flags, const double *__restrict__ exw,
           const double *__restrict__ exuh, const double *__restrict__ exvh, DeControl *ctl,
           DeQ *out, unsigned long long *__restrict__ nneg, const double *__restrict__ pdt,
-          const double *__restrict__ E = nullptr, int N = 0,
+          double host_dt, int euler, const double *__restrict__ E = nullptr, int N = 0,
           const double *__restrict__ vx = nullptr)
 {
     const int lb = xcd_block();
@@ -1923,6 +1932,13 @@ de_update(const int *__restrict__ scen, DeParams p, const DeQ *q, const double *
     double dt;
     if constexpr (DT == DE_DT_GIVEN) {
         dt = cb->dt;
+    } else if constexpr (DT == DE_DT_HOST) {
+        dt = host_dt;
+        if (lb == cb->bbeg && threadIdx.x == 0) {
+            cb->dt = dt;
+            if (euler)
+                cb->integral = de_flux_integral(cb->integral, dt, 1, cb->bflux0, 0.0, 0.0);
+        }
     } else {
         __shared__ double red[DE_BLOCK / 64];
         double m = 1.0e100;
@@ -2154,10 +2170,11 @@ __device__ __forceinline__ void de_reduce_rows(const double *__restrict__ src, i
 
 // A reduction to the control block outside device-controlled steps: MODE
 // DE_R_*, of the row (and for DE_R_FLUX0 the CFL timesteps and protect's
-// mass). src: the partials, or the chunk results (CHUNKS).
+// mass). src: the partials, or the chunk results (CHUNKS). integrate: the
+// method whose step it completes, or 0.
 template <int MODE, bool CHUNKS>
 __global__ void __launch_bounds__(DE_RED_THREADS)
-de_reduce(const double *__restrict__ src, int nblocks, int row, DeControl *ctl)
+de_reduce(const double *__restrict__ src, int nblocks, int row, int integrate, DeControl *ctl)
 {
     __shared__ double res[3][DE_RCHUNKS], red[DE_RED_THREADS / 64];
     const int sc = blockIdx.x, S = gridDim.x, t = threadIdx.x;
@@ -2191,6 +2208,9 @@ de_reduce(const double *__restrict__ src, int nblocks, int row, DeControl *ctl)
         else if (MODE == DE_R_MASS) cb->mass = sum[0];
         else if (MODE == DE_R_VOLUME) cb->volume = sum[0];
         else cb->bflux2 = sum[0];
+        if (integrate)
+            cb->integral = de_flux_integral(cb->integral, cb->dt, integrate, cb->bflux0,
+                                            cb->bflux1, cb->bflux2);
     }
 }
 
@@ -2199,15 +2219,6 @@ __device__ __forceinline__ DeControl *de_scenario(DeControl *ctl, int S)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     return s < S ? ctl + s : nullptr;
-}
-
-// boundary_flux_integral_operator.__call__ (boundary_flux_integral_operator.py:46-62)
-__device__ __forceinline__ double de_flux_integral(double integral, double dt, int method,
-                                                   double s0, double s1, double s2)
-{
-    if (method == 1) return integral + dt * s0;
-    if (method == 2) return integral + 0.5 * dt * (s0 + s1);
-    return integral + 1.0 / 6.0 * dt * (s0 + s1 + 4.0 * s2);
 }
 
 // End of a step, one workgroup per scenario: the boundary flux sums of the
@@ -2263,11 +2274,8 @@ struct DeBatchSetup {
     int stop_reached;  // a scenario already at its final or yield time takes no step
 };
 
-__global__ void de_setup_batch(DeControl *ctl, int S, const DeBatchSetup *__restrict__ setup)
+__device__ __forceinline__ void de_setup(DeControl *c, const DeBatchSetup &b)
 {
-    DeControl *c = de_scenario(ctl, S);
-    if (!c) return;
-    const DeBatchSetup b = setup[c - ctl];
     c->t = b.t;
     c->rec_min = b.rec_min;
     c->rec_max = b.rec_max;
@@ -2291,6 +2299,18 @@ __global__ void de_setup_batch(DeControl *ctl, int S, const DeBatchSetup *__rest
         if (c->t >= c->finaltime - c->eps) c->done = 1;
         else if (c->t >= c->yieldtime) c->done = 2;
     }
+}
+
+__global__ void de_setup_batch(DeControl *ctl, int S, const DeBatchSetup *__restrict__ setup)
+{
+    DeControl *c = de_scenario(ctl, S);
+    if (c) de_setup(c, setup[c - ctl]);
+}
+
+// a single scenario's, from the kernel's arguments
+__global__ void de_setup_one(DeControl *c, DeBatchSetup b)
+{
+    if (threadIdx.x == 0 && blockIdx.x == 0) de_setup(c, b);
 }
 
 // leave device-controlled mode: steps are live again

@@ -631,7 +631,7 @@ class Domain:
                 c = np.broadcast_to(c, (N,)).copy()
             else:
                 c = np.broadcast_to(np.asarray(value, np.float64), (N,)).copy()
-            vtx = np.repeat(c[:, None], 3, axis=1)
+            vtx = np.repeat(c[:, None], 3, axis=1) if name == "elevation" else None
         elif location == "vertices":
             if callable(value):
                 V = self.mesh.vertex_coordinates
@@ -1101,13 +1101,16 @@ class Domain:
         return 0
 
     def _chunk_estimate(self):
-        """Steps to the next yield or final time from the last timestep, so that
-        few launches of a run become no-ops."""
+        """Steps to the next yield or final time at the last CFL timestep (the
+        last step itself may have been cut short at a yield time), so that few
+        launches of a run become no-ops."""
         target = self.relative_yieldtime
         if self.relative_finaltime is not None:
             target = min(target, self.relative_finaltime)
-        if self.timestep > 0.0:
-            est = (target - self.relative_time) / self.timestep
+        flux = self.flux_timestep if self.fixed_flux_timestep is None else self.fixed_flux_timestep
+        dt = min(self.CFL * flux, self.evolve_max_timestep)
+        if dt > 0.0:
+            est = (target - self.relative_time) / dt
             return int(max(1, min(256, est + 2)))
         return 8
 
