@@ -60,6 +60,14 @@ class TimeControl(C.Structure):
                 ("default_order", C.c_int64)]
 
 
+class TileTables(C.Structure):
+    _u32, _i32 = C.POINTER(C.c_uint32), C.POINTER(C.c_int32)
+    _fields_ = [("capacity", C.c_int64), ("sizes", _ip), ("stencil", _u32), ("across", _u32),
+                ("nodes", _u32), ("cstart", _i32), ("hstart", _i32), ("estart", _i32),
+                ("esplit", _i32), ("nstart", _i32), ("cell", _i32), ("hstencil", _u32),
+                ("hcell", _u32), ("hnodes", _u32), ("edge", _u32), ("node", _dp)]
+
+
 class StepState(C.Structure):
     _fields_ = [("relative_time", C.c_double), ("timestep", C.c_double),
                 ("flux_timestep", C.c_double), ("recorded_min_timestep", C.c_double),
@@ -132,6 +140,8 @@ SIGNATURES = {
     "anuga_tile_order": (C.c_int, [C.c_int64, _dp, _ip, _ip]),
     "anuga_tile_halos": (C.c_int, [C.c_int64, C.POINTER(C.c_int32), _ip, C.c_int64,
                                    C.POINTER(C.c_int32), C.POINTER(C.c_uint32), _ip, _ip]),
+    "anuga_tile_tables": (C.c_int, [C.c_int64, C.POINTER(C.c_int32), _dp,
+                                    C.POINTER(TileTables)]),
     "anuga_tile_edges": (C.c_int, [C.c_int64, C.POINTER(C.c_int32), _ip, _ip, C.c_int64,
                                    C.POINTER(C.c_uint32), _ip]),
     "anuga_synchronize": (C.c_int, [C.c_void_p]),

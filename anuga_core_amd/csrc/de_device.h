@@ -115,13 +115,44 @@ struct DeTiles {
     const int *__restrict__ halo;       // the halo triangles of each tile
     const unsigned *__restrict__ slot;  // [N] 3 x 10 bits: halo slot of edge i, 1023: in the tile
     int hcap;                           // the largest halo (LDS stride)
-    // the edges whose flux a tile evaluates once (null: none built): each
-    // in-tile interior edge from its lower-numbered triangle, then each edge
-    // to the halo from the tile's side (DE_TE_* fields)
-    const int *__restrict__ estart;     // [tiles + 1] offsets into edge
-    const int *__restrict__ esplit;     // [tiles] the first edge to the halo
+};
+
+// The once-per-edge fused kernel's own tables of a tile (de_xflux_e). A tile's
+// cells are its DE_BLOCK triangles, then its halo, then the halo's neighbours
+// outside both; a cell's index is its place in that list, 10 bits. Nodes are
+// the distinct vertices of the tile's and the halo's triangles, 10 bits.
+// Halo edges are the tile's edge-list entries behind esplit, in that order.
+struct DeTileX {
+    const int *__restrict__ cstart;        // [tiles + 1] offsets into cell
+    const int *__restrict__ cell;          // the cells behind the tile's own
+    const int *__restrict__ nstart;        // [tiles + 1] offsets into node
+    const double2 *__restrict__ node;
+    // per triangle: its edges' neighbours as cell indices (3 x 10 bits, 1023:
+    // boundary edge); their edges j (3 x 2 bits, from bit 0) and, of a halo
+    // neighbour, the halo edge (3 x 8 bits, from bit 6); its nodes (3 x 10)
+    const unsigned *__restrict__ stencil;
+    const unsigned *__restrict__ across;
+    const unsigned *__restrict__ nodes;
+    // per halo edge: the halo triangle's stencil; its cell index (10 bits) and
+    // edge (2 bits, from bit 10); its nodes
+    const int *__restrict__ hstart;        // [tiles + 1] offsets
+    const unsigned *__restrict__ hstencil;
+    const unsigned *__restrict__ hcell;
+    const unsigned *__restrict__ hnodes;
+    int hecap, ncap;                       // the most halo edges and nodes of a tile (LDS strides)
+    // the edges whose flux the tile evaluates once: each in-tile interior edge
+    // from its lower-numbered triangle, then each edge to the halo from the
+    // tile's side (DE_TE_* fields)
+    const int *__restrict__ estart;        // [tiles + 1] offsets into edge
+    const int *__restrict__ esplit;        // [tiles] the first edge to the halo
     const unsigned *__restrict__ edge;
 };
+// cells of a tile behind its own (their LDS fits in the edge values' place),
+// its halo edges (one thread each, a wave left for the tile's edges; 8 bits),
+// its nodes
+#define DE_XCELLS_MAX (DE_BLOCK < 511 ? DE_BLOCK : 1022 - DE_BLOCK)
+#define DE_XHALO_MAX (DE_BLOCK - 64 < 256 ? DE_BLOCK - 64 : 256)
+#define DE_XNODES_MAX 384
 
 // Local flux updating (max_flux_update_frequency > 1): per half-edge state,
 // [3][N] in the internal order (half-edge (k, i) at i * N + k). e0..e2: the

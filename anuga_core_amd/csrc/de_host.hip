@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cmath>
 #include <cstdio>
@@ -89,6 +90,16 @@ struct RateOp {
     int vmode = 0;
 };
 
+// The tables of DeTileX for one scenario (its own triangle numbering; offsets
+// from 0). ok: within the kernel's limits; vertices: nodes were built.
+struct TileTables {
+    bool ok = false, vertices = false;
+    std::vector<int> cstart, cell, nstart, hstart, estart, esplit;
+    std::vector<double2> node;
+    std::vector<unsigned> stencil, across, nodes, hstencil, hcell, hnodes, edge;
+    int hecap = 0, ncap = 0;
+};
+
 struct anuga_domain {
     int N = 0, M = 0, nblocks = 0;   // N: internal triangles incl. padding; M: boundary edges
     int max_blocks = 0;              // the largest scenario's blocks
@@ -119,19 +130,19 @@ struct anuga_domain {
     int hcap = 0;
     // per scenario, until every mesh is set: tile offsets, halo (internal
     // ids), slots and largest halo (-1: no tiles)
-    std::vector<std::vector<int>> ts_start, ts_halo, ts_estart, ts_esplit;
-    std::vector<std::vector<unsigned>> ts_slot, ts_edge;
-    // tile edge lists of the once-per-edge kernel (null: not built); mirror:
+    std::vector<std::vector<int>> ts_start, ts_halo;
+    std::vector<std::vector<unsigned>> ts_slot;
+    // tables of the once-per-edge kernel (hecap == 0: not built); mirror:
     // every interior edge's normals and lengths mirror exactly (checked per
     // scenario at upload), which that kernel assumes
-    int *testart = nullptr, *tesplit = nullptr;
-    unsigned *tedge = nullptr;
+    DeTileX tx{};
+    std::vector<struct TileTables> ts_x;   // per scenario, until every mesh is set
     bool mirror = true;
     bool edge_once = true;     // ANUGA_HIP_EDGE_ONCE=0: the gather-every-side kernel
-    // vertex geometry: the fused FP64 kernel forms edge offsets, normals and
-    // lengths from each triangle's vertex coordinates (vx) instead of reading
-    // the stored records, where that reproduces every scenario's arrays bit
-    // for bit (ANUGA_HIP_VERTEX_GEOMETRY=0: the stored records)
+    // vertex geometry: that kernel forms edge offsets, normals and lengths
+    // from the vertices of the tile (its node list) instead of reading the
+    // stored records, where that reproduces every scenario's arrays bit for
+    // bit (ANUGA_HIP_VERTEX_GEOMETRY=0: the stored records)
     bool vgeom = true;
     std::vector<int> ts_hcap;
     bool e_stale = false;                // E does not hold the last extrapolation
@@ -678,7 +689,7 @@ template <int SUB>
 static void launch_xflux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
 {
     DeBoundary bc{d->bkind, d->bval, d->M, d->bsstride};
-    DeTiles tl{d->tstart, d->thalo, d->tslot, d->hcap, d->testart, d->tesplit, d->tedge};
+    DeTiles tl{d->tstart, d->thalo, d->tslot, d->hcap};
     if (d->mixed) {
         // FP64 centroid depth + 12 FP32 record components per triangle
         const size_t lds = ((size_t)DE_BLOCK + (size_t)d->hcap) * (sizeof(double) + 12 * sizeof(float));
@@ -694,14 +705,17 @@ static void launch_xflux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
                            d->stream, dev_mesh(d), dev_params(d->P), S, d->eta, tl, bc, d->flags,
                            d->ex[0], d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d), part_row(d, DE_P_MASS), d->dneg,
                            (double *)d->E);
-    } else if (d->mirror && d->tedge && d->edge_once) {
-        // each edge's flux once: tile and halo edge values, then the tile's
-        // centroid depths and beds; geometry from the vertices where it can be
-        const size_t lds = (14 * (size_t)DE_BLOCK + 12 * (size_t)d->hcap) * sizeof(double);
-        auto kern = (d->vgeom && d->vx) ? de_xflux_e<SUB, true> : de_xflux_e<SUB, false>;
-        hipLaunchKernelGGL(kern, dim3(d->nblocks), dim3(DE_BLOCK), lds, d->stream,
-                           dev_mesh(d), dev_params(d->P), S, d->eta, tl, bc, d->flags, d->ex[0],
-                           d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
+    } else if (d->mirror && d->tx.hecap && d->edge_once) {
+        // each edge's flux once: tile edge values (before them, the cells),
+        // halo edge values, the tile's centroid depths and beds, and the
+        // vertices and node words where the geometry comes from them
+        const bool vg = d->vgeom && d->tx.ncap;
+        const size_t lds = (14 * (size_t)DE_BLOCK + 4 * (size_t)d->tx.hecap) * sizeof(double) +
+                           (vg ? d->tx.ncap * sizeof(double2) + DE_BLOCK * sizeof(unsigned) : 0);
+        auto kern = vg ? de_xflux_e<SUB, true> : de_xflux_e<SUB, false>;
+        hipLaunchKernelGGL(kern, dim3(d->nblocks), dim3(DE_BLOCK), lds, d->stream, dev_mesh(d),
+                           dev_params(d->P), S, d->eta, d->tx, bc, d->flags, d->ex[0], d->ex[1],
+                           d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
                            part_row(d, DE_P_MASS), d->dneg);
     } else {
         const size_t lds = (12 * (size_t)DE_BLOCK + 12 * (size_t)d->hcap) * sizeof(double);
@@ -987,6 +1001,7 @@ static int launch_check(anuga_domain *d)
 // creation
 // ---------------------------------------------------------------------------
 extern "C" void anuga_destroy(anuga_domain *d);
+static void free_tile_tables(anuga_domain *d);
 
 // Allocate the buffers of S scenarios of ntri[s] triangles and nbnd[s]
 // boundary edges; no mesh is uploaded yet. On failure *out stays NULL and
@@ -1204,8 +1219,7 @@ static const int kMaxHalo = std::min(320, (65536 - 113 * DE_BLOCK - 1024) / 97 /
 // The tile metadata of triangles in internal order (nb: packed neighbours of
 // one scenario starting at 0). Returns the largest halo, or -1 when a
 // neighbour index is out of range; the caller refuses halos above kMaxHalo.
-// The tile edge lists of the once-per-edge fused kernel (de_xflux_e): per
-// tile, each edge between two tile triangles from its lower-numbered side and
+// The tile edge lists as anuga_tile_edges exports them: per tile, each edge between two tile triangles from its lower-numbered side and
 // each edge to the halo from the tile's side, ordered by edge index, then
 // triangle (consecutive entries read consecutive geometry). halo slots as
 // tile_halos assigns them.
@@ -1280,9 +1294,178 @@ static int tile_halos(int N, const int4 *hn, std::vector<int> &start, std::vecto
     return hcap;
 }
 
-// The tile metadata of scenario s (its nb records hn, internal ids), kept on
-// the host until every scenario's mesh is set.
-static int scenario_tiles(anuga_domain *d, int s, const std::vector<int4> &hn)
+// DeTileX's tables of tiles [b0, b1) of one scenario of N triangles (nb records
+// hn, its own numbering), appended to x; vx: the triangles' vertex coordinates
+// [N][6], or NULL. False: a tile exceeds the kernel's limits.
+static bool tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1, TileTables &x)
+{
+    // place of each cell of a tile (its triangle id), by open addressing
+    constexpr int HS = 4 * DE_XCELLS_MAX, NS = 4 * DE_XNODES_MAX;
+    std::vector<int> hkey(HS), hval(HS);
+    std::vector<int> nval(NS);
+    std::vector<std::array<int, 3>> hedge;   // halo edges: halo triangle, its edge
+    auto nbr = [&](int k, int i) { return i == 0 ? hn[k].x : (i == 1 ? hn[k].y : hn[k].z); };
+    auto word = [](const int f[3]) {
+        return (unsigned)f[0] | ((unsigned)f[1] << 10) | ((unsigned)f[2] << 20);
+    };
+    for (int b = b0; b < b1; b++) {
+        const int k0 = b * DE_BLOCK, k1 = std::min(N, k0 + DE_BLOCK);
+        const int cbase = (int)x.cell.size();
+        std::fill(hkey.begin(), hkey.end(), -1);
+        bool full = false;
+        auto place = [&](int n) {   // cell index of triangle n, appended if new
+            if (n >= k0 && n < k1) return n - k0;
+            unsigned h = (unsigned)n * 2654435761u;
+            for (;; h++) {
+                const unsigned s = h & (HS - 1);
+                if (hkey[s] == n) return hval[s];
+                if (hkey[s] < 0) {
+                    const int j = (int)x.cell.size() - cbase;
+                    if (j >= DE_XCELLS_MAX) {
+                        full = true;
+                        return 0;
+                    }
+                    hkey[s] = n;
+                    hval[s] = DE_BLOCK + j;
+                    x.cell.push_back(n);
+                    return hval[s];
+                }
+            }
+        };
+        // the edges inside the tile, then those to the halo, each by edge
+        // index, then triangle (consecutive entries read consecutive data)
+        x.estart.push_back((int)x.edge.size());
+        hedge.clear();
+        std::vector<unsigned> across(k1 - k0, 0);
+        for (int halo = 0; halo < 2; halo++) {
+            if (halo) x.esplit.push_back((int)x.edge.size());
+            for (int i = 0; i < 3; i++)
+                for (int k = k0; k < k1; k++) {
+                    const int v = nbr(k, i);
+                    if (v < 0) continue;
+                    const int n = v >> 2, j = v & 3;
+                    const bool out = n < k0 || n >= k1;
+                    if (!halo) across[k - k0] |= (unsigned)j << (2 * i);
+                    if (halo && out) {
+                        const int he = (int)hedge.size();
+                        if (he >= DE_XHALO_MAX) return false;
+                        across[k - k0] |= (unsigned)he << (6 + 8 * i);
+                        hedge.push_back({n, j, 0});
+                        x.edge.push_back(DE_TE_MAKE(k - k0, i, 1, 0, j));
+                    } else if (!halo && !out && k < n) {
+                        x.edge.push_back(DE_TE_MAKE(k - k0, i, 0, n - k0, j));
+                    }
+                }
+        }
+        // the halo's cells first, then the halo's neighbours'
+        for (const auto &e : hedge) place(e[0]);
+        auto stencil = [&](int k) {
+            int f[3];
+            for (int i = 0; i < 3; i++) f[i] = nbr(k, i) >= 0 ? place(nbr(k, i) >> 2) : 1023;
+            return word(f);
+        };
+        x.hstart.push_back((int)x.hstencil.size());
+        for (const auto &e : hedge) {
+            x.hstencil.push_back(stencil(e[0]));
+            x.hcell.push_back((unsigned)place(e[0]) | ((unsigned)e[1] << 10));
+        }
+        for (int k = k0; k < k1; k++) x.stencil.push_back(stencil(k));
+        if (full) return false;
+        x.across.insert(x.across.end(), across.begin(), across.end());
+        x.cstart.push_back(cbase);
+        x.hecap = std::max(x.hecap, (int)hedge.size());
+        if (!vx) continue;
+        // the distinct vertices (by their bits) of the tile and its halo
+        const int nbase = (int)x.node.size();
+        std::fill(nval.begin(), nval.end(), -1);
+        bool crowded = false;
+        auto node = [&](int k, int c) {
+            const double2 p = make_double2(vx[6 * (size_t)k + 2 * c], vx[6 * (size_t)k + 2 * c + 1]);
+            uint64_t u[2];
+            std::memcpy(u, &p, sizeof(u));
+            uint64_t h = (u[0] * 0x9e3779b97f4a7c15ull) ^ (u[1] * 0xc2b2ae3d27d4eb4full);
+            h ^= h >> 32;
+            for (;; h++) {
+                int &s = nval[h & (NS - 1)];
+                if (s < 0) {
+                    const int j = (int)x.node.size() - nbase;
+                    if (j >= DE_XNODES_MAX) {
+                        crowded = true;
+                        return 0;
+                    }
+                    s = j;
+                    x.node.push_back(p);
+                    return j;
+                }
+                if (!std::memcmp(&x.node[nbase + s], u, sizeof(u))) return s;
+            }
+        };
+        auto nodes = [&](int k) {
+            int f[3];
+            for (int c = 0; c < 3; c++) f[c] = node(k, c);
+            return word(f);
+        };
+        for (int k = k0; k < k1; k++) x.nodes.push_back(nodes(k));
+        for (const auto &e : hedge) x.hnodes.push_back(nodes(e[0]));
+        if (crowded) return false;
+        x.nstart.push_back(nbase);
+        x.ncap = std::max(x.ncap, (int)x.node.size() - nbase);
+    }
+    return true;
+}
+
+// The tables of a whole scenario, its tiles cut on several threads.
+static void scenario_tables(int N, const int4 *hn, const double *vx, TileTables &x)
+{
+    const int nt = (N + DE_BLOCK - 1) / DE_BLOCK;
+    const int T = std::max(1, std::min<int>({(int)std::thread::hardware_concurrency(), 16, nt / 16}));
+    std::vector<TileTables> part(T);
+    std::vector<char> ok(T, 0);
+    auto work = [&](int i) {
+        const int b0 = (int)((int64_t)nt * i / T), b1 = (int)((int64_t)nt * (i + 1) / T);
+        ok[i] = tile_tables(N, hn, vx, b0, b1, part[i]);
+    };
+    std::vector<std::thread> th;
+    for (int i = 1; i < T; i++) th.emplace_back(work, i);
+    work(0);
+    for (auto &t : th) t.join();
+    x = TileTables();
+    x.vertices = vx != nullptr;
+    for (int i = 0; i < T; i++)
+        if (!ok[i]) return;
+    x.ok = true;
+    if (T == 1) std::swap(x, part[0]);
+    x.ok = true;
+    x.vertices = vx != nullptr;
+    auto join = [](auto &to, const auto &from) { to.insert(to.end(), from.begin(), from.end()); };
+    auto offsets = [](std::vector<int> &to, const std::vector<int> &from, size_t base) {
+        for (int v : from) to.push_back((int)(v + base));
+    };
+    if (T > 1)
+        for (const TileTables &p : part) {
+            offsets(x.cstart, p.cstart, x.cell.size());
+            offsets(x.nstart, p.nstart, x.node.size());
+            offsets(x.hstart, p.hstart, x.hstencil.size());
+            offsets(x.estart, p.estart, x.edge.size());
+            offsets(x.esplit, p.esplit, x.edge.size());
+            join(x.cell, p.cell);
+            join(x.node, p.node);
+            join(x.stencil, p.stencil);
+            join(x.across, p.across);
+            join(x.nodes, p.nodes);
+            join(x.hstencil, p.hstencil);
+            join(x.hcell, p.hcell);
+            join(x.hnodes, p.hnodes);
+            join(x.edge, p.edge);
+            x.hecap = std::max(x.hecap, p.hecap);
+            x.ncap = std::max(x.ncap, p.ncap);
+        }
+}
+
+// The tile metadata of scenario s (its nb records hn, internal ids; hv: its
+// vertex coordinates, or NULL), kept on the host until every scenario's mesh
+// is set.
+static int scenario_tiles(anuga_domain *d, int s, const std::vector<int4> &hn, const double *hv)
 {
     const int N = (int)hn.size(), kb = d->kbeg[s];
     std::vector<int4> loc(hn);
@@ -1295,16 +1478,132 @@ static int scenario_tiles(anuga_domain *d, int s, const std::vector<int4> &hn)
         d->ts_start.resize(d->S);
         d->ts_halo.resize(d->S);
         d->ts_slot.resize(d->S);
-        d->ts_estart.resize(d->S);
-        d->ts_esplit.resize(d->S);
-        d->ts_edge.resize(d->S);
+        d->ts_x.resize(d->S);
         d->ts_hcap.assign(d->S, -1);
     }
     const int hcap = tile_halos(N, loc.data(), d->ts_start[s], d->ts_halo[s], d->ts_slot[s]);
     if (hcap < 0) return fail(d, ANUGA_E_ARG, "tiles: neighbour out of range");
-    tile_edges(N, loc.data(), d->ts_slot[s], d->ts_estart[s], d->ts_esplit[s], d->ts_edge[s]);
     for (int &n : d->ts_halo[s]) n += kb;
     d->ts_hcap[s] = hcap;
+    if (!d->mixed && d->edge_once) {
+        scenario_tables(N, loc.data(), d->vgeom ? hv : nullptr, d->ts_x[s]);
+        // too many nodes in a tile: the stored records
+        if (!d->ts_x[s].ok && d->vgeom && hv) scenario_tables(N, loc.data(), nullptr, d->ts_x[s]);
+        for (int &n : d->ts_x[s].cell) n += kb;
+    }
+    return ANUGA_OK;
+}
+
+// The tables share one device allocation (tx.cstart is its start).
+static void free_tile_tables(anuga_domain *d)
+{
+    if (d->tx.cstart) hipFree(const_cast<int *>(d->tx.cstart));
+    d->tx = DeTileX{};
+}
+
+// Assemble every scenario's TileTables into DeTileX's device arrays; none
+// (hecap 0) if a scenario exceeds the limits.
+static int upload_tile_tables(anuga_domain *d)
+{
+    free_tile_tables(d);
+    if (d->mixed || !d->edge_once || (int)d->ts_x.size() != d->S) return ANUGA_OK;
+    bool vertices = d->vgeom;
+    for (const TileTables &x : d->ts_x) {
+        if (!x.ok) return ANUGA_OK;
+        vertices = vertices && x.vertices;
+    }
+    TileTables a;
+    const TileTables *all = &d->ts_x[0];
+    // scenarios start on whole tiles; the padding behind them has no neighbours
+    if (d->S > 1) {
+        a.stencil.assign(d->N, 0x3fffffffu);
+        a.across.assign(d->N, 0u);
+        if (vertices) a.nodes.assign(d->N, 0u);
+        for (int s = 0; s < d->S; s++) {
+            const TileTables &x = d->ts_x[s];
+            auto join = [](auto &to, const auto &from) {
+                to.insert(to.end(), from.begin(), from.end());
+            };
+            auto offsets = [](std::vector<int> &to, const std::vector<int> &from, size_t base) {
+                for (int v : from) to.push_back((int)(v + base));
+            };
+            offsets(a.cstart, x.cstart, a.cell.size());
+            offsets(a.hstart, x.hstart, a.hstencil.size());
+            offsets(a.estart, x.estart, a.edge.size());
+            offsets(a.esplit, x.esplit, a.edge.size());
+            join(a.cell, x.cell);
+            join(a.hstencil, x.hstencil);
+            join(a.hcell, x.hcell);
+            join(a.edge, x.edge);
+            std::copy(x.stencil.begin(), x.stencil.end(), a.stencil.begin() + d->kbeg[s]);
+            std::copy(x.across.begin(), x.across.end(), a.across.begin() + d->kbeg[s]);
+            if (vertices) {
+                offsets(a.nstart, x.nstart, a.node.size());
+                join(a.node, x.node);
+                join(a.hnodes, x.hnodes);
+                std::copy(x.nodes.begin(), x.nodes.end(), a.nodes.begin() + d->kbeg[s]);
+            }
+            a.hecap = std::max(a.hecap, x.hecap);
+            a.ncap = std::max(a.ncap, x.ncap);
+        }
+        all = &a;
+    }
+    // one allocation; small tables cross in one copy
+    auto closed = [](std::vector<int> v, size_t end) {   // with the closing offset
+        v.push_back((int)end);
+        return v;
+    };
+    const std::vector<int> cstart = closed(all->cstart, all->cell.size()),
+                           hstart = closed(all->hstart, all->hstencil.size()),
+                           estart = closed(all->estart, all->edge.size()),
+                           nstart = closed(all->nstart, all->node.size());
+    struct Part {
+        const void **dst, *src;
+        size_t bytes, at;
+    };
+    std::vector<Part> parts;
+    size_t total = 0;
+    auto add = [&](auto &dst, const auto &src) {
+        const size_t bytes = src.size() * sizeof(src[0]);
+        parts.push_back({(const void **)&dst, src.data(), bytes, total});
+        total += (bytes + 255) / 256 * 256;
+    };
+    DeTileX x{};
+    add(x.cstart, cstart);
+    add(x.cell, all->cell);
+    add(x.stencil, all->stencil);
+    add(x.across, all->across);
+    add(x.hstart, hstart);
+    add(x.hstencil, all->hstencil);
+    add(x.hcell, all->hcell);
+    add(x.estart, estart);
+    add(x.esplit, all->esplit);
+    add(x.edge, all->edge);
+    if (vertices) {
+        add(x.nstart, nstart);
+        add(x.node, all->node);
+        add(x.nodes, all->nodes);
+        add(x.hnodes, all->hnodes);
+        x.ncap = (all->ncap + 1) & ~1;
+    }
+    char *base = nullptr;
+    HIPCHK(d, dalloc(&base, total));
+    d->tx.cstart = reinterpret_cast<const int *>(base);   // freed with the handle from here on
+    if (total <= (size_t)1 << 22) {
+        std::vector<char> all_bytes(total);
+        for (const Part &q : parts)
+            if (q.bytes) std::memcpy(all_bytes.data() + q.at, q.src, q.bytes);
+        HIPCHK(d, hipMemcpy(base, all_bytes.data(), total, hipMemcpyHostToDevice));
+    } else {
+        for (const Part &q : parts)
+            if (q.bytes) HIPCHK(d, hipMemcpy(base + q.at, q.src, q.bytes, hipMemcpyHostToDevice));
+    }
+    for (const Part &q : parts) *q.dst = base + q.at;
+    // the LDS stride of the halo edges: a multiple of 16, never zero
+    x.hecap = std::max((all->hecap + 15) / 16 * 16, 16);
+    d->tx = x;
+    d->ts_x.clear();
+    d->ts_x.shrink_to_fit();
     return ANUGA_OK;
 }
 
@@ -1320,11 +1619,6 @@ static int upload_tiles(anuga_domain *d)
     }
     if (d->tslot) HIPCHK(d, hipFree(d->tslot));
     d->tslot = nullptr;
-    if (d->testart) HIPCHK(d, hipFree(d->testart));
-    if (d->tesplit) HIPCHK(d, hipFree(d->tesplit));
-    if (d->tedge) HIPCHK(d, hipFree(d->tedge));
-    d->testart = d->tesplit = nullptr;
-    d->tedge = nullptr;
     if ((int)d->ts_hcap.size() != d->S) return ANUGA_OK;
     int hcap = 0;
     for (int s = 0; s < d->S; s++) {
@@ -1332,40 +1626,16 @@ static int upload_tiles(anuga_domain *d)
         hcap = std::max(hcap, d->ts_hcap[s]);
     }
     if (hcap > kMaxHalo) return ANUGA_OK;
-    std::vector<int> start(d->nblocks + 1, 0), halo, estart(d->nblocks + 1, 0),
-        esplit(d->nblocks, 0);
-    std::vector<unsigned> slot(d->N, 0x3fffffffu), edge;
+    std::vector<int> start(d->nblocks + 1, 0), halo;
+    std::vector<unsigned> slot(d->N, 0x3fffffffu);
     int b = 0;
     for (int s = 0; s < d->S; s++) {
-        const int b0 = d->kbeg[s] / DE_BLOCK, nt = (int)d->ts_start[s].size() - 1;
-        for (; b < b0; b++) {
-            start[b] = (int)halo.size();
-            estart[b] = esplit[b] = (int)edge.size();
-        }
-        for (int t = 0; t < nt; t++, b++) {
-            start[b] = (int)halo.size() + d->ts_start[s][t];
-            estart[b] = (int)edge.size() + d->ts_estart[s][t];
-            esplit[b] = (int)edge.size() + d->ts_esplit[s][t];
-        }
+        const int nt = (int)d->ts_start[s].size() - 1;
+        for (int t = 0; t < nt; t++, b++) start[b] = (int)halo.size() + d->ts_start[s][t];
         halo.insert(halo.end(), d->ts_halo[s].begin(), d->ts_halo[s].end());
-        edge.insert(edge.end(), d->ts_edge[s].begin(), d->ts_edge[s].end());
         std::copy(d->ts_slot[s].begin(), d->ts_slot[s].end(), slot.begin() + d->kbeg[s]);
     }
-    for (; b <= d->nblocks; b++) {
-        start[b] = (int)halo.size();
-        estart[b] = (int)edge.size();
-        if (b < d->nblocks) esplit[b] = (int)edge.size();
-    }
-    HIPCHK(d, dalloc(&d->testart, (size_t)d->nblocks + 1));
-    HIPCHK(d, dalloc(&d->tesplit, (size_t)d->nblocks));
-    HIPCHK(d, hipMemcpy(d->tesplit, esplit.data(), d->nblocks * sizeof(int),
-                        hipMemcpyHostToDevice));
-    HIPCHK(d, dalloc(&d->tedge, std::max<size_t>(edge.size(), 1)));
-    HIPCHK(d, hipMemcpy(d->testart, estart.data(), (d->nblocks + 1) * sizeof(int),
-                        hipMemcpyHostToDevice));
-    if (!edge.empty())
-        HIPCHK(d, hipMemcpy(d->tedge, edge.data(), edge.size() * sizeof(unsigned),
-                            hipMemcpyHostToDevice));
+    for (; b <= d->nblocks; b++) start[b] = (int)halo.size();
     HIPCHK(d, dalloc(&d->tstart, (size_t)d->nblocks + 1));
     HIPCHK(d, dalloc(&d->thalo, halo.size()));
     HIPCHK(d, dalloc(&d->tslot, (size_t)d->N));
@@ -1376,7 +1646,24 @@ static int upload_tiles(anuga_domain *d)
     HIPCHK(d, hipMemcpy(d->tslot, slot.data(), d->N * sizeof(unsigned), hipMemcpyHostToDevice));
     // the LDS stride: a multiple of 32, never zero
     d->hcap = std::max((hcap + 31) / 32 * 32, 32);
-    return ANUGA_OK;
+    return upload_tile_tables(d);
+}
+
+// Whether check(lo, hi) holds for ranges that cover [0, N), several threads at
+// once for larger N.
+template <class F>
+static bool all_of_ranges(int64_t N, F check)
+{
+    const int64_t per = 8192;
+    const int T = (int)std::max<int64_t>(
+        1, std::min<int64_t>({(int64_t)std::thread::hardware_concurrency(), 16, N / per}));
+    std::vector<char> ok(T, 0);
+    std::vector<std::thread> th;
+    auto work = [&](int i) { ok[i] = check(N * i / T, N * (i + 1) / T); };
+    for (int i = 1; i < T; i++) th.emplace_back(work, i);
+    work(0);
+    for (auto &t : th) t.join();
+    return std::all_of(ok.begin(), ok.end(), [](char c) { return c != 0; });
 }
 
 // Upload the validated mesh of scenario s (its own triangle and boundary
@@ -1385,11 +1672,10 @@ static int upload_tiles(anuga_domain *d)
 // neighbour's and the lengths are equal (true of normals and lengths formed
 // from the two vertices, general_mesh.py:202-232), so that one side's flux
 // gives the other's by negation.
-static bool mesh_mirrors(const anuga_mesh *mesh)
+static bool mesh_mirrors(const anuga_mesh *mesh, int64_t lo, int64_t hi)
 {
-    const int64_t N = mesh->number_of_elements;
     const double *nrm = mesh->normals, *el = mesh->edgelengths;
-    for (int64_t k = 0; k < N; k++)
+    for (int64_t k = lo; k < hi; k++)
         for (int i = 0; i < 3; i++) {
             const int64_t n = mesh->neighbours[3 * k + i];
             if (n < 0) continue;
@@ -1404,13 +1690,12 @@ static bool mesh_mirrors(const anuga_mesh *mesh)
 
 // Whether the mesh's edge midpoints, normals and lengths are the ones
 // general_mesh.py forms from its vertex coordinates (:202-232, :599-626),
-// bit for bit, so that the kernels may form them from the vertices.
-static bool geometry_from_vertices(const anuga_mesh *mesh)
+// bit for bit, on triangles [lo, hi), so that the kernels may form them from the vertices.
+static bool geometry_from_vertices(const anuga_mesh *mesh, int64_t lo, int64_t hi)
 {
     const double *V = mesh->vertex_coordinates;
-    if (!V) return false;
     const double *nrm = mesh->normals, *el = mesh->edgelengths, *em = mesh->edge_coordinates;
-    for (int64_t k = 0; k < mesh->number_of_elements; k++) {
+    for (int64_t k = lo; k < hi; k++) {
         const double *v = V + 6 * k;
         for (int i = 0; i < 3; i++) {
             const int a = (i + 1) % 3, b = (i + 2) % 3;
@@ -1431,12 +1716,18 @@ static bool geometry_from_vertices(const anuga_mesh *mesh)
 // coordinates, vx).
 static void check_vertex_geometry(anuga_domain *d, const anuga_mesh *mesh)
 {
-    if (!geometry_from_vertices(mesh)) d->vgeom = false;
+    if (!mesh->vertex_coordinates ||
+        !all_of_ranges(mesh->number_of_elements, [&](int64_t lo, int64_t hi) {
+            return geometry_from_vertices(mesh, lo, hi);
+        }))
+        d->vgeom = false;
 }
 
 static int upload_mesh(anuga_domain *d, int s, const anuga_mesh *mesh)
 {
-    if (!mesh_mirrors(mesh)) d->mirror = false;
+    if (!all_of_ranges(mesh->number_of_elements,
+                       [&](int64_t lo, int64_t hi) { return mesh_mirrors(mesh, lo, hi); }))
+        d->mirror = false;
     const int N = d->ntri[s], kb = d->kbeg[s], mb = d->mbeg[s];
     const int64_t *nbr = mesh->neighbours, *nbe = mesh->neighbour_edges;
     const int64_t *sur = mesh->surrogate_neighbours, *nob = mesh->number_of_boundaries;
@@ -1473,49 +1764,52 @@ static int upload_mesh(anuga_domain *d, int s, const anuga_mesh *mesh)
         const size_t NN = d->N;
         std::vector<DeGeoX64> gx(N);
         std::vector<double> a(3 * (size_t)N), b(3 * (size_t)N), c(3 * (size_t)N), r(N);
-        for (int p = 0; p < N; p++) {
-            const int64_t k = perm[p];
-            for (int i = 0; i < 3; i++) {
-                // xv - x and yv - y exactly as sw_domain_orig.c:2130-2135 forms them
-                gx[p].dxv[i] = em[6 * k + 2 * i] - cen[2 * k];
-                gx[p].dyv[i] = em[6 * k + 2 * i + 1] - cen[2 * k + 1];
-                a[(size_t)i * N + p] = nrm[6 * k + 2 * i];
-                b[(size_t)i * N + p] = nrm[6 * k + 2 * i + 1];
-                c[(size_t)i * N + p] = el[3 * k + i];
+        all_of_ranges(N, [&](int64_t lo, int64_t hi) {
+            for (int64_t p = lo; p < hi; p++) {
+                const int64_t k = perm[p];
+                for (int i = 0; i < 3; i++) {
+                    // xv - x and yv - y exactly as sw_domain_orig.c:2130-2135 forms them
+                    gx[p].dxv[i] = em[6 * k + 2 * i] - cen[2 * k];
+                    gx[p].dyv[i] = em[6 * k + 2 * i + 1] - cen[2 * k + 1];
+                    a[(size_t)i * N + p] = nrm[6 * k + 2 * i];
+                    b[(size_t)i * N + p] = nrm[6 * k + 2 * i + 1];
+                    c[(size_t)i * N + p] = el[3 * k + i];
+                }
+                r[p] = mesh->radii[k];
+                // the gradient's auxiliary geometry, in the kernel's operation order
+                // (this file is compiled without floating-point contraction)
+                double *g = gx[p].aux;
+                for (int j = 0; j < 6; j++) g[j] = 0.0;
+                if (nob[k] <= 1) {
+                    int64_t s[3];
+                    for (int i = 0; i < 3; i++) s[i] = sur[3 * k + i];
+                    const double dx1 = cen[2 * s[1]] - cen[2 * s[0]];
+                    const double dx2 = cen[2 * s[2]] - cen[2 * s[0]];
+                    const double dy1 = cen[2 * s[1] + 1] - cen[2 * s[0] + 1];
+                    const double dy2 = cen[2 * s[2] + 1] - cen[2 * s[0] + 1];
+                    const double area2 = dy2 * dx1 - dy1 * dx2;
+                    g[0] = dx1;
+                    g[1] = dx2;
+                    g[2] = dy1;
+                    g[3] = dy2;
+                    g[4] = area2;
+                    g[5] = 1.0 / area2;
+                } else if (nob[k] == 2) {
+                    int64_t s1 = -1;
+                    for (int i = 0; i < 3 && s1 < 0; i++)
+                        if (nbr[3 * k + i] >= 0) s1 = nbr[3 * k + i];
+                    const double dx1 = cen[2 * s1] - cen[2 * k];
+                    const double dy1 = cen[2 * s1 + 1] - cen[2 * k + 1];
+                    const double area2 = dx1 * dx1 + dy1 * dy1;
+                    double dx2 = 1.0 / area2;
+                    const double dy2 = dx2 * dy1;
+                    dx2 *= dx1;
+                    g[1] = dx2;
+                    g[3] = dy2;
+                }
             }
-            r[p] = mesh->radii[k];
-            // the gradient's auxiliary geometry, in the kernel's operation order
-            // (this file is compiled without floating-point contraction)
-            double *g = gx[p].aux;
-            for (int j = 0; j < 6; j++) g[j] = 0.0;
-            if (nob[k] <= 1) {
-                int64_t s[3];
-                for (int i = 0; i < 3; i++) s[i] = sur[3 * k + i];
-                const double dx1 = cen[2 * s[1]] - cen[2 * s[0]];
-                const double dx2 = cen[2 * s[2]] - cen[2 * s[0]];
-                const double dy1 = cen[2 * s[1] + 1] - cen[2 * s[0] + 1];
-                const double dy2 = cen[2 * s[2] + 1] - cen[2 * s[0] + 1];
-                const double area2 = dy2 * dx1 - dy1 * dx2;
-                g[0] = dx1;
-                g[1] = dx2;
-                g[2] = dy1;
-                g[3] = dy2;
-                g[4] = area2;
-                g[5] = 1.0 / area2;
-            } else if (nob[k] == 2) {
-                int64_t s1 = -1;
-                for (int i = 0; i < 3 && s1 < 0; i++)
-                    if (nbr[3 * k + i] >= 0) s1 = nbr[3 * k + i];
-                const double dx1 = cen[2 * s1] - cen[2 * k];
-                const double dy1 = cen[2 * s1 + 1] - cen[2 * k + 1];
-                const double area2 = dx1 * dx1 + dy1 * dy1;
-                double dx2 = 1.0 / area2;
-                const double dy2 = dx2 * dy1;
-                dx2 *= dx1;
-                g[1] = dx2;
-                g[3] = dy2;
-            }
-        }
+            return true;
+        });
         HIPCHK(d, hipMemcpy((DeGeoX64 *)d->gx + kb, gx.data(), N * sizeof(DeGeoX64),
                             hipMemcpyHostToDevice));
         for (int i = 0; i < 3; i++) {
@@ -1551,17 +1845,22 @@ static int upload_mesh(anuga_domain *d, int s, const anuga_mesh *mesh)
     std::copy(perm.begin(), perm.end(), d->perm.begin() + kb);
     if (!d->caller) HIPCHK(d, dalloc(&d->caller, (size_t)d->N));
     HIPCHK(d, hipMemcpy(d->caller + kb, perm.data(), N * sizeof(int), hipMemcpyHostToDevice));
+    std::vector<double> hv;
     if (mesh->vertex_coordinates && !d->mixed) {
-        std::vector<double> hv(6 * (size_t)N);
-        for (int p = 0; p < N; p++)
-            for (int j = 0; j < 6; j++) hv[6 * (size_t)p + j] = mesh->vertex_coordinates[6 * (size_t)perm[p] + j];
+        hv.resize(6 * (size_t)N);
+        all_of_ranges(N, [&](int64_t lo, int64_t hi) {
+            for (int64_t p = lo; p < hi; p++)
+                std::memcpy(&hv[6 * p], mesh->vertex_coordinates + 6 * (int64_t)perm[p],
+                            6 * sizeof(double));
+            return true;
+        });
         if (!d->vx) HIPCHK(d, dalloc(&d->vx, 6 * (size_t)d->N));
         HIPCHK(d, hipMemcpy(d->vx + 6 * (size_t)kb, hv.data(), 6 * (size_t)N * sizeof(double),
                             hipMemcpyHostToDevice));
     }
     if (d->vgeom) check_vertex_geometry(d, mesh);
     if (d->P.reorder == 2) {
-        int rc = scenario_tiles(d, s, hn);
+        int rc = scenario_tiles(d, s, hn, hv.empty() ? nullptr : hv.data());
         if (rc) return rc;
     }
     if (!d->mesh_set[s]) {
@@ -1983,7 +2282,7 @@ void anuga_destroy(anuga_domain *d)
                     d->scen, d->tstart, d->thalo, d->tslot, d->rw, d->rwd, d->caller, d->vx, d->node_start, d->node_tri, d->iperm_dev,
                     d->out_f32, d->gtri, d->gtimes, d->gvals, d->sub_idx, d->sub_val, d->eta, d->A, d->B, d->C, d->E, d->flags,
                     d->ex[0], d->ex[1], d->ex[2], d->bkind, d->bval, d->part, d->chunks, d->ctl, d->dsetup,
-                    d->hist, d->si[0], d->si[1], d->testart, d->tesplit, d->tedge,
+                    d->hist, d->si[0], d->si[1],
                     d->lts.e0, d->lts.e1, d->lts.e2, d->lts.pg, d->lts.et, d->lts.fuf,
                     d->lts.acf, d->lts.tmin, d->lts.unf};
     for (void *p : ptrs)
@@ -1993,6 +2292,7 @@ void anuga_destroy(anuga_domain *d)
         for (auto e : d->timers[t].start) hipEventDestroy(e);
         for (auto e : d->timers[t].stop) hipEventDestroy(e);
     }
+    free_tile_tables(d);
     delete d->adj;
     for (RateOp &o : d->ops) {
         void *q[] = {o.idx, o.rate, o.influx};
@@ -3206,6 +3506,41 @@ int anuga_tile_halos(int64_t N, const int32_t *nb, int64_t *start, int64_t halo_
     for (size_t b = 0; b < st.size(); b++) start[b] = st[b];
     for (size_t q = 0; q < h.size(); q++) halo[q] = h[q];
     for (int64_t k = 0; k < N; k++) slot[k] = sl[k];
+    return ANUGA_OK;
+}
+
+int anuga_tile_tables(int64_t N, const int32_t *nb, const double *vertex_coordinates,
+                      const anuga_tile_tables_out *o)
+{
+    if (N < 1 || N >= (int64_t(1) << 29) || !nb || !o) return ANUGA_E_ARG;
+    std::vector<int4> hn(N);
+    for (int64_t k = 0; k < N; k++) {
+        hn[k] = make_int4(nb[3 * k], nb[3 * k + 1], nb[3 * k + 2], 0);
+        for (int i = 0; i < 3; i++)
+            if (nb[3 * k + i] >= 0 && (nb[3 * k + i] >> 2) >= N) return ANUGA_E_ARG;
+    }
+    TileTables x;
+    scenario_tables((int)N, hn.data(), vertex_coordinates, x);
+    if (!x.ok) return ANUGA_E_STATE;
+    auto put = [](auto *to, const auto &from, size_t cap) {
+        if (!to || from.size() > cap) return false;
+        std::copy(from.begin(), from.end(), to);
+        return true;
+    };
+    const size_t nt = x.cstart.size(), cap = (size_t)o->capacity;
+    bool fits = put(o->stencil, x.stencil, N) && put(o->across, x.across, N) &&
+                put(o->cstart, x.cstart, nt) && put(o->cell, x.cell, cap) &&
+                put(o->hstart, x.hstart, nt) && put(o->hstencil, x.hstencil, cap) &&
+                put(o->hcell, x.hcell, cap) && put(o->estart, x.estart, nt) &&
+                put(o->esplit, x.esplit, nt) && put(o->edge, x.edge, cap);
+    if (fits && vertex_coordinates) {
+        fits = put(o->nodes, x.nodes, N) && put(o->hnodes, x.hnodes, cap) &&
+               put(o->nstart, x.nstart, nt) && x.node.size() <= cap && o->node;
+        if (fits) std::memcpy(o->node, x.node.data(), x.node.size() * sizeof(double2));
+    }
+    if (!fits) return ANUGA_E_ARG;
+    const size_t n[4] = {x.cell.size(), x.hstencil.size(), x.edge.size(), x.node.size()};
+    for (int i = 0; i < 4; i++) o->sizes[i] = (int64_t)n[i];
     return ANUGA_OK;
 }
 

@@ -87,23 +87,14 @@ struct DeExtrap {
 // general_mesh.py forms the arrays the reference's extrapolation reads
 // (:599-626 edge midpoints 0.5 (Va + Vb); sw_domain_orig.c:2112-2135 their
 // offsets from the stored centroid).
-// The three vertices of a triangle (its row of the per-triangle vertex
-// coordinates, the same doubles as the nodes they come from).
 struct DeVerts {
     double2 v0, v1, v2;
 };
 
-__device__ __forceinline__ DeVerts de_load_verts(const DeMesh &m, int k)
-{
-    const double2 *r = reinterpret_cast<const double2 *>(m.vx) + 3 * (size_t)k;
-    return DeVerts{r[0], r[1], r[2]};
-}
-
-__device__ __forceinline__ void de_vertex_offsets(const DeMesh &m, int k, const DeVerts &w,
+__device__ __forceinline__ void de_vertex_offsets(const double2 c, const DeVerts &w,
                                                   double dxv[3], double dyv[3])
 {
     const double2 v0 = w.v0, v1 = w.v1, v2 = w.v2;
-    const double2 c = m.cen[k];
     dxv[0] = 0.5 * (v1.x + v2.x) - c.x;
     dyv[0] = 0.5 * (v1.y + v2.y) - c.y;
     dxv[1] = 0.5 * (v2.x + v0.x) - c.x;
@@ -112,28 +103,191 @@ __device__ __forceinline__ void de_vertex_offsets(const DeMesh &m, int k, const 
     dyv[2] = 0.5 * (v0.y + v1.y) - c.y;
 }
 
-// Outward normal and length of edge i of triangle k from its vertices
-// (general_mesh.py:202-232: the edge opposite vertex i, (x, y) =
-// V[i+2] - V[i+1], l = sqrt(x^2 + y^2), normal (y / l, -(x / l))).
-__device__ __forceinline__ void de_vertex_normal(const DeMesh &m, int k, int i, double &n1,
+// Outward normal and length of an edge from va to vb (general_mesh.py:202-232:
+// of the edge opposite vertex i, (x, y) = V[i+2] - V[i+1],
+// l = sqrt(x^2 + y^2), normal (y / l, -(x / l))).
+__device__ __forceinline__ void de_vertex_normal(const double2 va, const double2 vb, double &n1,
                                                  double &n2, double &len)
 {
-    const double2 *r = reinterpret_cast<const double2 *>(m.vx) + 3 * (size_t)k;
-    const int a = i == 2 ? 0 : i + 1, b = i == 0 ? 2 : i - 1;
-    const double2 va = r[a], vb = r[b];
     const double xn = vb.x - va.x, yn = vb.y - va.y;
     len = sqrt(xn * xn + yn * yn);
     n1 = yn / len;
     n2 = -(xn / len);
 }
 
-// vk, qk, tvk: triangle k's neighbour record, state and vertices (VG),
-// loaded by the caller
-template <class T, bool VG = false>
+// Edge offsets and the gradient's auxiliary geometry of triangle k from the
+// stored record: the six numbers of DeGeoX64 (FP64), or formed from the FP32
+// surrogate offsets.
+template <class T>
+struct DeStoredGeo {
+    typename DeGeo<T>::X g;
+    __device__ __forceinline__ DeStoredGeo(const DeMesh &m, int k, T dxv[3], T dyv[3])
+        : g(static_cast<const typename DeGeo<T>::X *>(m.gx)[k])
+    {
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            dxv[i] = g.dxv[i];
+            dyv[i] = g.dyv[i];
+        }
+    }
+    __device__ __forceinline__ void aux(T &dx1, T &dx2, T &dy1, T &dy2, T &area2, T &inv) const
+    {
+        if constexpr (sizeof(T) == 8) {
+            dx1 = g.aux[0];
+            dx2 = g.aux[1];
+            dy1 = g.aux[2];
+            dy2 = g.aux[3];
+            area2 = g.aux[4];
+            inv = g.aux[5];
+        } else {
+            dx1 = g.rx[1] - g.rx[0];
+            dx2 = g.rx[2] - g.rx[0];
+            dy1 = g.ry[1] - g.ry[0];
+            dy2 = g.ry[2] - g.ry[0];
+            area2 = dy2 * dx1 - dy1 * dx2;
+            inv = de_rcp(area2);
+        }
+    }
+    __device__ __forceinline__ void line(bool e0, bool e1, T &dx2, T &dy2) const
+    {
+        if constexpr (sizeof(T) == 8) {
+            dx2 = g.aux[1];
+            dy2 = g.aux[3];
+        } else {
+            // selects on named copies: a select between members would load
+            // from a selected address, so the record would sit in scratch
+            const T x0 = g.rx[0], x1 = g.rx[1], x2 = g.rx[2];
+            const T y0 = g.ry[0], y1 = g.ry[1], y2 = g.ry[2];
+            const T dx1 = e0 ? x0 : (e1 ? x1 : x2);
+            const T dy1 = e0 ? y0 : (e1 ? y1 : y2);
+            const T area2 = dx1 * dx1 + dy1 * dy1;
+            dx2 = de_rcp(area2);
+            dy2 = dx2 * dy1;
+            dx2 *= dx1;
+        }
+    }
+};
+
+// The same from the centroids: the surrogate centroids c0, c1, c2 (ck, its
+// own, where an edge is a boundary edge).
+struct DeCentroidGeo {
+    double2 ck, c0, c1, c2;
+    // the surrogate centroids' triangle (sw_domain_orig.c:2130-2160)
+    __device__ __forceinline__ void aux(double &dx1, double &dx2, double &dy1, double &dy2,
+                                        double &area2, double &inv) const
+    {
+        dx1 = c1.x - c0.x;
+        dx2 = c2.x - c0.x;
+        dy1 = c1.y - c0.y;
+        dy2 = c2.y - c0.y;
+        area2 = dy2 * dx1 - dy1 * dx2;
+        inv = 1.0 / area2;
+    }
+    // toward the one interior neighbour (sw_domain_orig.c:2421-2450)
+    __device__ __forceinline__ void line(bool e0, bool e1, double &dx2, double &dy2) const
+    {
+        const double x0 = c0.x, x1 = c1.x, x2 = c2.x, y0 = c0.y, y1 = c1.y, y2 = c2.y;
+        const double cx = e0 ? x0 : (e1 ? x1 : x2), cy = e0 ? y0 : (e1 ? y1 : y2);
+        const double ddx = cx - ck.x, ddy = cy - ck.y;
+        const double a2 = ddx * ddx + ddy * ddy;
+        dx2 = 1.0 / a2;
+        dy2 = dx2 * ddy;
+        dx2 *= ddx;
+    }
+};
+
+// The limited jumps of a triangle whose own cell is x.c, from its surrogate
+// neighbours' cells; v, nbound: its neighbour record.
+template <class T, class Geo>
+__device__ __forceinline__ void de_extrap_jumps(const DeParams &p, const int v[3], int nbound,
+                                                const DeCell nb[3], const T dxv[3],
+                                                const T dyv[3], const Geo &geo, int *err,
+                                                DeExtrap<T> &x)
+{
+    const double mah = p.mah;
+    const DeCell &c = x.c;
+    T(&jw)[3] = x.jw, (&jh)[3] = x.jh, (&ju)[3] = x.ju, (&jv)[3] = x.jv;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        jw[i] = T(0.0);
+        jh[i] = T(0.0);
+        ju[i] = T(0.0);
+        jv[i] = T(0.0);
+    }
+    bool &constant = x.constant, &gw = x.gw, &gu = x.gu, &gv = x.gv;
+    constant = (nbound == 3);
+    gw = gu = gv = true;   // false: beta == 0, edge = centroid value
+    if (nbound <= 1) {
+        T dx1, dx2, dy1, dy2, area2, inv_area2;
+        geo.aux(dx1, dx2, dy1, dy2, area2, inv_area2);
+        if (area2 <= T(0.0)) {
+            constant = true;
+        } else {
+            const T a_tmp = T(0.3), b_tmp = T(0.1);
+            const T c_tmp = T(1.0) / (a_tmp - b_tmp);
+            const T d_tmp = T(1.0) - (c_tmp * a_tmp);
+            const T tmah = T(mah);
+            const T hc = T(c.h), h0 = T(nb[0].h), h1 = T(nb[1].h), h2 = T(nb[2].h);
+            const T hmin = fmin(fmin(h0, fmin(h1, h2)), hc);
+            const T hmax = fmax(fmax(h0, fmax(h1, h2)), hc);
+            T hfactor = fmax(T(0.0), fmin(de_div(c_tmp * fmax(hmin, T(0.0)), fmax(hc, T(1.0e-06))) + d_tmp,
+                                          fmin(de_div(c_tmp * fmax(hc, T(0.0)), fmax(hmax, T(1.0e-06))) + d_tmp,
+                                               T(1.0))));
+            hfactor = fmin(de_div(T(1.2) * fmax(hmin - tmah, T(0.0)), fmax(hmin, T(0.0)) + T(1.0) * tmah),
+                           hfactor);
+
+            T beta = T(p.bwd) + (T(p.bw) - T(p.bwd)) * hfactor;
+            gw = beta > T(0.0);
+            if (gw) {
+                de_aux_jumps<T>(c.w, nb[0].w, nb[1].w, nb[2].w, dx1, dx2, dy1, dy2, inv_area2,
+                                dxv, dyv, beta, jw);
+                de_aux_jumps<T>(c.h, nb[0].h, nb[1].h, nb[2].h, dx1, dx2, dy1, dy2, inv_area2,
+                                dxv, dyv, beta, jh);
+            }
+            beta = T(p.buhd) + (T(p.buh) - T(p.buhd)) * hfactor;
+            gu = beta > T(0.0);
+            if (gu)
+                de_aux_jumps<T>(c.u, nb[0].u, nb[1].u, nb[2].u, dx1, dx2, dy1, dy2, inv_area2,
+                                dxv, dyv, beta, ju);
+            beta = T(p.bvhd) + (T(p.bvh) - T(p.bvhd)) * hfactor;
+            gv = beta > T(0.0);
+            if (gv)
+                de_aux_jumps<T>(c.v, nb[0].v, nb[1].v, nb[2].v, dx1, dx2, dy1, dy2, inv_area2,
+                                dxv, dyv, beta, jv);
+        }
+    } else if (nbound == 2) {
+        // the first edge whose surrogate is not k itself (sw_domain_orig.c:2421-2439)
+        // selects rather than indexing, so the register arrays stay in registers
+        const bool e0 = v[0] >= 0, e1 = v[1] >= 0, e2 = v[2] >= 0;
+        if (!(e0 || e1 || e2)) {
+            atomicOr(err, DE_ERR_NO_NEIGHBOUR);
+            constant = true;
+        } else {
+            // field-wise selects on named copies: indexing the array here
+            // would place it in private (scratch) memory
+            const DeCell a0 = nb[0], a1 = nb[1], a2 = nb[2];
+            DeCell n1;
+            n1.w = e0 ? a0.w : (e1 ? a1.w : a2.w);
+            n1.h = e0 ? a0.h : (e1 ? a1.h : a2.h);
+            n1.u = e0 ? a0.u : (e1 ? a1.u : a2.u);
+            n1.v = e0 ? a0.v : (e1 ? a1.v : a2.v);
+            T dx2, dy2;
+            geo.line(e0, e1, dx2, dy2);
+            const T bw = T(p.bw);
+            de_line_jumps<T>(c.w, n1.w, dx2, dy2, dxv, dyv, bw, jw);
+            de_line_jumps<T>(c.h, n1.h, dx2, dy2, dxv, dyv, bw, jh);
+            de_line_jumps<T>(c.u, n1.u, dx2, dy2, dxv, dyv, bw, ju);
+            de_line_jumps<T>(c.v, n1.v, dx2, dy2, dxv, dyv, bw, jv);
+        }
+    }
+}
+
+// The whole extrapolation of triangle k, its neighbours gathered from memory.
+// vk, qk: its neighbour record and state, loaded by the caller.
+template <class T>
 __device__ __forceinline__ void de_extrap_cell(const DeMesh &m, const DeParams &p,
                                                const DeQ *__restrict__ q, int k, int4 vk,
-                                               DeQ qk, const DeVerts &tvk, int *err,
-                                               DeExtrap<T> &x)
+                                               DeQ qk, int *err, DeExtrap<T> &x)
 {
     const double mah = p.mah;
     const int v[3] = {vk.x, vk.y, vk.z};
@@ -202,145 +356,19 @@ __device__ __forceinline__ void de_extrap_cell(const DeMesh &m, const DeParams &
         }
     }
 
-    typename DeGeo<T>::X gx;
-    T dxv[3], dyv[3];
-    if constexpr (VG) {
-        de_vertex_offsets(m, k, tvk, dxv, dyv);
-    } else {
-        gx = static_cast<const typename DeGeo<T>::X *>(m.gx)[k];
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-            dxv[i] = gx.dxv[i];
-            dyv[i] = gx.dyv[i];
-        }
-    }
     // limited jumps from the centroid to the edges, per quantity
-    T(&jw)[3] = x.jw, (&jh)[3] = x.jh, (&ju)[3] = x.ju, (&jv)[3] = x.jv;
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        jw[i] = T(0.0);
-        jh[i] = T(0.0);
-        ju[i] = T(0.0);
-        jv[i] = T(0.0);
-    }
-    bool &constant = x.constant, &gw = x.gw, &gu = x.gu, &gv = x.gv;
-    constant = (nbound == 3);
-    gw = gu = gv = true;   // false: beta == 0, edge = centroid value
-    if (nbound <= 1) {
-        T dx1, dx2, dy1, dy2, area2, inv_area2;
-        if constexpr (VG) {
-            // the surrogate centroids' triangle (sw_domain_orig.c:2130-2160)
-            const double2 c0 = m.cen[sur[0]], c1 = m.cen[sur[1]], c2 = m.cen[sur[2]];
-            dx1 = c1.x - c0.x;
-            dx2 = c2.x - c0.x;
-            dy1 = c1.y - c0.y;
-            dy2 = c2.y - c0.y;
-            area2 = dy2 * dx1 - dy1 * dx2;
-            inv_area2 = 1.0 / area2;
-        } else if constexpr (sizeof(T) == 8) {
-            dx1 = gx.aux[0];
-            dx2 = gx.aux[1];
-            dy1 = gx.aux[2];
-            dy2 = gx.aux[3];
-            area2 = gx.aux[4];
-            inv_area2 = gx.aux[5];
-        } else {
-            dx1 = gx.rx[1] - gx.rx[0];
-            dx2 = gx.rx[2] - gx.rx[0];
-            dy1 = gx.ry[1] - gx.ry[0];
-            dy2 = gx.ry[2] - gx.ry[0];
-            area2 = dy2 * dx1 - dy1 * dx2;
-            inv_area2 = de_rcp(area2);
-        }
-        if (area2 <= T(0.0)) {
-            constant = true;
-        } else {
-            const T a_tmp = T(0.3), b_tmp = T(0.1);
-            const T c_tmp = T(1.0) / (a_tmp - b_tmp);
-            const T d_tmp = T(1.0) - (c_tmp * a_tmp);
-            const T tmah = T(mah);
-            const T hc = T(c.h), h0 = T(nb[0].h), h1 = T(nb[1].h), h2 = T(nb[2].h);
-            const T hmin = fmin(fmin(h0, fmin(h1, h2)), hc);
-            const T hmax = fmax(fmax(h0, fmax(h1, h2)), hc);
-            T hfactor = fmax(T(0.0), fmin(de_div(c_tmp * fmax(hmin, T(0.0)), fmax(hc, T(1.0e-06))) + d_tmp,
-                                          fmin(de_div(c_tmp * fmax(hc, T(0.0)), fmax(hmax, T(1.0e-06))) + d_tmp,
-                                               T(1.0))));
-            hfactor = fmin(de_div(T(1.2) * fmax(hmin - tmah, T(0.0)), fmax(hmin, T(0.0)) + T(1.0) * tmah),
-                           hfactor);
-
-            T beta = T(p.bwd) + (T(p.bw) - T(p.bwd)) * hfactor;
-            gw = beta > T(0.0);
-            if (gw) {
-                de_aux_jumps<T>(c.w, nb[0].w, nb[1].w, nb[2].w, dx1, dx2, dy1, dy2, inv_area2,
-                                dxv, dyv, beta, jw);
-                de_aux_jumps<T>(c.h, nb[0].h, nb[1].h, nb[2].h, dx1, dx2, dy1, dy2, inv_area2,
-                                dxv, dyv, beta, jh);
-            }
-            beta = T(p.buhd) + (T(p.buh) - T(p.buhd)) * hfactor;
-            gu = beta > T(0.0);
-            if (gu)
-                de_aux_jumps<T>(c.u, nb[0].u, nb[1].u, nb[2].u, dx1, dx2, dy1, dy2, inv_area2,
-                                dxv, dyv, beta, ju);
-            beta = T(p.bvhd) + (T(p.bvh) - T(p.bvhd)) * hfactor;
-            gv = beta > T(0.0);
-            if (gv)
-                de_aux_jumps<T>(c.v, nb[0].v, nb[1].v, nb[2].v, dx1, dx2, dy1, dy2, inv_area2,
-                                dxv, dyv, beta, jv);
-        }
-    } else if (nbound == 2) {
-        // the first edge whose surrogate is not k itself (sw_domain_orig.c:2421-2439)
-        // selects rather than indexing, so the register arrays stay in registers
-        const bool e0 = v[0] >= 0, e1 = v[1] >= 0, e2 = v[2] >= 0;
-        if (!(e0 || e1 || e2)) {
-            atomicOr(err, DE_ERR_NO_NEIGHBOUR);
-            constant = true;
-        } else {
-            // field-wise selects on named copies: indexing the array here
-            // would place it in private (scratch) memory
-            const DeCell a0 = nb[0], a1 = nb[1], a2 = nb[2];
-            DeCell n1;
-            n1.w = e0 ? a0.w : (e1 ? a1.w : a2.w);
-            n1.h = e0 ? a0.h : (e1 ? a1.h : a2.h);
-            n1.u = e0 ? a0.u : (e1 ? a1.u : a2.u);
-            n1.v = e0 ? a0.v : (e1 ? a1.v : a2.v);
-            T dx2, dy2;
-            if constexpr (VG) {
-                // toward the one interior neighbour (sw_domain_orig.c:2421-2450)
-                const int s1 = e0 ? sur[0] : (e1 ? sur[1] : sur[2]);
-                const double2 cs = m.cen[s1], ck = m.cen[k];
-                const double ddx = cs.x - ck.x, ddy = cs.y - ck.y;
-                const double a2 = ddx * ddx + ddy * ddy;
-                dx2 = 1.0 / a2;
-                dy2 = dx2 * ddy;
-                dx2 *= ddx;
-            } else if constexpr (sizeof(T) == 8) {
-                dx2 = gx.aux[1];
-                dy2 = gx.aux[3];
-            } else {
-                const T dx1 = e0 ? gx.rx[0] : (e1 ? gx.rx[1] : gx.rx[2]);
-                const T dy1 = e0 ? gx.ry[0] : (e1 ? gx.ry[1] : gx.ry[2]);
-                const T area2 = dx1 * dx1 + dy1 * dy1;
-                dx2 = de_rcp(area2);
-                dy2 = dx2 * dy1;
-                dx2 *= dx1;
-            }
-            const T bw = T(p.bw);
-            de_line_jumps<T>(c.w, n1.w, dx2, dy2, dxv, dyv, bw, jw);
-            de_line_jumps<T>(c.h, n1.h, dx2, dy2, dxv, dyv, bw, jh);
-            de_line_jumps<T>(c.u, n1.u, dx2, dy2, dxv, dyv, bw, ju);
-            de_line_jumps<T>(c.v, n1.v, dx2, dy2, dxv, dyv, bw, jv);
-        }
-    }
+    T dxv[3], dyv[3];
+    const DeStoredGeo<T> geo(m, k, dxv, dyv);
+    de_extrap_jumps<T>(p, v, nbound, nb, dxv, dyv, geo, err, x);
 }
 
 // the same, loading triangle k's records
-template <class T, bool VG = false>
+template <class T>
 __device__ __forceinline__ void de_extrap_cell(const DeMesh &m, const DeParams &p,
                                                const DeQ *__restrict__ q, int k, int *err,
                                                DeExtrap<T> &x)
 {
-    const DeVerts tvk = VG ? de_load_verts(m, k) : DeVerts{};
-    de_extrap_cell<T, VG>(m, p, q, k, m.nb[k], q[k], tvk, err, x);
+    de_extrap_cell<T>(m, p, q, k, m.nb[k], q[k], err, x);
 }
 
 // FP64 edge values of edge i (compile-time i, or a select on a run-time one):
@@ -1250,30 +1278,163 @@ __device__ __forceinline__ void de_block_partials(double dtmin, double bflux, do
     }
 }
 
+// the three 10-bit fields of a word
+__device__ __forceinline__ int de_field(unsigned w, int i) { return (int)((w >> (10 * i)) & 1023u); }
+
+// The protected cell of a triangle with state q (sw_domain_orig.c:1245-1276,
+// :2014-2064) before the dry-neighbour test: the velocity of a cell deeper
+// than mah, which that test may still zero.
+__device__ __forceinline__ DeCell de_wet_cell(const DeQ &q, double mah)
+{
+    DeCell c;
+    c.w = de_clamped(q.w, q.z, mah) ? q.z : q.w;
+    c.h = de_height(c.w, q.z);
+    c.u = 0.0;
+    c.v = 0.0;
+    if (c.h > mah) {
+        const double inv = 1.0 / c.h;
+        c.u = q.uh * inv;
+        c.v = q.vh * inv;
+    }
+    return c;
+}
+
+// The cells of a tile in LDS: [w, h, u, v, centroid x, y][2 DE_BLOCK]
+#define DE_XSTRIDE (2 * DE_BLOCK)
+__device__ __forceinline__ void de_put_cell(double *L, int j, const DeCell &v, const double2 &cen)
+{
+    L[j] = v.w;
+    L[DE_XSTRIDE + j] = v.h;
+    L[2 * DE_XSTRIDE + j] = v.u;
+    L[3 * DE_XSTRIDE + j] = v.v;
+    L[4 * DE_XSTRIDE + j] = cen.x;
+    L[5 * DE_XSTRIDE + j] = cen.y;
+}
+
+// What the extrapolation of a triangle reads of the cells: its own after the
+// dry-neighbour test, its surrogate neighbours', and their centroids (VG). v:
+// negative on boundary edges (only the signs are used).
+struct DeStencil {
+    DeCell own, nb[3];
+    double2 ck, c0, c1, c2;
+    int v[3], nbound;
+    bool keep;     // the momentum survives
+};
+
+// The stencil st of the triangle with cell `self` from the cells in LDS, as
+// de_extrap_cell forms it from the records in memory: the same operations on
+// the same values. The triangle's id k (of kp, if given) is read only where
+// it is dry.
+template <bool VG>
+__device__ __forceinline__ void de_read_stencil(const DeMesh &m, const DeParams &p,
+                                                const DeQ *__restrict__ q, const int *kp, int k,
+                                                unsigned st, int self, const double *L,
+                                                DeStencil &x)
+{
+    const double mah = p.mah;
+    x.own.w = L[self];
+    x.own.h = L[DE_XSTRIDE + self];
+    x.own.u = L[2 * DE_XSTRIDE + self];
+    x.own.v = L[3 * DE_XSTRIDE + self];
+    int idx[3];
+    x.nbound = 0;
+    bool dry_k = true;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const int f = de_field(st, i);
+        const bool edge = f == 1023;
+        x.v[i] = edge ? -1 : 0;
+        x.nbound += edge;
+        idx[i] = edge ? self : f;
+        x.nb[i].w = L[idx[i]];
+        x.nb[i].h = L[DE_XSTRIDE + idx[i]];
+        x.nb[i].u = L[2 * DE_XSTRIDE + idx[i]];
+        x.nb[i].v = L[3 * DE_XSTRIDE + idx[i]];
+        dry_k = dry_k && (edge || x.nb[i].h < mah);
+    }
+    if constexpr (VG) {
+        const double *cx = L + 4 * DE_XSTRIDE, *cy = L + 5 * DE_XSTRIDE;
+        x.ck = make_double2(cx[self], cy[self]);
+        x.c0 = make_double2(cx[idx[0]], cy[idx[0]]);
+        x.c1 = make_double2(cx[idx[1]], cy[idx[1]]);
+        x.c2 = make_double2(cx[idx[2]], cy[idx[2]]);
+    }
+    x.keep = x.own.h > mah && !dry_k;
+    if (!x.keep) {
+        x.own.u = x.own.v = 0.0;
+        // a boundary edge's surrogate is the triangle itself
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (x.v[i] < 0) x.nb[i].u = x.nb[i].v = 0.0;
+    }
+    if (x.own.h < mah && x.nbound < 3) {
+        // a wet neighbour keeps its velocity unless all of its own neighbours
+        // are dry; this triangle is one, so the others count only here
+        const int4 vk = m.nb[kp ? *kp : k];
+        const int vn[3] = {vk.x, vk.y, vk.z};
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (vn[i] >= 0 && x.nb[i].h > mah) {
+                const int4 vs = m.nb[vn[i] >> 2];
+                const int vv[3] = {vs.x, vs.y, vs.z};
+                bool dry = true;
+#pragma unroll
+                for (int r = 0; r < 3; r++)
+                    if (vv[r] >= 0) {
+                        const DeQ t = q[vv[r] >> 2];
+                        dry = dry && (de_height(t.w, t.z) < mah);
+                    }
+                if (dry) x.nb[i].u = x.nb[i].v = 0.0;
+            }
+    }
+}
+
+// The extrapolation of a stencil; nd: the nodes of word vi (VG), otherwise the
+// stored record of triangle k.
+template <bool VG>
+__device__ __forceinline__ void de_extrap_stencil(const DeMesh &m, const DeParams &p, int k,
+                                                  const DeStencil &s, const double2 *nd,
+                                                  unsigned vi, int *err, DeExtrap<double> &x)
+{
+    x.c = s.own;
+    double dxv[3], dyv[3];
+    if constexpr (VG) {
+        const DeVerts tv{nd[de_field(vi, 0)], nd[de_field(vi, 1)], nd[de_field(vi, 2)]};
+        de_vertex_offsets(s.ck, tv, dxv, dyv);
+        const DeCentroidGeo geo{s.ck, s.c0, s.c1, s.c2};
+        de_extrap_jumps<double>(p, s.v, s.nbound, s.nb, dxv, dyv, geo, err, x);
+    } else {
+        const DeStoredGeo<double> geo(m, k, dxv, dyv);
+        de_extrap_jumps<double>(p, s.v, s.nbound, s.nb, dxv, dyv, geo, err, x);
+    }
+}
+
 // One listed edge of a tile (de_xflux_e): its flux from the tile triangle's
-// side (the entry's halo bit: the neighbour is in the halo; otherwise in the
-// tile, and its side's pressure term and CFL bound are formed here too),
-// written over the LDS edge values that only this entry reads. The halo bit
-// is read at run time, so a wave can take edges of both kinds in one pass.
+// side, written over the LDS edge values that only this entry reads. he: the
+// halo edge it is (its neighbour in the halo), or negative: the neighbour is
+// in the tile, and its side's pressure term and CFL bound are formed here too.
 template <int SUBSTEP, bool VG>
 __device__ __forceinline__ void de_tile_edge(const DeMesh &m, const DeParams &p, unsigned en,
-                                             int k0, double *lds, double *hl,
-                                             const double *hz, int hcap, double &dtmin)
+                                             int he, int k0, double *lds, double *hl,
+                                             const double *hz, int hecap, const double2 *nd,
+                                             const unsigned *vis, double &dtmin)
 {
     constexpr int Q = 3 * DE_BLOCK;
     const double g = p.g, eps = p.eps;
     const int N = m.N;
     const int ta = DE_TE_T(en), ia = DE_TE_I(en), nb = DE_TE_N(en), jb = DE_TE_J(en);
-    const bool halo = DE_TE_HALO(en);
+    const bool halo = he >= 0;
     const int ka = k0 + ta;
     double *const A = lds + ia * DE_BLOCK + ta;
-    double *const R = halo ? hl + jb * hcap + nb : lds + jb * DE_BLOCK + nb;
-    const int rs = halo ? 3 * hcap : Q;
+    double *const R = halo ? hl + he : lds + jb * DE_BLOCK + nb;
+    const int rs = halo ? hecap : Q;
     const double ql0 = A[0], hle = A[Q], ql1 = A[2 * Q], ql2 = A[3 * Q];
     const double qr0 = R[0], hre = R[rs], qr1 = R[2 * rs], qr2 = R[3 * rs];
     double n1, n2, length;
     if constexpr (VG) {
-        de_vertex_normal(m, ka, ia, n1, n2, length);
+        const unsigned w = vis[ta];
+        const int a = ia == 2 ? 0 : ia + 1, b = ia == 0 ? 2 : ia - 1;
+        de_vertex_normal(nd[de_field(w, a)], nd[de_field(w, b)], n1, n2, length);
     } else {
         n1 = m.nx[ia * N + ka];
         n2 = m.ny[ia * N + ka];
@@ -1318,8 +1479,13 @@ __device__ __forceinline__ void de_tile_edge(const DeMesh &m, const DeParams &p,
 // options: no riverwalls, low_froude 0, flat friction; the mesh's normals and
 // lengths mirror exactly across every interior edge). VG: the geometry is
 // formed from the vertices. Phases, with a barrier after each:
-//  1. every thread extrapolates its triangle into LDS (de_extrap_cell, as
-//     de_xflux);
+//  0. the state of the tile, its halo and the halo's neighbours becomes cells
+//     in LDS (protected stage, depth, velocity, centroid), each formed once,
+//     with the vertices beside them;
+//  1. every thread extrapolates its triangle from the cells (de_extrap_jumps,
+//     as de_xflux), and one thread per halo edge reads that halo triangle's
+//     stencil into registers. The tile's edge values take the cells' place in
+//     LDS, one barrier later;
 //  2. the first waves extrapolate the halo while each thread of the others
 //     evaluates one edge inside the tile, from its lower-numbered side, which
 //     also forms the other side's pressure term (the reference's compute-
@@ -1332,124 +1498,173 @@ __device__ __forceinline__ void de_tile_edge(const DeMesh &m, const DeParams &p,
 //     wave speed identical); boundary edges are evaluated here, from the
 //     untouched edge values.
 // Each listed edge's results overwrite the LDS edge values only it reads.
-// Four waves per SIMD (at most 128 VGPRs), which the LDS allows too.
+//
+// Bound by instruction issue: the SIMDs issue VALU work 70% of the time, four
+// waves each (105 VGPRs; 34 KB of LDS per workgroup allow four workgroups per
+// CU). Against gathering every neighbour's state, centroid and vertices from
+// memory in phases 1 and 2 (4M triangles): 826 -> 403 MB of HBM reads per
+// launch, 960 -> 274 cache accesses and 1548 -> 1436 VALU instructions per
+// wave, 251 -> 212 us (substep 0) and 280 -> 235 us (substep 1). A workgroup
+// of five waves, the fifth for the halo in phase 1, took 410 us: its waves do
+// not spread evenly over four SIMDs, so two workgroups fit a CU instead of
+// four. 128 triangles per tile: 245 us.
 template <int SUBSTEP, bool VG = false>
 __global__ void __launch_bounds__(DE_BLOCK, 4)
 de_xflux_e(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__restrict__ eta,
-           DeTiles tl, DeBoundary bc, unsigned char *__restrict__ flags, double *__restrict__ exw,
+           DeTileX tx, DeBoundary bc, unsigned char *__restrict__ flags, double *__restrict__ exw,
            double *__restrict__ exuh, double *__restrict__ exvh, const DeQ *bk, DeQ *out,
            DeControl *ctl, double *__restrict__ part_dt, double *__restrict__ part_bf,
            double *__restrict__ part_mass, unsigned long long *__restrict__ nneg)
 {
     static_assert(DE_BLOCK >= 128, "the halo and the tile's edges share the workgroup's waves");
-    // [4 quantities][3 edges][DE_BLOCK] tile edge values, [4][3][hcap] halo,
-    // then [2][DE_BLOCK] the tile's centroid depths and beds
-    extern __shared__ double lds[];
+    // [6][2 DE_BLOCK] cells, then in their place [4 quantities][3 edges]
+    // [DE_BLOCK] tile edge values; [4][hecap] halo edge values; [2][DE_BLOCK]
+    // centroid depths and beds; VG: [ncap] nodes, [DE_BLOCK] node words
+    extern __shared__ double2 lds16[];
+    double *const lds = reinterpret_cast<double *>(lds16);
     __shared__ double red_dt[DE_BLOCK / 64], red_bf[DE_BLOCK / 64], red_m[DE_BLOCK / 64];
     const int lb = xcd_block();
     const int N = m.N, t = threadIdx.x;
     const int k0 = lb * DE_BLOCK, k = k0 + t;
-    // phase 1's own records, requested before the control block is read
-    // (bounded by the arrays' length, not yet by the scenario's end)
-    int4 vk1 = make_int4(-1, -1, -1, 3);
-    DeVerts tv1{};
-    DeQ qk1{0.0, 0.0, 0.0, 0.0};
+    const int hecap = tx.hecap;
+    double *const hl = lds + 12 * DE_BLOCK;
+    double *const hz = hl + 4 * hecap;
+    double2 *const nd = reinterpret_cast<double2 *>(hz + 2 * DE_BLOCK);
+    unsigned *const vis = reinterpret_cast<unsigned *>(nd + tx.ncap);
+    const int c0 = tx.cstart[lb], nc = tx.cstart[lb + 1] - c0;
+    const int h0 = tx.hstart[lb], nhe = tx.hstart[lb + 1] - h0;
+    const int e0 = tx.estart[lb], es = tx.esplit[lb], e1 = tx.estart[lb + 1];
+
+    // every record that phases 0 to 3 need, requested before the control block
+    // is read (bounded by the arrays' length, not yet by the scenario's end)
+    const int kc = t < nc ? tx.cell[c0 + t] : 0;
+    DeQ qk{0.0, 0.0, 0.0, 0.0};
+    double2 ck = make_double2(0.0, 0.0);
+    unsigned st = 0x3fffffffu, vi = 0;
     if (k < N) {
-        vk1 = m.nb[k];
-        qk1 = q[k];
-        if (VG) tv1 = de_load_verts(m, k);
+        qk = q[k];
+        ck = m.cen[k];
+        st = tx.stencil[k];
+        if (VG) vi = tx.nodes[k];
     }
-    // the edge-list entries of phases 2 and 3, loaded now so that their
-    // latency hides behind the extrapolation: hw waves take the halo in
-    // phase 2 (at least one wave left for the tile's edges), each thread of
-    // the others one edge inside the tile
-    const int h0 = tl.start[lb], nh = tl.start[lb + 1] - h0;
-    const int e0 = tl.estart[lb], es = tl.esplit[lb], e1 = tl.estart[lb + 1];
-    const int hw = min((nh + 63) >> 6, DE_BLOCK / 64 - 1);
+    double2 node = make_double2(0.0, 0.0);
+    int n0 = 0, nn = 0;
+    if (VG) {
+        n0 = tx.nstart[lb];
+        nn = tx.nstart[lb + 1] - n0;
+        if (t < nn) node = tx.node[n0 + t];
+    }
+    // phase 2: hw waves take the halo (at most one edge to it per thread),
+    // each thread of the others one edge inside the tile
+    const int hw = (nhe + 63) >> 6;
     const int e2 = e0 + t - 64 * hw, e3 = min(es, e0 + DE_BLOCK - 64 * hw) + t;
     const bool has2 = t >= 64 * hw && e2 < es;
-    // phase 2's item: a tile edge, or the first halo triangle of a halo thread
-    const unsigned en2 = has2 ? tl.edge[e2] : (t < nh && t < 64 * hw ? (unsigned)tl.halo[h0 + t] : 0u);
-    const unsigned en3 = e3 < e1 ? tl.edge[e3] : 0u;
+    const bool hal = t < nhe;
+    const unsigned en2 = has2 ? tx.edge[e2] : 0u, en3 = e3 < e1 ? tx.edge[e3] : 0u;
+    unsigned hst = 0, hc = 0, hvi = 0;
+    if (hal) {
+        hst = tx.hstencil[h0 + t];
+        hc = tx.hcell[h0 + t];
+        if (VG) hvi = tx.hnodes[h0 + t];
+    }
+    DeQ qc{0.0, 0.0, 0.0, 0.0};
+    double2 cc = make_double2(0.0, 0.0);
+    if (t < nc) {
+        qc = q[kc];
+        cc = m.cen[kc];
+    }
 
     DeControl *cb = de_ctl(ctl, m.scen, lb);
     if (cb->done) return;
     int *err = &cb->status;
     const double dt = SUBSTEP ? cb->dt : 0.0;
-    const int kend = cb->kend;
-    const int hcap = tl.hcap;
-    double *const hl = lds + 12 * DE_BLOCK;
-    double *const hz = hl + 12 * hcap;
+    const bool on = k < cb->kend;
     double mass = 0.0, dtmin = 1.0e100, bflux = 0.0;
     unsigned fk = 0;
     constexpr int Q = 3 * DE_BLOCK;   // stride between quantities of the tile
-    // phase 1
-    if (k < kend) {
-        DeExtrap<double> x;
-        de_extrap_cell<double, VG>(m, p, q, k, vk1, qk1, tv1, err, x);
-        mass = x.mass;
-        fk = x.flag;
-        flags[k] = (unsigned char)fk;
-        hz[t] = x.c.h;
-        hz[DE_BLOCK + t] = x.z;
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-            double ew, eh, euh, evh;
-            de_edge64(x, i, ew, eh, euh, evh);
-            lds[(0 + i) * DE_BLOCK + t] = ew;
-            lds[(3 + i) * DE_BLOCK + t] = eh;
-            lds[(6 + i) * DE_BLOCK + t] = euh;
-            lds[(9 + i) * DE_BLOCK + t] = evh;
-        }
+
+    // phase 0
+    de_put_cell(lds, t, de_wet_cell(qk, p.mah), ck);
+    hz[DE_BLOCK + t] = qk.z;
+    if (VG) {
+        vis[t] = vi;
+        if (t < nn) nd[t] = node;
+        for (int j = t + DE_BLOCK; j < nn; j += DE_BLOCK) nd[j] = tx.node[n0 + j];
     }
-    // phase 2's records, requested before the barrier: a halo thread's
-    // first triangle's neighbours
-    const bool hal2 = t < nh && t < 64 * hw;
-    int4 rec2 = make_int4(-1, -1, -1, 3);
-    if (hal2) rec2 = m.nb[en2];
+    if (t < nc) de_put_cell(lds, DE_BLOCK + t, de_wet_cell(qc, p.mah), cc);
+    __syncthreads();
+
+    // phase 1
+    double ev[4][3];
+    if (on) {
+        DeStencil s;
+        de_read_stencil<VG>(m, p, q, nullptr, k, st, t, lds, s);
+        const bool clamp = de_clamped(qk.w, qk.z, p.mah);
+        if (clamp) mass = (qk.z - qk.w) * m.area[k];
+        fk = (clamp ? DE_F_CLAMP : 0u) | (s.keep ? DE_F_KEEP : 0u);
+        flags[k] = (unsigned char)fk;
+        hz[t] = s.own.h;
+        DeExtrap<double> x;
+        de_extrap_stencil<VG>(m, p, k, s, nd, vi, err, x);
+#pragma unroll
+        for (int i = 0; i < 3; i++) de_edge64(x, i, ev[0][i], ev[1][i], ev[2][i], ev[3][i]);
+    }
+    DeStencil hs{};
+    int kh = 0;
+    if (hal) {
+        const int *kp = tx.cell + c0 + (int)(hc & 1023u) - DE_BLOCK;
+        if (!VG) kh = *kp;
+        de_read_stencil<VG>(m, p, q, kp, 0, hst, (int)(hc & 1023u), lds, hs);
+    }
+    __syncthreads();
+    // every cell has been read: the edge values take their place
+    if (on) {
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) lds[(3 * r + i) * DE_BLOCK + t] = ev[r][i];
+    }
     __syncthreads();
 
     // phase 2: the halo's extrapolation, and edges inside the tile
-    if (t < 64 * hw) {
-        for (int j = t; j < nh; j += 64 * hw) {
-            DeExtrap<double> x;
-            const int kh = j == t ? (int)en2 : tl.halo[h0 + j];
-            if (j != t) rec2 = m.nb[kh];   // a further halo triangle
-            const DeVerts tvh = VG ? de_load_verts(m, kh) : DeVerts{};
-            de_extrap_cell<double, VG>(m, p, q, kh, rec2, q[kh], tvh, err, x);
+    if (hal) {
+        DeExtrap<double> x;
+        de_extrap_stencil<VG>(m, p, kh, hs, nd, hvi, err, x);
+        // a branch per edge: a run-time choice between the registers of x
+        // would place x in scratch
+        const int jb = (int)(hc >> 10) & 3;
 #pragma unroll
-            for (int i = 0; i < 3; i++) {
+        for (int i = 0; i < 3; i++)
+            if (i == jb) {
                 double ew, eh, euh, evh;
                 de_edge64(x, i, ew, eh, euh, evh);
-                hl[(0 + i) * hcap + j] = ew;
-                hl[(3 + i) * hcap + j] = eh;
-                hl[(6 + i) * hcap + j] = euh;
-                hl[(9 + i) * hcap + j] = evh;
+                hl[t] = ew;
+                hl[hecap + t] = eh;
+                hl[2 * hecap + t] = euh;
+                hl[3 * hecap + t] = evh;
             }
-        }
     } else if (has2) {
-        de_tile_edge<SUBSTEP, VG>(m, p, en2, k0, lds, hl, hz, hcap, dtmin);
+        de_tile_edge<SUBSTEP, VG>(m, p, en2, -1, k0, lds, hl, hz, hecap, nd, vis, dtmin);
     }
     __syncthreads();
 
     // phase 3: the tile's remaining edges, then the edges to the halo
     if (e3 < e1) {
-        de_tile_edge<SUBSTEP, VG>(m, p, en3, k0, lds, hl, hz, hcap, dtmin);
+        de_tile_edge<SUBSTEP, VG>(m, p, en3, e3 - es, k0, lds, hl, hz, hecap, nd, vis, dtmin);
         for (int e = e3 + DE_BLOCK; e < e1; e += DE_BLOCK)
-            de_tile_edge<SUBSTEP, VG>(m, p, tl.edge[e], k0, lds, hl, hz, hcap, dtmin);
+            de_tile_edge<SUBSTEP, VG>(m, p, tx.edge[e], e - es, k0, lds, hl, hz, hecap, nd, vis,
+                                      dtmin);
     }
-    // phase 4's inputs, requested before the barrier (held from the
-    // kernel's start they cost registers in every phase)
-    DeQ qk4{0.0, 0.0, 0.0, 0.0}, bk_k{0.0, 0.0, 0.0, 0.0};
-    int4 vk4 = make_int4(-1, -1, -1, 3);
+    // phase 4's inputs, requested before the barrier (held from the kernel's
+    // start they cost registers in every phase)
+    DeQ q3{0.0, 0.0, 0.0, 0.0}, bk_k{0.0, 0.0, 0.0, 0.0};
     double eta_k = 0.0, area_k = 1.0;
-    unsigned sl_k = 0;
-    if (k < kend) {
-        qk4 = q[k];
-        vk4 = m.nb[k];
+    unsigned ac = 0;
+    if (on) {
+        ac = tx.across[k];
         area_k = m.area[k];
-        sl_k = tl.slot[k];
         if (SUBSTEP) {
+            q3 = q[k];
             eta_k = eta[k];
             bk_k = bk[k];
         }
@@ -1457,39 +1672,32 @@ de_xflux_e(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__rest
     __syncthreads();
 
     // phase 4: each triangle's three edges in local order
-    if (k < kend) {
-        const DeCentroid c = de_centroid(qk4, fk);
-        const int4 vk = vk4;
-        const int v[3] = {vk.x, vk.y, vk.z};
-        const unsigned sl = sl_k;
+    if (on) {
         double sw = 0.0, sx = 0.0, sy = 0.0;
 #pragma unroll
         for (int i = 0; i < 3; i++) {
             double *const A = lds + i * DE_BLOCK + t;
-            if (v[i] < 0) {
+            const int f = de_field(st, i);
+            if (f == 1023) {            // a boundary edge
+                const DeCentroid c = de_centroid(SUBSTEP ? q3 : q[k], fk);
+                const int4 vk = m.nb[k];
+                const int vb = i == 0 ? vk.x : (i == 1 ? vk.y : vk.z);
                 const double hc = de_height(c.w, c.z);
-                de_edge_flux<double, SUBSTEP, false>(m, p, bc, q, flags, N, k, i, v[i], c, hc,
+                de_edge_flux<double, SUBSTEP, false>(m, p, bc, q, flags, N, k, i, vb, c, hc,
                                                      c.z, A[0], A[Q], A[2 * Q], A[3 * Q], 0.0,
                                                      0.0, 0.0, 0.0, sw, sx, sy, bflux, dtmin);
                 continue;
             }
-            const int n = v[i] >> 2, j = v[i] & 3;
-            const unsigned s = (sl >> (10 * i)) & 1023u;
             double a0, a1, a2, b1, b2;
-            if (s != 1023u) {           // to the halo: this side's entry
+            if (f > t) {                // evaluated from this side
                 a0 = A[0];
                 a1 = A[Q];
                 a2 = A[2 * Q];
                 b1 = A[3 * Q];
-                b2 = hl[j * hcap + s];
-            } else if (k < n) {         // evaluated from this side
-                a0 = A[0];
-                a1 = A[Q];
-                a2 = A[2 * Q];
-                b1 = A[3 * Q];
-                b2 = lds[j * DE_BLOCK + (n - k0)];
+                b2 = f >= DE_BLOCK ? hl[(ac >> (6 + 8 * i)) & 255u]
+                                   : lds[((ac >> (2 * i)) & 3u) * DE_BLOCK + f];
             } else {                    // evaluated from the neighbour's side
-                const double *O = lds + j * DE_BLOCK + (n - k0);
+                const double *O = lds + ((ac >> (2 * i)) & 3u) * DE_BLOCK + f;
                 a0 = -O[0];
                 a1 = -O[Q];
                 a2 = -O[2 * Q];
@@ -1511,7 +1719,7 @@ de_xflux_e(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__rest
             exuh[k] = sx;
             exvh[k] = sy;
         } else {
-            const DeQ r = de_advance(c, eta_k, sw, sx, sy, dt, p, err, nneg);
+            const DeQ r = de_advance(de_centroid(q3, fk), eta_k, sw, sx, sy, dt, p, err, nneg);
             out[k] = de_rk_combine<SUBSTEP>(r, bk_k);
         }
     }
@@ -1741,7 +1949,7 @@ de_xflux_mixed(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__
 
     if (k < kend) {
         DeExtrap<float> x;
-        de_extrap_cell<float>(m, p, q, k, vk1, qk1, DeVerts{}, err, x);
+        de_extrap_cell<float>(m, p, q, k, vk1, qk1, err, x);
         mass = x.mass;
         fk = x.flag;
         flags[k] = (unsigned char)fk;

@@ -137,11 +137,13 @@ class Ensemble:
                  nrm=np.ascontiguousarray(mesh.normals), el=np.ascontiguousarray(mesh.edgelengths),
                  rad=np.ascontiguousarray(mesh.radii), area=np.ascontiguousarray(mesh.areas),
                  cen=np.ascontiguousarray(mesh.centroid_coordinates),
-                 em=np.ascontiguousarray(mesh.edge_midpoint_coordinates))
+                 em=np.ascontiguousarray(mesh.edge_midpoint_coordinates),
+                 vx=np.ascontiguousarray(mesh.vertex_coordinates))
         desc = _native.AnugaMesh(mesh.number_of_triangles, mesh.boundary_length,
                                  _ip(k["nb"]), _ip(k["nbe"]), _ip(k["sur"]), _ip(k["nob"]),
                                  _dptr(k["nrm"]), _dptr(k["el"]), _dptr(k["rad"]),
-                                 _dptr(k["area"]), _dptr(k["cen"]), _dptr(k["em"]))
+                                 _dptr(k["area"]), _dptr(k["cen"]), _dptr(k["em"]),
+                                 None if self.precision == "mixed" else _dptr(k["vx"]))
         self._call("anuga_ensemble_set_mesh", int(s), C.byref(desc))
         if keep:
             self._meshes[s] = mesh

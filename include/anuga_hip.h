@@ -476,6 +476,23 @@ int anuga_tile_order(int64_t N, const double *centroids, const int64_t *neighbou
 int anuga_tile_halos(int64_t N, const int32_t *nb, int64_t *start, int64_t halo_cap,
                      int32_t *halo, uint32_t *slot, int64_t *nhalo, int64_t *hcap);
 
+/* The tables of the once-per-edge fused kernel for triangles in internal order
+ * (nb as in anuga_tile_halos; vertex_coordinates (N,3,2), or NULL: no nodes),
+ * host only: what each workgroup reads, one entry per tile in the *start
+ * arrays (their last tile ends at sizes[]: cells, halo edges, edges, nodes).
+ * ANUGA_E_STATE where a tile exceeds the kernel's limits. */
+typedef struct {
+    int64_t capacity;          /* of cell, hstencil, hcell, hnodes, edge; node: pairs */
+    int64_t *sizes;            /* [4] */
+    uint32_t *stencil, *across, *nodes;                     /* [N] */
+    int32_t *cstart, *hstart, *estart, *esplit, *nstart;    /* [tiles] */
+    int32_t *cell;
+    uint32_t *hstencil, *hcell, *hnodes, *edge;
+    double *node;
+} anuga_tile_tables_out;
+int anuga_tile_tables(int64_t N, const int32_t *nb, const double *vertex_coordinates,
+                      const anuga_tile_tables_out *out);
+
 /* The edge lists of the fused kernel that evaluates each edge's flux once,
  * for the same tiles and packed neighbours as anuga_tile_halos: per tile
  * (estart: tiles + 1 offsets), each edge between two tile triangles from its

@@ -1,0 +1,139 @@
+"""The once-per-edge fused kernel's tables (CPU): every cell, node, halo edge
+and listed edge that a workgroup reads, replayed against the mesh, and its LDS
+extents against the launch's. Calls only host-side entry points."""
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from anuga_core_amd import _native
+from anuga_core_amd.mesh import Mesh, graded_square, rectangular, rectangular_cross
+from tests.test_tiles import BLOCK, tile_layout
+
+CELLS, HALO, NODES = BLOCK, min(BLOCK - 64, 256), 384      # DE_XCELLS_MAX, DE_XHALO_MAX, DE_XNODES_MAX
+
+
+def _tables(nb, vertices=None):
+    """The tables of packed neighbours nb [N][3], or None beyond the limits."""
+    N = len(nb)
+    nt = (N + BLOCK - 1) // BLOCK
+    cap = 3 * N + nt * (CELLS + NODES + HALO)
+    u = lambda n: np.zeros(n, np.uint32)  # noqa: E731
+    i = lambda n: np.zeros(n, np.int32)   # noqa: E731
+    a = dict(sizes=np.zeros(4, np.int64), stencil=u(N), across=u(N), nodes=u(N), cstart=i(nt),
+             hstart=i(nt), estart=i(nt), esplit=i(nt), nstart=i(nt), cell=i(cap),
+             hstencil=u(cap), hcell=u(cap), hnodes=u(cap), edge=u(cap), node=np.zeros(2 * cap))
+    fields = dict(_native.TileTables._fields_)
+    t = _native.TileTables(capacity=cap, **{k: v.ctypes.data_as(fields[k]) for k, v in a.items()})
+    vx = None if vertices is None else np.ascontiguousarray(vertices, np.float64)
+    nb = np.ascontiguousarray(nb, np.int32)
+    rc = _native.lib().anuga_tile_tables(
+        N, nb.ctypes.data_as(C.POINTER(C.c_int32)),
+        None if vx is None else vx.ctypes.data_as(C.POINTER(C.c_double)), C.byref(t))
+    if rc:
+        return None
+    for name, end, starts in (("cell", 0, "cstart"), ("hstencil", 1, "hstart"),
+                              ("edge", 2, "estart"), ("node", 3, "nstart")):
+        a[starts] = np.append(a[starts], a["sizes"][end])
+    a["node"] = a["node"].reshape(-1, 2)
+    return a
+
+
+def _field(w, i):
+    return (w.astype(np.int64) >> (10 * i)) & 1023
+
+
+def _replay(nb, a, vertices):
+    N = len(nb)
+    nb = nb.astype(np.int64)
+    for b in range((N + BLOCK - 1) // BLOCK):
+        k0, k1 = b * BLOCK, min(N, (b + 1) * BLOCK)
+        cells = np.full(2 * BLOCK, -1)
+        cells[:k1 - k0] = np.arange(k0, k1)
+        more = a["cell"][a["cstart"][b]:a["cstart"][b + 1]]
+        assert len(more) <= CELLS and len(np.unique(more)) == len(more)
+        assert not np.any((more >= k0) & (more < k1))
+        cells[BLOCK:BLOCK + len(more)] = more
+        es, e0, e1 = a["esplit"][b], a["estart"][b], a["estart"][b + 1]
+        h = slice(a["hstart"][b], a["hstart"][b + 1])
+        nhe = h.stop - h.start
+        assert nhe == e1 - es and nhe <= HALO
+        hcell = a["hcell"][h].astype(np.int64)
+        halo, hj = cells[hcell & 1023], hcell >> 10
+        assert np.all((hcell & 1023) >= BLOCK) and np.all(halo >= 0) and np.all(hj < 3)
+        k = np.arange(k0, k1)
+        for i in range(3):
+            # stencils: the neighbour's cell, 1023 on boundary edges
+            for st, tri in ((a["stencil"][k0:k1], k), (a["hstencil"][h], halo)):
+                f, v = _field(st, i), nb[tri, i]
+                assert np.array_equal(f == 1023, v < 0)
+                inner = v >= 0
+                assert np.array_equal(cells[f[inner]], v[inner] >> 2)
+            # across: the neighbour's edge, and the halo edge that faces it
+            f, v = _field(a["stencil"][k0:k1], i), nb[k, i]
+            ac = a["across"][k0:k1].astype(np.int64)
+            inner = v >= 0
+            assert np.array_equal(((ac >> (2 * i)) & 3)[inner], v[inner] & 3)
+            out = inner & (f >= BLOCK)
+            he = (ac >> (6 + 8 * i)) & 255
+            assert np.all(he[out] < nhe)
+            assert np.array_equal(halo[he[out]], v[out] >> 2)
+            assert np.array_equal(hj[he[out]], v[out] & 3)
+            # one listed entry per halo edge, in the halo edges' order
+            en = a["edge"][es + he[out]].astype(np.int64)
+            assert np.array_equal(en & 1023, k[out] - k0)
+            assert np.all((en >> 10) & 3 == i) and np.all((en >> 12) & 1 == 1)
+        # in-tile edges: each once, from its lower-numbered triangle
+        en = a["edge"][e0:es].astype(np.int64)
+        t, i, n, j = en & 1023, (en >> 10) & 3, (en >> 13) & 1023, (en >> 23) & 3
+        assert np.all((en >> 12) & 1 == 0) and np.all(t < n)
+        assert np.array_equal(nb[k0 + t, i], ((k0 + n) << 2) | j)
+        v = nb[k0:k1]
+        inside = (v >= 0) & ((v >> 2) >= k0) & ((v >> 2) < k1)
+        assert len(np.unique(t * 4 + i)) == len(en) == inside.sum() // 2
+        if vertices is None:
+            continue
+        nd = a["node"][a["nstart"][b]:a["nstart"][b + 1]]
+        assert len(nd) <= NODES and len(np.unique(nd, axis=0)) == len(nd)
+        for c in range(3):
+            assert np.array_equal(nd[_field(a["nodes"][k0:k1], c)], vertices[k0:k1, c])
+            assert np.array_equal(nd[_field(a["hnodes"][h], c)], vertices[halo, c])
+
+
+def _ordered(mesh):
+    nb = tile_layout(mesh)[0]
+    cen = np.ascontiguousarray(mesh.centroid_coordinates)
+    order = np.empty(len(nb), np.int64)
+    nbr = np.ascontiguousarray(mesh.neighbours, np.int64)
+    p64 = lambda x: x.ctypes.data_as(C.POINTER(C.c_int64))  # noqa: E731
+    assert _native.lib().anuga_tile_order(len(nb), cen.ctypes.data_as(C.POINTER(C.c_double)),
+                                          p64(nbr), p64(order)) == 0
+    return nb, mesh.vertex_coordinates.reshape(-1, 3, 2)[order]
+
+
+@pytest.mark.parametrize("make", [
+    lambda: rectangular_cross(1, 1), lambda: rectangular_cross(8, 8),
+    lambda: rectangular_cross(37, 53, 1000.0, 700.0), lambda: rectangular_cross(150, 150),
+    lambda: rectangular(1000, 1, 1000.0, 1.0), lambda: rectangular(128, 1), lambda: rectangular(3, 43),
+    lambda: graded_square(300.0, 9.0, 40.0, (100.0, 100.0, 200.0, 200.0), seed=3)])
+def test_tables_name_every_neighbour_edge_and_vertex(make):
+    nb, vertices = _ordered(Mesh(*make()))
+    a = _tables(nb, vertices)
+    assert a is not None
+    _replay(nb, a, vertices)
+    plain = _tables(nb)
+    for name in ("stencil", "across", "cell", "hstencil", "hcell", "edge"):
+        assert np.array_equal(plain[name][:len(a[name])], a[name][:len(plain[name])])
+
+
+def test_tables_refuse_scattered_tiles():
+    """Triangles in a random order: more cells than a tile's LDS holds."""
+    mesh = Mesh(*rectangular_cross(30, 30))
+    N = mesh.number_of_triangles
+    order = np.random.default_rng(0).permutation(N)
+    place = np.empty(N, np.int64)
+    place[order] = np.arange(N)
+    n, e = mesh.neighbours[order], mesh.neighbour_edges[order]
+    nb = np.where(n >= 0, (place[np.maximum(n, 0)] << 2) | e, -1)
+    assert _tables(nb) is None
