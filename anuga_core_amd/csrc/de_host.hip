@@ -2495,9 +2495,10 @@ static int add_operator(anuga_domain *d, int kind, int64_t n, const int64_t *ind
     }
     HIPCHK(d, hipStreamSynchronize(d->stream));
     HIPCHK(d, dalloc(&o.idx, (size_t)std::max(o.n, 1)));
-    HIPCHK(d, dalloc(&o.influx, 1));
+    const size_t parts = ((size_t)o.n + DE_BLOCK - 1) / DE_BLOCK;   // one per workgroup of de_rate
+    HIPCHK(d, dalloc(&o.influx, parts));
     HIPCHK(d, hipMemcpy(o.idx, idx.data(), std::max(o.n, 1) * sizeof(int), hipMemcpyHostToDevice));
-    HIPCHK(d, hipMemset(o.influx, 0, sizeof(double)));
+    HIPCHK(d, hipMemset(o.influx, 0, std::max<size_t>(parts, 1) * sizeof(double)));
     d->ops.push_back(o);
     rc = upload_rate(d, d->ops.back(), rates, rate, factor);
     if (rc) return rc;
@@ -2685,7 +2686,13 @@ int anuga_get_operator_influx(anuga_domain *d, int64_t id, double *cumulative)
     if (!d || !cumulative) return ANUGA_E_ARG;
     if (id < 0 || id >= (int64_t)d->ops.size()) return fail(d, ANUGA_E_ARG, "no such operator");
     HIPCHK(d, hipStreamSynchronize(d->stream));
-    HIPCHK(d, hipMemcpy(cumulative, d->ops[id].influx, sizeof(double), hipMemcpyDeviceToHost));
+    const RateOp &o = d->ops[id];
+    // an inlet keeps its sum; a rate operator one part per workgroup
+    const size_t parts = o.kind == 0 ? std::max(1, (o.n + DE_BLOCK - 1) / DE_BLOCK) : 1;
+    std::vector<double> h(parts);
+    HIPCHK(d, hipMemcpy(h.data(), o.influx, parts * sizeof(double), hipMemcpyDeviceToHost));
+    *cumulative = 0.0;
+    for (double x : h) *cumulative += x;
     return ANUGA_OK;
 }
 

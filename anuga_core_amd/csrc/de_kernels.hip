@@ -2766,8 +2766,10 @@ de_set_field(int n, const int *__restrict__ caller, const double *__restrict__ i
 // triangles after a step: local rate = factor * dt * rate; with all rates
 // >= 0 the stage rises by it; otherwise (`careful`) the loss is capped at the
 // depth and the momenta scale with the depth that remains. The inflow
-// (local rate * area) is accumulated for the volume balance (FP64 atomics:
-// a diagnostic, summed in no fixed order).
+// (local rate * area) is accumulated per workgroup, in influx[blockIdx.x],
+// and summed on the host when it is asked for. Atomic adds to one address were
+// the kernel's time (36k triangles: 11.5 us with one per triangle, 9.4 with one
+// per wave, 4.0 with none).
 // Set_stage_operator after a step (set_quantity.py:95-131, quantity
 // 'stage'): the stage centroid values of the region become the given values
 // (value[i], or value0 for all); momenta and bed unchanged.
@@ -2788,24 +2790,34 @@ de_rate(const DeControl *ctl, int n, const int *__restrict__ idx, const double *
 {
     if (ctl->done) return;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int k = idx[i];
-    const double r = rate ? rate[i] : rate0;
-    const double dt = ctl->dt;
-    DeQ q = S[k];
-    double lr = factor * dt * r;
-    if (!careful) {
-        q.w = q.w + lr;
-    } else {
-        const double h = q.w - q.z;
-        lr = fmax(lr, -h);
-        const double lf = lr < 0.0 ? (lr + h) / (h + 1.0e-10) : 1.0;
-        q.w = q.w + lr;
-        q.uh = q.uh * lf;
-        q.vh = q.vh * lf;
+    double gain = 0.0;
+    if (i < n) {
+        const int k = idx[i];
+        const double r = rate ? rate[i] : rate0;
+        const double dt = ctl->dt;
+        DeQ q = S[k];
+        double lr = factor * dt * r;
+        if (!careful) {
+            q.w = q.w + lr;
+        } else {
+            const double h = q.w - q.z;
+            lr = fmax(lr, -h);
+            const double lf = lr < 0.0 ? (lr + h) / (h + 1.0e-10) : 1.0;
+            q.w = q.w + lr;
+            q.uh = q.uh * lf;
+            q.vh = q.vh * lf;
+        }
+        S[k] = q;
+        gain = lr * area[k];
     }
-    S[k] = q;
-    atomicAdd(influx, lr * area[k]);
+    __shared__ double red[DE_BLOCK / 64];
+    gain = de_wave_sum_nz(gain);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = gain;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int j = 1; j < DE_BLOCK / 64; j++) gain += red[j];
+        influx[blockIdx.x] += gain;
+    }
 }
 
 // ---------------------------------------------------------------------------
