@@ -222,6 +222,8 @@ struct DeControl {
     int done;              // 1: finaltime reached, 2: yield time reached (steps become no-ops)
     int status;            // error bits, DE_ERR_*
     int hist_cap, method;  // method: timestep_fluxcalls (1 euler, 2 rk2, 3 rk3)
+    int pending;           // the last step's later boundary fluxes are not in the integral yet
+    int unused;
     // the scenario's triangles are [kbeg, kend) and its blocks [bbeg, bend) of
     // the internal numbering (fixed at creation)
     int kbeg, kend, bbeg, bend;

@@ -70,7 +70,7 @@ const int kHostHist = 512;
 // and 19.0 us a step, with a graph of one step 21.5 and 22.9, of 8 steps 17.4
 // and 18.7, of 32 steps 17.1 and 18.5; 90k triangles, DE1: 41.3, 45.2, 40.4,
 // 40.3. Capturing 8 steps takes 45 to 100 us once.
-const int kGraphSteps = 8, kGraphMin = 64;
+const int kGraphSteps = 8, kGraphMin = 64;   // an even count: see self_contained
 
 }  // namespace
 
@@ -180,6 +180,10 @@ struct anuga_domain {
     double *part = nullptr;   // [DE_P_ROWS][nblocks]
     double *chunks = nullptr; // [DE_P_ROWS][S][DE_RCHUNKS]: the reduction's first stage
     DeControl *ctl = nullptr; // [S] device step control
+    DeControl *ctl2 = nullptr;   // [S] the other set of self-contained steps, behind dneg
+    // the sets that the kernels read and take the later substeps' timestep
+    // from: ctl, but inside a self-contained step
+    DeControl *kctl = nullptr, *kdt = nullptr;
     unsigned long long *dneg = nullptr; // fix_negative count, behind ctl
     // one pinned allocation: the mirror of ctl and of the counter behind it,
     // then hsetup, hhist and the staging of the boundary values' three slots
@@ -630,11 +634,11 @@ static void launch_extrapolate(anuga_domain *d, DeQ *S)
     if (d->mixed)
         hipLaunchKernelGGL(de_extrapolate<float>, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->E, d->flags,
-                           part_row(d, DE_P_MASS), d->ctl);
+                           part_row(d, DE_P_MASS), d->kctl);
     else
         hipLaunchKernelGGL(de_extrapolate<double>, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->E, d->flags,
-                           part_row(d, DE_P_MASS), d->ctl);
+                           part_row(d, DE_P_MASS), d->kctl);
     timer_end(d, T_EXTRAP);
 }
 
@@ -653,18 +657,21 @@ static void launch_flux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
             hipLaunchKernelGGL((de_flux<double, SUB, true>), dim3(d->nblocks), dim3(DE_BLOCK), 0,
                                d->stream, dev_mesh(d), dev_params(d->P), S, d->eta,
                                (const double *)d->E, bc, d->flags, d->ex[0], d->ex[1],
-                               d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
+                               d->ex[2], bk, out, d->kctl, d->kdt,
+                               part_row(d, DE_P_DT), bflux_row<SUB>(d),
                                d->dneg);
         else
             hipLaunchKernelGGL((de_flux<double, SUB>), dim3(d->nblocks), dim3(DE_BLOCK), 0,
                                d->stream, dev_mesh(d), dev_params(d->P), S, d->eta,
                                (const double *)d->E, bc, d->flags, d->ex[0], d->ex[1],
-                               d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
+                               d->ex[2], bk, out, d->kctl, d->kdt,
+                               part_row(d, DE_P_DT), bflux_row<SUB>(d),
                                d->dneg);
     } else
         hipLaunchKernelGGL((de_flux_mixed<SUB>), dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->eta, (const DeEdgeRec32 *)d->E,
-                           bc, d->flags, d->ex[0], d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d), d->dneg);
+                           bc, d->flags, d->ex[0], d->ex[1], d->ex[2], bk, out, d->kctl, d->kdt,
+                           part_row(d, DE_P_DT), bflux_row<SUB>(d), d->dneg);
 }
 
 template <class T>
@@ -695,7 +702,8 @@ static void launch_xflux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
         const size_t lds = ((size_t)DE_BLOCK + (size_t)d->hcap) * (sizeof(double) + 12 * sizeof(float));
         hipLaunchKernelGGL(de_xflux_mixed<SUB>, dim3(d->nblocks), dim3(DE_BLOCK), lds, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->eta, tl, bc, d->flags, d->ex[0],
-                           d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
+                           d->ex[1], d->ex[2], bk, out, d->kctl, d->kdt,
+                           part_row(d, DE_P_DT), bflux_row<SUB>(d),
                            part_row(d, DE_P_MASS), d->dneg);
     } else if (d->rw || d->P.low_froude || d->P.use_sloped_mannings) {
         // the general instantiation: walls, low_froude, sloped friction
@@ -703,7 +711,8 @@ static void launch_xflux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
                            (((size_t)DE_BLOCK + d->hcap + 7) & ~(size_t)7);
         hipLaunchKernelGGL((de_xflux<SUB, true>), dim3(d->nblocks), dim3(DE_BLOCK), lds,
                            d->stream, dev_mesh(d), dev_params(d->P), S, d->eta, tl, bc, d->flags,
-                           d->ex[0], d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d), part_row(d, DE_P_MASS), d->dneg,
+                           d->ex[0], d->ex[1], d->ex[2], bk, out, d->kctl, d->kdt,
+                           part_row(d, DE_P_DT), bflux_row<SUB>(d), part_row(d, DE_P_MASS), d->dneg,
                            (double *)d->E);
     } else if (d->mirror && d->tx.hecap && d->edge_once) {
         // each edge's flux once: tile edge values (before them, the cells),
@@ -715,13 +724,15 @@ static void launch_xflux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
         auto kern = vg ? de_xflux_e<SUB, true> : de_xflux_e<SUB, false>;
         hipLaunchKernelGGL(kern, dim3(d->nblocks), dim3(DE_BLOCK), lds, d->stream, dev_mesh(d),
                            dev_params(d->P), S, d->eta, d->tx, bc, d->flags, d->ex[0], d->ex[1],
-                           d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
+                           d->ex[2], bk, out, d->kctl, d->kdt,
+                           part_row(d, DE_P_DT), bflux_row<SUB>(d),
                            part_row(d, DE_P_MASS), d->dneg);
     } else {
         const size_t lds = (12 * (size_t)DE_BLOCK + 12 * (size_t)d->hcap) * sizeof(double);
         hipLaunchKernelGGL(de_xflux<SUB>, dim3(d->nblocks), dim3(DE_BLOCK), lds, d->stream,
                            dev_mesh(d), dev_params(d->P), S, d->eta, tl, bc, d->flags, d->ex[0],
-                           d->ex[1], d->ex[2], bk, out, d->ctl, part_row(d, DE_P_DT), bflux_row<SUB>(d),
+                           d->ex[1], d->ex[2], bk, out, d->kctl, d->kdt,
+                           part_row(d, DE_P_DT), bflux_row<SUB>(d),
                            part_row(d, DE_P_MASS), d->dneg, (double *)d->E);
     }
 }
@@ -769,11 +780,14 @@ static void launch_update_t(anuga_domain *d, DeQ *S, DeQ *out, int dt, double ho
     auto kern = dt == DE_DT_GIVEN    ? de_update<SLOPED, DE_DT_GIVEN>
                 : dt == DE_DT_HOST   ? de_update<SLOPED, DE_DT_HOST>
                 : dt == DE_DT_DIRECT ? de_update<SLOPED, DE_DT_DIRECT>
+                : dt == DE_DT_STEP   ? de_update<SLOPED, DE_DT_STEP>
                                      : de_update<SLOPED, DE_DT_CHUNKS>;
-    hipLaunchKernelGGL(kern, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream, d->scen,
+    const DeStepEnd se{d->kdt, d->part, d->S == 1 ? d->hist : nullptr, d->nblocks,
+                       (int)d->P.timestep_fluxcalls};
+    const int control = dt == DE_DT_STEP ? d->S : 0;
+    hipLaunchKernelGGL(kern, dim3(d->nblocks + control), dim3(DE_BLOCK), 0, d->stream, d->scen,
                        dev_params(d->P), S, d->eta, d->flags, d->ex[0], d->ex[1], d->ex[2],
-                       d->ctl, out, d->dneg, pdt, host_dt,
-                       (int)(d->P.timestep_fluxcalls == 1), (const double *)d->E, d->N, d->vx);
+                       d->kctl, out, d->dneg, pdt, host_dt, se, (const double *)d->E, d->N, d->vx);
 }
 
 // dt: DE_DT_*, where the timestep comes from; host_dt: the timestep of
@@ -911,12 +925,26 @@ static void launch_operators(anuga_domain *d)
     for (const RateOp &o : d->ops) launch_operator(d, o);
 }
 
+// Whether device-controlled steps are self-contained: the update's control
+// workgroups end the step. Operators and gauges run between the last substep
+// and the end of a step, and many blocks are reduced by many workgroups.
+static bool self_contained(const anuga_domain *d)
+{
+    return reduce_direct(d) && d->ops.empty() && !d->G;
+}
+
 // One device-controlled step of every scenario: the substeps, the timestep on
 // the device and the end-of-step bookkeeping. Every kernel returns at once for
-// a scenario whose done flag is set.
-static void enqueue_device_step(anuga_domain *d)
+// a scenario whose done flag is set. Self-contained steps read one set of
+// control blocks and write the other; `odd`: this one reads ctl2.
+static void enqueue_device_step(anuga_domain *d, bool odd)
 {
     const bool rk = d->P.timestep_fluxcalls > 1;
+    const bool whole = self_contained(d);
+    if (whole) {
+        d->kctl = odd ? d->ctl2 : d->ctl;
+        d->kdt = odd ? d->ctl : d->ctl2;
+    }
     if (fused(d)) {
         launch_xflux(d, 0, d->A);
     } else {
@@ -926,13 +954,27 @@ static void enqueue_device_step(anuga_domain *d)
     if (!reduce_direct(d))
         hipLaunchKernelGGL((de_reduce_chunks<true, 0>), dim3(DE_RCHUNKS, d->S), dim3(256), 0,
                            d->stream, d->part, d->nblocks, 0, 0, 0, 1, d->ctl, d->chunks);
-    launch_update(d, d->A, rk ? d->B : d->A, reduce_direct(d) ? DE_DT_DIRECT : DE_DT_CHUNKS);
+    launch_update(d, d->A, rk ? d->B : d->A,
+                  whole ? DE_DT_STEP : (reduce_direct(d) ? DE_DT_DIRECT : DE_DT_CHUNKS));
     enqueue_later_substeps(d, false);
+    if (whole) {
+        d->kctl = d->kdt = d->ctl;
+        return;
+    }
     launch_operators(d);
     launch_finish(d);
     if (d->G)
         hipLaunchKernelGGL(de_sample_gauges<false>, dim3(1), dim3(256), 0, d->stream, d->ctl,
                            d->G, d->gtri, d->A, 0.0, d->gtimes, d->gvals);
+}
+
+// After `steps` self-contained steps: the control blocks back in ctl.
+static void flush_steps(anuga_domain *d, int64_t steps)
+{
+    const int m = (int)d->P.timestep_fluxcalls;
+    auto kern = m == 1 ? de_flush_step<1> : (m == 2 ? de_flush_step<2> : de_flush_step<3>);
+    hipLaunchKernelGGL(kern, dim3(d->S), dim3(DE_RED_THREADS), 0, d->stream, d->part, d->nblocks,
+                       d->ctl, d->ctl2, (int)(steps & 1));
 }
 
 static void drop_graph(anuga_domain *d)
@@ -949,7 +991,7 @@ static int enqueue_device_steps(anuga_domain *d, int64_t nsteps)
     const bool graph = d->use_graph && !d->timing && (d->graph_exec || nsteps >= kGraphMin);
     if (graph && !d->graph_exec) {
         HIPCHK(d, hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
-        for (int i = 0; i < kGraphSteps; i++) enqueue_device_step(d);
+        for (int i = 0; i < kGraphSteps; i++) enqueue_device_step(d, i & 1);
         hipGraph_t g = nullptr;
         HIPCHK(d, hipStreamEndCapture(d->stream, &g));
         d->graph = g;
@@ -959,7 +1001,8 @@ static int enqueue_device_steps(anuga_domain *d, int64_t nsteps)
     if (graph)
         for (; i + kGraphSteps <= nsteps; i += kGraphSteps)
             HIPCHK(d, hipGraphLaunch(d->graph_exec, d->stream));
-    for (; i < nsteps; i++) enqueue_device_step(d);
+    for (; i < nsteps; i++) enqueue_device_step(d, i & 1);
+    if (self_contained(d) && nsteps > 0) flush_steps(d, nsteps);
     return ANUGA_OK;
 }
 
@@ -1097,8 +1140,10 @@ static int domain_alloc(const anuga_params *params, int64_t S64, const int64_t *
     DCHK(dalloc(&d->part, DE_P_ROWS * (size_t)d->nblocks));
     DCHK(dalloc(&d->chunks, DE_P_ROWS * (size_t)S * DE_RCHUNKS));
     // the control blocks with the fix_negative counter behind them
-    DCHK(hipMalloc((void **)&d->ctl, S * sizeof(DeControl) + sizeof(unsigned long long)));
+    DCHK(hipMalloc((void **)&d->ctl, 2 * S * sizeof(DeControl) + sizeof(unsigned long long)));
     d->dneg = reinterpret_cast<unsigned long long *>(d->ctl + S);
+    d->ctl2 = reinterpret_cast<DeControl *>(d->dneg + 1);
+    d->kctl = d->kdt = d->ctl;
     DCHK(dalloc(&d->dsetup, S));
     static_assert(sizeof(DeControl) % 8 == 0 && sizeof(DeBatchSetup) % 8 == 0, "pinned layout");
     const size_t hctl_bytes = S * sizeof(DeControl) + sizeof(unsigned long long);
@@ -1152,6 +1197,7 @@ static int domain_alloc(const anuga_params *params, int64_t S64, const int64_t *
         c.bend = (c.kend + DE_BLOCK - 1) / DE_BLOCK;
     }
     DCHK(hipMemcpy(d->ctl, d->hctl, hctl_bytes, hipMemcpyHostToDevice));
+    DCHK(hipMemset(d->ctl2, 0, S * sizeof(DeControl)));
     {
         const char *g = std::getenv("ANUGA_HIP_GRAPH");
         d->use_graph = !(g && g[0] == '0');
@@ -2191,16 +2237,16 @@ static void adj_stages(anuga_domain *d, AdjRun *a, const DeQ *X)
                        pm, d->ctl);
     hipLaunchKernelGGL((de_flux<double, 0>), g, b, 0, d->stream, dev_mesh(d), p, X, d->eta,
                        a->E0, bc, a->f0, a->ex0, a->ex0 + N, a->ex0 + 2 * N, nullptr, nullptr,
-                       d->ctl,
+                       d->ctl, d->ctl,
                        part_row(d, DE_P_DT), part_row(d, DE_P_BF0), a->neg);
     hipLaunchKernelGGL((de_update<false, DE_DT_GIVEN>), g, b, 0, d->stream, d->scen, p, X, d->eta,
                        a->f0, a->ex0, a->ex0 + N, a->ex0 + 2 * N, d->ctl, a->S1, a->neg, nullptr,
-                       0.0, 0, nullptr, 0, nullptr);
+                       0.0, DeStepEnd{}, nullptr, 0, nullptr);
     hipLaunchKernelGGL(de_extrapolate<double>, g, b, 0, d->stream, dev_mesh(d), p, a->S1, a->E1,
                        a->f1, pm, d->ctl);
     hipLaunchKernelGGL((de_flux<double, 0>), g, b, 0, d->stream, dev_mesh(d), p, a->S1, d->eta,
                        a->E1, bc, a->f1, a->ex1, a->ex1 + N, a->ex1 + 2 * N, nullptr, nullptr,
-                       d->ctl,
+                       d->ctl, d->ctl,
                        part_row(d, DE_P_DT), part_row(d, DE_P_BF0), a->neg);
 }
 

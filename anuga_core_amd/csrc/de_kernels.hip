@@ -796,7 +796,8 @@ __global__ void __launch_bounds__(DE_BLOCK)
 de_flux(DeMesh m, DeParams p, const DeQ *q, const double *__restrict__ eta,
         const T *__restrict__ E, DeBoundary bc, const unsigned char *__restrict__ flags,
         double *__restrict__ exw, double *__restrict__ exuh, double *__restrict__ exvh,
-        const DeQ *bk, DeQ *out, DeControl *ctl, double *__restrict__ part_dt,
+        const DeQ *bk, DeQ *out, DeControl *ctl,
+        const DeControl *dctl, double *__restrict__ part_dt,
         double *__restrict__ part_bf, unsigned long long *__restrict__ nneg)
 {
     __shared__ double red_dt[DE_BLOCK / 64];
@@ -805,7 +806,7 @@ de_flux(DeMesh m, DeParams p, const DeQ *q, const double *__restrict__ eta,
     DeControl *cb = de_ctl(ctl, m.scen, lb);
     if (cb->done) return;
     int *err = &cb->status;
-    const double dt = SUBSTEP ? cb->dt : 0.0;
+    const double dt = SUBSTEP ? dctl[cb - ctl].dt : 0.0;
     const int N = m.N;
     const int k = lb * DE_BLOCK + threadIdx.x;
     double dtmin = 1.0e100, bflux = 0.0;
@@ -1095,7 +1096,8 @@ __global__ void __launch_bounds__(DE_BLOCK)
 de_xflux(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__restrict__ eta,
          DeTiles tl, DeBoundary bc, unsigned char *__restrict__ flags, double *__restrict__ exw,
          double *__restrict__ exuh, double *__restrict__ exvh, const DeQ *bk, DeQ *out,
-         DeControl *ctl, double *__restrict__ part_dt, double *__restrict__ part_bf,
+         DeControl *ctl,
+         const DeControl *dctl, double *__restrict__ part_dt, double *__restrict__ part_bf,
          double *__restrict__ part_mass, unsigned long long *__restrict__ nneg,
          double *__restrict__ Eg)
 {
@@ -1106,7 +1108,7 @@ de_xflux(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__restri
     DeControl *cb = de_ctl(ctl, m.scen, lb);
     if (cb->done) return;
     int *err = &cb->status;
-    const double dt = SUBSTEP ? cb->dt : 0.0;
+    const double dt = SUBSTEP ? dctl[cb - ctl].dt : 0.0;
     const int N = m.N, t = threadIdx.x;
     const int k0 = lb * DE_BLOCK, k = k0 + t;
     const int kend = cb->kend;
@@ -1513,7 +1515,8 @@ __global__ void __launch_bounds__(DE_BLOCK, 4)
 de_xflux_e(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__restrict__ eta,
            DeTileX tx, DeBoundary bc, unsigned char *__restrict__ flags, double *__restrict__ exw,
            double *__restrict__ exuh, double *__restrict__ exvh, const DeQ *bk, DeQ *out,
-           DeControl *ctl, double *__restrict__ part_dt, double *__restrict__ part_bf,
+           DeControl *ctl,
+           const DeControl *dctl, double *__restrict__ part_dt, double *__restrict__ part_bf,
            double *__restrict__ part_mass, unsigned long long *__restrict__ nneg)
 {
     static_assert(DE_BLOCK >= 128, "the halo and the tile's edges share the workgroup's waves");
@@ -1577,7 +1580,7 @@ de_xflux_e(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__rest
     DeControl *cb = de_ctl(ctl, m.scen, lb);
     if (cb->done) return;
     int *err = &cb->status;
-    const double dt = SUBSTEP ? cb->dt : 0.0;
+    const double dt = SUBSTEP ? dctl[cb - ctl].dt : 0.0;
     const bool on = k < cb->kend;
     double mass = 0.0, dtmin = 1.0e100, bflux = 0.0;
     unsigned fk = 0;
@@ -1830,7 +1833,8 @@ de_flux_mixed(DeMesh m, DeParams p, const DeQ *q, const double *__restrict__ eta
               const DeEdgeRec32 *__restrict__ E, DeBoundary bc,
               const unsigned char *__restrict__ flags, double *__restrict__ exw,
               double *__restrict__ exuh, double *__restrict__ exvh, const DeQ *bk, DeQ *out,
-              DeControl *ctl, double *__restrict__ part_dt, double *__restrict__ part_bf,
+              DeControl *ctl,
+              const DeControl *dctl, double *__restrict__ part_dt, double *__restrict__ part_bf,
               unsigned long long *__restrict__ nneg)
 {
     __shared__ double red_dt[DE_BLOCK / 64];
@@ -1839,7 +1843,7 @@ de_flux_mixed(DeMesh m, DeParams p, const DeQ *q, const double *__restrict__ eta
     DeControl *cb = de_ctl(ctl, m.scen, lb);
     if (cb->done) return;
     int *err = &cb->status;
-    const double dt = SUBSTEP ? cb->dt : 0.0;
+    const double dt = SUBSTEP ? dctl[cb - ctl].dt : 0.0;
     const int N = m.N;
     const int k = lb * DE_BLOCK + threadIdx.x;
     double dtmin = 1.0e100, bflux = 0.0;
@@ -1912,7 +1916,8 @@ __global__ void __launch_bounds__(DE_BLOCK, DE_MIXED_WAVES)
 de_xflux_mixed(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__restrict__ eta,
                DeTiles tl, DeBoundary bc, unsigned char *__restrict__ flags,
                double *__restrict__ exw, double *__restrict__ exuh, double *__restrict__ exvh,
-               const DeQ *bk, DeQ *out, DeControl *ctl, double *__restrict__ part_dt,
+               const DeQ *bk, DeQ *out, DeControl *ctl,
+               const DeControl *dctl, double *__restrict__ part_dt,
                double *__restrict__ part_bf, double *__restrict__ part_mass,
                unsigned long long *__restrict__ nneg)
 {
@@ -1934,7 +1939,7 @@ de_xflux_mixed(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__
     DeControl *cb = de_ctl(ctl, m.scen, lb);
     if (cb->done) return;
     int *err = &cb->status;
-    const double dt = SUBSTEP ? cb->dt : 0.0;
+    const double dt = SUBSTEP ? dctl[cb - ctl].dt : 0.0;
     const int kend = cb->kend;
     const int hcap = tl.hcap;
     double *const hct = lds, *const hch = lds + DE_BLOCK;
@@ -2043,6 +2048,63 @@ de_xflux_mixed(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__
                                part_mass, lb);
 }
 
+// Fixed-order reduction of the per-block partials part[row][nblocks], row
+// DE_P_*, into the control blocks. Each scenario's blocks split into
+// DE_RCHUNKS contiguous chunks; a chunk's partials are added in a fixed order,
+// then the chunk results. The order depends only on the scenario's block
+// count. Up to DE_DIRECT_BLOCKS blocks (a chunk of at most 64, one per lane)
+// one workgroup per scenario reduces them in a single launch (4.6 us, at any
+// such size); above, de_reduce_chunks gives each chunk its own workgroup so
+// that many CUs read the partials, and a second stage adds the chunk results.
+// Both give the same bits.
+#define DE_DIRECT_BLOCKS (64 * DE_RCHUNKS)
+
+// what a reduction leaves in the control block
+enum { DE_R_FLUX0 = 0, DE_R_FLUX1, DE_R_MASS, DE_R_VOLUME, DE_R_FLUX2 };
+
+#define DE_RED_THREADS 512
+// The sums of NR rows of one scenario's partials, by one workgroup of TH
+// threads (every thread gets them): the chunk results are read (CHUNKS) or
+// formed here, a wave per chunk and a lane per block.
+template <bool CHUNKS, int NR, int TH = DE_RED_THREADS>
+__device__ __forceinline__ void de_reduce_rows(const double *__restrict__ src, int nblocks,
+                                               const DeControl *cb, int sc, int S,
+                                               const int rows[3], double (*res)[DE_RCHUNKS],
+                                               double sum[3])
+{
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (!CHUNKS) {
+        const int b0 = cb->bbeg, b1 = cb->bend;
+        const int len = (b1 - b0 + DE_RCHUNKS - 1) / DE_RCHUNKS;
+        constexpr int PER = DE_RCHUNKS / (TH / 64);
+        double x[PER][3];
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            const int c = wv + j * (TH / 64);
+            const int i = b0 + c * len + lane;
+            const bool in = lane < len && i < b1;
+#pragma unroll
+            for (int r = 0; r < NR; r++)
+                x[j][r] = in ? src[(size_t)rows[r] * nblocks + i] : 0.0;
+        }
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+#pragma unroll
+            for (int r = 0; r < NR; r++) {
+                const double v = de_wave_sum_nz(x[j][r]);
+                if (lane == 0) res[r][wv + j * (TH / 64)] = v;
+            }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        double v = 0.0;
+        if (lane < DE_RCHUNKS)
+            v = CHUNKS ? src[((size_t)rows[r] * S + sc) * DE_RCHUNKS + lane] : res[r][lane];
+        sum[r] = __shfl(de_wave_sum_nz(v), 0, 64);
+    }
+}
+
 // boundary_flux_integral_operator.__call__ (boundary_flux_integral_operator.py:46-62)
 __device__ __forceinline__ double de_flux_integral(double integral, double dt, int method,
                                                    double s0, double s1, double s2)
@@ -2071,17 +2133,18 @@ __device__ __forceinline__ double de_clamped_timestep(const DeControl *c, double
 
 // the rest of update_timestep, by one thread of a scenario: the recorded
 // extremes, the small-step counter with its first-order switch and its
-// exception (reported as DE_ERR_SMALL_TIMESTEP), and the results
-__device__ __forceinline__ void de_commit_timestep(DeControl *c, double flux_dt, double ts,
-                                                   double dt)
+// exception (returned as DE_ERR_SMALL_TIMESTEP), and the results
+__device__ __forceinline__ int de_commit_timestep(DeControl *c, double flux_dt, double ts,
+                                                  double dt)
 {
+    int err = 0;
     c->rec_max = (c->rec_max > ts) ? c->rec_max : ts;      // max(timestep, recorded_max)
     c->rec_min = (c->rec_min < ts) ? c->rec_min : ts;      // min(timestep, recorded_min)
     if (ts < c->min_dt) {
         c->smallsteps += 1;
         if (c->smallsteps > c->max_smallsteps) {
             c->smallsteps = 0;
-            if (c->order == 1) atomicOr(&c->status, DE_ERR_SMALL_TIMESTEP);
+            if (c->order == 1) err = DE_ERR_SMALL_TIMESTEP;
             else c->order = 1;
         }
     } else {
@@ -2090,13 +2153,122 @@ __device__ __forceinline__ void de_commit_timestep(DeControl *c, double flux_dt,
     }
     c->flux_dt = flux_dt;
     c->dt = dt;
+    return err;
+}
+
+// what the control workgroups of de_update read and write (DE_DT_STEP); of
+// the host-sequenced steps the method alone
+struct DeStepEnd {
+    DeControl *next;
+    const double *part;
+    double *hist;
+    int nblocks, method;
+};
+
+// The end of a step at time t + dt: timestep history (one scenario only) and
+// the yield / final-time test of _evolve_base (generic_domain.py:1855-1895)
+// that turns the scenario's next steps into no-ops; returns DE_ERR_OVERSHOOT
+// or 0.
+__device__ __forceinline__ int de_end_step(DeControl *c, double t, double dt, double *hist)
+{
+    c->t = t + dt;
+    if (hist && c->nsteps < c->hist_cap) hist[c->nsteps] = dt;
+    c->nsteps += 1;
+    if (c->t >= c->finaltime - c->eps) {
+        c->done = 1;
+        return c->t > c->finaltime ? DE_ERR_OVERSHOOT : 0;
+    }
+    if (c->t >= c->yieldtime) c->done = 2;
+    return 0;
+}
+
+// The minimum of a scenario's CFL partials, formed by every thread of a
+// workgroup of DE_BLOCK threads.
+__device__ __forceinline__ double de_block_dt(const double *__restrict__ pdt, int b0, int b1,
+                                              double *red)
+{
+    double m = 1.0e100;
+    for (int i = b0 + (int)threadIdx.x; i < b1; i += DE_BLOCK) m = fmin(m, pdt[i]);
+    m = de_wave_min(m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = red[0];
+    for (int i = 1; i < DE_BLOCK / 64; i++) m = fmin(m, red[i]);
+    return m;
+}
+
+// A scenario's control workgroup in a self-contained step (DE_DT_STEP): the
+// next control block from this step's, the timestep and the boundary fluxes
+// that are known: of rk2 and rk3 the step's later ones are added one step
+// late, from the partials they left (pending), or by de_flush_step. The status
+// bits stay where the kernels set them.
+__device__ __forceinline__ void de_step_control(const DeControl *__restrict__ c, DeControl *next,
+                                                const double *__restrict__ part, int nblocks,
+                                                int method, double *hist, double *red,
+                                                double (*res)[DE_RCHUNKS])
+{
+    const bool live = !c->done;
+    double m = 0.0, sum[3] = {0.0, 0.0, 0.0};
+    if (live) {
+        m = de_block_dt(part + (size_t)DE_P_DT * nblocks, c->bbeg, c->bend, red);
+        const int rows[3] = {DE_P_BF0, DE_P_BF1, DE_P_BF2};
+        de_reduce_rows<false, 3, DE_BLOCK>(part, nblocks, c, 0, 1, rows, res, sum);
+    }
+    if (threadIdx.x) return;
+    DeControl n = *c;
+    n.status = next->status;
+    if (live) {
+        if (n.pending) {
+            n.bflux1 = sum[1];
+            n.bflux2 = sum[2];
+            n.integral = de_flux_integral(n.integral, n.dt, method, n.bflux0, n.bflux1, n.bflux2);
+        }
+        const double ts = de_cfl_timestep(&n, m), dt = de_clamped_timestep(&n, ts);
+        n.status |= de_commit_timestep(&n, m, ts, dt);
+        n.bflux0 = sum[0];
+        n.pending = method > 1;
+        if (method == 1) n.integral = de_flux_integral(n.integral, dt, 1, n.bflux0, 0.0, 0.0);
+        n.status |= de_end_step(&n, n.t, dt, hist);
+    }
+    *next = n;
+}
+
+// After the last self-contained step of a run: the boundary fluxes still
+// pending, and after an odd number of steps the control blocks of ctl2 back
+// into ctl, with the status bits of both.
+template <int METHOD>
+__global__ void __launch_bounds__(DE_RED_THREADS)
+de_flush_step(const double *__restrict__ part, int nblocks, DeControl *ctl, DeControl *ctl2,
+              int odd)
+{
+    __shared__ double res[3][DE_RCHUNKS];
+    const int sc = blockIdx.x, S = gridDim.x;
+    DeControl *c = ctl + sc;
+    const int status = c->status | ctl2[sc].status;
+    const int pending = odd ? ctl2[sc].pending : c->pending;
+    double sum[3] = {0.0, 0.0, 0.0};
+    const int rows[3] = {DE_P_BF0, DE_P_BF1, DE_P_BF2};
+    if (METHOD > 1 && pending)
+        de_reduce_rows<false, METHOD>(part, nblocks, c, sc, S, rows, res, sum);
+    if (threadIdx.x) return;
+    if (odd) *c = ctl2[sc];
+    c->status = status;
+    ctl2[sc].status = 0;
+    if (METHOD > 1 && pending) {
+        c->bflux1 = sum[1];
+        if (METHOD > 2) c->bflux2 = sum[2];
+        c->integral = de_flux_integral(c->integral, c->dt, METHOD, c->bflux0, c->bflux1,
+                                       c->bflux2);
+        c->pending = 0;
+    }
 }
 
 // where de_update takes the timestep from: the control block, the host (which
-// it then records, and for euler advances the boundary flux integral), or update_timestep over the minimum of the scenario's per-block CFL
-// partials, read directly (at most DE_DIRECT_BLOCKS of them) or as the chunk
-// results of de_reduce_chunks<0>
-enum { DE_DT_GIVEN = 0, DE_DT_HOST, DE_DT_DIRECT, DE_DT_CHUNKS };
+// it then records, and for euler advances the boundary flux integral), or update_timestep
+// over the minimum of the scenario's per-block CFL partials, read directly (at
+// most DE_DIRECT_BLOCKS of them) or as the chunk results of de_reduce_chunks.
+// DE_DT_STEP: directly, with the step's whole control in workgroups of its own.
+enum { DE_DT_GIVEN = 0, DE_DT_HOST, DE_DT_DIRECT, DE_DT_CHUNKS, DE_DT_STEP };
 
 // friction + update + fix_negative_cells from the explicit updates of substep 0;
 // `out` may alias `q` (Euler, in place: each thread reads then writes its own record).
@@ -2111,16 +2283,31 @@ enum { DE_DT_GIVEN = 0, DE_DT_HOST, DE_DT_DIRECT, DE_DT_CHUNKS };
 // steps from 13.7 to 10.3 ms. The minimum's loads and barrier hide behind the
 // triangle's own records, requested first: 66.5 us at 4M triangles, 67.0
 // without it.
+//
+// DE_DT_STEP: S more workgroups, behind the others, write each scenario's next
+// control block (de_step_control) while these advance their triangles, so that
+// a step needs no launch for its end: 18.2 -> 16.7 us a DE0 step of 40k
+// triangles, 39.5 -> 36.8 a DE1 step of 90k.
 template <bool SLOPED, int DT>
 __global__ void __launch_bounds__(DE_BLOCK)
 de_update(const int *__restrict__ scen, DeParams p, const DeQ *q, const double *__restrict__ eta,
           const unsigned char *__restrict__ flags, const double *__restrict__ exw,
           const double *__restrict__ exuh, const double *__restrict__ exvh, DeControl *ctl,
           DeQ *out, unsigned long long *__restrict__ nneg, const double *__restrict__ pdt,
-          double host_dt, int euler, const double *__restrict__ E = nullptr, int N = 0,
+          double host_dt, DeStepEnd se, const double *__restrict__ E = nullptr, int N = 0,
           const double *__restrict__ vx = nullptr)
 {
+    __shared__ double red[DE_BLOCK / 64];
     const int lb = xcd_block();
+    if constexpr (DT == DE_DT_STEP) {
+        __shared__ double res[3][DE_RCHUNKS];
+        if (lb >= se.nblocks) {
+            const int s = lb - se.nblocks;
+            de_step_control(ctl + s, se.next + s, se.part, se.nblocks, se.method, se.hist, red,
+                            res);
+            return;
+        }
+    }
     const int sc = scen ? scen[lb] : 0;
     DeControl *cb = ctl + sc;
     if (cb->done) return;
@@ -2144,26 +2331,19 @@ de_update(const int *__restrict__ scen, DeParams p, const DeQ *q, const double *
         dt = host_dt;
         if (lb == cb->bbeg && threadIdx.x == 0) {
             cb->dt = dt;
-            if (euler)
+            if (se.method == 1)
                 cb->integral = de_flux_integral(cb->integral, dt, 1, cb->bflux0, 0.0, 0.0);
         }
     } else {
-        __shared__ double red[DE_BLOCK / 64];
-        double m = 1.0e100;
-        if constexpr (DT == DE_DT_DIRECT) {
-            for (int i = cb->bbeg + (int)threadIdx.x; i < cb->bend; i += DE_BLOCK)
-                m = fmin(m, pdt[i]);
-        } else if (threadIdx.x < DE_RCHUNKS) {
-            m = pdt[(size_t)sc * DE_RCHUNKS + threadIdx.x];
-        }
-        m = de_wave_min(m);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-        __syncthreads();
-        m = red[0];
-        for (int i = 1; i < DE_BLOCK / 64; i++) m = fmin(m, red[i]);
+        const double m = DT == DE_DT_CHUNKS ? de_block_dt(pdt, sc * DE_RCHUNKS,
+                                                          (sc + 1) * DE_RCHUNKS, red)
+                                            : de_block_dt(pdt, cb->bbeg, cb->bend, red);
         const double ts = de_cfl_timestep(cb, m);
         dt = de_clamped_timestep(cb, ts);
-        if (lb == cb->bbeg && threadIdx.x == 0) de_commit_timestep(cb, m, ts, dt);
+        if (DT != DE_DT_STEP && lb == cb->bbeg && threadIdx.x == 0) {
+            const int e = de_commit_timestep(cb, m, ts, dt);
+            if (e) atomicOr(&cb->status, e);
+        }
     }
     if (!on) return;
     DeSlope sl{false, 0.0, 0.0};
@@ -2273,20 +2453,6 @@ de_fix_negative(int kend, DeQ *__restrict__ q, unsigned long long *__restrict__ 
     }
 }
 
-// Fixed-order reduction of the per-block partials part[row][nblocks], row
-// DE_P_*, into the control blocks. Each scenario's blocks split into
-// DE_RCHUNKS contiguous chunks; a chunk's partials are added in a fixed order,
-// then the chunk results. The order depends only on the scenario's block
-// count. Up to DE_DIRECT_BLOCKS blocks (a chunk of at most 64, one per lane)
-// one workgroup per scenario reduces them in a single launch (4.6 us, at any
-// such size); above, de_reduce_chunks gives each chunk its own workgroup so
-// that many CUs read the partials, and a second stage adds the chunk results.
-// Both give the same bits.
-#define DE_DIRECT_BLOCKS (64 * DE_RCHUNKS)
-
-// what a reduction leaves in the control block
-enum { DE_R_FLUX0 = 0, DE_R_FLUX1, DE_R_MASS, DE_R_VOLUME, DE_R_FLUX2 };
-
 // One workgroup per chunk (blockIdx.x) and scenario (blockIdx.y): the CFL
 // minimum if DT, and the sums of NR rows, each to chunks[row][scenario][chunk].
 // live: nothing for scenarios that are done.
@@ -2330,49 +2496,6 @@ de_reduce_chunks(const double *__restrict__ part, int nblocks, int r0, int r1, i
             for (int k = 1; k < 4; k++) red[r][0] += red[r][k];
             chunks[rows[r] * n + o] = red[r][0];
         }
-    }
-}
-
-#define DE_RED_THREADS 512
-// The sums of NR rows of one scenario's partials, by one workgroup of
-// DE_RED_THREADS threads (every thread gets them): the chunk results are read
-// (CHUNKS) or formed here, a wave per chunk and a lane per block.
-template <bool CHUNKS, int NR>
-__device__ __forceinline__ void de_reduce_rows(const double *__restrict__ src, int nblocks,
-                                               const DeControl *cb, int sc, int S,
-                                               const int rows[3], double (*res)[DE_RCHUNKS],
-                                               double sum[3])
-{
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (!CHUNKS) {
-        const int b0 = cb->bbeg, b1 = cb->bend;
-        const int len = (b1 - b0 + DE_RCHUNKS - 1) / DE_RCHUNKS;
-        constexpr int PER = DE_RCHUNKS / (DE_RED_THREADS / 64);
-        double x[PER][3];
-#pragma unroll
-        for (int j = 0; j < PER; j++) {
-            const int c = wv + j * (DE_RED_THREADS / 64);
-            const int i = b0 + c * len + lane;
-            const bool in = lane < len && i < b1;
-#pragma unroll
-            for (int r = 0; r < NR; r++)
-                x[j][r] = in ? src[(size_t)rows[r] * nblocks + i] : 0.0;
-        }
-#pragma unroll
-        for (int j = 0; j < PER; j++)
-#pragma unroll
-            for (int r = 0; r < NR; r++) {
-                const double v = de_wave_sum_nz(x[j][r]);
-                if (lane == 0) res[r][wv + j * (DE_RED_THREADS / 64)] = v;
-            }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int r = 0; r < NR; r++) {
-        double v = 0.0;
-        if (lane < DE_RCHUNKS)
-            v = CHUNKS ? src[((size_t)rows[r] * S + sc) * DE_RCHUNKS + lane] : res[r][lane];
-        sum[r] = __shfl(de_wave_sum_nz(v), 0, 64);
     }
 }
 
@@ -2429,11 +2552,10 @@ __device__ __forceinline__ DeControl *de_scenario(DeControl *ctl, int S)
     return s < S ? ctl + s : nullptr;
 }
 
-// End of a step, one workgroup per scenario: the boundary flux sums of the
-// METHOD's substeps and their integral (boundary_flux_integral_operator.py:
-// 39-49), relative_time += dt, timestep history (one scenario only), and the
-// yield / final-time test of _evolve_base (generic_domain.py:1855-1895) that
-// turns the scenario's next steps into no-ops.
+// End of a step that is not self-contained (operators, gauges, more than
+// DE_DIRECT_BLOCKS blocks), one workgroup per scenario: the boundary flux sums
+// of the METHOD's substeps and their integral (boundary_flux_integral_operator
+// .py:39-49), and de_end_step.
 template <int METHOD, bool CHUNKS>
 __global__ void __launch_bounds__(DE_RED_THREADS)
 de_finish_step(const double *__restrict__ src, int nblocks, DeControl *ctl, double *hist)
@@ -2451,15 +2573,8 @@ de_finish_step(const double *__restrict__ src, int nblocks, DeControl *ctl, doub
     if (METHOD > 2) c->bflux2 = sum[2];
     const double dt = c->dt;
     c->integral = de_flux_integral(c->integral, dt, METHOD, sum[0], sum[1], sum[2]);
-    c->t = c->t + dt;
-    if (hist && c->nsteps < c->hist_cap) hist[c->nsteps] = dt;
-    c->nsteps += 1;
-    if (c->t >= c->finaltime - c->eps) {
-        if (c->t > c->finaltime) atomicOr(&c->status, DE_ERR_OVERSHOOT);
-        c->done = 1;
-    } else if (c->t >= c->yieldtime) {
-        c->done = 2;
-    }
+    const int e = de_end_step(c, c->t, dt, hist);
+    if (e) atomicOr(&c->status, e);
 }
 
 // host-controlled steps (one scenario): the host computed dt
@@ -2502,6 +2617,7 @@ __device__ __forceinline__ void de_setup(DeControl *c, const DeBatchSetup &b)
     c->method = b.method;
     c->nsteps = 0;
     c->gstep = 0;
+    c->pending = 0;
     c->done = 0;
     if (b.stop_reached) {
         if (c->t >= c->finaltime - c->eps) c->done = 1;
