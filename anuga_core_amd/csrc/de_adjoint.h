@@ -6,11 +6,10 @@
 // order, is restated once more over a scalar type T, so that it can run with
 // T = double (the value; bit-identical to the production kernels, checked
 // against the oracle on the CPU) and with T = Dual<K> (forward-mode
-// derivatives along K tangent directions). The adjoint kernels evaluate a
-// cell with dual numbers seeded on one group of inputs at a time and
-// contract the output tangents with the output adjoints: a vector-Jacobian
-// product per cell, exact for the piecewise-smooth function the forward
-// computes (branches are taken on the value part, as the forward takes them).
+// derivatives along K tangent directions). The adjoint kernels apply
+// vector-Jacobian products written by hand as reverse sweeps (adj_*_vjp),
+// exact for the piecewise-smooth function the forward computes (branches are
+// taken as the forward takes them); the duals check them.
 //
 // Functions are __host__ __device__ so that tests can run them on the CPU.
 #pragma once
@@ -572,16 +571,6 @@ struct AdjView {
     double dt;
 };
 
-// accumulate into an adjoint: several triangles add to the same entry
-ADJ_HD void adj_add(double *a, double v)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    atomicAdd(a, v);
-#else
-    *a += v;
-#endif
-}
-
 ADJ_HD void adj_neighbours(const AdjView &m, int k, int v[3], int sur[3])
 {
 #pragma unroll
@@ -750,19 +739,71 @@ ADJ_HD void adj_fwd_advance(const AdjView &m, const double *S, const unsigned ch
 }
 
 // ---- adjoints ----------------------------------------------------------------------
-// Map an adjoint of the centroid values (w, uh, vh, z after the flags) onto
-// the raw state of triangle k and the bed.
+// An adjoint of the centroid values (w, uh, vh, z after the flags) added to
+// that of the raw state ls and the bed lz of the triangle.
+ADJ_HD void adj_add_centroid(unsigned f, const double lc[4], double ls[3], double &lz)
+{
+    const double g[4] = {(f & ADJ_F_CLAMP) ? 0.0 : lc[0], (f & ADJ_F_KEEP) ? lc[1] : 0.0,
+                         (f & ADJ_F_KEEP) ? lc[2] : 0.0,
+                         lc[3] + ((f & ADJ_F_CLAMP) ? lc[0] : 0.0)};
+    for (int c = 0; c < 3; c++)
+        if (g[c] != 0.0) ls[c] += g[c];
+    if (g[3] != 0.0) lz += g[3];
+}
+
 ADJ_HD void adj_scatter_centroid(unsigned f, const double lc[4], double *lamS, double *zbar,
                                  int N, int k)
 {
-    const double lw = (f & ADJ_F_CLAMP) ? 0.0 : lc[0];
-    const double lz = lc[3] + ((f & ADJ_F_CLAMP) ? lc[0] : 0.0);
-    const double lu = (f & ADJ_F_KEEP) ? lc[1] : 0.0;
-    const double lv = (f & ADJ_F_KEEP) ? lc[2] : 0.0;
-    if (lw != 0.0) adj_add(lamS + k, lw);
-    if (lu != 0.0) adj_add(lamS + N + k, lu);
-    if (lv != 0.0) adj_add(lamS + 2 * (size_t)N + k, lv);
-    if (lz != 0.0) adj_add(zbar + k, lz);
+    double ls[3] = {lamS[k], lamS[N + k], lamS[2 * (size_t)N + k]}, lz = zbar[k];
+    adj_add_centroid(f, lc, ls, lz);
+    for (int c = 0; c < 3; c++) lamS[(size_t)c * N + k] = ls[c];
+    zbar[k] = lz;
+}
+
+// The update of a triangle with centroid values c, friction eta and explicit
+// updates ex by reverse mode: lam_out (w, uh, vh of the result) -> the adjoints
+// g of c (0..3), eta (4) and ex (5..7). The same derivatives as adj_advance_cell
+// on duals; the quotient (S q) / q of the semi-implicit update is S.
+ADJ_HD void adj_advance_vjp(const double c[4], double eta, const double ex[3], double dt,
+                            const AdjParams &p, const double lam_out[3], double g[8])
+{
+    const double h = c[0] - c[3];
+    const bool rough = eta > p.mah && h >= p.mah;
+    double mag = 0.0, P = 1.0, S = 0.0;
+    if (rough) {
+        mag = sqrt(c[1] * c[1] + c[2] * c[2]);
+        P = de_pow_7_3(h);
+        S = (-p.g * eta * eta * mag) / P;
+    }
+    const double rw = c[0] + dt * ex[0];
+    for (int j = 0; j < 8; j++) g[j] = 0.0;
+    if (rw - c[3] < 0.0) {
+        g[3] = lam_out[0];
+        return;
+    }
+    g[0] = lam_out[0];
+    g[5] = dt * lam_out[0];
+    double gS = 0.0;
+#pragma unroll
+    for (int j = 1; j < 3; j++) {
+        const double si = c[j] == 0.0 ? 0.0 : (S * c[j]) / c[j];
+        const double den = 1.0 - dt * si;
+        const double r = (c[j] + dt * ex[j]) / den;
+        const double gn = lam_out[j] / den;
+        g[j] = gn;
+        g[5 + j] = dt * gn;
+        if (c[j] != 0.0) gS += dt * (gn * r);
+    }
+    if (rough) {
+        const double gS0 = gS / P, gP = -(gS * S) / P;
+        g[4] = gS0 * (-p.g * (eta + eta) * mag);
+        const double gm = mag > 0.0 ? gS0 * (-p.g * eta * eta) / mag : 0.0;
+        g[1] += gm * c[1];
+        g[2] += gm * c[2];
+        const double gh = gP * ((7.0 / 3.0) * P / h);
+        g[0] += gh;
+        g[3] -= gh;
+    }
 }
 
 // Update of triangle k: lam_out (w, uh, vh of the result) -> adjoints of the
@@ -773,27 +814,15 @@ ADJ_HD void adj_bwd_advance(const AdjView &m, const double *S, const unsigned ch
                             const double lam_out[3], int k, double *lamS, double *zbar,
                             double *nbar, double *lam_ex)
 {
-    typedef Dual<4> D;
     const int N = m.N;
     double q[4] = {S[4 * k], S[4 * k + 1], S[4 * k + 2], S[4 * k + 3]}, c[4];
     const unsigned f = fl[k];
     adj_centroid<double>(q, f, c);
-    const double in[8] = {c[0], c[1], c[2], c[3], m.eta[k], exw[k], exuh[k], exvh[k]};
+    const double ex[3] = {exw[k], exuh[k], exvh[k]};
     double g[8];
-    for (int pass = 0; pass < 2; pass++) {
-        D x[8];
-        for (int j = 0; j < 8; j++) {
-            x[j] = D(in[j]);
-            if (j / 4 == pass) x[j].d[j % 4] = 1.0;
-        }
-        D o[3];
-        adj_advance_cell<D>(x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7], m.dt, m.p, o);
-        for (int t = 0; t < 4; t++)
-            g[4 * pass + t] = lam_out[0] * o[0].d[t] + lam_out[1] * o[1].d[t] + lam_out[2] * o[2].d[t];
-    }
-    const double lc[4] = {g[0], g[1], g[2], g[3]};
-    adj_scatter_centroid(f, lc, lamS, zbar, N, k);
-    if (g[4] != 0.0) adj_add(nbar + k, g[4]);
+    adj_advance_vjp(c, m.eta[k], ex, m.dt, m.p, lam_out, g);
+    adj_scatter_centroid(f, g, lamS, zbar, N, k);
+    if (g[4] != 0.0) nbar[k] += g[4];
     lam_ex[k] = g[5];
     lam_ex[N + k] = g[6];
     lam_ex[2 * (size_t)N + k] = g[7];
@@ -848,7 +877,7 @@ ADJ_HD void adj_bwd_flux(const AdjView &m, const double *S, const unsigned char 
                     const size_t slot = pass == 0 ? (size_t)i * N + k
                                                   : (size_t)(v[i] & 3) * N + (v[i] >> 2);
                     for (int t = 0; t < KF; t++)
-                        if (gj[t] != 0.0) adj_add(lamE + (size_t)(s0 + t) * 3 * N + slot, gj[t]);
+                        if (gj[t] != 0.0) lamE[(size_t)(s0 + t) * 3 * N + slot] += gj[t];
                 }
             }
         }
@@ -863,103 +892,120 @@ ADJ_HD void adj_bwd_flux(const AdjView &m, const double *S, const unsigned char 
 // it is frozen), accumulated from the outputs back to the inputs in one
 // sweep instead of one forward pass per group of input tangents.
 
-// adj_limit's reverse: g (adjoint of the limited jumps, in) -> gd (of the
-// unlimited jumps d), gqmin, gqmax, gbeta (added to).
-ADJ_HD void adj_rev_limit(const double d[3], double qmin, double qmax, double beta,
-                          double freeze, const double g[3], double gd[3], double &gqmin,
-                          double &gqmax, double &gbeta)
+// adj_limit of the jumps d and what its reverse needs: the least ratio r, the
+// edge src that gave it (-1: none) and whether phi varies with them.
+struct AdjLimit {
+    double d[3], r, phi;
+    int src;
+    bool live;
+};
+
+ADJ_HD void adj_limit_state(AdjLimit &l, double qmin, double qmax, double beta, double freeze)
 {
     const double tiny = 1.0e-100;
     double r = 1000.0, r0 = 1.0;
-    int rsrc = -1, r0src = -1, rnum = 0, r0num = 0;
+    int src = -1, r0src = -1;
+#pragma unroll
     for (int i = 0; i < 3; i++) {
-        if (d[i] < -tiny) {
-            r0 = qmin / d[i];
-            r0src = i;
-            r0num = 1;
-        }
-        if (d[i] > tiny) {
-            r0 = qmax / d[i];
-            r0src = i;
-            r0num = 2;
-        }
+        const bool neg = l.d[i] < -tiny, some = neg || l.d[i] > tiny;
+        const double x = (neg ? qmin : qmax) / l.d[i];
+        r0 = some ? x : r0;
+        r0src = some ? i : r0src;
         if (r0 <= r) {
             r = r0;
-            rsrc = r0src;
-            rnum = r0num;
+            src = r0src;
         }
     }
     const double rb = r * beta;
-    const bool live = rb <= 1.0 &&
-                      !(freeze > 0.0 && fabs(d[0]) < freeze && fabs(d[1]) < freeze &&
-                        fabs(d[2]) < freeze);
-    const double phi = rb <= 1.0 ? rb : 1.0;
+    l.r = r;
+    l.src = src;
+    l.live = rb <= 1.0 && !(freeze > 0.0 && fabs(l.d[0]) < freeze && fabs(l.d[1]) < freeze &&
+                            fabs(l.d[2]) < freeze);
+    l.phi = rb <= 1.0 ? rb : 1.0;
+}
+
+// adj_limit's reverse: g (adjoint of the limited jumps, in) -> gd (of the
+// unlimited jumps d), gqmin, gqmax, gbeta (added to).
+ADJ_HD void adj_rev_limit(const AdjLimit &l, double beta, const double g[3], double gd[3],
+                          double &gqmin, double &gqmax, double &gbeta)
+{
     double gphi = 0.0;
+#pragma unroll
     for (int i = 0; i < 3; i++) {
-        gd[i] = g[i] * phi;
-        gphi += g[i] * d[i];
+        gd[i] = g[i] * l.phi;
+        gphi += g[i] * l.d[i];
     }
-    if (!live) return;
+    if (!l.live) return;
     const double gr = gphi * beta;
-    gbeta += gphi * r;
-    if (rsrc < 0) return;
-    const double ib = 1.0 / d[rsrc];
-    const double gnum = gr * ib;
-    gd[rsrc] += -(r * gr) * ib;
-    if (rnum == 1) gqmin += gnum;
+    gbeta += gphi * l.r;
+    if (l.src < 0) return;
+    const double ds = l.src == 0 ? l.d[0] : (l.src == 1 ? l.d[1] : l.d[2]);
+    const double ib = 1.0 / ds;
+    const double gnum = gr * ib, gds = -(l.r * gr) * ib;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+        if (i == l.src) gd[i] += gds;
+    if (ds < 0.0) gqmin += gnum;
     else gqmax += gnum;
 }
 
-// adj_aux_jumps' reverse: g (adjoint of d) -> gq[4] (qk, q0, q1, q2), gbeta
-// (added to)
-ADJ_HD void adj_rev_aux(double qk, double q0, double q1, double q2, double dx1, double dx2,
-                        double dy1, double dy2, double inv_area2, const double dxv[3],
-                        const double dyv[3], double beta, double freeze, const double g[3],
-                        double gq[4], double &gbeta)
+struct AdjTrue { static constexpr bool value = true; };
+struct AdjFalse { static constexpr bool value = false; };
+
+// adj_aux_jumps of one quantity and what its reverse needs: which of dq0 (0),
+// dq0 + dq1 (1), dq0 + dq2 (2) or zero (3) is the greatest and the least
+struct AdjAux {
+    AdjLimit l;
+    int mx, mn;
+};
+
+ADJ_HD void adj_aux_state(AdjAux &x, double qk, double q0, double q1, double q2,
+                          const AdjExtrapGeo &gm, double inv_area2, double beta, double freeze)
 {
     const double dq0 = q0 - qk, dq1 = q1 - q0, dq2 = q2 - q0;
-    double a = dy2 * dq1 - dy1 * dq2;
+    double a = gm.dy2 * dq1 - gm.dy1 * dq2;
     a *= inv_area2;
-    double b = dx1 * dq2 - dx2 * dq1;
+    double b = gm.dx1 * dq2 - gm.dx2 * dq1;
     b *= inv_area2;
-    double d[3];
-    for (int i = 0; i < 3; i++) d[i] = a * dxv[i] + b * dyv[i];
+#pragma unroll
+    for (int i = 0; i < 3; i++) x.l.d[i] = a * gm.dxv[i] + b * gm.dyv[i];
     const double s1 = dq0 + dq1, s2 = dq0 + dq2;
     // qmax = max(max(dq0, max(s1, s2)), 0), each max passing its first on ties
     const int mx_in = s1 >= s2 ? 1 : 2;
     const double mxv = mx_in == 1 ? s1 : s2;
     const int mx_o = dq0 >= mxv ? 0 : mx_in;
     const double mxo = mx_o == 0 ? dq0 : mxv;
-    const bool mx_live = mxo >= 0.0;
-    const double qmax = mx_live ? mxo : 0.0;
+    x.mx = mxo >= 0.0 ? mx_o : 3;
+    const double qmax = mxo >= 0.0 ? mxo : 0.0;
     const int mn_in = s1 <= s2 ? 1 : 2;
     const double mnv = mn_in == 1 ? s1 : s2;
     const int mn_o = dq0 <= mnv ? 0 : mn_in;
     const double mno = mn_o == 0 ? dq0 : mnv;
-    const bool mn_live = mno <= 0.0;
-    const double qmin = mn_live ? mno : 0.0;
+    x.mn = mno <= 0.0 ? mn_o : 3;
+    const double qmin = mno <= 0.0 ? mno : 0.0;
+    adj_limit_state(x.l, qmin, qmax, beta, freeze);
+}
+
+// adj_aux_jumps' reverse: g (adjoint of the limited jumps) -> gq[4] (qk, q0,
+// q1, q2), gbeta (added to)
+ADJ_HD void adj_rev_aux(const AdjAux &x, const AdjExtrapGeo &gm, double inv_area2, double beta,
+                        const double g[3], double gq[4], double &gbeta)
+{
     double gd[3], gqmin = 0.0, gqmax = 0.0;
-    adj_rev_limit(d, qmin, qmax, beta, freeze, g, gd, gqmin, gqmax, gbeta);
-    double gdq0 = 0.0, gs1 = 0.0, gs2 = 0.0;
-    if (mx_live) {
-        if (mx_o == 0) gdq0 += gqmax;
-        else if (mx_o == 1) gs1 += gqmax;
-        else gs2 += gqmax;
-    }
-    if (mn_live) {
-        if (mn_o == 0) gdq0 += gqmin;
-        else if (mn_o == 1) gs1 += gqmin;
-        else gs2 += gqmin;
-    }
+    adj_rev_limit(x.l, beta, g, gd, gqmin, gqmax, gbeta);
+    double gdq0 = (x.mx == 0 ? gqmax : 0.0) + (x.mn == 0 ? gqmin : 0.0);
+    const double gs1 = (x.mx == 1 ? gqmax : 0.0) + (x.mn == 1 ? gqmin : 0.0);
+    const double gs2 = (x.mx == 2 ? gqmax : 0.0) + (x.mn == 2 ? gqmin : 0.0);
     double ga = 0.0, gb = 0.0;
+#pragma unroll
     for (int i = 0; i < 3; i++) {
-        ga += gd[i] * dxv[i];
-        gb += gd[i] * dyv[i];
+        ga += gd[i] * gm.dxv[i];
+        gb += gd[i] * gm.dyv[i];
     }
     ga *= inv_area2;
     gb *= inv_area2;
-    const double gdq1 = ga * dy2 - gb * dx2 + gs1;
-    const double gdq2 = gb * dx1 - ga * dy1 + gs2;
+    const double gdq1 = ga * gm.dy2 - gb * gm.dx2 + gs1;
+    const double gdq2 = gb * gm.dx1 - ga * gm.dy1 + gs2;
     gdq0 += gs1 + gs2;
     gq[0] -= gdq0;
     gq[1] += gdq0 - gdq1 - gdq2;
@@ -975,12 +1021,13 @@ ADJ_HD void adj_rev_line(double qk, double q1, double dx2, double dy2, const dou
 {
     const double dq1 = q1 - qk;
     const double a = dq1 * dx2, b = dq1 * dy2;
-    double d[3];
-    for (int i = 0; i < 3; i++) d[i] = a * dxv[i] + b * dyv[i];
+    AdjLimit l;
+    for (int i = 0; i < 3; i++) l.d[i] = a * dxv[i] + b * dyv[i];
     const bool up = dq1 >= 0.0;
     const double qmin = up ? 0.0 : dq1, qmax = up ? dq1 : 0.0;
     double gd[3], gqmin = 0.0, gqmax = 0.0, gbeta = 0.0;
-    adj_rev_limit(d, qmin, qmax, beta, freeze, g, gd, gqmin, gqmax, gbeta);
+    adj_limit_state(l, qmin, qmax, beta, freeze);
+    adj_rev_limit(l, beta, g, gd, gqmin, gqmax, gbeta);
     double gdq1 = up ? gqmax : gqmin;
     for (int i = 0; i < 3; i++) gdq1 += (gd[i] * dxv[i]) * dx2 + (gd[i] * dyv[i]) * dy2;
     gq1 += gdq1;
@@ -989,7 +1036,9 @@ ADJ_HD void adj_rev_line(double qk, double q1, double dx2, double dy2, const dou
 
 // The vector-Jacobian product of adj_extrap_cell: lo[4 i + t] (adjoints of
 // ew, eh, euh, evh on edge i) -> gs[4 j + c] (adjoints of w, uh, vh, z of
-// stencil slot j).
+// stencil slot j). The limiters of u and v are reversed as soon as they are
+// formed, the one of h is kept from its forward values to its reverse, and w
+// has no forward part: four limiters with their divisions, not seven.
 ADJ_HD void adj_extrap_vjp(const double w[4], const double uh[4], const double vh[4],
                            const double z[4], const unsigned fl[4], const AdjExtrapGeo &gm,
                            const AdjParams &p, const double lo[12], double gs[16])
@@ -1019,9 +1068,7 @@ ADJ_HD void adj_extrap_vjp(const double w[4], const double uh[4], const double v
             nv[i] = vh[i + 1] * ninv[i];
         }
     }
-    // forward values: the jumps (limited), as adj_extrap_cell forms them
-    double jw[3] = {0.0, 0.0, 0.0}, jh[3] = {0.0, 0.0, 0.0};
-    double ju[3] = {0.0, 0.0, 0.0}, jv[3] = {0.0, 0.0, 0.0};
+    // forward values: the limiters' slopes, as adj_extrap_cell forms them
     bool constant = gm.nbound == 3, gw = true, gu = true, gv = true;
     bool aux = false, line = false;
     double area2 = 0.0, inv_area2 = 0.0, hfactor = 0.0, bw_ = 0.0, bu_ = 0.0, bv_ = 0.0;
@@ -1080,22 +1127,10 @@ ADJ_HD void adj_extrap_vjp(const double w[4], const double uh[4], const double v
             inv_area2 = 1.0 / area2;
             bw_ = p.bwd + (p.bw - p.bwd) * hfactor;
             gw = bw_ > 0.0;
-            if (gw) {
-                adj_aux_jumps<double>(cw, nw[0], nw[1], nw[2], gm.dx1, gm.dx2, gm.dy1, gm.dy2,
-                                      inv_area2, gm.dxv, gm.dyv, bw_, jw, p.freeze);
-                adj_aux_jumps<double>(ch, nh[0], nh[1], nh[2], gm.dx1, gm.dx2, gm.dy1, gm.dy2,
-                                      inv_area2, gm.dxv, gm.dyv, bw_, jh, p.freeze);
-            }
             bu_ = p.buhd + (p.buh - p.buhd) * hfactor;
             gu = bu_ > 0.0;
-            if (gu)
-                adj_aux_jumps<double>(cu, nu[0], nu[1], nu[2], gm.dx1, gm.dx2, gm.dy1, gm.dy2,
-                                      inv_area2, gm.dxv, gm.dyv, bu_, ju, p.freeze);
             bv_ = p.bvhd + (p.bvh - p.bvhd) * hfactor;
             gv = bv_ > 0.0;
-            if (gv)
-                adj_aux_jumps<double>(cv, nv[0], nv[1], nv[2], gm.dx1, gm.dx2, gm.dy1, gm.dy2,
-                                      inv_area2, gm.dxv, gm.dyv, bv_, jv, p.freeze);
         }
     } else if (gm.nbound == 2) {
         if (!(gm.interior[0] || gm.interior[1] || gm.interior[2])) {
@@ -1107,66 +1142,93 @@ ADJ_HD void adj_extrap_vjp(const double w[4], const double uh[4], const double v
             ldx2 = 1.0 / la2;
             ldy2 = ldx2 * gm.ly;
             ldx2 *= gm.lx;
-            adj_line_jumps<double>(cw, nw[lsel], ldx2, ldy2, gm.dxv, gm.dyv, p.bw, jw, p.freeze);
-            adj_line_jumps<double>(ch, nh[lsel], ldx2, ldy2, gm.dxv, gm.dyv, p.bw, jh, p.freeze);
-            adj_line_jumps<double>(cu, nu[lsel], ldx2, ldy2, gm.dxv, gm.dyv, p.bw, ju, p.freeze);
-            adj_line_jumps<double>(cv, nv[lsel], ldx2, ldy2, gm.dxv, gm.dyv, p.bw, jv, p.freeze);
         }
     }
-    // reverse: the edge values
+    // reverse: the edge values and the jumps
     const bool kw = !(constant || !gw), ku = !(constant || !gu), kv = !(constant || !gv);
     double gcw = 0.0, gch = 0.0, gcu = 0.0, gcv = 0.0;
-    double gjw[3], gjh[3], gju[3], gjv[3];
-    for (int i = 0; i < 3; i++) {
-        const double eh = kw ? ch + jh[i] : ch;
-        const double eu = ku ? cu + ju[i] : cu;
-        const double ev = kv ? cv + jv[i] : cv;
-        const double lw = lo[4 * i], lh = lo[4 * i + 1], lu = lo[4 * i + 2], lv = lo[4 * i + 3];
-        const double geh = lh + lu * eu + lv * ev;
-        const double geu = lu * eh, gev = lv * eh;
-        gcw += lw;
-        gch += geh;
-        gcu += geu;
-        gcv += gev;
-        gjw[i] = kw ? lw : 0.0;
-        gjh[i] = kw ? geh : 0.0;
-        gju[i] = ku ? geu : 0.0;
-        gjv[i] = kv ? gev : 0.0;
-    }
-    // reverse: the jumps
     double gnw[3] = {0.0, 0.0, 0.0}, gnh[3] = {0.0, 0.0, 0.0};
     double gnu[3] = {0.0, 0.0, 0.0}, gnv[3] = {0.0, 0.0, 0.0};
+    double gbw = 0.0, gbu = 0.0, gbv = 0.0;
+    const auto sweep = [&](auto on_line) {
+        constexpr bool LINE = decltype(on_line)::value;
+        // the limited jumps of one quantity (qk, q), their state in x
+        const auto jumps = [&](double qk, const double q[3], double beta, bool some, AdjAux &x,
+                               double j[3]) {
+            for (int i = 0; i < 3; i++) j[i] = 0.0;
+            if constexpr (LINE) {
+                adj_line_jumps<double>(qk, q[lsel], ldx2, ldy2, gm.dxv, gm.dyv, p.bw, j, p.freeze);
+            } else if (aux && some) {
+                adj_aux_state(x, qk, q[0], q[1], q[2], gm, inv_area2, beta, p.freeze);
+                for (int i = 0; i < 3; i++) j[i] = x.l.d[i] * x.l.phi;
+            }
+        };
+        // their reverse: gj -> gqk, gq, gbeta
+        const auto reverse = [&](double qk, const double q[3], double beta, bool some,
+                                 const AdjAux &x, const double gj[3], double &gqk, double gq[3],
+                                 double &gbeta) {
+            if constexpr (LINE) {
+                double gk = 0.0, g1 = 0.0;
+                adj_rev_line(qk, q[lsel], ldx2, ldy2, gm.dxv, gm.dyv, p.bw, p.freeze, gj, gk, g1);
+                gqk += gk;
+                for (int i = 0; i < 3; i++)
+                    if (i == lsel) gq[i] += g1;
+            } else if (aux && some) {
+                double g4[4] = {0.0, 0.0, 0.0, 0.0};
+                adj_rev_aux(x, gm, inv_area2, beta, gj, g4, gbeta);
+                gqk += g4[0];
+                for (int i = 0; i < 3; i++) gq[i] += g4[i + 1];
+            }
+        };
+        AdjAux xh, xq;
+        double j[3], eh[3], geh[3], gj[3];
+        jumps(ch, nh, bw_, gw, xh, j);
+        for (int i = 0; i < 3; i++) {
+            eh[i] = kw ? ch + j[i] : ch;
+            geh[i] = lo[4 * i + 1];
+        }
+        // euh = eu eh
+        jumps(cu, nu, bu_, gu, xq, j);
+        for (int i = 0; i < 3; i++) {
+            const double lu = lo[4 * i + 2], eu = ku ? cu + j[i] : cu;
+            const double geu = lu * eh[i];
+            geh[i] += lu * eu;
+            gcu += geu;
+            gj[i] = ku ? geu : 0.0;
+        }
+        reverse(cu, nu, bu_, gu, xq, gj, gcu, gnu, gbu);
+        // evh = ev eh
+        jumps(cv, nv, bv_, gv, xq, j);
+        for (int i = 0; i < 3; i++) {
+            const double lv = lo[4 * i + 3], ev = kv ? cv + j[i] : cv;
+            const double gev = lv * eh[i];
+            geh[i] += lv * ev;
+            gcv += gev;
+            gj[i] = kv ? gev : 0.0;
+        }
+        reverse(cv, nv, bv_, gv, xq, gj, gcv, gnv, gbv);
+        // ew
+        if (!LINE && aux && gw)
+            adj_aux_state(xq, cw, nw[0], nw[1], nw[2], gm, inv_area2, bw_, p.freeze);
+        for (int i = 0; i < 3; i++) {
+            gcw += lo[4 * i];
+            gj[i] = kw ? lo[4 * i] : 0.0;
+        }
+        reverse(cw, nw, bw_, gw, xq, gj, gcw, gnw, gbw);
+        // eh
+        for (int i = 0; i < 3; i++) {
+            gch += geh[i];
+            gj[i] = kw ? geh[i] : 0.0;
+        }
+        reverse(ch, nh, bw_, gw, xh, gj, gch, gnh, gbw);
+    };
+    if (line) sweep(AdjTrue{});
+    else sweep(AdjFalse{});
     if (aux) {
         double ghf = 0.0;
-        if (gw) {
-            double gq[4] = {0.0, 0.0, 0.0, 0.0}, gb = 0.0;
-            adj_rev_aux(cw, nw[0], nw[1], nw[2], gm.dx1, gm.dx2, gm.dy1, gm.dy2, inv_area2,
-                        gm.dxv, gm.dyv, bw_, p.freeze, gjw, gq, gb);
-            gcw += gq[0];
-            for (int i = 0; i < 3; i++) gnw[i] += gq[i + 1];
-            double gq2[4] = {0.0, 0.0, 0.0, 0.0};
-            adj_rev_aux(ch, nh[0], nh[1], nh[2], gm.dx1, gm.dx2, gm.dy1, gm.dy2, inv_area2,
-                        gm.dxv, gm.dyv, bw_, p.freeze, gjh, gq2, gb);
-            gch += gq2[0];
-            for (int i = 0; i < 3; i++) gnh[i] += gq2[i + 1];
-            ghf += gb * (p.bw - p.bwd);
-        }
-        if (gu) {
-            double gq[4] = {0.0, 0.0, 0.0, 0.0}, gb = 0.0;
-            adj_rev_aux(cu, nu[0], nu[1], nu[2], gm.dx1, gm.dx2, gm.dy1, gm.dy2, inv_area2,
-                        gm.dxv, gm.dyv, bu_, p.freeze, gju, gq, gb);
-            gcu += gq[0];
-            for (int i = 0; i < 3; i++) gnu[i] += gq[i + 1];
-            ghf += gb * (p.buh - p.buhd);
-        }
-        if (gv) {
-            double gq[4] = {0.0, 0.0, 0.0, 0.0}, gb = 0.0;
-            adj_rev_aux(cv, nv[0], nv[1], nv[2], gm.dx1, gm.dx2, gm.dy1, gm.dy2, inv_area2,
-                        gm.dxv, gm.dyv, bv_, p.freeze, gjv, gq, gb);
-            gcv += gq[0];
-            for (int i = 0; i < 3; i++) gnv[i] += gq[i + 1];
-            ghf += gb * (p.bvh - p.bvhd);
-        }
+        if (gw) ghf += gbw * (p.bw - p.bwd);
+        if (gu) ghf += gbu * (p.buh - p.buhd);
+        if (gv) ghf += gbv * (p.bvh - p.bvhd);
         // hfactor -> ch, hmin, hmax
         double ghmin = 0.0, ghmax = 0.0;
         const double gC = c_sel ? ghf : 0.0, ghf1 = c_sel ? 0.0 : ghf;
@@ -1189,23 +1251,6 @@ ADJ_HD void adj_extrap_vjp(const double w[4], const double uh[4], const double v
         else gnh[hmin_src] += ghmin;
         if (hmax_src == 3) gch += ghmax;
         else gnh[hmax_src] += ghmax;
-    } else if (line) {
-        double gqk = 0.0, gq1 = 0.0;
-        adj_rev_line(cw, nw[lsel], ldx2, ldy2, gm.dxv, gm.dyv, p.bw, p.freeze, gjw, gqk, gq1);
-        gcw += gqk;
-        gnw[lsel] += gq1;
-        gqk = gq1 = 0.0;
-        adj_rev_line(ch, nh[lsel], ldx2, ldy2, gm.dxv, gm.dyv, p.bw, p.freeze, gjh, gqk, gq1);
-        gch += gqk;
-        gnh[lsel] += gq1;
-        gqk = gq1 = 0.0;
-        adj_rev_line(cu, nu[lsel], ldx2, ldy2, gm.dxv, gm.dyv, p.bw, p.freeze, gju, gqk, gq1);
-        gcu += gqk;
-        gnu[lsel] += gq1;
-        gqk = gq1 = 0.0;
-        adj_rev_line(cv, nv[lsel], ldx2, ldy2, gm.dxv, gm.dyv, p.bw, p.freeze, gjv, gqk, gq1);
-        gcv += gqk;
-        gnv[lsel] += gq1;
     }
     // reverse: the cells -> the raw state of each slot
     if (keep0) {
@@ -1504,23 +1549,20 @@ ADJ_HD void adj_edge_vjp(const AdjView &m, int k, int i, const double L[4], cons
     gC[3] += gzc;
 }
 
-// adj_bwd_flux by reverse mode: the same additions from one sweep of
-// adj_edge_vjp per edge.
-ADJ_HD void adj_bwd_flux_rev(const AdjView &m, const double *S, const unsigned char *fl,
-                             const double *E, const double *lam_ex, int k, double *lamE,
-                             double *lamS, double *zbar)
+// The flux of triangle k with centroid values c by reverse mode: the adjoints
+// lex of its explicit updates -> its own edge values' (own(i, g)), those of
+// the neighbour's across each interior edge (other(i, g); g: w, h, uh, vh) and
+// its centroid values' (lc), from one sweep of adj_edge_vjp per edge.
+template <class Own, class Other>
+ADJ_HD void adj_flux_vjp(const AdjView &m, const double *E, const double c[4],
+                         const double lex[3], int k, const int v[3], Own own, Other other,
+                         double lc[4])
 {
-    const int N = m.N;
-    int v[3], sur[3];
-    adj_neighbours(m, k, v, sur);
-    double q[4] = {S[4 * k], S[4 * k + 1], S[4 * k + 2], S[4 * k + 3]}, c[4];
-    const unsigned f = fl[k];
-    adj_centroid<double>(q, f, c);
     const double inv_area = 1.0 / m.area[k];
-    const double lw = lam_ex[k] * inv_area, lx = lam_ex[N + k] * inv_area;
-    const double ly = lam_ex[2 * (size_t)N + k] * inv_area;
+    const double lw = lex[0] * inv_area, lx = lex[1] * inv_area;
+    const double ly = lex[2] * inv_area;
     const double lo[5] = {lw, lx, ly, -lx, -ly};
-    double lc[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int t = 0; t < 4; t++) lc[t] = 0.0;
     for (int i = 0; i < 3; i++) {
         double L[4], R[4], dir[3];
         int kind;
@@ -1528,22 +1570,40 @@ ADJ_HD void adj_bwd_flux_rev(const AdjView &m, const double *S, const unsigned c
         double gL[4] = {0.0, 0.0, 0.0, 0.0}, gR[4] = {0.0, 0.0, 0.0, 0.0};
         double gC[4] = {0.0, 0.0, 0.0, 0.0};
         adj_edge_vjp(m, k, i, L, R, c, kind, dir, lo, gL, gR, gC);
-        const size_t own = (size_t)i * N + k;
-        for (int t = 0; t < 4; t++)
-            if (gL[t] != 0.0) adj_add(lamE + (size_t)t * 3 * N + own, gL[t]);
-        if (kind < 0) {
-            const size_t nbs = (size_t)(v[i] & 3) * N + (v[i] >> 2);
-            for (int t = 0; t < 4; t++)
-                if (gR[t] != 0.0) adj_add(lamE + (size_t)t * 3 * N + nbs, gR[t]);
-        }
+        own(i, gL);
+        if (kind < 0) other(i, gR);
         for (int t = 0; t < 4; t++) lc[t] += gC[t];
     }
+}
+
+// adj_bwd_flux by reverse mode
+ADJ_HD void adj_bwd_flux_rev(const AdjView &m, const double *S, const unsigned char *fl,
+                             const double *E, const double *lam_ex, int k, double *lamE,
+                             double *lamS, double *zbar)
+{
+    const int N = m.N;
+    int v[3], sur[3];
+    adj_neighbours(m, k, v, sur);
+    double q[4] = {S[4 * k], S[4 * k + 1], S[4 * k + 2], S[4 * k + 3]}, c[4], lc[4];
+    const unsigned f = fl[k];
+    adj_centroid<double>(q, f, c);
+    const double lex[3] = {lam_ex[k], lam_ex[N + k], lam_ex[2 * (size_t)N + k]};
+    const auto own = [&](int i, const double g[4]) {
+        for (int t = 0; t < 4; t++)
+            if (g[t] != 0.0) lamE[(size_t)t * 3 * N + (size_t)i * N + k] += g[t];
+    };
+    const auto other = [&](int i, const double g[4]) {
+        for (int t = 0; t < 4; t++)
+            if (g[t] != 0.0)
+                lamE[(size_t)t * 3 * N + (size_t)(v[i] & 3) * N + (v[i] >> 2)] += g[t];
+    };
+    adj_flux_vjp(m, E, c, lex, k, v, own, other, lc);
     adj_scatter_centroid(f, lc, lamS, zbar, N, k);
 }
 
 // Extrapolation of triangle k: lamE (its edge values) -> the adjoints of the
 // raw state of k and of its surrogate neighbours (and of their beds), stored
-// per stencil slot: X[(4 slot + c) N + k], slot 0 for k itself (a boundary
+// per stencil slot: X[4 (slot N + k) + c], slot 0 for k itself (a boundary
 // edge's surrogate is k and counts there), slot 1 + i for the neighbour
 // across edge i, c over w, uh, vh, z. adj_gather_extrap then sums each
 // triangle's contributions in a fixed order, so the result does not depend on
@@ -1567,7 +1627,7 @@ ADJ_HD void adj_bwd_extrap(const AdjView &m, const double *S, const unsigned cha
             lo[4 * i + t] = lamE[(size_t)t * 3 * N + (size_t)i * N + k];
             any = any || lo[4 * i + t] != 0.0;
         }
-    for (int j = 0; j < 16; j++) X[(size_t)j * N + k] = 0.0;
+    for (int j = 0; j < 16; j++) X[4 * ((size_t)(j >> 2) * N + k) + (j & 3)] = 0.0;
     if (!any) return;
     unsigned f[4];
     for (int j = 0; j < 4; j++) f[j] = fl[id[j]];
@@ -1607,26 +1667,21 @@ ADJ_HD void adj_bwd_extrap(const AdjView &m, const double *S, const unsigned cha
             for (int i = 0; i < 3; i++)
                 a += lo[4 * i] * ew[i].d[c] + lo[4 * i + 1] * eh[i].d[c] +
                      lo[4 * i + 2] * euh[i].d[c] + lo[4 * i + 3] * evh[i].d[c];
-            X[(size_t)(4 * slot + c0 + c) * N + k] = a;
+            X[4 * ((size_t)slot * N + k) + c0 + c] = a;
         }
     }
 }
 
-// adj_bwd_extrap by reverse mode: the same stores into X from one sweep of
-// adj_extrap_vjp.
-ADJ_HD void adj_bwd_extrap_rev(const AdjView &m, const double *S, const unsigned char *fl,
-                               const double *lamE, int k, double *X)
+// adj_bwd_extrap by reverse mode, from one sweep of adj_extrap_vjp: the
+// adjoints lo of the edge values (4 per edge: w, h, uh, vh) -> the same stores
+// into X.
+ADJ_HD void adj_store_extrap(const AdjView &m, const double *S, const unsigned char *fl,
+                             const double lo[12], int k, const int v[3], const int sur[3],
+                             double *X)
 {
     const int N = m.N;
-    int v[3], sur[3];
-    adj_neighbours(m, k, v, sur);
-    double lo[12];
     bool any = false;
-    for (int i = 0; i < 3; i++)
-        for (int t = 0; t < 4; t++) {
-            lo[4 * i + t] = lamE[(size_t)t * 3 * N + (size_t)i * N + k];
-            any = any || lo[4 * i + t] != 0.0;
-        }
+    for (int j = 0; j < 12; j++) any = any || lo[j] != 0.0;
     double out[16];
     for (int j = 0; j < 16; j++) out[j] = 0.0;
     if (any) {
@@ -1651,24 +1706,48 @@ ADJ_HD void adj_bwd_extrap_rev(const AdjView &m, const double *S, const unsigned
                 else out[c] += gs[4 * (i + 1) + c];
             }
     }
-    for (int j = 0; j < 16; j++) X[(size_t)j * N + k] = out[j];
+    for (int j = 0; j < 16; j++) X[4 * ((size_t)(j >> 2) * N + k) + (j & 3)] = out[j];
+}
+
+ADJ_HD void adj_bwd_extrap_rev(const AdjView &m, const double *S, const unsigned char *fl,
+                               const double *lamE, int k, double *X)
+{
+    const size_t N = m.N;
+    int v[3], sur[3];
+    adj_neighbours(m, k, v, sur);
+    double lo[12];
+    for (int i = 0; i < 3; i++)
+        for (int t = 0; t < 4; t++) lo[4 * i + t] = lamE[t * 3 * N + i * N + k];
+    adj_store_extrap(m, S, fl, lo, k, v, sur, X);
 }
 
 // The extrapolation adjoints that reach triangle t (adj_bwd_extrap's X): its
 // own stencil's, then those of its neighbours across edges 0, 1, 2, added to
-// the state adjoint lamS and the bed adjoint zbar.
+// the adjoints of its state ls and its bed lz.
+ADJ_HD void adj_sum_extrap(const AdjView &m, const double *X, int t, const int v[3], double ls[3],
+                           double &lz)
+{
+    const int N = m.N;
+    double a[4];
+    for (int c = 0; c < 4; c++) a[c] = X[4 * (size_t)t + c];
+    for (int i = 0; i < 3; i++) {
+        if (v[i] < 0) continue;
+        const double *x = X + 4 * ((size_t)(1 + (v[i] & 3)) * N + (v[i] >> 2));
+        for (int c = 0; c < 4; c++) a[c] += x[c];
+    }
+    for (int c = 0; c < 3; c++)
+        if (!(a[c] == 0.0)) ls[c] += a[c];
+    if (!(a[3] == 0.0)) lz += a[3];
+}
+
 ADJ_HD void adj_gather_extrap(const AdjView &m, const double *X, int t, double *lamS,
                               double *zbar)
 {
     const int N = m.N;
     int v[3], sur[3];
     adj_neighbours(m, t, v, sur);
-    for (int c = 0; c < 4; c++) {
-        double a = X[(size_t)c * N + t];
-        for (int i = 0; i < 3; i++)
-            if (v[i] >= 0) a += X[(size_t)(4 * (1 + (v[i] & 3)) + c) * N + (v[i] >> 2)];
-        if (a == 0.0) continue;
-        if (c < 3) lamS[(size_t)c * N + t] += a;
-        else zbar[t] += a;
-    }
+    double ls[3] = {lamS[t], lamS[N + t], lamS[2 * (size_t)N + t]}, lz = zbar[t];
+    adj_sum_extrap(m, X, t, v, ls, lz);
+    for (int c = 0; c < 3; c++) lamS[(size_t)c * N + t] = ls[c];
+    zbar[t] = lz;
 }

@@ -239,14 +239,15 @@ struct AdjRun {
     DeQ *S1 = nullptr;         // first-stage state of the step being reversed
     double *E0 = nullptr, *E1 = nullptr, *ex0 = nullptr, *ex1 = nullptr;
     unsigned char *f0 = nullptr, *f1 = nullptr;
-    double *lam = nullptr, *lamn = nullptr, *lam1 = nullptr, *lamE = nullptr, *lam_ex = nullptr;
-    double *lamX = nullptr;    // [16][N] the extrapolation adjoint per stencil slot
+    double *lam = nullptr, *lam1 = nullptr;
+    double *lamE = nullptr, *lamN = nullptr;   // [3][N][4] adjoints of edge values: own, neighbours'
+    double *lamX = nullptr;    // [4][N][4] the extrapolation adjoint per stencil slot
     double *zbar = nullptr, *nbar = nullptr, *rec = nullptr;
     int *gauges = nullptr;
     unsigned long long *neg = nullptr;   // fix_negative count of recomputed steps (ignored)
     ~AdjRun()
     {
-        void *p[] = {ckpt, seg, S1, E0, E1, ex0, ex1, f0, f1, lam, lamn, lam1, lamE, lam_ex, lamX,
+        void *p[] = {ckpt, seg, S1, E0, E1, ex0, ex1, f0, f1, lam, lam1, lamE, lamN, lamX,
                      zbar, nbar, rec, gauges, neg};
         for (void *q : p)
             if (q) hipFree(q);
@@ -2208,21 +2209,22 @@ static AdjView adj_view(const anuga_domain *d, double dt)
     return m;
 }
 
-// one DE1 step of X in place with the timestep already in ctl->dt (the
-// production kernels; d->B, d->E, d->flags and d->ex serve as scratch)
-static void step_fixed(anuga_domain *d, DeQ *X)
+// one DE1 step of X to `out` (which may be X) with the timestep already in
+// ctl->dt (the production kernels; d->B, d->E, d->flags and d->ex serve as
+// scratch)
+static void step_fixed(anuga_domain *d, DeQ *X, DeQ *out)
 {
     if (fused(d)) {
         launch_xflux(d, 0, X);
         launch_update(d, X, d->B);
-        launch_xflux(d, 1, d->B, X, X);
+        launch_xflux(d, 1, d->B, X, out);
         return;
     }
     launch_extrapolate(d, X);
     launch_flux(d, 0, X);
     launch_update(d, X, d->B);
     launch_extrapolate(d, d->B);
-    launch_flux(d, 1, d->B, X, X);
+    launch_flux(d, 1, d->B, X, out);
 }
 
 // the stage quantities of the step from X into the adjoint's buffers
@@ -2232,54 +2234,37 @@ static void adj_stages(anuga_domain *d, AdjRun *a, const DeQ *X)
     const size_t N = d->N;
     DeBoundary bc{d->bkind, d->bval, d->M, 0};
     const DeParams p = dev_params(d->P);
-    double *pm = part_row(d, DE_P_MASS);
-    hipLaunchKernelGGL(de_extrapolate<double>, g, b, 0, d->stream, dev_mesh(d), p, X, a->E0, a->f0,
-                       pm, d->ctl);
-    hipLaunchKernelGGL((de_flux<double, 0>), g, b, 0, d->stream, dev_mesh(d), p, X, d->eta,
-                       a->E0, bc, a->f0, a->ex0, a->ex0 + N, a->ex0 + 2 * N, nullptr, nullptr,
-                       d->ctl, d->ctl,
-                       part_row(d, DE_P_DT), part_row(d, DE_P_BF0), a->neg);
-    hipLaunchKernelGGL((de_update<false, DE_DT_GIVEN>), g, b, 0, d->stream, d->scen, p, X, d->eta,
-                       a->f0, a->ex0, a->ex0 + N, a->ex0 + 2 * N, d->ctl, a->S1, a->neg, nullptr,
-                       0.0, DeStepEnd{}, nullptr, 0, nullptr);
-    hipLaunchKernelGGL(de_extrapolate<double>, g, b, 0, d->stream, dev_mesh(d), p, a->S1, a->E1,
-                       a->f1, pm, d->ctl);
-    hipLaunchKernelGGL((de_flux<double, 0>), g, b, 0, d->stream, dev_mesh(d), p, a->S1, d->eta,
-                       a->E1, bc, a->f1, a->ex1, a->ex1 + N, a->ex1 + 2 * N, nullptr, nullptr,
-                       d->ctl, d->ctl,
-                       part_row(d, DE_P_DT), part_row(d, DE_P_BF0), a->neg);
+    const DeMesh m = dev_mesh(d);
+    double *pm = part_row(d, DE_P_MASS), *pt = part_row(d, DE_P_DT), *pf = part_row(d, DE_P_BF0);
+    hipLaunchKernelGGL(de_extrapolate<double>, g, b, 0, d->stream, m, p, X, a->E0, a->f0, pm,
+                       d->ctl);
+    hipLaunchKernelGGL((de_flux<double, 0, false, true>), g, b, 0, d->stream, m, p, X, d->eta,
+                       a->E0, bc, a->f0, a->ex0, a->ex0 + N, a->ex0 + 2 * N, nullptr, a->S1,
+                       d->ctl, d->ctl, pt, pf, a->neg);
+    hipLaunchKernelGGL(de_extrapolate<double>, g, b, 0, d->stream, m, p, a->S1, a->E1, a->f1, pm,
+                       d->ctl);
+    hipLaunchKernelGGL((de_flux<double, 0>), g, b, 0, d->stream, m, p, a->S1, d->eta, a->E1, bc,
+                       a->f1, a->ex1, a->ex1 + N, a->ex1 + 2 * N, nullptr, nullptr, d->ctl, d->ctl,
+                       pt, pf, a->neg);
 }
 
 // lam (adjoint of the step's result, [3][N]) -> adjoint of its start X
 static int adj_step(anuga_domain *d, AdjRun *a, const DeQ *X)
 {
     const dim3 g(d->nblocks), b(DE_BLOCK);
-    const size_t N = d->N;
     const AdjView m = adj_view(d, a->dt);
     const double *Sx = reinterpret_cast<const double *>(X);
     const double *S1 = reinterpret_cast<const double *>(a->S1);
     adj_stages(d, a, X);
-    // the final saxpy: half to the step's start directly, half through the stages
-    hipLaunchKernelGGL(adj_k_scale, dim3((3 * N + DE_BLOCK - 1) / DE_BLOCK), b, 0, d->stream,
-                       (int)(3 * N), 0.5, a->lam, a->lamn);
-    HIPCHK(d, hipMemsetAsync(a->lam1, 0, 3 * N * sizeof(double), d->stream));
     // second stage: S2 = advance(S1)
-    hipLaunchKernelGGL(adj_k_advance, g, b, 0, d->stream, m, S1, a->f1, a->ex1, a->ex1 + N,
-                       a->ex1 + 2 * N, a->lam, 0.5, a->lam1, a->zbar, a->nbar, a->lam_ex);
-    HIPCHK(d, hipMemsetAsync(a->lamE, 0, 12 * N * sizeof(double), d->stream));
-    hipLaunchKernelGGL(adj_k_flux, g, b, 0, d->stream, m, S1, a->f1, a->E1, a->lam_ex, a->lamE,
-                       a->lam1, a->zbar);
-    hipLaunchKernelGGL(adj_k_extrap, g, b, 0, d->stream, m, S1, a->f1, a->lamE, a->lamX);
-    hipLaunchKernelGGL(adj_k_extrap_gather, g, b, 0, d->stream, m, a->lamX, a->lam1, a->zbar);
+    hipLaunchKernelGGL(adj_k_stage<true>, g, b, 0, d->stream, m, S1, a->f1, a->E1, a->ex1,
+                       a->lamX, a->lam, a->lam1, a->lamE, a->lamN, a->zbar, a->nbar);
+    hipLaunchKernelGGL(adj_k_extrap, g, b, 0, d->stream, m, S1, a->f1, a->lamE, a->lamN, a->lamX);
     // first stage: S1 = advance(X)
-    hipLaunchKernelGGL(adj_k_advance, g, b, 0, d->stream, m, Sx, a->f0, a->ex0, a->ex0 + N,
-                       a->ex0 + 2 * N, a->lam1, 1.0, a->lamn, a->zbar, a->nbar, a->lam_ex);
-    HIPCHK(d, hipMemsetAsync(a->lamE, 0, 12 * N * sizeof(double), d->stream));
-    hipLaunchKernelGGL(adj_k_flux, g, b, 0, d->stream, m, Sx, a->f0, a->E0, a->lam_ex, a->lamE,
-                       a->lamn, a->zbar);
-    hipLaunchKernelGGL(adj_k_extrap, g, b, 0, d->stream, m, Sx, a->f0, a->lamE, a->lamX);
-    hipLaunchKernelGGL(adj_k_extrap_gather, g, b, 0, d->stream, m, a->lamX, a->lamn, a->zbar);
-    std::swap(a->lam, a->lamn);
+    hipLaunchKernelGGL(adj_k_stage<false>, g, b, 0, d->stream, m, Sx, a->f0, a->E0, a->ex0,
+                       a->lamX, a->lam, a->lam1, a->lamE, a->lamN, a->zbar, a->nbar);
+    hipLaunchKernelGGL(adj_k_extrap, g, b, 0, d->stream, m, Sx, a->f0, a->lamE, a->lamN, a->lamX);
+    hipLaunchKernelGGL(adj_k_extrap_gather, g, b, 0, d->stream, m, a->lamX, a->lam, a->zbar);
     return launch_check(d);
 }
 
@@ -3789,11 +3774,10 @@ int anuga_adjoint_record(anuga_domain *d, int64_t nsteps, double dt, int64_t che
     ACHK(dalloc(&a->f0, N));
     ACHK(dalloc(&a->f1, N));
     ACHK(dalloc(&a->lam, n3));
-    ACHK(dalloc(&a->lamn, n3));
     ACHK(dalloc(&a->lam1, n3));
     ACHK(dalloc(&a->lamE, 4 * n3));
     ACHK(dalloc(&a->lamX, 16 * (size_t)N));
-    ACHK(dalloc(&a->lam_ex, n3));
+    ACHK(dalloc(&a->lamN, 4 * n3));
     ACHK(dalloc(&a->zbar, N));
     ACHK(dalloc(&a->nbar, N));
     ACHK(dalloc(&a->rec, std::max<int64_t>(a->nobs * G, 1)));
@@ -3806,7 +3790,7 @@ int anuga_adjoint_record(anuga_domain *d, int64_t nsteps, double dt, int64_t che
     hipLaunchKernelGGL(de_set_dt, dim3(1), dim3(64), 0, d->stream, d->ctl, dt);
     HIPCHK(d, hipMemcpyAsync(a->ckpt, d->A, N * sizeof(DeQ), hipMemcpyDeviceToDevice, d->stream));
     for (int64_t s = 1; s <= nsteps; s++) {
-        step_fixed(d, d->A);
+        step_fixed(d, d->A, d->A);
         if (s % a->every == 0 && s < nsteps)
             HIPCHK(d, hipMemcpyAsync(a->ckpt + (s / a->every) * (size_t)N, d->A, N * sizeof(DeQ),
                                      hipMemcpyDeviceToDevice, d->stream));
@@ -3847,8 +3831,7 @@ int anuga_adjoint_gradient(anuga_domain *d, const double *dloss_dstage, double *
                                  hipMemcpyDeviceToDevice, d->stream));
         for (int64_t t = 1; t < s1 - s0; t++) {
             DeQ *x = a->seg + t * (size_t)N;
-            HIPCHK(d, hipMemcpyAsync(x, x - N, N * sizeof(DeQ), hipMemcpyDeviceToDevice, d->stream));
-            step_fixed(d, x);
+            step_fixed(d, x - N, x);
         }
         for (int64_t s = s1; s > s0; s--) {
             if (a->G > 0 && s % a->obs_every == 0)

@@ -788,10 +788,11 @@ __device__ __forceinline__ void de_edge_flux(const DeMesh &m, const DeParams &p,
 // SUBSTEP 0: writes explicit updates; SUBSTEP > 0: advances with the
 // scenario's dt and writes de_rk_combine<SUBSTEP>(advanced, bk) to out (out
 // may be bk, or q itself: each thread reads its own q and bk before writing).
+// STAGE: substep 0 writes the explicit updates and advances with dt to out.
 // GENERAL: the instantiation for riverwalls, low_froude 1/2 and sloped
 // friction (runtime switches), so that the common kernel carries none of
 // their registers.
-template <class T, int SUBSTEP, bool GENERAL = false>
+template <class T, int SUBSTEP, bool GENERAL = false, bool STAGE = false>
 __global__ void __launch_bounds__(DE_BLOCK)
 de_flux(DeMesh m, DeParams p, const DeQ *q, const double *__restrict__ eta,
         const T *__restrict__ E, DeBoundary bc, const unsigned char *__restrict__ flags,
@@ -806,7 +807,7 @@ de_flux(DeMesh m, DeParams p, const DeQ *q, const double *__restrict__ eta,
     DeControl *cb = de_ctl(ctl, m.scen, lb);
     if (cb->done) return;
     int *err = &cb->status;
-    const double dt = SUBSTEP ? dctl[cb - ctl].dt : 0.0;
+    const double dt = SUBSTEP || STAGE ? dctl[cb - ctl].dt : 0.0;
     const int N = m.N;
     const int k = lb * DE_BLOCK + threadIdx.x;
     double dtmin = 1.0e100, bflux = 0.0;
@@ -846,6 +847,8 @@ de_flux(DeMesh m, DeParams p, const DeQ *q, const double *__restrict__ eta,
             exw[k] = sw;
             exuh[k] = sx;
             exvh[k] = sy;
+            if constexpr (STAGE)
+                out[k] = de_advance(c, eta[k], sw, sx, sy, dt, p, err, nneg);
         } else {
             DeSlope sl{false, 0.0, 0.0};
             if constexpr (GENERAL)

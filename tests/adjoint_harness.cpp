@@ -170,7 +170,7 @@ void harness_adjoint(int N, int M, const int *nb, const double *cen, const doubl
     }
 }
 
-// the extrapolation's vector-Jacobian product per stencil slot (X, [16][N])
+// the extrapolation's vector-Jacobian product per stencil slot (X, [4][N][4])
 // for the edge-value adjoints wt ([4][3][N]), by forward-mode duals and by
 // the reverse sweep
 void harness_extrap_products(int N, int M, const int *nb, const double *cen, const double *gx,
@@ -188,6 +188,29 @@ void harness_extrap_products(int N, int M, const int *nb, const double *cen, con
     }
 }
 
+
+// the update's vector-Jacobian product for n cells (in: centroid w, uh, vh, z,
+// friction, three explicit updates; lam: w, uh, vh of the result) by
+// forward-mode duals and by the reverse sweep: 8 values per cell
+void harness_advance_products(int n, const double *prm, double dt, const double *in,
+                              const double *lam, double *out_dual, double *out_rev)
+{
+    typedef Dual<8> D;
+    const AdjParams p{prm[0], prm[1], prm[2], prm[3], prm[4], prm[5], prm[6], prm[7], prm[8],
+                      g_freeze};
+    for (int k = 0; k < n; k++) {
+        const double *x = in + 8 * k, *l = lam + 3 * k;
+        D d[8], o[3];
+        for (int j = 0; j < 8; j++) {
+            d[j] = D(x[j]);
+            d[j].d[j] = 1.0;
+        }
+        adj_advance_cell<D>(d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7], dt, p, o);
+        for (int j = 0; j < 8; j++)
+            out_dual[8 * k + j] = l[0] * o[0].d[j] + l[1] * o[1].d[j] + l[2] * o[2].d[j];
+        adj_advance_vjp(x, x[4], x + 5, dt, p, l, out_rev + 8 * k);
+    }
+}
 
 // the flux's vector-Jacobian product both ways on the edge values of S:
 // wt [3][N] weights the explicit updates; out_* receive lamE [4][3][N] then

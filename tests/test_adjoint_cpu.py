@@ -410,3 +410,38 @@ def test_reverse_flux_product_equals_dual(harness, case):
         scale = np.abs(d).max()
         assert scale > 0
         assert np.max(np.abs(r - d)) <= 1e-11 * scale, np.max(np.abs(r - d)) / scale
+
+
+@pytest.mark.parametrize("case", ["wet", "shallow", "still", "drained"])
+def test_reverse_update_product_equals_dual(harness, case):
+    """The update's hand-written reverse sweep (adj_advance_vjp) gives the
+    forward-mode dual product's adjoints to rounding: with friction, below the
+    depth and the friction coefficient that switch it off, with a momentum
+    component or both zero, and where the update is reset to the bed."""
+    rng = np.random.default_rng(11)
+    n = 300
+    x = np.zeros((n, 8))
+    x[:, 3] = rng.uniform(-1.0, 1.0, n)
+    x[:, 0] = x[:, 3] + rng.uniform(0.05, 2.0, n)
+    x[:, 1:3] = rng.uniform(-1.0, 1.0, (n, 2))
+    x[:, 4] = rng.uniform(0.01, 0.05, n)
+    x[:, 5:] = rng.uniform(-0.5, 0.5, (n, 3))
+    if case == "shallow":
+        x[::2, 0] = x[::2, 3] + 1.0e-7
+        x[1::2, 4] = 0.0
+    elif case == "still":
+        x[::3, 1] = 0.0
+        x[1::3, 1:3] = 0.0
+    elif case == "drained":
+        x[:, 5] = -30.0
+    lam = rng.standard_normal((n, 3))
+    dual, rev = np.zeros((n, 8)), np.zeros((n, 8))
+    dp = lambda a: a.ctypes.data_as(C.POINTER(C.c_double))
+    harness.harness_advance_products(n, DE1.ctypes.data_as(C.POINTER(C.c_double)),
+                                     C.c_double(0.1), dp(x), dp(lam), dp(dual), dp(rev))
+    for j in range(8):
+        # some 30 roundings of 2^-53 in terms that are not above the greatest
+        # adjoint of their input by more than the cancellation of the friction
+        # term with its quotient (a factor 1e2 here)
+        scale = max(np.abs(dual[:, j]).max(), 1.0e-300)
+        assert np.max(np.abs(rev[:, j] - dual[:, j])) <= 1e-12 * scale, j
