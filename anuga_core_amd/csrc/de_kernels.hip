@@ -1445,6 +1445,13 @@ __device__ __forceinline__ void de_tile_edge(const DeMesh &m, const DeParams &p,
         n2 = m.ny[ia * N + ka];
         length = m.len[ia * N + ka];
     }
+    // the CFL radii, requested before the flux that decides whether they are
+    // used: 206.0 -> 200.7 us substep 0 at 4M triangles
+    double ra = 0.0, rb = 0.0;
+    if (SUBSTEP == 0) {
+        ra = m.radius[ka];
+        rb = halo ? ra : m.radius[k0 + nb];
+    }
     const double zl = ql0 - hle, zr = qr0 - hre;
     const double z_half = fmax(zl, zr);
     const double h_left = fmax(hle + zl - z_half, 0.0);
@@ -1467,7 +1474,7 @@ __device__ __forceinline__ void de_tile_edge(const DeMesh &m, const DeParams &p,
     const bool cfl = SUBSTEP == 0 && speed > eps;
     if (cfl) {
         tt = 1.0 / fmax(speed, eps);
-        dtmin = fmin(dtmin, m.radius[ka] * tt);
+        dtmin = fmin(dtmin, ra * tt);
     }
     if (!halo) {
         // the other side: its own depths and bed, the same flux
@@ -1476,7 +1483,7 @@ __device__ __forceinline__ void de_tile_edge(const DeMesh &m, const DeParams &p,
                                                  (hre + hcb) * (zr - zcb)) + pflux);
         R[rs] = n1 * pgb;
         R[2 * rs] = n2 * pgb;
-        if (cfl) dtmin = fmin(dtmin, m.radius[k0 + nb] * tt);
+        if (cfl) dtmin = fmin(dtmin, rb * tt);
     }
 }
 
@@ -1509,7 +1516,8 @@ __device__ __forceinline__ void de_tile_edge(const DeMesh &m, const DeParams &p,
 // CU). Against gathering every neighbour's state, centroid and vertices from
 // memory in phases 1 and 2 (4M triangles): 826 -> 403 MB of HBM reads per
 // launch, 960 -> 274 cache accesses and 1548 -> 1436 VALU instructions per
-// wave, 251 -> 212 us (substep 0) and 280 -> 235 us (substep 1). A workgroup
+// wave, 251 -> 212 us (substep 0) and 280 -> 235 us (substep 1); with two
+// divisions a limiter and the CFL radii requested early 201 and 227. A workgroup
 // of five waves, the fifth for the halo in phase 1, took 410 us: its waves do
 // not spread evenly over four SIMDs, so two workgroups fit a CU instead of
 // four. 128 triangles per tile: 245 us.
