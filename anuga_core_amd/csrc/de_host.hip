@@ -235,7 +235,8 @@ struct AdjRun {
     int G = 0;
     double dt = 0.0;
     DeQ *ckpt = nullptr;       // [nckpt][N]: state at steps 0, every, 2 every, ...
-    DeQ *seg = nullptr;        // [every][N]: the states of one segment, recomputed
+    DeQ *seg = nullptr;        // [every][N]: the states of one segment
+    int64_t held = -1;         // which one seg holds (the last one, as recorded)
     DeQ *S1 = nullptr;         // first-stage state of the step being reversed
     double *E0 = nullptr, *E1 = nullptr, *ex0 = nullptr, *ex1 = nullptr;
     unsigned char *f0 = nullptr, *f1 = nullptr;
@@ -3789,17 +3790,26 @@ int anuga_adjoint_record(anuga_domain *d, int64_t nsteps, double dt, int64_t che
     ensure_live(d);
     hipLaunchKernelGGL(de_set_dt, dim3(1), dim3(64), 0, d->stream, d->ctl, dt);
     HIPCHK(d, hipMemcpyAsync(a->ckpt, d->A, N * sizeof(DeQ), hipMemcpyDeviceToDevice, d->stream));
+    // the last segment's states are left where the adjoint wants them first
+    const int64_t last = (a->nckpt - 1) * a->every;
     for (int64_t s = 1; s <= nsteps; s++) {
-        step_fixed(d, d->A, d->A);
+        if (s - 1 == last)
+            HIPCHK(d, hipMemcpyAsync(a->seg, d->A, N * sizeof(DeQ), hipMemcpyDeviceToDevice,
+                                     d->stream));
+        step_fixed(d, s > last ? a->seg + (s - 1 - last) * (size_t)N : d->A,
+                   s > last && s < nsteps ? a->seg + (s - last) * (size_t)N : d->A);
         if (s % a->every == 0 && s < nsteps)
             HIPCHK(d, hipMemcpyAsync(a->ckpt + (s / a->every) * (size_t)N, d->A, N * sizeof(DeQ),
                                      hipMemcpyDeviceToDevice, d->stream));
         if (G > 0 && s % obs_every == 0)
             hipLaunchKernelGGL(adj_k_gauges, dim3((G + 63) / 64), dim3(64), 0, d->stream, G,
-                               a->gauges, d->A, a->rec + (s / obs_every - 1) * (size_t)G);
+                               a->gauges, s > last && s < nsteps ? a->seg + (s - last) * (size_t)N
+                                                                 : d->A,
+                               a->rec + (s / obs_every - 1) * (size_t)G);
     }
     rc = launch_check(d);
     if (rc) return rc;
+    a->held = a->nckpt - 1;
     rc = sync_scalars(d);
     if (rc) return rc;
     if (G > 0)
@@ -3827,11 +3837,15 @@ int anuga_adjoint_gradient(anuga_domain *d, const double *dloss_dstage, double *
     hipLaunchKernelGGL(de_set_dt, dim3(1), dim3(64), 0, d->stream, d->ctl, a->dt);
     for (int64_t j = a->nckpt - 1; j >= 0; j--) {
         const int64_t s0 = j * a->every, s1 = std::min(s0 + a->every, a->nsteps);
-        HIPCHK(d, hipMemcpyAsync(a->seg, a->ckpt + j * (size_t)N, N * sizeof(DeQ),
-                                 hipMemcpyDeviceToDevice, d->stream));
-        for (int64_t t = 1; t < s1 - s0; t++) {
-            DeQ *x = a->seg + t * (size_t)N;
-            step_fixed(d, x - N, x);
+        if (a->held != j) {
+            a->held = -1;
+            HIPCHK(d, hipMemcpyAsync(a->seg, a->ckpt + j * (size_t)N, N * sizeof(DeQ),
+                                     hipMemcpyDeviceToDevice, d->stream));
+            for (int64_t t = 1; t < s1 - s0; t++) {
+                DeQ *x = a->seg + t * (size_t)N;
+                step_fixed(d, x - N, x);
+            }
+            a->held = j;
         }
         for (int64_t s = s1; s > s0; s--) {
             if (a->G > 0 && s % a->obs_every == 0)

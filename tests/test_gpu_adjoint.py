@@ -213,3 +213,27 @@ def test_torch_autograd_two_forwards_before_backward():
         gn, _, _ = d.adjoint_gradient(2.0 * rec)
         assert np.allclose(t.grad.numpy(), gn, rtol=1e-12, atol=1e-18)
     assert not np.allclose(na.grad.numpy(), nb.grad.numpy())
+
+
+@pytest.mark.parametrize("every", [1, 4, 7, 30, 50])
+def test_gpu_gradient_twice_from_one_record(every):
+    """The recorded run leaves its last segment's states where the adjoint
+    starts; a second gradient recomputes them from the checkpoint. The same
+    bits from both, and from any distance of checkpoints."""
+    print("adjoint twice, checkpoints every", every, flush=True)
+    mesh, q, bc = _wet_case(9)
+    init = _initial(mesh, q)
+    rng = np.random.default_rng(8)
+    gauges = rng.choice(mesh.number_of_triangles, 5, replace=False)
+    dL = rng.standard_normal((10, 5))
+    out = []
+    for distance in (10, every):
+        d = _domain(mesh, q, bc, init)
+        rec = d.adjoint_record(30, 0.15, gauges, 3, checkpoint_every=distance)
+        out.append([rec, d.get_quantity("stage").centroid_values.copy()])
+        out[-1] += list(d.adjoint_gradient(dL))
+        out.append(out[-1][:2] + list(d.adjoint_gradient(dL)))
+        d.close()
+    for o in out[1:]:
+        for a, b in zip(o, out[0]):
+            assert np.array_equal(a, b)
