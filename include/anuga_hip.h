@@ -399,8 +399,8 @@ typedef struct anuga_step_state {
  * generic_domain.py:1914-2051) with update_timestep evaluated on the device,
  * so the run needs one host synchronisation at its end. Stops early, exactly
  * where _evolve_base would yield (relative_yieldtime) or finish
- * (relative_finaltime - epsilon); the remaining launches are no-ops. One step
- * is captured once into a HIP graph and replayed (unless ANUGA_HIP_GRAPH=0 or
+ * (relative_finaltime - epsilon); the remaining launches are no-ops. Long runs
+ * replay a HIP graph of a few steps, captured once (unless ANUGA_HIP_GRAPH=0 or
  * kernel timing is on). dt_history (may be NULL) receives the timesteps taken. */
 int anuga_evolve_steps(anuga_domain *d, int64_t max_steps, const anuga_time_control *tc,
                        anuga_step_state *state, double *dt_history);
