@@ -979,8 +979,15 @@ static void flush_steps(anuga_domain *d, int64_t steps)
                        d->ctl, d->ctl2, (int)(steps & 1));
 }
 
+// The steps to come are not those recorded: the adjoint recomputes every segment.
+static void forward_changes(anuga_domain *d)
+{
+    if (d->adj) d->adj->held = -1;
+}
+
 static void drop_graph(anuga_domain *d)
 {
+    forward_changes(d);
     if (d->graph_exec) hipGraphExecDestroy(d->graph_exec);
     if (d->graph) hipGraphDestroy(d->graph);
     d->graph_exec = nullptr;
@@ -1958,6 +1965,7 @@ static int set_centroids(anuga_domain *d, int s, int quantity, const double *val
     const int slot = record_slot(quantity);
     if (slot < 0 && quantity != ANUGA_FRICTION)
         return fail(d, ANUGA_E_ARG, "quantity cannot be set");
+    if (slot < 0) forward_changes(d);
     double *v = d->eta + kb, *v2 = nullptr;
     int stride = 1;
     if (slot >= 0) {
@@ -2027,6 +2035,7 @@ static int set_boundary(anuga_domain *d, int s, const int32_t *kind, const doubl
             for (int q = 0; q < 3; q++) v[(size_t)q * M + j] = dirichlet_values[3 * (size_t)j + q];
         }
     }
+    forward_changes(d);
     HIPCHK(d, hipStreamSynchronize(d->stream));
     HIPCHK(d, hipMemcpy(d->bkind + mb, k.data(), M, hipMemcpyHostToDevice));
     if (d->hbkind.empty()) d->hbkind.assign(std::max(MT, 1), 0);
@@ -2455,6 +2464,7 @@ int anuga_set_boundary_values(anuga_domain *d, int64_t slot, const double *value
     if (slot < 0 || slot > 2) return fail(d, ANUGA_E_ARG, "slot must be 0, 1 or 2");
     if (M > 0 && !values) return fail(d, ANUGA_E_ARG, "values is NULL");
     if (M == 0) return ANUGA_OK;
+    forward_changes(d);
     // through pinned staging, in stream order: nothing waits unless the slot's
     // last upload may still be on its way
     if (d->bval_sent[slot]) {

@@ -1511,7 +1511,7 @@ __device__ __forceinline__ void de_tile_edge(const DeMesh &m, const DeParams &p,
 //     untouched edge values.
 // Each listed edge's results overwrite the LDS edge values only it reads.
 //
-// Bound by instruction issue: the SIMDs issue VALU work 70% of the time, four
+// Bound by instruction issue: the SIMDs issue VALU work some 80% of the time, four
 // waves each (105 VGPRs; 34 KB of LDS per workgroup allow four workgroups per
 // CU). Against gathering every neighbour's state, centroid and vertices from
 // memory in phases 1 and 2 (4M triangles): 826 -> 403 MB of HBM reads per

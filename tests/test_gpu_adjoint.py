@@ -237,3 +237,20 @@ def test_gpu_gradient_twice_from_one_record(every):
     for o in out[1:]:
         for a, b in zip(o, out[0]):
             assert np.array_equal(a, b)
+
+
+def test_gpu_gradient_after_a_change_of_friction():
+    """Friction set between a record and its gradient enters every recomputed
+    segment, the last one too: a second gradient, which recomputes all of
+    them, gives the same bits."""
+    print("adjoint after a change of friction", flush=True)
+    mesh, q, bc = _wet_case(9)
+    init = _initial(mesh, q)
+    gauges = np.arange(0, mesh.number_of_triangles, 40)
+    d = _domain(mesh, q, bc, init)
+    rec = d.adjoint_record(12, 0.15, gauges, 3, checkpoint_every=5)
+    dL = np.ones(rec.shape)
+    d.set_quantity("friction", 2.0 * q["friction"], location="centroids")
+    first, second = d.adjoint_gradient(dL), d.adjoint_gradient(dL)
+    for a, b in zip(first, second):
+        assert np.array_equal(a, b)
