@@ -65,7 +65,8 @@ class TileTables(C.Structure):
     _fields_ = [("capacity", C.c_int64), ("sizes", _ip), ("stencil", _u32), ("across", _u32),
                 ("nodes", _u32), ("cstart", _i32), ("hstart", _i32), ("estart", _i32),
                 ("esplit", _i32), ("nstart", _i32), ("cell", _i32), ("hstencil", _u32),
-                ("hcell", _u32), ("hnodes", _u32), ("edge", _u32), ("node", _dp)]
+                ("hcell", _u32), ("hnodes", _u32), ("edge", _u32), ("node", _dp),
+                ("crowded", C.POINTER(C.c_uint8))]
 
 
 class StepState(C.Structure):

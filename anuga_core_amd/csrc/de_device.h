@@ -117,6 +117,7 @@ struct DeTiles {
     const int *__restrict__ halo;       // the halo triangles of each tile
     const unsigned *__restrict__ slot;  // [N] 3 x 10 bits: halo slot of edge i, 1023: in the tile
     int hcap;                           // the largest halo (LDS stride)
+    const int *__restrict__ list;       // the tiles of the launch (null: all)
 };
 
 // The once-per-edge fused kernel's own tables of a tile (de_xflux_e). A tile's
@@ -148,10 +149,14 @@ struct DeTileX {
     const int *__restrict__ estart;        // [tiles + 1] offsets into edge
     const int *__restrict__ esplit;        // [tiles] the first edge to the halo
     const unsigned *__restrict__ edge;
+    // [tiles] 1: a crowded tile, beyond the limits below. It has no entries
+    // here and runs de_xflux, which gathers from memory. Null: there are none
+    const unsigned char *__restrict__ crowded;
 };
 // cells of a tile behind its own (their LDS fits in the edge values' place),
 // its halo edges (one thread each, a wave left for the tile's edges; 8 bits),
-// its nodes
+// its nodes. Compact tiles have about 90 cells, 50 halo edges and 170 nodes;
+// meshes graded by orders of magnitude have a few tiles beyond the limits.
 #define DE_XCELLS_MAX (DE_BLOCK < 511 ? DE_BLOCK : 1022 - DE_BLOCK)
 #define DE_XHALO_MAX (DE_BLOCK - 64 < 256 ? DE_BLOCK - 64 : 256)
 #define DE_XNODES_MAX 384

@@ -72,6 +72,14 @@ const int kHostHist = 512;
 // 40.3. Capturing 8 steps takes 45 to 100 us once.
 const int kGraphSteps = 8, kGraphMin = 64;   // an even count: see self_contained
 
+// Tiles within the once-per-edge kernel's limits from which a second launch
+// for the crowded ones pays (tables_pay). The launch takes 10 us a substep
+// however few they are; a tile that runs the gather kernel for its sake costs
+// 5 ns. A grid with a dozen crowded tiles, DE1, gather kernel alone and two
+// launches: 128.8 and 135.3 us a step at 0.64M triangles, 157.0 and 156.8 at
+// 0.81M, 209.8 and 178.1 at 1.0M, 401.5 and 297.8 at 2.0M.
+const int kCrowdedMin = 3200;
+
 }  // namespace
 
 // a Rate_operator's device data
@@ -91,13 +99,16 @@ struct RateOp {
 };
 
 // The tables of DeTileX for one scenario (its own triangle numbering; offsets
-// from 0). ok: within the kernel's limits; vertices: nodes were built.
+// from 0). vertices: nodes were built. crowded: per tile, 1 beyond the
+// kernel's limits; by_nodes: how many of those for their nodes alone.
 struct TileTables {
-    bool ok = false, vertices = false;
+    bool vertices = false;
     std::vector<int> cstart, cell, nstart, hstart, estart, esplit;
     std::vector<double2> node;
     std::vector<unsigned> stencil, across, nodes, hstencil, hcell, hnodes, edge;
-    int hecap = 0, ncap = 0;
+    std::vector<unsigned char> crowded;
+    int hecap = 0, ncap = 0, by_nodes = 0;
+    int ncrowded() const { return (int)std::count(crowded.begin(), crowded.end(), 1); }
 };
 
 struct anuga_domain {
@@ -137,6 +148,8 @@ struct anuga_domain {
     // scenario at upload), which that kernel assumes
     DeTileX tx{};
     std::vector<struct TileTables> ts_x;   // per scenario, until every mesh is set
+    int *xlist = nullptr;                  // the crowded tiles, in tx's allocation
+    int nxlist = 0;
     bool mirror = true;
     bool edge_once = true;     // ANUGA_HIP_EDGE_ONCE=0: the gather-every-side kernel
     // vertex geometry: that kernel forms edge offsets, normals and lengths
@@ -698,7 +711,15 @@ template <int SUB>
 static void launch_xflux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
 {
     DeBoundary bc{d->bkind, d->bval, d->M, d->bsstride};
-    DeTiles tl{d->tstart, d->thalo, d->tslot, d->hcap};
+    DeTiles tl{d->tstart, d->thalo, d->tslot, d->hcap, nullptr};
+    // the plain gather kernel, over nb tiles of tl
+    auto gather = [&](int nb) {
+        const size_t lds = (12 * (size_t)DE_BLOCK + 12 * (size_t)d->hcap) * sizeof(double);
+        hipLaunchKernelGGL(de_xflux<SUB>, dim3(nb), dim3(DE_BLOCK), lds, d->stream, dev_mesh(d),
+                           dev_params(d->P), S, d->eta, tl, bc, d->flags, d->ex[0], d->ex[1],
+                           d->ex[2], bk, out, d->kctl, d->kdt, part_row(d, DE_P_DT),
+                           bflux_row<SUB>(d), part_row(d, DE_P_MASS), d->dneg, (double *)d->E);
+    };
     if (d->mixed) {
         // FP64 centroid depth + 12 FP32 record components per triangle
         const size_t lds = ((size_t)DE_BLOCK + (size_t)d->hcap) * (sizeof(double) + 12 * sizeof(float));
@@ -729,13 +750,12 @@ static void launch_xflux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
                            d->ex[2], bk, out, d->kctl, d->kdt,
                            part_row(d, DE_P_DT), bflux_row<SUB>(d),
                            part_row(d, DE_P_MASS), d->dneg);
+        if (d->nxlist) {
+            tl.list = d->xlist;
+            gather(d->nxlist);
+        }
     } else {
-        const size_t lds = (12 * (size_t)DE_BLOCK + 12 * (size_t)d->hcap) * sizeof(double);
-        hipLaunchKernelGGL(de_xflux<SUB>, dim3(d->nblocks), dim3(DE_BLOCK), lds, d->stream,
-                           dev_mesh(d), dev_params(d->P), S, d->eta, tl, bc, d->flags, d->ex[0],
-                           d->ex[1], d->ex[2], bk, out, d->kctl, d->kdt,
-                           part_row(d, DE_P_DT), bflux_row<SUB>(d),
-                           part_row(d, DE_P_MASS), d->dneg, (double *)d->E);
+        gather(d->nblocks);
     }
 }
 
@@ -1351,8 +1371,8 @@ static int tile_halos(int N, const int4 *hn, std::vector<int> &start, std::vecto
 
 // DeTileX's tables of tiles [b0, b1) of one scenario of N triangles (nb records
 // hn, its own numbering), appended to x; vx: the triangles' vertex coordinates
-// [N][6], or NULL. False: a tile exceeds the kernel's limits.
-static bool tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1, TileTables &x)
+// [N][6], or NULL. A tile beyond the kernel's limits gets no entries.
+static void tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1, TileTables &x)
 {
     // place of each cell of a tile (its triangle id), by open addressing
     constexpr int HS = 4 * DE_XCELLS_MAX, NS = 4 * DE_XNODES_MAX;
@@ -1365,7 +1385,9 @@ static bool tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1,
     };
     for (int b = b0; b < b1; b++) {
         const int k0 = b * DE_BLOCK, k1 = std::min(N, k0 + DE_BLOCK);
-        const int cbase = (int)x.cell.size();
+        const int cbase = (int)x.cell.size(), ebase = (int)x.edge.size();
+        const int hbase = (int)x.hstencil.size(), nbase = (int)x.node.size();
+        const size_t kbase = x.stencil.size();
         std::fill(hkey.begin(), hkey.end(), -1);
         bool full = false;
         auto place = [&](int n) {   // cell index of triangle n, appended if new
@@ -1389,11 +1411,11 @@ static bool tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1,
         };
         // the edges inside the tile, then those to the halo, each by edge
         // index, then triangle (consecutive entries read consecutive data)
-        x.estart.push_back((int)x.edge.size());
         hedge.clear();
         std::vector<unsigned> across(k1 - k0, 0);
+        int esplit = ebase;
         for (int halo = 0; halo < 2; halo++) {
-            if (halo) x.esplit.push_back((int)x.edge.size());
+            if (halo) esplit = (int)x.edge.size();
             for (int i = 0; i < 3; i++)
                 for (int k = k0; k < k1; k++) {
                     const int v = nbr(k, i);
@@ -1403,7 +1425,10 @@ static bool tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1,
                     if (!halo) across[k - k0] |= (unsigned)j << (2 * i);
                     if (halo && out) {
                         const int he = (int)hedge.size();
-                        if (he >= DE_XHALO_MAX) return false;
+                        if (he >= DE_XHALO_MAX) {
+                            full = true;
+                            continue;
+                        }
                         across[k - k0] |= (unsigned)he << (6 + 8 * i);
                         hedge.push_back({n, j, 0});
                         x.edge.push_back(DE_TE_MAKE(k - k0, i, 1, 0, j));
@@ -1419,19 +1444,13 @@ static bool tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1,
             for (int i = 0; i < 3; i++) f[i] = nbr(k, i) >= 0 ? place(nbr(k, i) >> 2) : 1023;
             return word(f);
         };
-        x.hstart.push_back((int)x.hstencil.size());
         for (const auto &e : hedge) {
             x.hstencil.push_back(stencil(e[0]));
             x.hcell.push_back((unsigned)place(e[0]) | ((unsigned)e[1] << 10));
         }
         for (int k = k0; k < k1; k++) x.stencil.push_back(stencil(k));
-        if (full) return false;
         x.across.insert(x.across.end(), across.begin(), across.end());
-        x.cstart.push_back(cbase);
-        x.hecap = std::max(x.hecap, (int)hedge.size());
-        if (!vx) continue;
         // the distinct vertices (by their bits) of the tile and its halo
-        const int nbase = (int)x.node.size();
         std::fill(nval.begin(), nval.end(), -1);
         bool crowded = false;
         auto node = [&](int k, int c) {
@@ -1460,13 +1479,44 @@ static bool tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1,
             for (int c = 0; c < 3; c++) f[c] = node(k, c);
             return word(f);
         };
-        for (int k = k0; k < k1; k++) x.nodes.push_back(nodes(k));
-        for (const auto &e : hedge) x.hnodes.push_back(nodes(e[0]));
-        if (crowded) return false;
+        if (vx) {
+            for (int k = k0; k < k1; k++) x.nodes.push_back(nodes(k));
+            for (const auto &e : hedge) x.hnodes.push_back(nodes(e[0]));
+        }
+        x.crowded.push_back(full || crowded);
+        if (full || crowded) {
+            x.by_nodes += !full;
+            x.cell.resize(cbase);
+            x.edge.resize(ebase);
+            x.hstencil.resize(hbase);
+            x.hcell.resize(hbase);
+            std::fill(x.stencil.begin() + kbase, x.stencil.end(), 0x3fffffffu);
+            std::fill(x.across.begin() + kbase, x.across.end(), 0u);
+            if (vx) {
+                x.node.resize(nbase);
+                x.hnodes.resize(hbase);
+                std::fill(x.nodes.begin() + kbase, x.nodes.end(), 0u);
+            }
+            hedge.clear();
+            esplit = ebase;
+        }
+        x.cstart.push_back(cbase);
+        x.estart.push_back(ebase);
+        x.esplit.push_back(esplit);
+        x.hstart.push_back(hbase);
+        x.hecap = std::max(x.hecap, (int)hedge.size());
+        if (!vx) continue;
         x.nstart.push_back(nbase);
         x.ncap = std::max(x.ncap, (int)x.node.size() - nbase);
     }
-    return true;
+}
+
+// Whether nt tiles, nc of them crowded, run as two launches: the once-per-edge
+// kernel and, over the crowded tiles, the gather kernel. Otherwise all of them
+// run the gather kernel.
+static bool tables_pay(int nt, int nc)
+{
+    return nc == 0 || nt - nc >= kCrowdedMin;
 }
 
 // The tables of a whole scenario, its tiles cut on several threads.
@@ -1475,22 +1525,16 @@ static void scenario_tables(int N, const int4 *hn, const double *vx, TileTables 
     const int nt = (N + DE_BLOCK - 1) / DE_BLOCK;
     const int T = std::max(1, std::min<int>({(int)std::thread::hardware_concurrency(), 16, nt / 16}));
     std::vector<TileTables> part(T);
-    std::vector<char> ok(T, 0);
     auto work = [&](int i) {
         const int b0 = (int)((int64_t)nt * i / T), b1 = (int)((int64_t)nt * (i + 1) / T);
-        ok[i] = tile_tables(N, hn, vx, b0, b1, part[i]);
+        tile_tables(N, hn, vx, b0, b1, part[i]);
     };
     std::vector<std::thread> th;
     for (int i = 1; i < T; i++) th.emplace_back(work, i);
     work(0);
     for (auto &t : th) t.join();
     x = TileTables();
-    x.vertices = vx != nullptr;
-    for (int i = 0; i < T; i++)
-        if (!ok[i]) return;
-    x.ok = true;
     if (T == 1) std::swap(x, part[0]);
-    x.ok = true;
     x.vertices = vx != nullptr;
     auto join = [](auto &to, const auto &from) { to.insert(to.end(), from.begin(), from.end()); };
     auto offsets = [](std::vector<int> &to, const std::vector<int> &from, size_t base) {
@@ -1512,8 +1556,10 @@ static void scenario_tables(int N, const int4 *hn, const double *vx, TileTables 
             join(x.hcell, p.hcell);
             join(x.hnodes, p.hnodes);
             join(x.edge, p.edge);
+            join(x.crowded, p.crowded);
             x.hecap = std::max(x.hecap, p.hecap);
             x.ncap = std::max(x.ncap, p.ncap);
+            x.by_nodes += p.by_nodes;
         }
 }
 
@@ -1541,10 +1587,12 @@ static int scenario_tiles(anuga_domain *d, int s, const std::vector<int4> &hn, c
     for (int &n : d->ts_halo[s]) n += kb;
     d->ts_hcap[s] = hcap;
     if (!d->mixed && d->edge_once) {
-        scenario_tables(N, loc.data(), d->vgeom ? hv : nullptr, d->ts_x[s]);
-        // too many nodes in a tile: the stored records
-        if (!d->ts_x[s].ok && d->vgeom && hv) scenario_tables(N, loc.data(), nullptr, d->ts_x[s]);
-        for (int &n : d->ts_x[s].cell) n += kb;
+        TileTables &x = d->ts_x[s];
+        scenario_tables(N, loc.data(), d->vgeom ? hv : nullptr, x);
+        // too many tiles with too many nodes: the stored records
+        if (x.by_nodes && !tables_pay((int)x.crowded.size(), x.ncrowded()))
+            scenario_tables(N, loc.data(), nullptr, x);
+        for (int &n : x.cell) n += kb;
     }
     return ANUGA_OK;
 }
@@ -1554,18 +1602,31 @@ static void free_tile_tables(anuga_domain *d)
 {
     if (d->tx.cstart) hipFree(const_cast<int *>(d->tx.cstart));
     d->tx = DeTileX{};
+    d->xlist = nullptr;
+    d->nxlist = 0;
 }
 
-// Assemble every scenario's TileTables into DeTileX's device arrays; none
-// (hecap 0) if a scenario exceeds the limits.
+// Assemble every scenario's TileTables into DeTileX's device arrays and list
+// the crowded tiles; none (hecap 0) where the tables do not pay.
 static int upload_tile_tables(anuga_domain *d)
 {
     free_tile_tables(d);
     if (d->mixed || !d->edge_once || (int)d->ts_x.size() != d->S) return ANUGA_OK;
     bool vertices = d->vgeom;
-    for (const TileTables &x : d->ts_x) {
-        if (!x.ok) return ANUGA_OK;
+    std::vector<int> list;
+    std::vector<unsigned char> crowded(d->nblocks, 0);
+    for (int s = 0; s < d->S; s++) {
+        const TileTables &x = d->ts_x[s];
         vertices = vertices && x.vertices;
+        for (size_t b = 0; b < x.crowded.size(); b++)
+            if (x.crowded[b]) {
+                list.push_back(d->kbeg[s] / DE_BLOCK + (int)b);
+                crowded[list.back()] = 1;
+            }
+    }
+    if (!tables_pay(d->nblocks, (int)list.size())) {
+        d->ts_x.clear();
+        return ANUGA_OK;
     }
     TileTables a;
     const TileTables *all = &d->ts_x[0];
@@ -1624,6 +1685,7 @@ static int upload_tile_tables(anuga_domain *d)
         total += (bytes + 255) / 256 * 256;
     };
     DeTileX x{};
+    const int *xlist = nullptr;
     add(x.cstart, cstart);
     add(x.cell, all->cell);
     add(x.stencil, all->stencil);
@@ -1634,6 +1696,10 @@ static int upload_tile_tables(anuga_domain *d)
     add(x.estart, estart);
     add(x.esplit, all->esplit);
     add(x.edge, all->edge);
+    if (!list.empty()) {
+        add(x.crowded, crowded);
+        add(xlist, list);
+    }
     if (vertices) {
         add(x.nstart, nstart);
         add(x.node, all->node);
@@ -1657,6 +1723,8 @@ static int upload_tile_tables(anuga_domain *d)
     // the LDS stride of the halo edges: a multiple of 16, never zero
     x.hecap = std::max((all->hecap + 15) / 16 * 16, 16);
     d->tx = x;
+    d->xlist = const_cast<int *>(xlist);
+    d->nxlist = (int)list.size();
     d->ts_x.clear();
     d->ts_x.shrink_to_fit();
     return ANUGA_OK;
@@ -3570,7 +3638,7 @@ int anuga_tile_tables(int64_t N, const int32_t *nb, const double *vertex_coordin
     }
     TileTables x;
     scenario_tables((int)N, hn.data(), vertex_coordinates, x);
-    if (!x.ok) return ANUGA_E_STATE;
+    if (!o->crowded && x.ncrowded()) return ANUGA_E_STATE;
     auto put = [](auto *to, const auto &from, size_t cap) {
         if (!to || from.size() > cap) return false;
         std::copy(from.begin(), from.end(), to);
@@ -3587,6 +3655,7 @@ int anuga_tile_tables(int64_t N, const int32_t *nb, const double *vertex_coordin
                put(o->nstart, x.nstart, nt) && x.node.size() <= cap && o->node;
         if (fits) std::memcpy(o->node, x.node.data(), x.node.size() * sizeof(double2));
     }
+    if (o->crowded) fits = fits && put(o->crowded, x.crowded, nt);
     if (!fits) return ANUGA_E_ARG;
     const size_t n[4] = {x.cell.size(), x.hstencil.size(), x.edge.size(), x.node.size()};
     for (int i = 0; i < 4; i++) o->sizes[i] = (int64_t)n[i];

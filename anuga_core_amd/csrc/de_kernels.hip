@@ -1107,7 +1107,7 @@ de_xflux(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__restri
     // [4 quantities][3 edges][DE_BLOCK] tile edge values, then [4][3][hcap] halo
     extern __shared__ double lds[];
     __shared__ double red_dt[DE_BLOCK / 64], red_bf[DE_BLOCK / 64], red_m[DE_BLOCK / 64];
-    const int lb = xcd_block();
+    const int lb = tl.list ? tl.list[xcd_block()] : xcd_block();
     DeControl *cb = de_ctl(ctl, m.scen, lb);
     if (cb->done) return;
     int *err = &cb->status;
@@ -1589,7 +1589,7 @@ de_xflux_e(DeMesh m, DeParams p, const DeQ *__restrict__ q, const double *__rest
     }
 
     DeControl *cb = de_ctl(ctl, m.scen, lb);
-    if (cb->done) return;
+    if (cb->done || (tx.crowded && tx.crowded[lb])) return;
     int *err = &cb->status;
     const double dt = SUBSTEP ? dctl[cb - ctl].dt : 0.0;
     const bool on = k < cb->kend;

@@ -480,7 +480,8 @@ int anuga_tile_halos(int64_t N, const int32_t *nb, int64_t *start, int64_t halo_
  * (nb as in anuga_tile_halos; vertex_coordinates (N,3,2), or NULL: no nodes),
  * host only: what each workgroup reads, one entry per tile in the *start
  * arrays (their last tile ends at sizes[]: cells, halo edges, edges, nodes).
- * ANUGA_E_STATE where a tile exceeds the kernel's limits. */
+ * A tile beyond the kernel's limits is left to another kernel: it is 1 in
+ * crowded and has no entries; ANUGA_E_STATE where crowded is NULL. */
 typedef struct {
     int64_t capacity;          /* of cell, hstencil, hcell, hnodes, edge; node: pairs */
     int64_t *sizes;            /* [4] */
@@ -489,6 +490,7 @@ typedef struct {
     int32_t *cell;
     uint32_t *hstencil, *hcell, *hnodes, *edge;
     double *node;
+    uint8_t *crowded;                                       /* [tiles], or NULL */
 } anuga_tile_tables_out;
 int anuga_tile_tables(int64_t N, const int32_t *nb, const double *vertex_coordinates,
                       const anuga_tile_tables_out *out);

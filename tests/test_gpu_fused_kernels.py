@@ -1,0 +1,78 @@
+"""The fused FP64 kernels that meshes, options and limits choose between give
+the same bits: the once-per-edge kernel with its geometry from the vertices,
+the same with the stored geometry, and the gather kernel, over every tile or
+over the crowded ones only."""
+
+import numpy as np
+import pytest
+
+from anuga_core_amd.boundaries import (Dirichlet_boundary, Reflective_boundary,
+                                       Transmissive_boundary)
+from anuga_core_amd.domain import Domain
+from anuga_core_amd.mesh import Mesh, rectangular_cross
+from tests.test_tile_tables import _ordered, _tables
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ("stage", "xmomentum", "ymomentum")
+KINDS = (lambda d: Reflective_boundary(d), lambda d: Dirichlet_boundary([0.3, 0.2, -0.1]),
+         lambda d: Transmissive_boundary(d))
+
+
+def _inputs(mesh, seed):
+    """Hills, partly above the water, and moving water."""
+    rng = np.random.default_rng(seed)
+    N = mesh.number_of_triangles
+    x, y = mesh.centroid_coordinates.T
+    z = 0.6 * np.sin(x / 2.3) * np.cos(y / 3.1) - 0.3
+    wet = rng.random(N) < 0.9
+    return dict(elevation=z, stage=np.where(wet, np.maximum(z, 0.1 * rng.random(N)), z),
+                friction=0.03 * rng.random(N), xmomentum=0.2 * wet * rng.standard_normal(N),
+                ymomentum=0.2 * wet * rng.standard_normal(N))
+
+
+def _run(mesh, q, alg, steps):
+    d = Domain(mesh=mesh)
+    d.set_flow_algorithm(alg)
+    d.set_evolve_min_timestep(0.0)
+    for n, v in q.items():
+        d.set_quantity(n, v, location="centroids")
+    d.set_boundary({t: KINDS[i % 3](d) for i, t in enumerate(sorted(d.get_boundary_tags()))})
+    for n in steps:
+        d.evolve_steps(n)
+    return ([d.get_quantity(n).centroid_values for n in NAMES], d.dt_history,
+            d.get_boundary_flux_integral())
+
+
+def _same(a, b):
+    assert a[1] == b[1] and a[2] == b[2]
+    for x, y in zip(a[0], b[0]):
+        assert np.array_equal(x, y)
+
+
+def _stacked_sheets(n, sheets=25, m=6):
+    """A grid of 4 n n triangles and, beside it, a stack of sheets over one
+    another: a tile there holds a piece of every sheet, with its surroundings."""
+    p0, t0 = (np.asarray(a) for a in rectangular_cross(n, n, float(n), float(n))[:2])
+    p1, t1 = (np.asarray(a) for a in rectangular_cross(m, m, float(m), float(m))[:2])
+    points = [p0] + [p1 + [n + 10.0, 0.0]] * sheets
+    triangles = [t0] + [t1 + len(p0) + i * len(p1) for i in range(sheets)]
+    return Mesh(np.concatenate(points), np.concatenate(triangles))
+
+
+@pytest.mark.parametrize("alg", ["DE0", "DE1", "DE2"])
+@pytest.mark.parametrize("n", [40, 460])
+def test_crowded_tiles_leave_the_others_on_the_fast_kernel(monkeypatch, n, alg):
+    """Below and above the number of tiles from which the crowded ones get a
+    launch of their own, against the gather kernel over all tiles."""
+    print("case crowded tiles %d %s" % (n, alg), flush=True)
+    mesh = _stacked_sheets(n)
+    if alg == "DE0":
+        a = _tables(*_ordered(mesh), crowded=True)
+        assert 0 < a["crowded"].sum() < 40
+    q = _inputs(mesh, n)
+    runs = []
+    for once in ("1", "0"):
+        monkeypatch.setenv("ANUGA_HIP_EDGE_ONCE", once)
+        runs.append(_run(mesh, q, alg, (3, 67) if n < 100 else (3,)))
+    _same(*runs)

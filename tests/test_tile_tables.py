@@ -14,8 +14,9 @@ from tests.test_tiles import BLOCK, tile_layout
 CELLS, HALO, NODES = BLOCK, min(BLOCK - 64, 256), 384      # DE_XCELLS_MAX, DE_XHALO_MAX, DE_XNODES_MAX
 
 
-def _tables(nb, vertices=None):
-    """The tables of packed neighbours nb [N][3], or None beyond the limits."""
+def _tables(nb, vertices=None, crowded=False):
+    """The tables of packed neighbours nb [N][3], or None beyond the limits;
+    crowded: with the tiles beyond them marked instead."""
     N = len(nb)
     nt = (N + BLOCK - 1) // BLOCK
     cap = 3 * N + nt * (CELLS + NODES + HALO)
@@ -24,6 +25,8 @@ def _tables(nb, vertices=None):
     a = dict(sizes=np.zeros(4, np.int64), stencil=u(N), across=u(N), nodes=u(N), cstart=i(nt),
              hstart=i(nt), estart=i(nt), esplit=i(nt), nstart=i(nt), cell=i(cap),
              hstencil=u(cap), hcell=u(cap), hnodes=u(cap), edge=u(cap), node=np.zeros(2 * cap))
+    if crowded:
+        a["crowded"] = np.zeros(nt, np.uint8)
     fields = dict(_native.TileTables._fields_)
     t = _native.TileTables(capacity=cap, **{k: v.ctypes.data_as(fields[k]) for k, v in a.items()})
     vx = None if vertices is None else np.ascontiguousarray(vertices, np.float64)
@@ -49,6 +52,12 @@ def _replay(nb, a, vertices):
     nb = nb.astype(np.int64)
     for b in range((N + BLOCK - 1) // BLOCK):
         k0, k1 = b * BLOCK, min(N, (b + 1) * BLOCK)
+        if "crowded" in a and a["crowded"][b]:
+            # no entries, so that the kernel's first loads stay in bounds
+            assert all(a[s][b] == a[s][b + 1] for s in ("cstart", "hstart", "estart"))
+            assert a["esplit"][b] == a["estart"][b]
+            assert np.all(a["stencil"][k0:k1] == 0x3fffffff) and not np.any(a["across"][k0:k1])
+            continue
         cells = np.full(2 * BLOCK, -1)
         cells[:k1 - k0] = np.arange(k0, k1)
         more = a["cell"][a["cstart"][b]:a["cstart"][b + 1]]
@@ -137,3 +146,39 @@ def test_tables_refuse_scattered_tiles():
     n, e = mesh.neighbours[order], mesh.neighbour_edges[order]
     nb = np.where(n >= 0, (place[np.maximum(n, 0)] << 2) | e, -1)
     assert _tables(nb) is None
+
+
+def _limits(nb, vertices, b):
+    """Cells, halo edges and nodes of tile b."""
+    k0, k1 = b * BLOCK, min(len(nb), (b + 1) * BLOCK)
+    n = np.where(nb >= 0, nb >> 2, -1).astype(np.int64)
+    out = lambda v: v[(v >= 0) & ((v < k0) | (v >= k1))]  # noqa: E731
+    edges = out(n[k0:k1].ravel())
+    halo = np.unique(edges)
+    cells = np.unique(np.concatenate([halo, out(n[halo].ravel())]))
+    tri = np.concatenate([np.arange(k0, k1), halo])
+    return len(cells), len(edges), len(np.unique(vertices[tri].reshape(-1, 2), axis=0))
+
+
+@pytest.mark.parametrize("tiles", [(0,), (3, 9, 17), tuple(range(8, 25))])
+def test_only_crowded_tiles_go_without_tables(tiles):
+    """A few tiles whose triangles are scattered over the mesh: these alone
+    are marked; every other tile's tables are whole."""
+    nb, vertices = _ordered(Mesh(*rectangular_cross(53, 41, 53.0, 41.0)))
+    N = len(nb)
+    among = np.concatenate([np.arange(b * BLOCK, (b + 1) * BLOCK) for b in tiles + (30,)])
+    order = np.arange(N)
+    order[among] = np.random.default_rng(len(tiles)).permutation(among)
+    place = np.empty(N, np.int64)
+    place[order] = np.arange(N)
+    n = nb[order].astype(np.int64)
+    nb = np.where(n >= 0, (place[np.maximum(n, 0) >> 2] << 2) | (n & 3), -1)
+    vertices = vertices[order]
+    nt = (N + BLOCK - 1) // BLOCK
+    sizes = np.array([_limits(nb, vertices, b) for b in range(nt)])
+    want = (sizes > (CELLS, HALO, NODES)).any(axis=1)
+    assert 2 <= want.sum() < nt
+    a = _tables(nb, vertices, crowded=True)
+    assert np.array_equal(a["crowded"], want.astype(np.uint8))
+    _replay(nb, a, vertices)
+    assert _tables(nb, vertices) is None
