@@ -214,7 +214,9 @@ struct anuga_domain {
     hipGraphExec_t graph_exec = nullptr;
     bool use_graph = true;
 
-    double host_dt = 0.0;     // the timestep of the last first substep (substate 1)
+    // the timestep of the last first substep (substate 1), NaN where the
+    // control block has taken another since
+    double host_dt = 0.0;
     int substate = 0;         // 0: at a step boundary (state in A); 1: rk2 substep state in B
     // per-operation calls (the reference's call order): the semi-implicit
     // momentum updates (allocated on first use), whether B holds a backup of
@@ -2305,6 +2307,39 @@ static void step_fixed(anuga_domain *d, DeQ *X, DeQ *out)
     launch_flux(d, 1, d->B, X, out);
 }
 
+// While it lives, fixed steps take their scratch from the record's stage
+// buffers: the handle's own may hold the first half of a step (the substep's
+// state, its updates and edge values, a backup) that the caller has yet to end.
+struct AdjScratch {
+    anuga_domain *const d;
+    DeQ *const B;
+    void *const E;
+    unsigned char *const flags;
+    double *const ex[3];
+    unsigned long long *const dneg;
+    const bool e_stale, backup_valid;
+    AdjScratch(anuga_domain *h, AdjRun *a)
+        : d(h), B(h->B), E(h->E), flags(h->flags), ex{h->ex[0], h->ex[1], h->ex[2]}, dneg(h->dneg),
+          e_stale(h->e_stale), backup_valid(h->backup_valid)
+    {
+        d->B = a->S1;
+        d->E = a->E0;
+        d->flags = a->f0;
+        for (int q = 0; q < 3; q++) d->ex[q] = a->ex0 + q * (size_t)d->N;
+        d->dneg = a->neg;
+    }
+    ~AdjScratch()
+    {
+        d->B = B;
+        d->E = E;
+        d->flags = flags;
+        for (int q = 0; q < 3; q++) d->ex[q] = ex[q];
+        d->dneg = dneg;
+        d->e_stale = e_stale;
+        d->backup_valid = backup_valid;
+    }
+};
+
 // the stage quantities of the step from X into the adjoint's buffers
 static void adj_stages(anuga_domain *d, AdjRun *a, const DeQ *X)
 {
@@ -3914,12 +3949,14 @@ int anuga_adjoint_gradient(anuga_domain *d, const double *dloss_dstage, double *
     HIPCHK(d, hipMemsetAsync(a->nbar, 0, N * sizeof(double), d->stream));
     ensure_live(d);
     hipLaunchKernelGGL(de_set_dt, dim3(1), dim3(64), 0, d->stream, d->ctl, a->dt);
+    d->host_dt = NAN;   // a step that waits for its later substeps sets its own again
     for (int64_t j = a->nckpt - 1; j >= 0; j--) {
         const int64_t s0 = j * a->every, s1 = std::min(s0 + a->every, a->nsteps);
         if (a->held != j) {
             a->held = -1;
             HIPCHK(d, hipMemcpyAsync(a->seg, a->ckpt + j * (size_t)N, N * sizeof(DeQ),
                                      hipMemcpyDeviceToDevice, d->stream));
+            const AdjScratch scratch(d, a);
             for (int64_t t = 1; t < s1 - s0; t++) {
                 DeQ *x = a->seg + t * (size_t)N;
                 step_fixed(d, x - N, x);

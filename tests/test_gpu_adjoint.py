@@ -254,3 +254,47 @@ def test_gpu_gradient_after_a_change_of_friction():
     first, second = d.adjoint_gradient(dL), d.adjoint_gradient(dL)
     for a, b in zip(first, second):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("every", [1, 4, 12])
+def test_gpu_gradient_inside_a_step(every):
+    """A gradient between the halves of a host-sequenced step, between its
+    flux and its update, and behind a backup leaves the step as it was, and
+    is the gradient that the same record gives outside of one."""
+    print("adjoint inside a step, checkpoints every", every, flush=True)
+    mesh, q, bc = _wet_case(9)
+    init = _initial(mesh, q)
+    gauges = np.arange(0, mesh.number_of_triangles, 40)
+    runs = []
+    for inside in (False, True):
+        d = _domain(mesh, q, bc, init)
+        rec = d.adjoint_record(12, 0.15, gauges, 3, checkpoint_every=every)
+        dL = np.ones(rec.shape)
+        grads = [] if inside else 3 * [d.adjoint_gradient(dL)]
+        d._compute_fluxes()
+        if inside:
+            grads.append(d.adjoint_gradient(dL))
+        d.timestep = 0.07
+        d._call("anuga_update_conserved_quantities", C.c_double(d.timestep), None)
+        if inside:
+            grads.append(d.adjoint_gradient(dL))
+        d._call("anuga_rk2_second_substep", C.c_double(d.timestep), None)
+        out = [d.get_quantity(n).centroid_values for n in ("stage", "xmomentum", "ymomentum")]
+        d.backup_conserved_quantities()
+        d.distribute_to_vertices_and_edges()
+        if inside:
+            grads.append(d.adjoint_gradient(dL))
+        d.compute_fluxes()
+        d.compute_forcing_terms()
+        d.update_conserved_quantities()
+        d.saxpy_conserved_quantities(0.5, 0.5)
+        out += [d.get_quantity(n).centroid_values for n in ("stage", "xmomentum", "ymomentum")]
+        runs.append((out, d.get_boundary_flux_integral(), grads))
+        d.close()
+    (a, ia, ga), (b, ib, gb) = runs
+    assert ia == ib
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
+    for g, h in zip(ga, gb):
+        for x, y in zip(g, h):
+            assert np.array_equal(x, y)
