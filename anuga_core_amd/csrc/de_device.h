@@ -103,8 +103,7 @@ struct DeMesh {
     // the caller's index of each triangle within its scenario (the
     // reference's loop order, for the low-Froude sums)
     const int *__restrict__ caller;
-    // the vertex coordinates [N][3] (x, y): sloped friction, and the fused
-    // FP64 kernel's geometry where it reproduces the mesh's arrays
+    // the vertex coordinates [N][3] (x, y), for sloped friction
     const double *__restrict__ vx;
 };
 

@@ -148,6 +148,10 @@ struct anuga_domain {
     // scenario at upload), which that kernel assumes
     DeTileX tx{};
     std::vector<struct TileTables> ts_x;   // per scenario, until every mesh is set
+    // vx holds the vertex coordinates where sloped friction reads them or the
+    // tables do not hold them; ts_kept: per scenario, only its tables do
+    bool vx_given = false;
+    std::vector<char> ts_kept;
     int *xlist = nullptr;                  // the crowded tiles, in tx's allocation
     int nxlist = 0;
     bool mirror = true;
@@ -541,7 +545,7 @@ static int check_params(anuga_domain *d, const anuga_params *p)
         return fail(d, ANUGA_E_ARG, "use_sloped_mannings must be 0 or 1");
     if (p->precision == ANUGA_PRECISION_MIXED && (p->low_froude || p->use_sloped_mannings))
         return fail(d, ANUGA_E_ARG, "low_froude and sloped friction need the FP64 path");
-    if (d && p->use_sloped_mannings && !d->vx)
+    if (d && p->use_sloped_mannings && !d->vx_given)
         return fail(d, ANUGA_E_ARG, "sloped friction needs the mesh's vertex_coordinates");
     if (p->extrapolate_velocity_second_order != 1)
         return fail(d, ANUGA_E_ARG, "extrapolate_velocity_second_order must be 1 (DE algorithms)");
@@ -1626,10 +1630,7 @@ static int upload_tile_tables(anuga_domain *d)
                 crowded[list.back()] = 1;
             }
     }
-    if (!tables_pay(d->nblocks, (int)list.size())) {
-        d->ts_x.clear();
-        return ANUGA_OK;
-    }
+    if (!tables_pay(d->nblocks, (int)list.size())) return ANUGA_OK;
     TileTables a;
     const TileTables *all = &d->ts_x[0];
     // scenarios start on whole tiles; the padding behind them has no neighbours
@@ -1727,8 +1728,6 @@ static int upload_tile_tables(anuga_domain *d)
     d->tx = x;
     d->xlist = const_cast<int *>(xlist);
     d->nxlist = (int)list.size();
-    d->ts_x.clear();
-    d->ts_x.shrink_to_fit();
     return ANUGA_OK;
 }
 
@@ -1837,8 +1836,7 @@ static bool geometry_from_vertices(const anuga_mesh *mesh, int64_t lo, int64_t h
 }
 
 // The vertex geometry stays on only while every scenario's arrays are
-// formed from its vertices (the kernels then read the per-triangle vertex
-// coordinates, vx).
+// formed from its vertices (the kernels then read the tiles' nodes).
 static void check_vertex_geometry(anuga_domain *d, const anuga_mesh *mesh)
 {
     if (!mesh->vertex_coordinates ||
@@ -1846,6 +1844,45 @@ static void check_vertex_geometry(anuga_domain *d, const anuga_mesh *mesh)
             return geometry_from_vertices(mesh, lo, hi);
         }))
         d->vgeom = false;
+}
+
+static int upload_vertices(anuga_domain *d, int s, const std::vector<double> &v)
+{
+    if (!d->vx) HIPCHK(d, dalloc(&d->vx, 6 * (size_t)d->N));
+    HIPCHK(d, hipMemcpy(d->vx + 6 * (size_t)d->kbeg[s], v.data(), v.size() * sizeof(double),
+                        hipMemcpyHostToDevice));
+    return ANUGA_OK;
+}
+
+// With every mesh set: the vertex coordinates that only the tables hold go to
+// vx where the tables were not installed or other scenarios are there.
+static int settle_vertices(anuga_domain *d)
+{
+    if (d->tx.ncap && !d->vx) return ANUGA_OK;
+    for (int s = 0; s < d->S; s++) {
+        if (!d->ts_kept[s]) continue;
+        const TileTables &x = d->ts_x[s];
+        std::vector<double> v(6 * (size_t)d->ntri[s]);
+        for (size_t k = 0; k < x.nodes.size(); k++)
+            for (int c = 0; c < 3; c++) {
+                const double2 p = x.node[x.nstart[k / DE_BLOCK] + ((x.nodes[k] >> (10 * c)) & 1023u)];
+                v[6 * k + 2 * c] = p.x;
+                v[6 * k + 2 * c + 1] = p.y;
+            }
+        int rc = upload_vertices(d, s, v);
+        if (rc) return rc;
+    }
+    return ANUGA_OK;
+}
+
+// The vertex coordinates for sloped friction, where they are not there yet.
+static int ensure_vertices(anuga_domain *d)
+{
+    if (d->vx || !d->vx_given || !d->tx.ncap) return ANUGA_OK;
+    HIPCHK(d, dalloc(&d->vx, 6 * (size_t)d->N));
+    hipLaunchKernelGGL(de_node_vertices, dim3(d->nblocks), dim3(DE_BLOCK), 0, d->stream, d->N,
+                       d->tx, (double2 *)d->vx);
+    return launch_check(d);
 }
 
 static int upload_mesh(anuga_domain *d, int s, const anuga_mesh *mesh)
@@ -1979,20 +2016,31 @@ static int upload_mesh(anuga_domain *d, int s, const anuga_mesh *mesh)
                             6 * sizeof(double));
             return true;
         });
-        if (!d->vx) HIPCHK(d, dalloc(&d->vx, 6 * (size_t)d->N));
-        HIPCHK(d, hipMemcpy(d->vx + 6 * (size_t)kb, hv.data(), 6 * (size_t)N * sizeof(double),
-                            hipMemcpyHostToDevice));
+        d->vx_given = true;
     }
     if (d->vgeom) check_vertex_geometry(d, mesh);
     if (d->P.reorder == 2) {
         int rc = scenario_tiles(d, s, hn, hv.empty() ? nullptr : hv.data());
         if (rc) return rc;
     }
+    d->ts_kept.resize(d->S, 0);
+    d->ts_kept[s] = !d->P.use_sloped_mannings && (int)d->ts_x.size() == d->S &&
+                    d->ts_x[s].vertices && d->ts_x[s].ncrowded() == 0;
+    if (!hv.empty() && !d->ts_kept[s]) {
+        int rc = upload_vertices(d, s, hv);
+        if (rc) return rc;
+    }
     if (!d->mesh_set[s]) {
         d->mesh_set[s] = 1;
         d->meshes_missing--;
     }
-    if (d->P.reorder == 2 && d->meshes_missing == 0) return upload_tiles(d);
+    if (d->P.reorder == 2 && d->meshes_missing == 0) {
+        int rc = upload_tiles(d);
+        if (!rc) rc = settle_vertices(d);
+        d->ts_x.clear();
+        d->ts_x.shrink_to_fit();
+        return rc;
+    }
     return ANUGA_OK;
 }
 
@@ -2462,6 +2510,10 @@ int anuga_set_params(anuga_domain *d, const anuga_params *params)
     if (d->lts_M > 1 && (params->low_froude || params->use_sloped_mannings))
         return fail(d, ANUGA_E_STATE, "local flux updating runs without low_froude or sloped "
                                       "friction");
+    if (params->use_sloped_mannings) {
+        rc = ensure_vertices(d);
+        if (rc) return rc;
+    }
     if (std::memcmp(params, &d->P, sizeof(anuga_params)) != 0) drop_graph(d);
     // a new method restarts the per-operation flux substep count, as the
     // reference's static base_call does (sw_domain_orig.c:791-794)

@@ -2855,6 +2855,19 @@ de_gather_f32(int N, const int *__restrict__ iperm, const double *__restrict__ v
 // ---------------------------------------------------------------------------
 // whole quantities between the internal and the caller's order
 // ---------------------------------------------------------------------------
+// The vertex coordinates of the n triangles of the tiles in tx, from the
+// tiles' nodes: sloped friction alone reads them, so they take their 48 B per
+// triangle when it is first asked for.
+__global__ void __launch_bounds__(DE_BLOCK)
+de_node_vertices(int n, DeTileX tx, double2 *__restrict__ vx)
+{
+    const int k = blockIdx.x * DE_BLOCK + threadIdx.x;
+    if (k >= n) return;
+    const double2 *nd = tx.node + tx.nstart[blockIdx.x];
+    const unsigned w = tx.nodes[k];
+    for (int c = 0; c < 3; c++) vx[3 * (size_t)k + c] = nd[de_field(w, c)];
+}
+
 // One centroid quantity of n triangles (internal order, caller[k] the
 // caller's index of triangle k): v[k * stride], or the depth of the records
 // at v (HEIGHT), to out in the caller's order, so that 8 B per triangle cross

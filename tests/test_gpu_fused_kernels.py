@@ -5,6 +5,7 @@ over the crowded ones only."""
 
 import numpy as np
 import pytest
+import torch
 
 from anuga_core_amd.boundaries import (Dirichlet_boundary, Reflective_boundary,
                                        Transmissive_boundary)
@@ -76,3 +77,39 @@ def test_crowded_tiles_leave_the_others_on_the_fast_kernel(monkeypatch, n, alg):
         monkeypatch.setenv("ANUGA_HIP_EDGE_ONCE", once)
         runs.append(_run(mesh, q, alg, (3, 67) if n < 100 else (3,)))
     _same(*runs)
+
+
+def _sloped(mesh, q):
+    d = Domain(mesh=mesh)
+    d.set_flow_algorithm("DE1")
+    for n, v in q.items():
+        d.set_quantity(n, v, location="centroids")
+    d.set_boundary({t: Reflective_boundary(d) for t in d.get_boundary_tags()})
+    d.evolve_steps(2)
+    before = torch.cuda.mem_get_info()[0]
+    d.set_sloped_mannings_function(True)
+    d.evolve_steps(1)
+    taken = before - torch.cuda.mem_get_info()[0]
+    d.evolve_steps(4)
+    return taken, [d.get_quantity(n).centroid_values for n in NAMES]
+
+
+@pytest.mark.parametrize("mesh", [lambda: Mesh(*rectangular_cross(201, 197, 201.0, 197.0)),
+                                  lambda: _stacked_sheets(200)])
+def test_vertex_coordinates_are_formed_for_sloped_friction(monkeypatch, mesh):
+    """Only sloped friction reads the vertex coordinates per triangle: they
+    take their 48 B when it is first set, formed from the nodes of the tiles.
+    Meshes without such nodes (here: the gather kernel over all tiles) have
+    them from the start, and the same steps."""
+    print("case sloped friction set late", flush=True)
+    mesh = mesh()
+    q = _inputs(mesh, 2)
+    crowded = mesh.number_of_triangles != 4 * 201 * 197
+    taken, a = _sloped(mesh, q)
+    # allocations come in pieces of 2 MiB
+    assert abs(taken - (0 if crowded else 48 * mesh.number_of_triangles)) <= 2 << 21
+    monkeypatch.setenv("ANUGA_HIP_EDGE_ONCE", "0")
+    taken, b = _sloped(mesh, q)
+    assert abs(taken) <= 2 << 21
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
