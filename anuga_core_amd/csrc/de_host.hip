@@ -18,10 +18,12 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <memory>
 #include <string>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -1375,6 +1377,33 @@ static int tile_halos(int N, const int4 *hn, std::vector<int> &start, std::vecto
     return hcap;
 }
 
+// work(0) to work(T - 1), each on a thread of its own as far as threads can be
+// started, the rest on this one; an exception of any of them reaches the caller.
+template <class F>
+static void on_threads(int T, F work)
+{
+    std::vector<std::exception_ptr> failed(T);
+    auto guarded = [&](int i) {
+        try {
+            work(i);
+        } catch (...) {
+            failed[i] = std::current_exception();
+        }
+    };
+    std::vector<std::thread> th;
+    th.reserve(T);
+    int i = 1;
+    try {
+        for (; i < T; i++) th.emplace_back(guarded, i);
+    } catch (const std::system_error &) {
+    }
+    for (; i < T; i++) guarded(i);
+    guarded(0);
+    for (auto &t : th) t.join();
+    for (const auto &f : failed)
+        if (f) std::rethrow_exception(f);
+}
+
 // DeTileX's tables of tiles [b0, b1) of one scenario of N triangles (nb records
 // hn, its own numbering), appended to x; vx: the triangles' vertex coordinates
 // [N][6], or NULL. A tile beyond the kernel's limits gets no entries.
@@ -1531,14 +1560,10 @@ static void scenario_tables(int N, const int4 *hn, const double *vx, TileTables 
     const int nt = (N + DE_BLOCK - 1) / DE_BLOCK;
     const int T = std::max(1, std::min<int>({(int)std::thread::hardware_concurrency(), 16, nt / 16}));
     std::vector<TileTables> part(T);
-    auto work = [&](int i) {
+    on_threads(T, [&](int i) {
         const int b0 = (int)((int64_t)nt * i / T), b1 = (int)((int64_t)nt * (i + 1) / T);
         tile_tables(N, hn, vx, b0, b1, part[i]);
-    };
-    std::vector<std::thread> th;
-    for (int i = 1; i < T; i++) th.emplace_back(work, i);
-    work(0);
-    for (auto &t : th) t.join();
+    });
     x = TileTables();
     if (T == 1) std::swap(x, part[0]);
     x.vertices = vx != nullptr;
@@ -1782,11 +1807,7 @@ static bool all_of_ranges(int64_t N, F check)
     const int T = (int)std::max<int64_t>(
         1, std::min<int64_t>({(int64_t)std::thread::hardware_concurrency(), 16, N / per}));
     std::vector<char> ok(T, 0);
-    std::vector<std::thread> th;
-    auto work = [&](int i) { ok[i] = check(N * i / T, N * (i + 1) / T); };
-    for (int i = 1; i < T; i++) th.emplace_back(work, i);
-    work(0);
-    for (auto &t : th) t.join();
+    on_threads(T, [&](int i) { ok[i] = check(N * i / T, N * (i + 1) / T); });
     return std::all_of(ok.begin(), ok.end(), [](char c) { return c != 0; });
 }
 

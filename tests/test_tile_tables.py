@@ -3,6 +3,10 @@ and listed edge that a workgroup reads, replayed against the mesh, and its LDS
 extents against the launch's. Calls only host-side entry points."""
 
 import ctypes as C
+import os
+import resource
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -182,3 +186,40 @@ def test_only_crowded_tiles_go_without_tables(tiles):
     assert np.array_equal(a["crowded"], want.astype(np.uint8))
     _replay(nb, a, vertices)
     assert _tables(nb, vertices) is None
+
+
+NO_THREADS = """
+import resource, sys
+sys.path.insert(0, %r)
+from anuga_core_amd.mesh import Mesh, rectangular_cross
+from tests.test_tile_tables import _ordered, _replay, _tables
+nb, vertices = _ordered(Mesh(*rectangular_cross(60, 60, 60.0, 60.0)))
+pages = int(open("/proc/self/statm").read().split()[0])
+resource.setrlimit(resource.RLIMIT_AS, (pages * resource.getpagesize() + (1 << 30),) * 2)
+import threading
+try:
+    threading.Thread(target=int).start()
+    print("a thread was started")
+except RuntimeError:
+    pass
+_replay(nb, _tables(nb, vertices), vertices)
+print("whole")
+"""
+
+
+def test_tables_without_threads():
+    """Where no thread can be started the calling one cuts every tile: stacks
+    of 4 GiB do not fit the address space that is left."""
+    def limit():
+        hard = resource.getrlimit(resource.RLIMIT_STACK)[1]
+        resource.setrlimit(resource.RLIMIT_STACK, (4 << 30, hard))
+
+    if 0 <= resource.getrlimit(resource.RLIMIT_STACK)[1] < 4 << 30:
+        pytest.skip("the stack limit cannot be raised")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", NO_THREADS % root], preexec_fn=limit, text=True,
+                       env=dict(os.environ, OMP_NUM_THREADS="1", OPENBLAS_NUM_THREADS="1"),
+                       capture_output=True, timeout=120)
+    if "a thread was started" in r.stdout:
+        pytest.skip("threads start all the same")
+    assert r.returncode == 0 and r.stdout == "whole\n", r.stderr[-2000:]
