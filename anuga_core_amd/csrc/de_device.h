@@ -10,6 +10,7 @@
 #include <stdint.h>
 
 #include "de_limit.h"
+#include "de_shape.h"
 
 // threads per workgroup of the per-triangle kernels (a multiple of 64)
 #ifndef DE_BLOCK

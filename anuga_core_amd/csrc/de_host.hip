@@ -1410,7 +1410,7 @@ static void on_threads(int T, F work)
 static void tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1, TileTables &x)
 {
     // place of each cell of a tile (its triangle id), by open addressing
-    constexpr int HS = 4 * DE_XCELLS_MAX, NS = 4 * DE_XNODES_MAX;
+    constexpr int HS = de_hash_slots(DE_XCELLS_MAX), NS = de_hash_slots(DE_XNODES_MAX);
     std::vector<int> hkey(HS), hval(HS);
     std::vector<int> nval(NS);
     std::vector<std::array<int, 3>> hedge;   // halo edges: halo triangle, its edge
