@@ -2087,24 +2087,26 @@ __device__ __forceinline__ void de_reduce_rows(const double *__restrict__ src, i
     if (!CHUNKS) {
         const int b0 = cb->bbeg, b1 = cb->bend;
         const int len = (b1 - b0 + DE_RCHUNKS - 1) / DE_RCHUNKS;
-        constexpr int PER = DE_RCHUNKS / (TH / 64);
+        constexpr int W = TH / 64, PER = de_wave_passes(W, DE_RCHUNKS);
         double x[PER][3];
 #pragma unroll
         for (int j = 0; j < PER; j++) {
-            const int c = wv + j * (TH / 64);
+            const int c = de_wave_chunk(wv, j, W, DE_RCHUNKS);
             const int i = b0 + c * len + lane;
-            const bool in = lane < len && i < b1;
+            const bool in = c >= 0 && lane < len && i < b1;
 #pragma unroll
             for (int r = 0; r < NR; r++)
                 x[j][r] = in ? src[(size_t)rows[r] * nblocks + i] : 0.0;
         }
 #pragma unroll
-        for (int j = 0; j < PER; j++)
+        for (int j = 0; j < PER; j++) {
+            const int c = de_wave_chunk(wv, j, W, DE_RCHUNKS);
 #pragma unroll
             for (int r = 0; r < NR; r++) {
                 const double v = de_wave_sum_nz(x[j][r]);
-                if (lane == 0) res[r][wv + j * (TH / 64)] = v;
+                if (lane == 0 && c >= 0) res[r][c] = v;
             }
+        }
         __syncthreads();
     }
 #pragma unroll

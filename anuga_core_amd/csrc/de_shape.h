@@ -16,3 +16,12 @@ DE_SHAPE_FN int de_hash_slots(int n)
     while (s < 2 * n) s *= 2;
     return s;
 }
+
+// A workgroup of `waves` waves forms `chunks` chunks in de_wave_passes passes:
+// the chunk of a wave in pass j, or -1 in the last pass where there is none.
+DE_SHAPE_FN int de_wave_passes(int waves, int chunks) { return (chunks + waves - 1) / waves; }
+DE_SHAPE_FN int de_wave_chunk(int wave, int j, int waves, int chunks)
+{
+    const int c = wave + j * waves;
+    return chunks % waves == 0 || c < chunks ? c : -1;
+}

@@ -12,6 +12,8 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 SOURCE = r"""
 #include "de_shape.h"
 extern "C" int hash_slots(int n) { return de_hash_slots(n); }
+extern "C" int wave_passes(int w, int n) { return de_wave_passes(w, n); }
+extern "C" int wave_chunk(int v, int j, int w, int n) { return de_wave_chunk(v, j, w, n); }
 """
 
 
@@ -33,3 +35,13 @@ def test_a_probe_reaches_a_free_slot(lib):
         s = lib.hash_slots(n)
         reached = {i & (s - 1) for i in range(s)}
         assert len(reached) == s and 2 * n <= s <= max(4 * n, 2)
+
+
+def test_every_chunk_is_formed_once(lib):
+    """Workgroups of any number of waves, three, five and six (192, 320 and 384
+    threads) among them, which do not divide the reduction's 32 chunks."""
+    for chunks in (1, 31, 32, 33):
+        for waves in range(1, 17):
+            got = [lib.wave_chunk(v, j, waves, chunks) for v in range(waves)
+                   for j in range(lib.wave_passes(waves, chunks))]
+            assert sorted(c for c in got if c >= 0) == list(range(chunks))
