@@ -750,8 +750,7 @@ static void launch_xflux_t(anuga_domain *d, DeQ *S, DeQ *bk, DeQ *out)
         // halo edge values, the tile's centroid depths and beds, and the
         // vertices and node words where the geometry comes from them
         const bool vg = d->vgeom && d->tx.ncap;
-        const size_t lds = (14 * (size_t)DE_BLOCK + 4 * (size_t)d->tx.hecap) * sizeof(double) +
-                           (vg ? d->tx.ncap * sizeof(double2) + DE_BLOCK * sizeof(unsigned) : 0);
+        const size_t lds = de_edge_lds(DE_BLOCK, d->tx.hecap, vg ? d->tx.ncap : 0);
         auto kern = vg ? de_xflux_e<SUB, true> : de_xflux_e<SUB, false>;
         hipLaunchKernelGGL(kern, dim3(d->nblocks), dim3(DE_BLOCK), lds, d->stream, dev_mesh(d),
                            dev_params(d->P), S, d->eta, d->tx, bc, d->flags, d->ex[0], d->ex[1],
@@ -1291,13 +1290,13 @@ static int validate_mesh(anuga_domain *d, const anuga_mesh *mesh, int64_t N, int
 // for tile b (triangles [b DE_BLOCK, (b + 1) DE_BLOCK)), the neighbour
 // triangles outside the tile, each once, in order of first appearance; per
 // triangle, each edge's slot in its tile's list (1023: the neighbour is in
-// the tile). No tiles (hcap 0) if a halo exceeds kMaxHalo
-// so that every fused kernel's LDS stays within 64 KB per workgroup: 96 B
-// per halo entry and up to 113 B per tile triangle (the once-per-edge
-// kernel's edge values, centroid depths and beds; the general
-// instantiation's flag byte), the static reduction arrays, and the halo
-// stride rounded up to a multiple of 32.
-static const int kMaxHalo = std::min(320, (65536 - 113 * DE_BLOCK - 1024) / 97 / 32 * 32);
+// the tile). No tiles (hcap 0) if a halo exceeds kMaxHalo, so that the LDS of
+// the gather kernels stays within DE_LDS_MAX: 97 B per halo entry and tile
+// triangle (the edge values and the general instantiation's flag byte), 16 B
+// more per tile triangle to spare, the reduction arrays, and the halo stride
+// rounded up to a multiple of 32. The once-per-edge kernel's LDS has limits of its own
+// (de_tables_fit).
+static const int kMaxHalo = std::min(320, (DE_LDS_MAX - 113 * DE_BLOCK - 1024) / 97 / 32 * 32);
 
 // The tile metadata of triangles in internal order (nb: packed neighbours of
 // one scenario starting at 0). Returns the largest halo, or -1 when a
@@ -1692,6 +1691,12 @@ static int upload_tile_tables(anuga_domain *d)
         }
         all = &a;
     }
+    // the LDS strides: of the halo edges a multiple of 16, never zero
+    const int hecap = std::max((all->hecap + 15) / 16 * 16, 16);
+    const int ncap = vertices ? (all->ncap + 1) & ~1 : 0;
+    const int fit = de_tables_fit(DE_BLOCK, hecap, ncap);
+    if (!fit) return ANUGA_OK;
+    vertices = fit == 2;
     // one allocation; small tables cross in one copy
     auto closed = [](std::vector<int> v, size_t end) {   // with the closing offset
         v.push_back((int)end);
@@ -1733,7 +1738,7 @@ static int upload_tile_tables(anuga_domain *d)
         add(x.node, all->node);
         add(x.nodes, all->nodes);
         add(x.hnodes, all->hnodes);
-        x.ncap = (all->ncap + 1) & ~1;
+        x.ncap = ncap;
     }
     char *base = nullptr;
     HIPCHK(d, dalloc(&base, total));
@@ -1748,8 +1753,7 @@ static int upload_tile_tables(anuga_domain *d)
             if (q.bytes) HIPCHK(d, hipMemcpy(base + q.at, q.src, q.bytes, hipMemcpyHostToDevice));
     }
     for (const Part &q : parts) *q.dst = base + q.at;
-    // the LDS stride of the halo edges: a multiple of 16, never zero
-    x.hecap = std::max((all->hecap + 15) / 16 * 16, 16);
+    x.hecap = hecap;
     d->tx = x;
     d->xlist = const_cast<int *>(xlist);
     d->nxlist = (int)list.size();

@@ -25,3 +25,24 @@ DE_SHAPE_FN int de_wave_chunk(int wave, int j, int waves, int chunks)
     const int c = wave + j * waves;
     return chunks % waves == 0 || c < chunks ? c : -1;
 }
+
+// LDS of a workgroup of a fused kernel: at most 64 KB.
+#define DE_LDS_MAX 65536
+
+// Bytes of LDS that de_xflux_e asks for at its launch, with tiles of `block`
+// triangles, at most hecap halo edges and ncap nodes a tile (0: no nodes), and
+// those that it has of its own (three values of each wave).
+DE_SHAPE_FN int de_edge_lds(int block, int hecap, int ncap)
+{
+    return 8 * (14 * block + 4 * hecap) + (ncap ? 16 * ncap + 4 * block : 0);
+}
+DE_SHAPE_FN int de_edge_lds_static(int block) { return 3 * 8 * (block / 64); }
+
+// What of the tables fits: 2 with the nodes, 1 without them, 0 nothing.
+DE_SHAPE_FN int de_tables_fit(int block, int hecap, int ncap)
+{
+    const int most = DE_LDS_MAX - de_edge_lds_static(block);
+    return ncap && de_edge_lds(block, hecap, ncap) <= most ? 2
+           : de_edge_lds(block, hecap, 0) <= most          ? 1
+                                                           : 0;
+}

@@ -12,6 +12,9 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 SOURCE = r"""
 #include "de_shape.h"
 extern "C" int hash_slots(int n) { return de_hash_slots(n); }
+extern "C" int edge_lds(int b, int h, int n) { return de_edge_lds(b, h, n); }
+extern "C" int edge_lds_static(int b) { return de_edge_lds_static(b); }
+extern "C" int tables_fit(int b, int h, int n) { return de_tables_fit(b, h, n); }
 extern "C" int wave_passes(int w, int n) { return de_wave_passes(w, n); }
 extern "C" int wave_chunk(int v, int j, int w, int n) { return de_wave_chunk(v, j, w, n); }
 """
@@ -45,3 +48,25 @@ def test_every_chunk_is_formed_once(lib):
             got = [lib.wave_chunk(v, j, waves, chunks) for v in range(waves)
                    for j in range(lib.wave_passes(waves, chunks))]
             assert sorted(c for c in got if c >= 0) == list(range(chunks))
+
+
+@pytest.mark.parametrize("block", [128, 192, 256, 320, 384, 512])
+def test_tables_whose_lds_does_not_fit_are_left_out(lib, block):
+    """Tiles of 512 triangles with 64 halo edges and 330 nodes would take 66
+    KB; the default tiles fit at every limit of the tables."""
+    for hecap in range(16, 257, 16):
+        for ncap in range(0, 385, 2):
+            fit = lib.tables_fit(block, hecap, ncap)
+            both, bare = (lib.edge_lds(block, hecap, n) + lib.edge_lds_static(block)
+                          for n in (ncap, 0))
+            if ncap and both <= 65536:
+                assert fit == 2
+            else:
+                assert fit == (bare <= 65536)
+            if block <= 256:
+                assert fit == (2 if ncap else 1)
+    assert lib.tables_fit(512, 64, 330) == 1 and lib.tables_fit(512, 256, 0) == 0
+    # the LDS that the kernel lays out: cells under the edge values, halo edge
+    # values, depths and beds; nodes on 16 B and the triangles' node words
+    assert lib.edge_lds(256, 64, 0) == 8 * (12 * 256 + 4 * 64 + 2 * 256)
+    assert lib.edge_lds(256, 64, 180) == lib.edge_lds(256, 64, 0) + 16 * 180 + 4 * 256
