@@ -3741,7 +3741,8 @@ int anuga_tile_halos(int64_t N, const int32_t *nb, int64_t *start, int64_t halo_
 int anuga_tile_tables(int64_t N, const int32_t *nb, const double *vertex_coordinates,
                       const anuga_tile_tables_out *o)
 {
-    if (N < 1 || N >= (int64_t(1) << 29) || !nb || !o) return ANUGA_E_ARG;
+    if (N < 1 || N >= (int64_t(1) << 29) || !nb || !o || !o->sizes || o->capacity < 0)
+        return ANUGA_E_ARG;
     std::vector<int4> hn(N);
     for (int64_t k = 0; k < N; k++) {
         hn[k] = make_int4(nb[3 * k], nb[3 * k + 1], nb[3 * k + 2], 0);
@@ -3756,7 +3757,10 @@ int anuga_tile_tables(int64_t N, const int32_t *nb, const double *vertex_coordin
         std::copy(from.begin(), from.end(), to);
         return true;
     };
+    // every length is checked before the first array is written
     const size_t nt = x.cstart.size(), cap = (size_t)o->capacity;
+    for (size_t n : {x.cell.size(), x.hstencil.size(), x.edge.size(), x.node.size()})
+        if (n > cap) return ANUGA_E_ARG;
     bool fits = put(o->stencil, x.stencil, N) && put(o->across, x.across, N) &&
                 put(o->cstart, x.cstart, nt) && put(o->cell, x.cell, cap) &&
                 put(o->hstart, x.hstart, nt) && put(o->hstencil, x.hstencil, cap) &&

@@ -18,9 +18,10 @@ from tests.test_tiles import BLOCK, tile_layout
 CELLS, HALO, NODES = BLOCK, min(BLOCK - 64, 256), 384      # DE_XCELLS_MAX, DE_XHALO_MAX, DE_XNODES_MAX
 
 
-def _tables(nb, vertices=None, crowded=False):
+def _tables(nb, vertices=None, crowded=False, refused=None, **fields):
     """The tables of packed neighbours nb [N][3], or None beyond the limits;
-    crowded: with the tiles beyond them marked instead."""
+    crowded: with the tiles beyond them marked instead. refused: the arrays,
+    after a call with these fields that returns this error."""
     N = len(nb)
     nt = (N + BLOCK - 1) // BLOCK
     cap = 3 * N + nt * (CELLS + NODES + HALO)
@@ -31,13 +32,17 @@ def _tables(nb, vertices=None, crowded=False):
              hstencil=u(cap), hcell=u(cap), hnodes=u(cap), edge=u(cap), node=np.zeros(2 * cap))
     if crowded:
         a["crowded"] = np.zeros(nt, np.uint8)
-    fields = dict(_native.TileTables._fields_)
-    t = _native.TileTables(capacity=cap, **{k: v.ctypes.data_as(fields[k]) for k, v in a.items()})
+    types = dict(_native.TileTables._fields_)
+    given = {k: v.ctypes.data_as(types[k]) for k, v in a.items()}
+    t = _native.TileTables(**{**dict(capacity=cap), **given, **fields})
     vx = None if vertices is None else np.ascontiguousarray(vertices, np.float64)
     nb = np.ascontiguousarray(nb, np.int32)
     rc = _native.lib().anuga_tile_tables(
         N, nb.ctypes.data_as(C.POINTER(C.c_int32)),
         None if vx is None else vx.ctypes.data_as(C.POINTER(C.c_double)), C.byref(t))
+    if refused is not None:
+        assert rc == refused
+        return a
     if rc:
         return None
     for name, end, starts in (("cell", 0, "cstart"), ("hstencil", 1, "hstart"),
@@ -223,3 +228,14 @@ def test_tables_without_threads():
     if "a thread was started" in r.stdout:
         pytest.skip("threads start all the same")
     assert r.returncode == 0 and r.stdout == "whole\n", r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("field,value", [("capacity", -1), ("capacity", 10), ("sizes", None),
+                                         ("stencil", None), ("edge", None), ("node", None)])
+def test_tables_refuse_a_bad_description(field, value):
+    """Negative and small capacities and missing arrays are refused, with
+    nothing written behind an array's end."""
+    nb, vertices = _ordered(Mesh(*rectangular_cross(30, 30)))
+    a = _tables(nb, vertices, refused=-1, **{field: value})
+    if field == "capacity":
+        assert not any(np.any(v) for v in a.values())
