@@ -16,6 +16,7 @@ import numpy as np
 import pytest
 
 from anuga_core_amd.domain import Domain
+from anuga_core_amd.operators import Rate_operator
 from oracle.kernels import OracleKernels
 from oracle.oracle_domain import OracleDomain
 from tests import scenarios as S
@@ -221,23 +222,42 @@ def test_device_timestep_matches_host_timestep(builder, kw, ys, ft):
     assert ia == ib
 
 
-def test_graph_replay_matches_eager(monkeypatch):
+@pytest.mark.parametrize("alg", ["DE0", "DE1", "DE2"])
+@pytest.mark.parametrize("form", ["plain", "rain", "gauges", "many"])
+def test_graph_replay_matches_eager(monkeypatch, form, alg):
     """The same device-controlled steps with and without HIP graph replay,
-    interleaved with eager host work (reads, volume reductions) between runs."""
-    print("case graph_vs_eager", flush=True)
+    interleaved with eager host work (reads, volume reductions) between runs:
+    runs long enough for a graph (64 steps) that end inside one (8 steps), then
+    short ones on the graph that is there. The steps end themselves (plain), or
+    an operator or gauges run before their end, or (many: above 2048 blocks)
+    chunk workgroups reduce their partials."""
+    print("case graph_vs_eager %s %s" % (form, alg), flush=True)
+    mesh, _, q, bc = S.hills_de1(m=364 if form == "many" else 20,
+                                 n=364 if form == "many" else 20, seed=4)
     res = []
     for graph in ("1", "0"):
         monkeypatch.setenv("ANUGA_HIP_GRAPH", graph)
-        mesh, alg, q, bc = S.hills_de1(m=20, n=20, seed=4)
         d = S.setup(Domain(mesh=mesh), alg, q, bc)
+        if form == "rain":
+            rain = Rate_operator(d, rate=1.0e-3)
+        elif form == "gauges":
+            d.set_gauges(triangles=[3, 700, 1599])
         vals = []
-        for _ in range(4):
-            d.evolve_steps(13)
-            vals.append((d.get_quantity("stage").centroid_values, d.get_water_volume(),
-                         list(d.dt_history)))
+        for steps in (69, 13, 8, 101, 3):
+            d.evolve_steps(steps)
+            vals.append((d.get_quantity("stage").centroid_values,
+                         d.get_quantity("xmomentum").centroid_values, d.get_water_volume(),
+                         list(d.dt_history), d.get_time(), d.get_boundary_flux_integral()))
+        if form == "rain":
+            vals.append((rain.get_cumulative_influx(),))
+        elif form == "gauges":
+            ts = d.get_gauge_timeseries()
+            assert len(ts["time"]) >= 194
+            vals.append(tuple(ts[k] for k in sorted(ts)))
         res.append(vals)
     for a, b in zip(*res):
-        assert np.array_equal(a[0], b[0]) and a[1] == b[1] and a[2] == b[2]
+        for x, y in zip(a, b):
+            assert np.array_equal(x, y)
 
 
 def _error_report(a, b):
