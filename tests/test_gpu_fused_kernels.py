@@ -10,7 +10,8 @@ import torch
 from anuga_core_amd.boundaries import (Dirichlet_boundary, Reflective_boundary,
                                        Transmissive_boundary)
 from anuga_core_amd.domain import Domain
-from anuga_core_amd.mesh import Mesh, rectangular_cross
+from anuga_core_amd.ensemble import Ensemble
+from anuga_core_amd.mesh import Mesh, graded_square, rectangular_cross
 from tests.test_tile_tables import _ordered, _tables
 
 pytestmark = pytest.mark.gpu
@@ -32,8 +33,8 @@ def _inputs(mesh, seed):
                 ymomentum=0.2 * wet * rng.standard_normal(N))
 
 
-def _run(mesh, q, alg, steps):
-    d = Domain(mesh=mesh)
+def _run(mesh, q, alg, steps, **options):
+    d = Domain(mesh=mesh, **options)
     d.set_flow_algorithm(alg)
     d.set_evolve_min_timestep(0.0)
     for n, v in q.items():
@@ -112,4 +113,70 @@ def test_vertex_coordinates_are_formed_for_sloped_friction(monkeypatch, mesh):
     taken, b = _sloped(mesh, q)
     assert abs(taken) <= 2 << 21
     for x, y in zip(a, b):
+        assert np.array_equal(x, y)
+
+
+# the switches of the two kernels that a mesh within the limits leaves unused:
+# stored geometry (vertices that do not reproduce the mesh's arrays) and the
+# gather kernel (normals that do not mirror, tiles beyond the limits)
+KERNELS = [("ANUGA_HIP_VERTEX_GEOMETRY", "0"), ("ANUGA_HIP_EDGE_ONCE", "0")]
+MESHES = {"graded": lambda: Mesh(*graded_square(300.0, 9.0, 40.0, (100.0, 100.0, 200.0, 200.0),
+                                                seed=3)),
+          "ragged": lambda: Mesh(*rectangular_cross(37, 53, 60.0, 70.0)),
+          "tiny": lambda: Mesh(*rectangular_cross(1, 1, 1.0, 1.0))}
+
+
+@pytest.mark.parametrize("name,value", KERNELS)
+@pytest.mark.parametrize("alg", ["DE0", "DE1", "DE2"])
+@pytest.mark.parametrize("mesh", sorted(MESHES))
+def test_kernels_give_the_same_bits(monkeypatch, mesh, alg, name, value):
+    print("case %s %s %s" % (mesh, alg, name), flush=True)
+    mesh = MESHES[mesh]()
+    q = _inputs(mesh, 7)
+    usual = _run(mesh, q, alg, (5, 68))
+    monkeypatch.setenv(name, value)
+    _same(_run(mesh, q, alg, (5, 68)), usual)
+
+
+@pytest.mark.parametrize("name,value", KERNELS)
+@pytest.mark.parametrize("alg", ["DE0", "DE1"])
+def test_ensemble_kernels_give_the_same_bits(monkeypatch, alg, name, value):
+    print("case ensemble %s %s" % (alg, name), flush=True)
+    meshes = [MESHES[m]() for m in ("tiny", "ragged", "graded", "tiny")]
+    runs = []
+    for switch in (False, True):
+        if switch:
+            monkeypatch.setenv(name, value)
+        e = Ensemble(meshes, flow_algorithm=alg)
+        for s, mesh in enumerate(meshes):
+            tags = sorted(mesh.get_boundary_tags())
+            kinds = ["reflective", ("dirichlet", [0.3, 0.2, -0.1]), "transmissive"]
+            e.set_scenario(s, mesh, _inputs(mesh, s), {t: kinds[i % 3] for i, t in enumerate(tags)})
+        e.evolve_steps(3)
+        e.evolve_steps(67)
+        runs.append(([e.get_quantity(s, n) for s in range(len(meshes)) for n in NAMES],
+                     [e.get_time(s) for s in range(len(meshes))],
+                     list(e.get_boundary_flux_integrals())))
+    _same(*runs)
+
+
+@pytest.mark.parametrize("alg", ["DE0", "DE1", "DE2"])
+@pytest.mark.parametrize("sides", [1, 2])
+def test_meshes_whose_geometry_is_their_own(sides, alg):
+    """Lengths that the vertices do not give, on both sides of an edge (the
+    once-per-edge kernel reads the stored geometry) and on one (an edge has two
+    fluxes: the gather kernel), against the separate kernels."""
+    print("case own geometry %d %s" % (sides, alg), flush=True)
+    mesh = MESHES["graded"]()
+    el = mesh.edgelengths.copy()
+    for k in range(5, mesh.number_of_triangles, 97):
+        n, j = mesh.neighbours[k, 1], mesh.neighbour_edges[k, 1]
+        el[k, 1] = np.nextafter(el[k, 1], np.inf)
+        if n >= 0 and sides == 2:
+            el[n, j] = el[k, 1]
+    mesh.edgelengths = el
+    q = _inputs(mesh, 11)
+    a, b = (_run(mesh, q, alg, (5, 68), reorder=r) for r in ("tiles", "rcm"))
+    assert a[1] == b[1]
+    for x, y in zip(a[0], b[0]):
         assert np.array_equal(x, y)
