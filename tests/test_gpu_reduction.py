@@ -44,8 +44,6 @@ def _domain(mesh, q, alg):
 @pytest.mark.parametrize("m,n", [(1, 1), (128, 1), (128, 32), (129, 32), (1024, 256),
                                  (1025, 256)])
 def test_device_steps_equal_host_steps(m, n, alg):
-    if m > 1000 and alg != "DE1":
-        pytest.skip("the large meshes run one algorithm")
     mesh = Mesh(*rectangular(m, n, float(m), float(n)))
     q = _inputs(mesh, m + n)
     runs = []
