@@ -143,8 +143,6 @@ SIGNATURES = {
                                    C.POINTER(C.c_int32), C.POINTER(C.c_uint32), _ip, _ip]),
     "anuga_tile_tables": (C.c_int, [C.c_int64, C.POINTER(C.c_int32), _dp,
                                     C.POINTER(TileTables)]),
-    "anuga_tile_edges": (C.c_int, [C.c_int64, C.POINTER(C.c_int32), _ip, _ip, C.c_int64,
-                                   C.POINTER(C.c_uint32), _ip]),
     "anuga_synchronize": (C.c_int, [C.c_void_p]),
     "anuga_kernel_timing": (C.c_int, [C.c_void_p, C.c_char_p, _dp, _ip]),
     "anuga_reset_kernel_timing": (C.c_int, [C.c_void_p, C.c_int]),

@@ -175,11 +175,11 @@ struct DeLts {
     unsigned char *unf;
 };
 
-// one entry of a tile's edge list: the tile triangle t and its edge i, the
-// neighbour's position (tile triangle or halo slot) and edge j
+// one entry of a tile's edge list: the tile triangle t and its edge i, whether
+// the edge leads to the halo, the neighbour's place in the tile (0: halo) and
+// edge j
 #define DE_TE_T(e) ((int)((e) & 1023u))
 #define DE_TE_I(e) ((int)(((e) >> 10) & 3u))
-#define DE_TE_HALO(e) (((e) >> 12) & 1u)
 #define DE_TE_N(e) ((int)(((e) >> 13) & 1023u))
 #define DE_TE_J(e) ((int)(((e) >> 23) & 3u))
 #define DE_TE_MAKE(t, i, halo, n, j) \

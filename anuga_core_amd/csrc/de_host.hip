@@ -1301,41 +1301,6 @@ static const int kMaxHalo = std::min(320, (DE_LDS_MAX - 113 * DE_BLOCK - 1024) /
 // The tile metadata of triangles in internal order (nb: packed neighbours of
 // one scenario starting at 0). Returns the largest halo, or -1 when a
 // neighbour index is out of range; the caller refuses halos above kMaxHalo.
-// The tile edge lists as anuga_tile_edges exports them: per tile, each edge between two tile triangles from its lower-numbered side and
-// each edge to the halo from the tile's side, ordered by edge index, then
-// triangle (consecutive entries read consecutive geometry). halo slots as
-// tile_halos assigns them.
-static void tile_edges(int N, const int4 *hn, const std::vector<unsigned> &slot,
-                       std::vector<int> &estart, std::vector<int> &esplit,
-                       std::vector<unsigned> &edges)
-{
-    const int nt = (N + DE_BLOCK - 1) / DE_BLOCK;
-    estart.assign(nt + 1, 0);
-    esplit.assign(nt, 0);
-    edges.clear();
-    edges.reserve((size_t)N * 5 / 3 + 64);
-    for (int b = 0; b < nt; b++) {
-        estart[b] = (int)edges.size();
-        const int k0 = b * DE_BLOCK, k1 = std::min(N, k0 + DE_BLOCK);
-        // the edges inside the tile first, then the edges to the halo
-        for (int halo = 0; halo < 2; halo++) {
-            if (halo) esplit[b] = (int)edges.size();
-            for (int i = 0; i < 3; i++)
-                for (int k = k0; k < k1; k++) {
-                    const int v = i == 0 ? hn[k].x : (i == 1 ? hn[k].y : hn[k].z);
-                    if (v < 0) continue;
-                    const int n = v >> 2, j = v & 3;
-                    const unsigned s = (slot[k] >> (10 * i)) & 1023u;
-                    if (halo && s != 1023u)
-                        edges.push_back(DE_TE_MAKE(k - k0, i, 1, s, j));
-                    else if (!halo && s == 1023u && k < n)
-                        edges.push_back(DE_TE_MAKE(k - k0, i, 0, n - k0, j));
-                }
-        }
-    }
-    estart[nt] = (int)edges.size();
-}
-
 static int tile_halos(int N, const int4 *hn, std::vector<int> &start, std::vector<int> &halo,
                       std::vector<unsigned> &slot)
 {
@@ -3696,25 +3661,6 @@ int anuga_tile_order(int64_t N, const double *centroids, const int64_t *neighbou
             if (neighbours[i] >= N) return ANUGA_E_ARG;
     const std::vector<int> o = tile_order((int)N, centroids, neighbours);
     for (int64_t k = 0; k < N; k++) order[k] = o[k];
-    return ANUGA_OK;
-}
-
-int anuga_tile_edges(int64_t N, const int32_t *nb, int64_t *estart, int64_t *esplit,
-                     int64_t edge_cap, uint32_t *edges, int64_t *nedges)
-{
-    if (N < 0 || N >= (int64_t(1) << 29) || (N > 0 && !nb) || !estart || !esplit || !nedges)
-        return ANUGA_E_ARG;
-    std::vector<int4> hn(N);
-    for (int64_t k = 0; k < N; k++) hn[k] = make_int4(nb[3 * k], nb[3 * k + 1], nb[3 * k + 2], 0);
-    std::vector<int> st, h, est, esp;
-    std::vector<unsigned> sl, e;
-    if (tile_halos((int)N, hn.data(), st, h, sl) < 0) return ANUGA_E_ARG;
-    tile_edges((int)N, hn.data(), sl, est, esp, e);
-    *nedges = (int64_t)e.size();
-    if ((int64_t)e.size() > edge_cap || (!edges && !e.empty())) return ANUGA_E_ARG;
-    for (size_t b = 0; b < est.size(); b++) estart[b] = est[b];
-    for (size_t b = 0; b < esp.size(); b++) esplit[b] = esp[b];
-    for (size_t q = 0; q < e.size(); q++) edges[q] = e[q];
     return ANUGA_OK;
 }
 

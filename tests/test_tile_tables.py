@@ -1,6 +1,7 @@
 """The once-per-edge fused kernel's tables (CPU): every cell, node, halo edge
-and listed edge that a workgroup reads, replayed against the mesh, and its LDS
-extents against the launch's. Calls only host-side entry points."""
+and listed edge that a workgroup reads, replayed against the mesh, and the
+kernel's phases (anuga_core_amd/csrc/de_kernels.hip, de_xflux_e) over the LDS
+they share. Calls only host-side entry points."""
 
 import ctypes as C
 import os
@@ -173,6 +174,8 @@ def _limits(nb, vertices, b):
 def test_only_crowded_tiles_go_without_tables(tiles):
     """A few tiles whose triangles are scattered over the mesh: these alone
     are marked; every other tile's tables are whole."""
+    if BLOCK != 256:
+        pytest.skip("sized for 256-triangle tiles")
     nb, vertices = _ordered(Mesh(*rectangular_cross(53, 41, 53.0, 41.0)))
     N = len(nb)
     among = np.concatenate([np.arange(b * BLOCK, (b + 1) * BLOCK) for b in tiles + (30,)])
@@ -239,3 +242,181 @@ def test_tables_refuse_a_bad_description(field, value):
     a = _tables(nb, vertices, refused=-1, **{field: value})
     if field == "capacity":
         assert not any(np.any(v) for v in a.values())
+
+
+class Lds:
+    """The LDS of a workgroup, holding tokens. Between two barriers no address
+    that one thread writes may be read or written by another."""
+
+    def __init__(self, size):
+        self.size, self.at = size, {}
+        self.barrier()
+
+    def barrier(self):
+        self.writer, self.readers = {}, {}
+
+    def put(self, thread, a, token):
+        assert 0 <= a < self.size
+        assert self.writer.setdefault(a, thread) == thread, "two writers of %d" % a
+        assert self.readers.get(a, {thread}) == {thread}, "%d is written as it is read" % a
+        self.at[a] = token
+
+    def get(self, thread, a):
+        assert 0 <= a < self.size
+        assert self.writer.get(a, thread) == thread, "%d is read as it is written" % a
+        self.readers.setdefault(a, set()).add(thread)
+        return self.at[a]
+
+
+def _phases(nb, a):
+    """Every phase of de_xflux_e with tokens in place of values: what each
+    thread reads is what the phase needs, from the slots that the tables name.
+    Returns the number of edges evaluated."""
+    N, nt = len(nb), (len(nb) + BLOCK - 1) // BLOCK
+    hecap = max((int(np.diff(a["hstart"]).max()) + 15) // 16 * 16, 16)
+    Q, XS, HL, HZ = 3 * BLOCK, 2 * BLOCK, 12 * BLOCK, 12 * BLOCK + 4 * hecap
+    a = {k: v.astype(np.int64).tolist() for k, v in a.items() if k not in ("node", "sizes")}
+    nb = nb.astype(np.int64).tolist()
+    field = lambda w, i: (w >> (10 * i)) & 1023  # noqa: E731
+    evaluated = 0
+    for b in range(nt):
+        if "crowded" in a and a["crowded"][b]:
+            continue
+        k0, kn = b * BLOCK, min(N - b * BLOCK, BLOCK)
+        cells = a["cell"][a["cstart"][b]:a["cstart"][b + 1]]
+        h0, nhe = a["hstart"][b], a["hstart"][b + 1] - a["hstart"][b]
+        e0, es, e1 = a["estart"][b], a["esplit"][b], a["estart"][b + 1]
+        hw = (nhe + 63) // 64
+        halo = [(cells[(w & 1023) - BLOCK], w >> 10) for w in a["hcell"][h0:h0 + nhe]]
+        lds = Lds(HZ + 2 * BLOCK)
+        # 0: the cells; the tile's beds
+        for t in range(BLOCK):
+            k = k0 + t if t < kn else None
+            for q in range(6):
+                lds.put(t, q * XS + t, ("cell", k, q))
+                if t < len(cells):
+                    lds.put(t, q * XS + BLOCK + t, ("cell", cells[t], q))
+            lds.put(t, HZ + BLOCK + t, ("bed", k))
+        lds.barrier()
+
+        # 1: the stencils of the tile's triangles and of the halo edges'
+        def read(t, self, tri, st):
+            for place, want in [(self, tri)] + [
+                    (self if field(st, i) == 1023 else field(st, i),
+                     tri if v < 0 else v >> 2) for i, v in enumerate(nb[tri])]:
+                for q in range(6):
+                    assert lds.get(t, q * XS + place) == ("cell", want, q)
+
+        for t in range(kn):
+            read(t, t, k0 + t, a["stencil"][k0 + t])
+            lds.put(t, HZ + t, ("depth", k0 + t))
+        for t, (tri, _) in enumerate(halo):
+            read(t, a["hcell"][h0 + t] & 1023, tri, a["hstencil"][h0 + t])
+        lds.barrier()
+        # the edge values take the cells' place
+        for t in range(kn):
+            for i in range(3):
+                for r in range(4):
+                    lds.put(t, (3 * r + i) * BLOCK + t, ("value", k0 + t, i, r))
+        lds.barrier()
+
+        def edge(thread, e):
+            en, he = a["edge"][e], e - es
+            t, i, n, j = en & 1023, (en >> 10) & 3, (en >> 13) & 1023, (en >> 23) & 3
+            A = i * BLOCK + t
+            R, rs = (HL + he, hecap) if he >= 0 else (j * BLOCK + n, Q)
+            side = (k0 + t, i)
+            other = halo[he] if he >= 0 else (k0 + n, j)
+            assert nb[side[0]][i] == (other[0] << 2) | other[1]
+            for r in range(4):
+                assert lds.get(thread, A + r * Q) == ("value",) + side + (r,)
+                assert lds.get(thread, R + r * rs) == ("value",) + other + (r,)
+            for m in (t, n) if he < 0 else (t,):
+                assert lds.get(thread, HZ + m) == ("depth", k0 + m)
+                assert lds.get(thread, HZ + BLOCK + m) == ("bed", k0 + m)
+            for r, name in enumerate(("a0", "a1", "a2", "b1")):
+                lds.put(thread, A + r * Q, (name,) + side)
+            lds.put(thread, R, ("b2",) + side)
+            if he < 0:
+                lds.put(thread, R + rs, ("c1",) + side)
+                lds.put(thread, R + 2 * rs, ("c2",) + side)
+
+        # 2: the halo's edge values; edges inside the tile on the other waves
+        done = []
+        for t, (tri, j) in enumerate(halo):
+            for r in range(4):
+                lds.put(t, HL + r * hecap + t, ("value", tri, j, r))
+        for t in range(64 * hw, BLOCK):
+            e = e0 + t - 64 * hw
+            if e < es:
+                edge(t, e)
+                done.append(e)
+        lds.barrier()
+        # 3: the edges that are left
+        for t in range(BLOCK):
+            for e in range(min(es, e0 + BLOCK - 64 * hw) + t, e1, BLOCK):
+                edge(t, e)
+                done.append(e)
+        assert sorted(done) == list(range(e0, e1))
+        evaluated += len(done)
+        lds.barrier()
+        # 4: every triangle's three edges, by the roles that the words give
+        for t in range(kn):
+            k = k0 + t
+            ac = a["across"][k]
+            for i in range(3):
+                A, f, v = i * BLOCK + t, field(a["stencil"][k], i), nb[k][i]
+                if f == 1023:
+                    assert v < 0
+                    got = [lds.get(t, A + r * Q) for r in range(4)]
+                    want = [("value", k, i, r) for r in range(4)]
+                elif f > t:
+                    far = HL + ((ac >> (6 + 8 * i)) & 255) if f >= BLOCK else \
+                        ((ac >> (2 * i)) & 3) * BLOCK + f
+                    got = [lds.get(t, A + r * Q) for r in range(4)] + [lds.get(t, far)]
+                    want = [(x, k, i) for x in ("a0", "a1", "a2", "b1", "b2")]
+                else:
+                    far = ((ac >> (2 * i)) & 3) * BLOCK + f
+                    got = [lds.get(t, far + r * Q) for r in range(3)] + \
+                        [lds.get(t, A + Q), lds.get(t, A + 2 * Q)]
+                    want = [(x, v >> 2, v & 3) for x in ("a0", "a1", "a2")] + \
+                        [(x, v >> 2, v & 3) for x in ("c1", "c2")]
+                assert got == want, (k, i, got, want)
+    return evaluated
+
+
+@pytest.mark.parametrize("make,per_triangle", [
+    (lambda: rectangular_cross(40, 40, 1000.0, 700.0), (1.4, 1.8)),
+    (lambda: rectangular_cross(37, 53, 1000.0, 700.0), None),
+    (lambda: rectangular_cross(1, 1), None), (lambda: rectangular_cross(8, 8), None),
+    (lambda: rectangular(128, 1), None),
+    (lambda: graded_square(600.0, 40.0, 300.0, (150.0, 150.0, 450.0, 450.0), seed=1), None)])
+def test_lds_of_every_phase(make, per_triangle):
+    nb, _ = _ordered(Mesh(*make()))
+    n = _phases(nb, _tables(nb))
+    if per_triangle:   # about 1.6 evaluated edges per triangle instead of 3
+        assert per_triangle[0] < n / len(nb) < per_triangle[1]
+
+
+def test_lds_of_tiles_at_the_limits():
+    """Tiles with scattered triangles, up to nearly as many cells as the tables
+    take, beside crowded ones that are left out."""
+    if BLOCK != 256:
+        pytest.skip("sized for 256-triangle tiles")
+    nb, _ = _ordered(Mesh(*rectangular_cross(53, 41, 53.0, 41.0)))
+    N = len(nb)
+    rng = np.random.default_rng(3)
+    order = np.arange(N)
+    for b in range(0, 30, 2):   # exchange more and more triangles of two tiles
+        m = 12 + b
+        i, j = (rng.choice(np.arange(t * BLOCK, (t + 1) * BLOCK), m, replace=False)
+                for t in (b, b + 1))
+        order[i], order[j] = order[j], order[i].copy()
+    place = np.empty(N, np.int64)
+    place[order] = np.arange(N)
+    n = nb[order].astype(np.int64)
+    nb = np.where(n >= 0, (place[np.maximum(n, 0) >> 2] << 2) | (n & 3), -1)
+    a = _tables(nb, crowded=True)
+    assert a["crowded"].any() and np.diff(a["cstart"]).max() > 0.9 * CELLS
+    _replay(nb, a, None)
+    _phases(nb, a)
