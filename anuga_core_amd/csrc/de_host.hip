@@ -74,6 +74,13 @@ const int kHostHist = 512;
 // 40.3. Capturing 8 steps takes 45 to 100 us once.
 const int kGraphSteps = 8, kGraphMin = 64;   // an even count: see self_contained
 
+// Quantities of up to so many triangles cross between the device and pinned
+// memory of the handle inside the kernel that reorders them; larger ones are
+// copied, from and to the caller's memory. Reading and setting the stage, us:
+// 12.9 and 13.4 in the kernel, 27.3 and 19.4 copied at 1600 triangles, 41.9
+// and 41.7, 50.3 and 42.7 at 90k, 164 and 139, 171 and 111 at 360k.
+const int kPinnedField = 1 << 16;
+
 // Tiles within the once-per-edge kernel's limits from which a second launch
 // for the crowded ones pays (tables_pay). The launch takes 10 us a substep
 // however few they are; a tile that runs the gather kernel for its sake costs
@@ -205,13 +212,16 @@ struct anuga_domain {
     DeControl *kctl = nullptr, *kdt = nullptr;
     unsigned long long *dneg = nullptr; // fix_negative count, behind ctl
     // one pinned allocation: the mirror of ctl and of the counter behind it,
-    // then hsetup, hhist and the staging of the boundary values' three slots
+    // then hsetup, hhist, the staging of the boundary values' three slots and
+    // that of a quantity
     DeControl *hctl = nullptr;          // [S] host mirror of ctl
     unsigned long long *hneg = nullptr; // host mirror of *dneg
     DeBatchSetup *dsetup = nullptr;     // [S] time control of a step run
     DeBatchSetup *hsetup = nullptr;     // [S] staging of dsetup
     double *hhist = nullptr;            // [kHostHist] the history of a run of steps
     double *hbval = nullptr;            // [3][3][M] boundary values on their way to bval
+    double *hfield = nullptr;           // [hfield_cap] one quantity in the caller's order
+    int hfield_cap = 0;
     bool bval_sent[3] = {false, false, false};   // slot not known to have arrived
     double *hist = nullptr;             // device timestep history of a step run (S == 1)
     int64_t hist_cap = 0;
@@ -1184,13 +1194,16 @@ static int domain_alloc(const anuga_params *params, int64_t S64, const int64_t *
     static_assert(sizeof(DeControl) % 8 == 0 && sizeof(DeBatchSetup) % 8 == 0, "pinned layout");
     const size_t hctl_bytes = S * sizeof(DeControl) + sizeof(unsigned long long);
     const size_t hsetup_bytes = S * sizeof(DeBatchSetup);
+    d->hfield_cap = std::min(*std::max_element(d->ntri.begin(), d->ntri.end()), kPinnedField);
     DCHK(hipHostMalloc((void **)&d->hctl,
-                       hctl_bytes + hsetup_bytes + (kHostHist + 9 * (size_t)M) * sizeof(double),
+                       hctl_bytes + hsetup_bytes +
+                           (kHostHist + 9 * (size_t)M + d->hfield_cap) * sizeof(double),
                        hipHostMallocDefault));
     d->hneg = reinterpret_cast<unsigned long long *>(d->hctl + S);
     d->hsetup = reinterpret_cast<DeBatchSetup *>(d->hneg + 1);
     d->hhist = reinterpret_cast<double *>(d->hsetup + S);
     d->hbval = d->hhist + kHostHist;
+    d->hfield = d->hbval + 9 * (size_t)M;
     if (S > 1) {
         DCHK(dalloc(&d->scen, d->nblocks));
         std::vector<int> bs(d->nblocks, 0);
@@ -2064,8 +2077,9 @@ static int scenario_ok(anuga_domain *d, int64_t s)
     return ANUGA_OK;
 }
 
-// One quantity of scenario s crosses as 8 B per triangle through the device
-// staging buffer `field` in the caller's order; a kernel reorders it.
+// One quantity of scenario s crosses as 8 B per triangle through a staging
+// buffer in the caller's order (field on the device, or hfield in pinned
+// memory: kPinnedField); a kernel reorders it.
 static int set_centroids(anuga_domain *d, int s, int quantity, const double *values)
 {
     if (!values) return fail(d, ANUGA_E_ARG, "values is NULL");
@@ -2082,10 +2096,12 @@ static int set_centroids(anuga_domain *d, int s, int quantity, const double *val
         v = reinterpret_cast<double *>((d->substate ? d->B : d->A) + kb) + slot;
         if (slot == 3) v2 = reinterpret_cast<double *>((d->substate ? d->A : d->B) + kb) + slot;
     }
-    HIPCHK(d, hipMemcpyAsync(d->field, values, N * sizeof(double), hipMemcpyHostToDevice,
-                             d->stream));
+    const bool pinned = N <= d->hfield_cap;
+    if (pinned) std::memcpy(d->hfield, values, N * sizeof(double));
+    else HIPCHK(d, hipMemcpyAsync(d->field, values, N * sizeof(double), hipMemcpyHostToDevice,
+                                  d->stream));
     hipLaunchKernelGGL(de_set_field, dim3((N + DE_BLOCK - 1) / DE_BLOCK), dim3(DE_BLOCK), 0,
-                       d->stream, N, d->caller + kb, d->field, stride, v, v2);
+                       d->stream, N, d->caller + kb, pinned ? d->hfield : d->field, stride, v, v2);
     if (slot == 3 && d->mixed)
         // bed offsets of the mixed flux's local datum
         hipLaunchKernelGGL(de_bed_offsets, dim3((N + DE_BLOCK - 1) / DE_BLOCK), dim3(DE_BLOCK), 0,
@@ -2102,13 +2118,16 @@ static int download_field(anuga_domain *d, int kb, int n, const double *v, int s
                           double *values, bool height = false)
 {
     auto kern = height ? de_get_field<true> : de_get_field<false>;
+    const bool pinned = n <= d->hfield_cap;
     hipLaunchKernelGGL(kern, dim3((n + DE_BLOCK - 1) / DE_BLOCK), dim3(DE_BLOCK), 0, d->stream, n,
-                       d->caller + kb, v, stride, d->field);
+                       d->caller + kb, v, stride, pinned ? d->hfield : d->field);
     int rc = launch_check(d);
     if (rc) return rc;
-    HIPCHK(d, hipMemcpyAsync(values, d->field, n * sizeof(double), hipMemcpyDeviceToHost,
-                             d->stream));
+    if (!pinned)
+        HIPCHK(d, hipMemcpyAsync(values, d->field, n * sizeof(double), hipMemcpyDeviceToHost,
+                                 d->stream));
     HIPCHK(d, hipStreamSynchronize(d->stream));
+    if (pinned) std::memcpy(values, d->hfield, n * sizeof(double));
     return ANUGA_OK;
 }
 

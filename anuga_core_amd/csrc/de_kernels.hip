@@ -2876,7 +2876,8 @@ de_node_vertices(int n, DeTileX tx, double2 *__restrict__ vx)
 // to the host, in the order the host keeps them. Bound by the PCIe copy that
 // follows: of 4M triangles 28 us here and 1.8 ms for the whole access, which
 // took 30 ms when the host downloaded the 32 B records and reordered them
-// (setting a quantity: 45 -> 10.7 ms, most of it numpy's).
+// (setting a quantity: 45 -> 10.7 ms, most of it numpy's). Of small meshes out
+// is pinned host memory: 1600 triangles 27.3 -> 12.9 us without the copy.
 template <bool HEIGHT>
 __global__ void __launch_bounds__(DE_BLOCK)
 de_get_field(int n, const int *__restrict__ caller, const double *__restrict__ v, int stride,

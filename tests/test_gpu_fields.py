@@ -1,7 +1,8 @@
 """Centroid quantities between the caller's and the library's order on the
 device (de_set_field, de_get_field), against the values as they were given:
-copies, so bit for bit, at sizes around one workgroup and for every quantity,
-in a single scenario and in an ensemble whose scenarios start on workgroup
+copies, so bit for bit, at sizes around one workgroup and around the size up
+to which pinned memory takes the place of copies, and for every quantity, in a
+single scenario and in an ensemble whose scenarios start on workgroup
 boundaries."""
 
 import numpy as np
@@ -30,7 +31,7 @@ def _same(a, b):
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
-@pytest.mark.parametrize("cells", [1, 127, 128, 129, 300])
+@pytest.mark.parametrize("cells", [1, 127, 128, 129, 300, 32768, 32769])
 def test_domain_fields_round_trip(cells, precision):
     mesh = Mesh(*rectangular(cells, 1, float(cells), 1.0))
     d = Domain(mesh=mesh, precision=precision)
@@ -44,7 +45,7 @@ def test_domain_fields_round_trip(cells, precision):
 
 
 def test_ensemble_fields_round_trip():
-    meshes = [Mesh(*rectangular(c, 1, float(c), 1.0)) for c in (128, 1, 200, 127)]
+    meshes = [Mesh(*rectangular(c, 1, float(c), 1.0)) for c in (128, 1, 200, 32769, 127)]
     e = Ensemble(meshes)
     qs = [_values(m.number_of_triangles, 10 + s) for s, m in enumerate(meshes)]
     for s, m in enumerate(meshes):
