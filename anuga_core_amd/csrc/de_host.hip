@@ -1395,6 +1395,12 @@ static void tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1,
     auto word = [](const int f[3]) {
         return (unsigned)f[0] | ((unsigned)f[1] << 10) | ((unsigned)f[2] << 20);
     };
+    const size_t nt = b1 - b0, n = std::min(N, b1 * DE_BLOCK) - b0 * DE_BLOCK;
+    for (auto *v : {&x.stencil, &x.across, &x.nodes}) v->reserve(n);
+    for (auto *v : {&x.hstencil, &x.hcell, &x.hnodes}) v->reserve(64 * nt);
+    x.edge.reserve(n * 5 / 3 + 64 * nt);
+    x.cell.reserve(128 * nt);
+    if (vx) x.node.reserve(192 * nt);
     for (int b = b0; b < b1; b++) {
         const int k0 = b * DE_BLOCK, k1 = std::min(N, k0 + DE_BLOCK);
         const int cbase = (int)x.cell.size(), ebase = (int)x.edge.size();
@@ -1469,9 +1475,7 @@ static void tile_tables(int N, const int4 *hn, const double *vx, int b0, int b1,
             const double2 p = make_double2(vx[6 * (size_t)k + 2 * c], vx[6 * (size_t)k + 2 * c + 1]);
             uint64_t u[2];
             std::memcpy(u, &p, sizeof(u));
-            uint64_t h = (u[0] * 0x9e3779b97f4a7c15ull) ^ (u[1] * 0xc2b2ae3d27d4eb4full);
-            h ^= h >> 32;
-            for (;; h++) {
+            for (uint64_t h = de_hash_bits(u[0], u[1]) >> 32;; h++) {
                 int &s = nval[h & (NS - 1)];
                 if (s < 0) {
                     const int j = (int)x.node.size() - nbase;
@@ -1535,7 +1539,7 @@ static bool tables_pay(int nt, int nc)
 static void scenario_tables(int N, const int4 *hn, const double *vx, TileTables &x)
 {
     const int nt = (N + DE_BLOCK - 1) / DE_BLOCK;
-    const int T = std::max(1, std::min<int>({(int)std::thread::hardware_concurrency(), 16, nt / 16}));
+    const int T = std::max(1, std::min<int>({(int)std::thread::hardware_concurrency(), 16, nt / 8}));
     std::vector<TileTables> part(T);
     on_threads(T, [&](int i) {
         const int b0 = (int)((int64_t)nt * i / T), b1 = (int)((int64_t)nt * (i + 1) / T);

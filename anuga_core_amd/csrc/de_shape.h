@@ -2,6 +2,8 @@
 // kernels, the host and CPU tests.
 #pragma once
 
+#include <stdint.h>
+
 #if defined(__HIPCC__)
 #define DE_SHAPE_FN __host__ __device__ constexpr
 #else
@@ -15,6 +17,17 @@ DE_SHAPE_FN int de_hash_slots(int n)
     int s = 2;
     while (s < 2 * n) s *= 2;
     return s;
+}
+
+// Hash of two doubles' bits, to be used from bit 32 up. Round coordinates
+// differ in a few high bits only, and a product carries bits upwards: without
+// the shifts, those of a grid have the low bits of their products in common
+// and crowd into few slots.
+DE_SHAPE_FN uint64_t de_hash_bits(uint64_t a, uint64_t b)
+{
+    uint64_t h = (a ^ (a >> 32)) * 0x9e3779b97f4a7c15ull + (b ^ (b >> 29)) * 0xc2b2ae3d27d4eb4full;
+    h ^= h >> 32;
+    return h * 0x9e3779b97f4a7c15ull;
 }
 
 // A workgroup of `waves` waves forms `chunks` chunks in de_wave_passes passes:

@@ -5,6 +5,7 @@ import ctypes as C
 import os
 import subprocess
 
+import numpy as np
 import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
@@ -12,6 +13,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 SOURCE = r"""
 #include "de_shape.h"
 extern "C" int hash_slots(int n) { return de_hash_slots(n); }
+extern "C" uint64_t hash_bits(uint64_t a, uint64_t b) { return de_hash_bits(a, b); }
 extern "C" int edge_lds(int b, int h, int n) { return de_edge_lds(b, h, n); }
 extern "C" int edge_lds_static(int b) { return de_edge_lds_static(b); }
 extern "C" int tables_fit(int b, int h, int n) { return de_tables_fit(b, h, n); }
@@ -27,7 +29,9 @@ def lib(tmp_path_factory):
     src.write_text(SOURCE)
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I" + CSRC, "-o", str(so),
                     str(src)], check=True)
-    return C.CDLL(str(so))
+    lib = C.CDLL(str(so))
+    lib.hash_bits.restype = C.c_uint64
+    return lib
 
 
 def test_a_probe_reaches_a_free_slot(lib):
@@ -70,3 +74,15 @@ def test_tables_whose_lds_does_not_fit_are_left_out(lib, block):
     # values, depths and beds; nodes on 16 B and the triangles' node words
     assert lib.edge_lds(256, 64, 0) == 8 * (12 * 256 + 4 * 64 + 2 * 256)
     assert lib.edge_lds(256, 64, 180) == lib.edge_lds(256, 64, 0) + 16 * 180 + 4 * 256
+
+
+@pytest.mark.parametrize("x0,dx", [(0.0, 1.0), (0.0, 10.0), (0.0, 0.1), (-3.0, 2.0 ** -7),
+                                   (500000.0, 25.0), (0.0, 1.0 / 3.0)])
+def test_hashes_of_grid_points_spread(lib, x0, dx):
+    """384 points of a grid, round coordinates among them, over 1024 slots
+    occupy about as many as random ones (320 expected, 9 the deviation)."""
+    x = x0 + dx * np.arange(16.0)
+    y = 2.0 * x0 + dx * np.arange(24.0)
+    p = np.stack(np.meshgrid(x, y), axis=-1).reshape(-1, 2).view(np.uint64).tolist()
+    slots = {(lib.hash_bits(C.c_uint64(a), C.c_uint64(b)) >> 32) & 1023 for a, b in p}
+    assert len(slots) > 320 - 6 * 9
