@@ -2895,14 +2895,15 @@ int anuga_get_operator_influx(anuga_domain *d, int64_t id, double *cumulative)
 {
     if (!d || !cumulative) return ANUGA_E_ARG;
     if (id < 0 || id >= (int64_t)d->ops.size()) return fail(d, ANUGA_E_ARG, "no such operator");
-    HIPCHK(d, hipStreamSynchronize(d->stream));
     const RateOp &o = d->ops[id];
     // an inlet keeps its sum; a rate operator one part per workgroup
-    const size_t parts = o.kind == 0 ? std::max(1, (o.n + DE_BLOCK - 1) / DE_BLOCK) : 1;
-    std::vector<double> h(parts);
-    HIPCHK(d, hipMemcpy(h.data(), o.influx, parts * sizeof(double), hipMemcpyDeviceToHost));
-    *cumulative = 0.0;
-    for (double x : h) *cumulative += x;
+    const int parts = o.kind == 0 ? std::max(1, (o.n + DE_BLOCK - 1) / DE_BLOCK) : 1;
+    hipLaunchKernelGGL(de_sum_parts, dim3(1), dim3(DE_SUM_THREADS), 0, d->stream, parts, o.influx,
+                       d->hfield);
+    int rc = launch_check(d);
+    if (rc) return rc;
+    HIPCHK(d, hipStreamSynchronize(d->stream));
+    *cumulative = d->hfield[0];
     return ANUGA_OK;
 }
 

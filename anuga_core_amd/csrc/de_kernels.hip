@@ -2910,7 +2910,7 @@ de_set_field(int n, const int *__restrict__ caller, const double *__restrict__ i
 // >= 0 the stage rises by it; otherwise (`careful`) the loss is capped at the
 // depth and the momenta scale with the depth that remains. The inflow
 // (local rate * area) is accumulated per workgroup, in influx[blockIdx.x],
-// and summed on the host when it is asked for. Atomic adds to one address were
+// and summed when it is asked for (de_sum_parts). Atomic adds to one address were
 // the kernel's time (36k triangles: 11.5 us with one per triangle, 9.4 with one
 // per wave, 4.0 with none).
 // Set_stage_operator after a step (set_quantity.py:95-131, quantity
@@ -2924,6 +2924,27 @@ de_set_stage(const DeControl *ctl, int n, const int *__restrict__ idx,
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     S[idx[i]].w = value ? value[i] : value0;
+}
+
+// The sum of n parts by one workgroup, in a fixed order, to pinned host memory:
+// 8 B cross instead of the parts: 21.9 -> 15.0 us a read at 4M triangles, which
+// have 15,625, and 12 to 13 either way at 400.
+#define DE_SUM_THREADS 1024
+__global__ void __launch_bounds__(DE_SUM_THREADS)
+de_sum_parts(int n, const double *__restrict__ part, double *__restrict__ sum)
+{
+    __shared__ double red[DE_SUM_THREADS / 64];
+    double a[4] = {0.0, 0.0, 0.0, 0.0};   // four loads on their way at a time
+    for (int i = threadIdx.x; i < n; i += 4 * DE_SUM_THREADS)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (i + j * DE_SUM_THREADS < n) a[j] += part[i + j * DE_SUM_THREADS];
+    double s = de_wave_sum_nz((a[0] + a[1]) + (a[2] + a[3]));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x) return;
+    for (int j = 1; j < DE_SUM_THREADS / 64; j++) s += red[j];
+    *sum = s;
 }
 
 __global__ void __launch_bounds__(DE_BLOCK)

@@ -10,7 +10,9 @@ import math
 import numpy as np
 import pytest
 
+from anuga_core_amd.boundaries import Reflective_boundary
 from anuga_core_amd.domain import Domain
+from anuga_core_amd.mesh import Mesh, rectangular
 from anuga_core_amd.operators import Rate_operator
 from oracle.kernels import OracleKernels
 from oracle.oracle_domain import OracleDomain, OracleRateOperator
@@ -163,3 +165,21 @@ def test_constant_inlet_runs_on_the_device():
     added = op.get_cumulative_influx()
     assert added == pytest.approx(2.0 * d.get_time(), rel=1e-12)
     assert d.get_water_volume() - v0 == pytest.approx(added, rel=1e-9)
+
+
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 32768, 131072, 131073, 600000])
+def test_influx_of_many_workgroups(n):
+    """The inflow is kept as one part per workgroup and summed by one: of 2,
+    256, 258 triangles and, from 262144 on, above one part per thread, each part and the last one counted."""
+    print("case influx of many workgroups", n, flush=True)
+    mesh = Mesh(*rectangular(n, 1, float(n), 1.0))
+    N = mesh.number_of_triangles
+    d = Domain(mesh=mesh)
+    d.set_quantity("stage", 1.0, location="centroids")
+    d.set_boundary({t: Reflective_boundary(d) for t in d.get_boundary_tags()})
+    rate = 1.0e-3 * (1.0 + np.arange(N) % 7)
+    op = Rate_operator(d, rate=rate)
+    d.evolve_steps(3)
+    want = math.fsum(rate * mesh.areas) * d.get_time()
+    # three steps' roundings of a part and a tree of at most 40 more
+    assert abs(op.get_cumulative_influx() - want) <= 50 * 2.0 ** -53 * want
